@@ -17,7 +17,7 @@ stops at the final LayerNorm) with the token ids already resident in HBM.  Print
 line.  Beside the whole-forward numbers it carries
   * "roofline": the dominant kernel (the ffn1 GEMM, M=153600 N=3072 K=768, GELU epilogue) timed
     live with events around each of its calls inside the timed region (a call is one launch of
-    the persistent kernel plus, at this shape, one of the small-tile kernel for the last 768
+    the persistent kernel plus, at this shape, one of the tile kernel for the last 768
     rows); achieved = 2*M*N*K / mean duration against the 2.5 PFLOP/s dense fp16 MFMA peak;
   * "cpu_baseline": the plain PyTorch fp32 forward of the same architecture (the stand-in for the
     reference's CPU-side comparator, HF GPT2Model in fp32) on this box's host cores, at the
@@ -441,8 +441,8 @@ def main():
                    "tokens_per_step": tokens, "n_layer": arch["n_layer"], "n_embd": h,
                    "n_head": arch["n_head"]},
         # one ffn1 call = gemm_stream_kernel on the row tiles that fill whole rounds of the
-        # persistent workgroups + gemm_kernel<128,128> on the rows left over (none for some shapes)
-        "roofline": {"kernel": f"ffn1 GEMM, both launches of a call (gemm_stream_kernel + small-tile gemm_kernel for the last rows: M={tokens} N={4 * h} K={h}, bias+GELU epilogue)",
+        # persistent workgroups + gemm_tile_kernel on the rows left over (none for some shapes)
+        "roofline": {"kernel": f"ffn1 GEMM, both launches of a call (gemm_stream_kernel + gemm_tile_kernel for the last rows: M={tokens} N={4 * h} K={h}, bias+GELU epilogue)",
                      "bound": "mfma", "achieved": round(achieved, 1), "peak": PEAK_FP16 / 1e12,
                      "unit": "TFLOP/s", "frac": round(achieved * 1e12 / PEAK_FP16, 4),
                      "avg_ms": round(ffn1_ms, 4), "calls": len(ffn1_events),

@@ -1,0 +1,198 @@
+// What the GEMM translation units share: the epilogue description, the direct global->LDS loads
+// with their hand-counted waits, the tile order, and the CU count of the persistent launches.
+#pragma once
+#include <stdlib.h>
+
+#include "common.h"
+#include "launch.h"
+
+namespace gptmi {
+
+struct EpiDev {
+  const void* bias;
+  const void* residual;
+  void* out;
+  void* q;
+  void* k;
+  void* v;
+  int64_t L;
+  int heads;
+  int d;
+  int gelu;
+  int vec_ok;  // pointers and N allow 4-element vector accesses
+  int tile_vec; // gemm_tile_kernel: N, head size and every pointer allow 16-byte accesses
+  int vec8_ok; // fp16 output: N, head size and the output pointers also allow 16-byte stores
+  int m_off;   // head-major scatter: row 0 of this launch is row m_off of the [B*L] token rows
+  DropoutArgs drop;  // p > 0: dropout between GELU and residual (gemm_tile_kernel only)
+};
+
+// LayerNorm in the operand prologue (gemm_tile_kernel<..., LNA = true>): weight, bias, epsilon and
+// the lanes per row the LayerNorm kernel would use for rows of this width (the sums are then
+// formed in the same order and the normalised operand has the same bits as that kernel's output).
+struct LnArgs {
+  const void* w;
+  const void* b;
+  float eps;
+  int lpr;
+};
+
+// Direct global->LDS load of 16 bytes per lane: lane l's bytes land at LDS
+// byte offset lds_off + 16*l (lds_off is wavefront-uniform and travels in M0).
+// Issued as inline assembly so that the compiler's wait-count tracking does not
+// see an LDS-writing memory instruction in flight: with the builtin, every LDS
+// wait inside the pipelined loop degrades to "wait for everything".  Completion
+// is tracked by hand with vmcnt (wait_vmcnt) ahead of the workgroup barrier.
+__device__ __forceinline__ void lds_dma16(const void* gsrc, unsigned lds_off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(lds_off), "v"(gsrc)
+               : "memory", "m0");
+}
+
+// The same with a wavefront-uniform 64-bit base in scalar registers and a 32-bit per-lane
+// byte offset: one VGPR per load instead of an address pair, and the k-step is a scalar add.
+__device__ __forceinline__ void lds_dma16_base(const void* base, unsigned lane_off,
+                                               unsigned lds_off) {
+  // s_mov + s_nop 3 = 5 wait states between a VALU write of `base` (v_readfirstlane, should
+  // the compiler ever have to move it out of a vector register) and the load that reads it
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_off), "v"(lane_off), "s"(base)
+               : "memory", "m0");
+}
+
+// Streaming store of 4 or 8 output elements at (wavefront-uniform 64-bit base) + (32-bit lane
+// offset).  Written as assembly because the compiler otherwise materialises one 64-bit address
+// pair per store of an unrolled epilogue and spills.  Two hazards the compiler handles for its
+// own instructions and cannot see inside assembly:
+//   * a scalar register written by a VALU instruction (v_readfirstlane) must not be read by a
+//     memory instruction within the next 5 wait states -- the leading s_nop 4 covers a base
+//     that the compiler had to move out of a vector register;
+//   * a store of more than 64 bits reads its data registers a little after issue -- the
+//     trailing s_nop 1 keeps the next VALU instruction from overwriting them.
+__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, h4 v) {
+  asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2 nt"
+               :
+               : "v"(lane_off), "v"(v), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, f4 v) {
+  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
+               :
+               : "v"(lane_off), "v"(v), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, h8 v) {
+  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
+               :
+               : "v"(lane_off), "v"(v), "s"(base)
+               : "memory");
+}
+
+// Workgroup barrier that does not drain the vector-memory counter: the
+// compiler's own barrier waits for vmcnt(0), which would serialise the
+// global->LDS prefetch of the younger pipeline stages behind it.
+__device__ __forceinline__ void block_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N <= 63, "vmcnt is a 6-bit counter");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <typename T> struct Pack4;
+template <> struct Pack4<_Float16> { typedef h4 type; };
+template <> struct Pack4<float> { typedef f4 type; };
+
+// Address of out[m][n] (plain) or of the q/k/v element that column n of row m
+// scatters to (qkv mode; n is a multiple of 4 and head sizes are too, so 4
+// consecutive columns stay inside one head).
+template <typename T, bool QKV>
+__device__ __forceinline__ T* out_ptr(const EpiDev& ep, int64_t m, int n, int N) {
+  if constexpr (!QKV) {
+    return (T*)ep.out + (m * (int64_t)N + n);
+  } else {
+    // m < 2^31 (checked by the launcher) and L <= m's range: 32-bit divisions
+    const unsigned hd = (unsigned)(ep.heads * ep.d);
+    const unsigned which = (unsigned)n / hd;
+    const unsigned within = (unsigned)n - which * hd;
+    const unsigned head = within / (unsigned)ep.d;
+    const unsigned dd = within - head * (unsigned)ep.d;
+    const unsigned L = (unsigned)ep.L;
+    const unsigned b = (unsigned)m / L;
+    const unsigned l = (unsigned)m - b * L;
+    T* base = (T*)(which == 0 ? ep.q : (which == 1 ? ep.k : ep.v));
+    return base + ((((int64_t)b * ep.heads + head) * ep.L + l) * ep.d + dd);
+  }
+}
+
+// Head-major destination of column n, row 0 of batch 0: q/k/v base + (head * L + 0) * d + dd.
+template <typename T>
+__device__ __forceinline__ T* qkv_column_base(const EpiDev& ep, int n) {
+  const unsigned hd = (unsigned)(ep.heads * ep.d);
+  const unsigned which = (unsigned)n / hd;
+  const unsigned within = (unsigned)n - which * hd;
+  const unsigned head = within / (unsigned)ep.d;
+  const unsigned dd = within - head * (unsigned)ep.d;
+  T* base = (T*)(which == 0 ? ep.q : (which == 1 ? ep.k : ep.v));
+  return base + ((int64_t)head * ep.L * ep.d + dd);
+}
+
+// XCD-aware tile id: workgroup ids are dealt round-robin over the 8 XCDs, so id
+// p runs on XCD p % 8.  The remap hands every XCD a contiguous range of tiles.
+__device__ __forceinline__ int xcd_tile(int pid, int num_tiles) {
+  const int per = (num_tiles + 7) >> 3;
+  int tall = num_tiles & 7;
+  if (tall == 0) tall = 8;
+  const int xcd = pid & 7, loc = pid >> 3;
+  return xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
+}
+
+// Width, in column tiles, of the groups the tile order walks through.  The weight panels of
+// one group (group_w * BN rows of Kp halves) should stay in a 4 MB L2 beside the activation
+// panels in flight, so they get about 2.4 MB; every group re-reads the activations once, so
+// the groups are as few and as even as that allows.  Panels too long for two of them to fit
+// (large K) keep the plain column-fastest order.
+inline int column_group(int tiles_n, int bn, int Kp) {
+  const int64_t panel = (int64_t)bn * Kp * 2;
+  const int fit = (int)((2400 << 10) / panel);
+  if (fit < 2 || tiles_n <= fit) return tiles_n;
+  const int groups = (tiles_n + fit - 1) / fit;
+  return (tiles_n + groups - 1) / groups;
+}
+
+// CUs of the current device rounded down to a multiple of 8 (workgroup id % 8 = XCD for every
+// tile of a persistent launch), or a negative error code.  The environment variable
+// GPTMI_MAX_WORKGROUPS (read once) caps the number: a measurement knob -- with fewer persistent
+// workgroups than CUs the chip's power management holds a higher clock, which is how one tells a
+// kernel that is bound by the power budget from one that is bound by its own schedule.
+inline int cu_count() {
+  static int num_cus = 0;  // idempotent one-time setup; a race only repeats it
+  if (num_cus == 0) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus < 8) {
+      set_error("gemm: cannot query the CU count");
+      return -4;
+    }
+    if (const char* cap = getenv("GPTMI_MAX_WORKGROUPS")) {
+      const int c = atoi(cap);
+      if (c >= 8 && c < cus) cus = c;
+    }
+    num_cus = cus - cus % 8;
+  }
+  return num_cus;
+}
+
+// One workgroup per output tile (gemm_tile.hip), every size, type and epilogue; the LayerNorm
+// prologue form of it; and what the cost model says a launch takes, in microseconds.
+int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                     bool f16, bool qkv, hipStream_t st);
+int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
+                               const LnArgs& ln, bool qkv, hipStream_t st);
+float gemm_tile_cost(int64_t M, int N, int Kp, int cus);
+
+}  // namespace gptmi

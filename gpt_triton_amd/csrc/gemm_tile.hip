@@ -1,0 +1,584 @@
+// GEMM on one workgroup per output tile, for problems that do not fill the persistent 256 x 256
+// kernels of gemm.hip: a few rows up to a few thousand.
+//
+//   C[M][N] = A[M][Kp] . Bt[N][Kp]^T,  out = dropout(gelu?(C + bias)) + residual
+//
+// (reference: fused_ffn_kernel, kernels.py:169-257, and the q/k/v relayout of
+// matmul_and_split_qkv, kernels.py:347-367.)  With A = LayerNorm(x) where asked for (LNA).
+//
+// What bounds it.  At these sizes a workgroup's own path through its k-tiles does: a barrier, an
+// LDS round trip and a memory round trip per k-tile that no other workgroup of the CU hides.  So
+//   * WK groups of wavefronts split K inside the workgroup: group g multiplies the 64-wide
+//     k-slices g, g + WK, ..., so a "k-step" of the workgroup is WK slices wide and the number of
+//     barriers and round trips falls by WK.  The groups' partial sums meet in LDS at the end and are
+//     added in group order (deterministic, and the same whichever tile a row falls into);
+//   * the fragments of the whole next k-step are read from LDS (into a second register set) while the
+//     current one is multiplied, one read behind every MFMA or two, so an LDS round trip has the time
+//     of a k-step, not of one slice;
+//   * NST k-steps are in LDS or on their way; a stage is refilled as soon as its fragments are in
+//     registers.
+//   * The epilogue goes through a row-major fp32 tile in LDS: every thread owns 16 bytes of the
+//     output at a time (8 halves or 4 floats), so loads and stores are whole lines whatever the
+//     tile's shape, a ragged last row costs one comparison, and residual, GELU, dropout and the
+//     head-major scatter are the same few lines for every configuration.
+#include <type_traits>
+
+#include "gemm_common.h"
+#include "layernorm.h"
+
+namespace gptmi {
+
+namespace {
+
+// LayerNorm of the BM rows from m0 on into the LDS panel, as fp16 operands: element k of row r
+// goes to k-slice k / 64, row r's 128 bytes there, 16-byte unit (k % 64) / 8 ^ key(r).  A row is
+// spread over LPR lanes as in layernorm_vec_kernel (same sums, same bits); rows past the end
+// repeat the last row.
+template <int BM, int NT, typename T, int LPR, int CH>
+__device__ __forceinline__ void normalise_rows(const T* __restrict__ x, int M, int H, int m0,
+                                               const LnArgs& ln, char* panel, int tid) {
+  constexpr int VN = 16 / sizeof(T);
+  typedef T V __attribute__((ext_vector_type(VN)));
+  typedef _Float16 HV __attribute__((ext_vector_type(VN)));
+  constexpr int RPP = NT / LPR;  // rows per pass
+  constexpr int PASSES = BM / RPP;
+  static_assert(PASSES >= 1 && BM % RPP == 0, "row passes");
+  const int nchunks = H / VN, ll = tid & (LPR - 1), rsub = tid / LPR;
+  const V* wv = reinterpret_cast<const V*>(ln.w);
+  const V* bv = reinterpret_cast<const V*>(ln.b);
+  // the rows of G passes are requested together: one memory round trip for them (long rows: two
+  // passes at a time, and the parameters per row from L1, or the registers do not hold them)
+  constexpr bool LONG = CH > 4;
+  constexpr int G = LONG && PASSES > 2 ? 2 : PASSES;
+  static_assert(PASSES % G == 0, "pass groups");
+  V tw[CH], tb[CH];
+  auto params = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int c = ll + i * LPR;
+      if (c < nchunks) {
+        tw[i] = wv[c];
+        tb[i] = bv[c];
+      }
+    }
+  };
+  if constexpr (!LONG) params();
+#pragma unroll(LONG ? 1 : 2)
+  for (int p0 = 0; p0 < PASSES; p0 += G) {
+    V t[G][CH];
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      int row = m0 + (p0 + p) * RPP + rsub;
+      row = row < M ? row : M - 1;
+      const V* xr = reinterpret_cast<const V*>(x + (size_t)row * H);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int c = ll + i * LPR;
+        if (c < nchunks) t[p][i] = xr[c];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      const int r = (p0 + p) * RPP + rsub;
+      float v[CH][VN], sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const bool in = ll + i * LPR < nchunks;
+#pragma unroll
+        for (int j = 0; j < VN; ++j) {
+          v[i][j] = in ? (float)t[p][i][j] : 0.f;
+          if (in) sum += v[i][j];
+        }
+      }
+      float mean, rstd;
+      layernorm_stats<CH, VN, LPR>(v, sum, ll, nchunks, H, ln.eps, mean, rstd);
+      if constexpr (LONG) params();
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int c = ll + i * LPR;
+        if (c < nchunks) {
+          HV o;
+#pragma unroll
+          for (int j = 0; j < VN; ++j)
+            o[j] = (_Float16)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+          const int k = c * VN, unit = (k & 63) >> 3;
+          *reinterpret_cast<HV*>(panel + (k >> 6) * (BM * 128) + r * 128 +
+                                 ((unit ^ ((r >> 1) & 7)) << 4) + (k & 7) * 2) = o;
+        }
+      }
+    }
+  }
+}
+
+template <int BM, int NT, typename T>
+__device__ __forceinline__ void normalise_panel(const T* x, int M, int H, int m0, const LnArgs& ln,
+                                                char* panel, int tid) {
+  const int need = (H / (16 / (int)sizeof(T)) + ln.lpr - 1) / ln.lpr;  // chunks per lane
+#define GPTMI_LN_ROWS(L)                                                       \
+  do {                                                                         \
+    if (need <= 1) normalise_rows<BM, NT, T, L, 1>(x, M, H, m0, ln, panel, tid);      \
+    else if (need <= 2) normalise_rows<BM, NT, T, L, 2>(x, M, H, m0, ln, panel, tid); \
+    else if (need <= 3) normalise_rows<BM, NT, T, L, 3>(x, M, H, m0, ln, panel, tid); \
+    else if (need <= 4) normalise_rows<BM, NT, T, L, 4>(x, M, H, m0, ln, panel, tid); \
+    else normalise_rows<BM, NT, T, L, 8>(x, M, H, m0, ln, panel, tid);                \
+  } while (0)
+  if (ln.lpr == 32) GPTMI_LN_ROWS(32);
+  else GPTMI_LN_ROWS(64);
+#undef GPTMI_LN_ROWS
+}
+
+// One shape of workgroup: BM x BN output tile on WM x WN wavefronts times WK groups that split K,
+// NST k-steps of LDS stages.
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int NST_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, NST = NST_;
+  static constexpr int THREADS = 64 * WM_ * WN_ * WK_;
+};
+
+// T: storage type of bias, residual and output (and of x with LNA).
+// WIDE: rows of 2^22 elements and more (64-bit lane addresses).
+template <class C, typename T, bool QKV, bool LNA, bool DROP, bool WIDE>
+__global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
+    const void* __restrict__ Av, const _Float16* __restrict__ Bt, int M, int N, int Kp,
+    int tiles_m, int tiles_n, int group_w, EpiDev ep, LnArgs ln) {
+  constexpr int BM = C::BM, BN = C::BN, WM = C::WM, WN = C::WN, WK = C::WK, NST = C::NST;
+  constexpr int TG = 64 * WM * WN, NT = TG * WK;  // threads per k-group, per workgroup
+  constexpr int TM = BM / WM, TN = BN / WN, MB = TM / 16, NB = TN / 16;
+  constexpr int A_IT = LNA ? 0 : BM * 8 / TG, B_IT = BN * 8 / TG, LPT = A_IT + B_IT;
+  constexpr int A_N = A_IT ? A_IT : 1;
+  constexpr int B_AT = LNA ? 0 : BM * 128;     // byte offset of the weight rows inside a slice
+  constexpr int SLICE = B_AT + BN * 128;       // one group's 64-wide k-slice
+  constexpr int STAGE = SLICE * WK;
+  static_assert((LNA || (BM * 8) % TG == 0) && (BN * 8) % TG == 0, "tile/threads mismatch");
+  static_assert(TM % 16 == 0 && TN % 16 == 0, "16 x 16 MFMA blocks");
+  static_assert(NST >= 2 && (NST - 2) * LPT <= 63, "vmcnt range");
+
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = wave / (WM * WN), w = wave % (WM * WN);
+  const int wm = w % WM, wn = w / WM;
+  const int tg = tid % TG;
+
+  const int tile = xcd_tile(blockIdx.x, tiles_m * tiles_n);
+  const int grp = tile / (tiles_m * group_w);
+  const int in_grp = tile - grp * tiles_m * group_w;
+  const int grp_w = min(group_w, tiles_n - grp * group_w);
+  const int m0 = (in_grp / grp_w) * BM, n0 = (grp * group_w + in_grp % grp_w) * BN;
+
+  // ---- direct global->LDS loads ------------------------------------------------------------
+  // Load `it` of a thread: 16-byte slot it * TG + tg of its group's slice: row slot / 8, position
+  // slot % 8, which holds source unit (slot % 8) ^ ((row >> 1) & 7).  Rows past the matrix edge
+  // re-read the last row (their products are never stored).
+  typedef typename std::conditional<WIDE, size_t, unsigned>::type Off;
+  auto row_off = [&](int r0, int rows, int s) __attribute__((always_inline)) {
+    const int r = s >> 3;
+    return (Off)(min(r0 + r, rows - 1) - r0) * (Off)Kp * 2u + (Off)(((s & 7) ^ ((r >> 1) & 7)) * 16);
+  };
+  Off a_off[A_N], b_off[B_IT];
+#pragma unroll
+  for (int it = 0; it < A_IT; ++it) a_off[it] = row_off(m0, M, it * TG + tg);
+#pragma unroll
+  for (int it = 0; it < B_IT; ++it) b_off[it] = row_off(n0, N, it * TG + tg);
+  const int KT = Kp / 64, ST = (KT + WK - 1) / WK;  // k-slices, k-steps
+  const char* a_base = (const char*)Av + (size_t)m0 * Kp * 2;
+  const char* b_base = (const char*)(Bt + (size_t)n0 * Kp);
+  const unsigned wave_off = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem) +
+                            (unsigned)g * SLICE + (unsigned)w * 1024u;
+  // a group without a slice in the last k-step loads the last slice again and multiplies nothing
+  auto issue_one = [&](int t, int stage, int n) __attribute__((always_inline)) {
+    const size_t koff = (size_t)min(t * WK + g, KT - 1) * 128;
+    const unsigned at = wave_off + (unsigned)stage * STAGE;
+    const char* base = (n < A_IT ? a_base : b_base) + koff;
+    const Off off = n < A_IT ? a_off[n < A_IT ? n : 0] : b_off[n < A_IT ? 0 : n - A_IT];
+    const unsigned lds = at + (n < A_IT ? n * (TG * 16) : B_AT + (n - A_IT) * (TG * 16));
+    if constexpr (WIDE) lds_dma16(base + off, lds);
+    else lds_dma16_base(base, off, lds);
+  };
+  // The loads of a k-step are dealt over the second half of one k-step (the first L1 of them) and
+  // the first half of the next: a burst arrives faster than the texture unit takes it (16 cycles a
+  // load and CU), and the wavefronts then stall on issue with their MFMAs behind it.
+  constexpr int L1 = LPT / 2;
+#pragma unroll
+  for (int s = 0; s < NST; ++s)
+    if (s < ST) {
+#pragma unroll
+      for (int n = 0; n < (s + 1 < NST ? LPT : L1); ++n) issue_one(s, s, n);
+    }
+
+  // acc[i][j]: columns 16 i.., rows 16 j.. of the wavefront's sub-tile; a lane holds the 4
+  // columns 4 (lane / 16) + 0..3 of row lane % 16
+  f4 acc[NB][MB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+
+  // Fragments of v_mfma_f32_16x16x32_f16: row lane % 16 of a block, 16-byte unit lane / 16 of a
+  // 32-wide half slice.  16 consecutive lanes read 16 rows at one unit: no bank conflicts.
+  const int lrow = lane & 15, lq = lane >> 4, fkey = (lrow >> 1) & 7;
+  const int a_row = (wm * TM + lrow) * 128, b_row = B_AT + (wn * TN + lrow) * 128;
+  const char* panel = smem + NST * STAGE;
+  h8 fa[2][MB], fb[2][NB];  // [half slice][block]
+  constexpr int NR = MB + NB, NM = MB * NB;  // fragment reads, MFMAs per half slice
+  constexpr int RPM = (NR + (NM + 1) / 2 - 1) / ((NM + 1) / 2);  // reads behind an MFMA: all behind the first half of them
+  auto read_one = [&](int t, int stage, int half, int n) __attribute__((always_inline)) {
+    const char* st = smem + stage * STAGE + g * SLICE;
+    const int un = ((half * 4 + lq) ^ fkey) << 4;
+    if (n < MB) {
+      const char* sa = LNA ? panel + (size_t)min(t * WK + g, KT - 1) * (BM * 128) : st;
+      fa[half][n < MB ? n : 0] = *reinterpret_cast<const h8*>(sa + a_row + n * 2048 + un);
+    } else {
+      fb[half][n < MB ? 0 : n - MB] = *reinterpret_cast<const h8*>(st + b_row + (n - MB) * 2048 + un);
+    }
+  };
+  auto mfma_one = [&](int half, int n) __attribute__((always_inline)) {
+    const int j = n / NB, ii = n % NB;
+    const int i = (j & 1) ? NB - 1 - ii : ii;  // one operand changes per MFMA
+    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[half][i], fa[half][j], acc[i][j], 0, 0, 0);
+  };
+  // the k-steps younger than the one that must have landed: `younger` of them, LPT loads each
+  auto wait_landed = [&](int younger) __attribute__((always_inline)) {
+    if (younger <= 0) wait_vmcnt<0>();
+    else if (younger == 1 || NST < 3) wait_vmcnt<LPT>();
+    else if (younger == 2 || NST < 4) wait_vmcnt<2 * LPT>();
+    else if (younger == 3 || NST < 5) wait_vmcnt<3 * LPT>();
+    else wait_vmcnt<4 * LPT>();
+  };
+  // a group of one wavefront reads only what it loaded itself
+  auto meet = [&]() __attribute__((always_inline)) {
+    if constexpr (WM * WN > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+
+  if constexpr (LNA) {
+    normalise_panel<BM, NT, T>((const T*)Av, M, Kp, m0, ln, smem + NST * STAGE, tid);
+    wait_vmcnt<0>();
+    __syncthreads();
+  } else {
+    // k-step 0; behind it min(NST, ST) - 1 more, the last of them in part if it is the NST-th
+    if (ST >= NST) wait_vmcnt<(NST - 2) * LPT + L1>();
+    else wait_landed(ST - 1);
+    meet();
+  }
+#pragma unroll
+  for (int n = 0; n < NR; ++n) read_one(0, 0, 0, n);
+
+  // ---- bias and residual of the chunks this thread will store, requested behind the first k-steps
+  // (the counted waits of the loop then wait for these too, once, and otherwise for no more than
+  // they name; at the end of the loop they would cost a memory round trip of their own)
+  constexpr int CW = 16 / (int)sizeof(T);  // output columns per 16 bytes
+  constexpr int CPR = BN / CW, CHUNKS = BM * CPR, IT = (CHUNKS + NT - 1) / NT;
+  static_assert(NT % CPR == 0, "a thread keeps its columns");
+  typedef T TV __attribute__((ext_vector_type(CW)));
+  const int cc = tid % CPR, n = n0 + cc * CW, r_first = tid / CPR;
+  constexpr int RSTEP = NT / CPR;
+  const bool col_ok = n < N && (CHUNKS >= NT || tid < CHUNKS);
+  // `vec`: N, head size and pointers allow 16-byte accesses; otherwise element by element
+  const bool vec = ep.tile_vec;
+  auto load_chunk = [&](const T* p) __attribute__((always_inline)) {
+    TV v;
+    if (vec) v = *reinterpret_cast<const TV*>(p);
+    else {
+#pragma unroll
+      for (int e = 0; e < CW; ++e) v[e] = n + e < N ? p[e] : (T)0.f;
+    }
+    return v;
+  };
+  TV bias_v, res_v[IT];
+#pragma unroll
+  for (int e = 0; e < CW; ++e) bias_v[e] = (T)0.f;
+  if (ep.bias && col_ok) bias_v = load_chunk((const T*)ep.bias + n);
+  const bool res = !QKV && ep.residual != nullptr;
+  if (res && col_ok) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int m = m0 + r_first + it * RSTEP;
+      if (m < M) res_v[it] = load_chunk((const T*)ep.residual + ((int64_t)m * N + n));
+    }
+  }
+
+  // One k-step: the MFMAs of its first half with the fragment reads of its second half dealt
+  // between them; the barrier that publishes k-step t + 1 and frees this stage; the MFMAs of the
+  // second half with the reads of the next k-step's first half and the refill of this stage
+  // with k-step t + NST.
+  int stage = 0, st_prev = NST - 1;
+  auto step = [&](auto load0, auto load1, int t) __attribute__((always_inline)) {
+    constexpr bool LOAD0 = decltype(load0)::value, LOAD1 = decltype(load1)::value;
+    const int st_next = stage + 1 == NST ? 0 : stage + 1;
+#pragma unroll
+    for (int q = 0; q < NM; ++q) {
+      mfma_one(0, q);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = q * RPM; n < (q + 1) * RPM && n < NR; ++n) read_one(t, stage, 1, n);
+      if constexpr (LOAD0) {
+#pragma unroll
+        for (int n = q * (LPT - L1) / NM; n < (q + 1) * (LPT - L1) / NM; ++n)
+          issue_one(t + NST - 1, st_prev, L1 + n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (LOAD0) wait_vmcnt<(NST - 2) * LPT>();
+    else wait_landed(ST - 2 - t);
+    meet();
+#pragma unroll
+    for (int q = 0; q < NM; ++q) {
+      mfma_one(1, q);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = q * RPM; n < (q + 1) * RPM && n < NR; ++n) read_one(t + 1, st_next, 0, n);
+      if constexpr (LOAD1) {
+#pragma unroll
+        for (int n = q * L1 / NM; n < (q + 1) * L1 / NM; ++n) issue_one(t + NST, stage, n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    st_prev = stage;
+    stage = st_next;
+  };
+  std::true_type yes;
+  std::false_type no;
+  int t = 0;
+  for (; t + NST < ST; ++t) step(yes, yes, t);
+  if (t + 1 < ST && t + NST == ST) step(yes, no, t++);
+  for (; t + 1 < ST; ++t) step(no, no, t);
+
+  // ---- last k-step
+  if (KT % WK == 0 || t * WK + g < KT) {
+#pragma unroll
+    for (int n = 0; n < NR; ++n) read_one(t, stage, 1, n);
+#pragma unroll
+    for (int q = 0; q < 2 * NM; ++q) mfma_one(q / NM, q % NM);
+  }
+
+  // ---- the groups' sums into LDS, row-major fp32: 16-byte unit u of row r at u ^ key(r), the key
+  // such that the 16 rows a quarter wavefront writes fall on 16 different 16-byte slots
+  __syncthreads();
+  constexpr int UPR = BN / 4;  // 16-byte units per row
+  auto unit_at = [&](int r, int u) __attribute__((always_inline)) {
+    return UPR >= 16 ? u ^ (r & 15) : u ^ ((r >> 1) & (UPR - 1));
+  };
+  {
+    char* mine = smem + g * (BM * BN * 4);
+#pragma unroll
+    for (int j = 0; j < MB; ++j)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int r = wm * TM + j * 16 + lrow, u = (wn * TN + i * 16) / 4 + lq;
+        *reinterpret_cast<f4*>(mine + r * (BN * 4) + (unit_at(r, u) << 4)) = acc[i][j];
+      }
+  }
+  __syncthreads();
+  if (!col_ok) return;
+
+  T* col = nullptr;  // head-major scatter: row 0 of batch 0 at this thread's columns
+  if constexpr (QKV) col = qkv_column_base<T>(ep, n);
+  const int64_t batch_stride = (int64_t)ep.heads * ep.L * ep.d;
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int r = r_first + it * RSTEP, m = m0 + r;
+    if (m >= M) break;
+    float z[CW];
+#pragma unroll
+    for (int u = 0; u < CW / 4; ++u) {
+      const int at = r * (BN * 4) + (unit_at(r, cc * (CW / 4) + u) << 4);
+      f4 s = *reinterpret_cast<const f4*>(smem + at);
+#pragma unroll
+      for (int k = 1; k < WK; ++k) s += *reinterpret_cast<const f4*>(smem + k * (BM * BN * 4) + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z[u * 4 + e] = s[e];
+    }
+#pragma unroll
+    for (int e = 0; e < CW; ++e) {
+      z[e] += (float)bias_v[e];
+      if (ep.gelu) z[e] = gelu_new(z[e]);
+    }
+    if constexpr (DROP) {
+      unsigned off[CW];
+#pragma unroll
+      for (int e = 0; e < CW; ++e) off[e] = (unsigned)((uint64_t)m * (uint64_t)N + (uint64_t)(n + e));
+      dropout_apply<CW>(ep.drop, off, z);
+    }
+    TV o;
+#pragma unroll
+    for (int e = 0; e < CW; ++e) o[e] = (T)(res ? z[e] + (float)res_v[it][e] : z[e]);
+    T* dst;
+    if constexpr (QKV) {
+      const unsigned mt = (unsigned)(m + ep.m_off), b = mt / (unsigned)ep.L, l = mt - b * (unsigned)ep.L;
+      dst = col + ((int64_t)b * batch_stride + (int64_t)l * ep.d);
+    } else {
+      dst = (T*)ep.out + ((int64_t)m * N + n);
+    }
+    if (vec) *reinterpret_cast<TV*>(dst) = o;
+    else {
+#pragma unroll
+      for (int e = 0; e < CW; ++e)
+        if (n + e < N) dst[e] = o[e];
+    }
+  }
+}
+
+template <class C, typename T, bool QKV, bool LNA, bool DROP, bool WIDE = false>
+int launch_tile_cfg(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                    const LnArgs& ln, hipStream_t st) {
+  auto kern = gemm_tile_kernel<C, T, QKV, LNA, DROP, WIDE>;
+  constexpr int stages = C::NST * ((LNA ? 0 : C::BM) + C::BN) * 128 * C::WK, sums = C::BM * C::BN * 4 * C::WK;
+  static_assert(stages <= 160 * 1024 && sums <= 160 * 1024, "LDS");
+  const size_t panel = LNA ? (size_t)C::BM * Kp * 2 : 0;
+  const size_t smem = stages + panel > (size_t)sums ? stages + panel : (size_t)sums;
+  static bool attr_done = false;  // idempotent; a race only repeats the call
+  if (!attr_done) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) {
+      set_error("hipFuncSetAttribute(160 KB LDS): %s", hipGetErrorString(e));
+      return -4;
+    }
+    attr_done = true;
+  }
+  const int64_t tiles_m = (M + C::BM - 1) / C::BM, tiles_n = ((int64_t)N + C::BN - 1) / C::BN;
+  if (tiles_m * tiles_n > 0x7fffffffll) {
+    set_error("gemm: %lld x %lld output tiles exceed the grid", (long long)tiles_m, (long long)tiles_n);
+    return -2;
+  }
+  const int group_w = column_group((int)tiles_n, C::BN, Kp);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(C::THREADS), smem, st, A,
+                     (const _Float16*)Bt, (int)M, N, Kp, (int)tiles_m, (int)tiles_n, group_w, ep, ln);
+  return 0;
+}
+
+// The menu, with the two numbers of the cost model: a launch of ceil(tiles / CUs) = R rounds takes
+// about launch + R (fixed + k_slices * slice) microseconds.  Fitted to 16 products of the four GPT-2
+// widths at 19 row counts from 8 to 20000 (weights from HBM, activations warm), where the model's
+// choice is 0.5 % slower than the best of the menu on average and 13 % at worst.  What the numbers
+// say: a workgroup takes in 40 to 48 bytes per clock whatever its shape, so a tile costs its
+// operand bytes -- small tiles win while they fill the 256 CUs once, large ones as soon as they do.
+//                    BM   BN  WM WN WK NST
+typedef Tile< 32,  16, 1, 1, 4, 4> T32x16;
+typedef Tile< 32,  32, 1, 1, 4, 4> T32x32;
+typedef Tile< 64,  32, 2, 1, 4, 3> T64x32;
+typedef Tile< 64,  64, 2, 2, 2, 4> T64x64;
+typedef Tile< 64, 128, 2, 2, 2, 3> T64x128;
+typedef Tile<128, 128, 2, 4, 1, 4> T128x128;
+typedef Tile<192, 128, 4, 2, 1, 3> T192x128;
+typedef Tile<128, 256, 2, 4, 1, 3> T128x256;
+struct TileCost {
+  int bm, bn, wk;
+  float launch, fixed, slice;
+};
+constexpr TileCost kTiles[] = {
+    {32, 16, 4, 2.18f, 1.36f, 0.057f},  {32, 32, 4, 1.98f, 1.34f, 0.086f},
+    {64, 32, 4, 1.82f, 1.45f, 0.131f},  {64, 64, 2, 1.55f, 1.37f, 0.189f},
+    {64, 128, 2, 0.99f, 2.09f, 0.305f}, {128, 128, 1, 0.f, 3.89f, 0.435f},
+    {192, 128, 1, 0.f, 5.01f, 0.556f},  {128, 256, 1, 0.f, 5.77f, 0.655f},
+};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+
+inline float cost_of(const TileCost& c, int64_t M, int N, int Kp, int cus) {
+  const int64_t tiles = ((M + c.bm - 1) / c.bm) * (((int64_t)N + c.bn - 1) / c.bn);
+  const int64_t rounds = (tiles + cus - 1) / cus;
+  return c.launch + (float)rounds * (c.fixed + (float)(Kp / 64) * c.slice);
+}
+
+inline int pick_tile(int64_t M, int N, int Kp, int cus, float* cost) {
+  int best = 0;
+  float least = cost_of(kTiles[0], M, N, Kp, cus);
+  for (int i = 1; i < kNumTiles; ++i) {
+    const float c = cost_of(kTiles[i], M, N, Kp, cus);
+    if (c < least) least = c, best = i;
+  }
+  if (cost) *cost = least;
+  return best;
+}
+
+template <typename T, bool QKV, bool DROP>
+int launch_pick(int i, const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                hipStream_t st) {
+  const LnArgs ln = {};
+  switch (i) {
+    case 0: return launch_tile_cfg<T32x16, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 1: return launch_tile_cfg<T32x32, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 2: return launch_tile_cfg<T64x32, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 3: return launch_tile_cfg<T64x64, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 4: return launch_tile_cfg<T64x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 5: return launch_tile_cfg<T128x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 6: return launch_tile_cfg<T192x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    default: return launch_tile_cfg<T128x256, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+  }
+}
+
+// rows of 2^22 elements and more: 64-bit addresses, one tile shape
+constexpr int kWideK = 1 << 22;
+
+}  // namespace
+
+float gemm_tile_cost(int64_t M, int N, int Kp, int cus) {
+  float cost;
+  pick_tile(M, N, Kp, cus, &cost);
+  return cost;
+}
+
+template <typename T, bool QKV>
+static int launch_tile_t(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                         hipStream_t st) {
+  const int cus = cu_count();
+  if (cus < 0) return cus;
+  if constexpr (!QKV) {
+    if (ep.drop.p > 0.f) {
+      if (Kp >= kWideK)
+        return launch_tile_cfg<T32x32, T, false, false, true, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+      return launch_pick<T, false, true>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+    }
+  }
+  if (Kp >= kWideK)
+    return launch_tile_cfg<T32x32, T, QKV, false, false, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+  return launch_pick<T, QKV, false>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+}
+
+int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                     bool f16, bool qkv, hipStream_t st) {
+  if (f16)
+    return qkv ? launch_tile_t<_Float16, true>(A, Bt, M, N, Kp, ep, st)
+               : launch_tile_t<_Float16, false>(A, Bt, M, N, Kp, ep, st);
+  return qkv ? launch_tile_t<float, true>(A, Bt, M, N, Kp, ep, st)
+             : launch_tile_t<float, false>(A, Bt, M, N, Kp, ep, st);
+}
+
+// ---- LayerNorm prologue ----------------------------------------------------------------------
+// 32-row tiles on 8 wavefronts: the LDS panel of the normalised rows takes 64 * K bytes (100 KB at
+// GPT-2 XL's 1600), three stages of weight rows 48 KB beside it.  K is split over as many groups as
+// the plain launch of these sizes splits it, so that the sums, too, are formed in the same order.
+namespace {
+typedef Tile<32,  32, 1, 2, 4, 3> Ln32x32;
+typedef Tile<32,  64, 1, 4, 2, 3> Ln32x64;
+typedef Tile<32, 128, 1, 8, 1, 3> Ln32x128;
+constexpr int kLnStages = 3 * 128 * 128;
+
+template <bool QKV>
+int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiDev& ep, const LnArgs& ln,
+              hipStream_t st) {
+  const int cus = cu_count();
+  if (cus < 0) return cus;
+  switch (kTiles[pick_tile(M, N, K, cus, nullptr)].wk) {
+    case 4: return launch_tile_cfg<Ln32x32, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 2: return launch_tile_cfg<Ln32x64, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    default: return launch_tile_cfg<Ln32x128, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+  }
+}
+}  // namespace
+
+bool gemm_layernorm_supported(int64_t M, int H) {
+  if (H <= 0 || H % 64 != 0 || M <= 0) return false;
+  const int nchunks = H / 8, lpr = lanes_per_row(nchunks);
+  return (nchunks + lpr - 1) / lpr <= 8 && (size_t)kLnStages + 64 * (size_t)H <= 160 * 1024;
+}
+
+int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
+                               const LnArgs& ln, bool qkv, hipStream_t st) {
+  return qkv ? launch_ln<true>(x, Bt, M, N, H, ep, ln, st) : launch_ln<false>(x, Bt, M, N, H, ep, ln, st);
+}
+
+}  // namespace gptmi
