@@ -2,6 +2,7 @@
 // operand packing for the GEMM, and dispatch to the kernel launchers.
 #include "../../include/gptmi.h"
 
+#include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -179,6 +180,93 @@ static int check_linear_args(const void* x, const void* W, const void* out, int6
   return GPTMI_OK;
 }
 
+// ---- whole blocks ------------------------------------------------------------------------------
+// A transformer block's launches behind one call.  Intermediate matrices live in the caller's
+// workspace, all of them fp16: for fp16 storage that is the storage type, for fp32 storage it is the
+// rounding that the next product (or the attention) applies to its operands anyway -- LayerNorm, q, k,
+// v, the attention's output and the GELU's output are each written once in fp16 instead of in fp32 and
+// again by a pack pass, with the same bits at the end.
+
+// Carves 256-byte aligned pieces out of a workspace.
+struct Carver {
+  char* base;
+  size_t used;
+  void* take(size_t bytes) {
+    void* p = base ? base + used : nullptr;
+    used += (size_t)round_up((int64_t)bytes, 256);
+    return p;
+  }
+};
+
+// The weight image a product reads: the caller's (packed), or one built into `ws`.
+static const void* weight_image(const void* W, void* ws, int64_t N, int64_t K, int wlayout, bool f16,
+                                hipStream_t st) {
+  if (wlayout == GPTMI_W_PACKED) return W;
+  launch_pack_transpose(W, ws, (int)K, (int)N, (int)round_up(K, 64), f16, st);
+  return ws;
+}
+static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
+  return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
+}
+
+struct AttentionPlan {
+  void *normed, *q, *k, *v, *merged, *w_qkv, *w_proj;
+  size_t total;
+};
+static AttentionPlan plan_attention(void* ws, int64_t M, int64_t h, int wlayout) {
+  Carver c = {(char*)ws, 0};
+  AttentionPlan p;
+  const size_t mat = (size_t)(M * h * 2);
+  p.normed = c.take(mat);
+  p.q = c.take(mat);
+  p.k = c.take(mat);
+  p.v = c.take(mat);
+  p.merged = c.take(mat);
+  p.w_qkv = c.take(image_bytes(3 * h, h, wlayout));
+  p.w_proj = c.take(image_bytes(h, h, wlayout));
+  p.total = c.used;
+  return p;
+}
+
+struct MlpPlan {
+  void *normed, *inner, *w1, *w2;
+  size_t total;
+};
+static MlpPlan plan_mlp(void* ws, int64_t M, int64_t h, int64_t inner, int wlayout) {
+  Carver c = {(char*)ws, 0};
+  MlpPlan p;
+  p.normed = c.take((size_t)(M * h * 2));
+  p.inner = c.take((size_t)(M * inner * 2));
+  p.w1 = c.take(image_bytes(inner, h, wlayout));
+  p.w2 = c.take(image_bytes(h, inner, wlayout));
+  p.total = c.used;
+  return p;
+}
+
+// What the block functions take: row widths that are multiples of 64 (every operand is then read in
+// place), up to the LayerNorm kernel's 8192.
+static int check_block(const char* what, int64_t M, int64_t h, float p, int wlayout, int dtype,
+                       const void* ws, size_t ws_bytes, size_t need) {
+  if (M <= 0 || h <= 0 || !dtype_ok(dtype) || (wlayout != GPTMI_W_KN && wlayout != GPTMI_W_PACKED)) {
+    set_error("%s: invalid argument", what);
+    return GPTMI_ERR_INVALID;
+  }
+  if (h % 64 != 0 || h > 8192) {
+    set_error("%s: row width %lld is not a multiple of 64 up to 8192", what, (long long)h);
+    return GPTMI_ERR_UNSUPPORTED;
+  }
+  if (!dropout_ok(p)) {
+    set_error("%s: dropout probability %g outside [0, 1)", what, (double)p);
+    return GPTMI_ERR_INVALID;
+  }
+  if (ws == nullptr || ws_bytes < need || ((uintptr_t)ws & 255) != 0) {
+    set_error("%s: workspace of %zu bytes, 256-byte aligned, needed (%zu given)", what, need,
+              ws ? ws_bytes : (size_t)0);
+    return GPTMI_ERR_WORKSPACE;
+  }
+  return GPTMI_OK;
+}
+
 }  // namespace gptmi
 
 using namespace gptmi;
@@ -239,7 +327,7 @@ int gptmi_embed_layernorm(const int64_t* ids, const void* wte, const void* wpe,
                               st)) {
     // rows the fused kernel does not hold in registers: the two kernels, same results
     launch_embed(ids, wte, wpe, emb, B * L, L, V, (int)H, Dropout{0.0f, 1337}, f16, st);
-    launch_layernorm(emb, ln_w, ln_b, out, B * L, (int)H, eps, f16, st);
+    launch_layernorm(emb, ln_w, ln_b, out, B * L, (int)H, eps, f16, false, st);
   }
   return check_launch("embed_layernorm");
 }
@@ -254,7 +342,7 @@ int gptmi_layernorm(const void* x, const void* w, const void* b, void* out, int6
     set_error("layernorm: H=%lld beyond the supported 8192", (long long)H);
     return GPTMI_ERR_UNSUPPORTED;
   }
-  launch_layernorm(x, w, b, out, M, (int)H, eps, dtype == GPTMI_F16, (hipStream_t)stream);
+  launch_layernorm(x, w, b, out, M, (int)H, eps, dtype == GPTMI_F16, false, (hipStream_t)stream);
   return check_launch("layernorm");
 }
 
@@ -479,6 +567,121 @@ int gptmi_flash_attn(const void* q, const void* k, const void* v, void* out, int
                              dtype == GPTMI_F16, (hipStream_t)stream);
   if (rc) return rc;
   return check_launch("flash_attn");
+}
+
+size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d,
+                                             int wlayout) {
+  if (B <= 0 || L <= 0 || heads <= 0 || d <= 0) return 0;
+  return plan_attention(nullptr, B * L, heads * d, wlayout).total;
+}
+
+int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
+                          const void* W_qkv, const void* b_qkv, const void* W_proj, const void* b_proj,
+                          void* out, int64_t B, int64_t L, int64_t heads, int64_t d, float p,
+                          uint64_t seed, int fuse_layernorm, int wlayout, void* workspace,
+                          size_t workspace_bytes, int dtype, void* stream) {
+  if (!x || !ln_w || !ln_b || !W_qkv || !W_proj || !out || B <= 0 || L <= 0 || heads <= 0 || d <= 0) {
+    set_error("attention_block: invalid argument");
+    return GPTMI_ERR_INVALID;
+  }
+  const int64_t M = B * L, h = heads * d;
+  const AttentionPlan pl = plan_attention(workspace, M, h, wlayout);
+  int rc = check_block("attention_block", M, h, p, wlayout, dtype, workspace, workspace_bytes, pl.total);
+  if (rc) return rc;
+  const bool f16 = dtype == GPTMI_F16;
+  hipStream_t st = (hipStream_t)stream;
+  const void* Bq = weight_image(W_qkv, pl.w_qkv, 3 * h, h, wlayout, f16, st);
+  const void* Bp = weight_image(W_proj, pl.w_proj, h, h, wlayout, f16, st);
+  if (((uintptr_t)x & 15) || ((uintptr_t)normed & 15) || ((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
+    set_error("attention_block: x and the weights must be 16-byte aligned");
+    return GPTMI_ERR_INVALID;
+  }
+  GemmEpilogue ep = {};
+  ep.bias = b_qkv;
+  ep.q = pl.q;
+  ep.k = pl.k;
+  ep.v = pl.v;
+  ep.L = L;
+  ep.heads = (int)heads;
+  ep.d = (int)d;
+  ep.qkv = true;
+  ep.f16 = f16;
+  ep.out_f16 = true;
+  if (fuse_layernorm && !normed) {
+    if (!f16 || !gemm_layernorm_supported(M, (int)h)) {
+      set_error("attention_block: the LayerNorm prologue takes fp16 storage and the row widths of "
+                "gptmi_layernorm_linear_supported");
+      return GPTMI_ERR_UNSUPPORTED;
+    }
+    rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
+  } else {
+    const void* A = pl.normed;
+    if (!normed) launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)h, eps, f16, true, st);
+    else if (f16) A = normed;
+    else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, false, st);
+    rc = launch_gemm(A, Bq, M, (int)(3 * h), (int)h, ep, st);
+  }
+  if (rc) return rc;
+  const Dropout drop = {p, seed};
+  const float scale = (float)(1.0 / sqrt((double)d));
+  rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
+           : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
+  if (rc) return rc;
+  GemmEpilogue eo = {};
+  eo.bias = b_proj;
+  eo.residual = x;
+  eo.out = out;
+  eo.drop = drop;
+  eo.f16 = f16;
+  rc = launch_gemm(pl.merged, Bp, M, (int)h, (int)h, eo, st);
+  if (rc) return rc;
+  return check_launch("attention_block");
+}
+
+size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int wlayout) {
+  if (M <= 0 || H <= 0 || inner <= 0) return 0;
+  return plan_mlp(nullptr, M, H, inner, wlayout).total;
+}
+
+int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
+                    const void* b1, const void* W2, const void* b2, void* out, int64_t M, int64_t H,
+                    int64_t inner, float p, uint64_t seed, int wlayout, void* workspace,
+                    size_t workspace_bytes, int dtype, void* stream) {
+  if (!x || !ln_w || !ln_b || !W1 || !W2 || !out || inner <= 0 || inner % 64 != 0 || inner > kMaxN) {
+    set_error("mlp_block: invalid argument");
+    return GPTMI_ERR_INVALID;
+  }
+  const MlpPlan pl = plan_mlp(workspace, M, H, inner, wlayout);
+  int rc = check_block("mlp_block", M, H, p, wlayout, dtype, workspace, workspace_bytes, pl.total);
+  if (rc) return rc;
+  const bool f16 = dtype == GPTMI_F16;
+  hipStream_t st = (hipStream_t)stream;
+  const void* B1 = weight_image(W1, pl.w1, inner, H, wlayout, f16, st);
+  const void* B2 = weight_image(W2, pl.w2, H, inner, wlayout, f16, st);
+  if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
+    set_error("mlp_block: the weights must be 16-byte aligned");
+    return GPTMI_ERR_INVALID;
+  }
+  launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)H, eps, f16, true, st);
+  const Dropout drop = {p, seed};
+  GemmEpilogue e1 = {};
+  e1.bias = b1;
+  e1.out = pl.inner;
+  e1.gelu = 1;
+  e1.drop = drop;
+  e1.f16 = f16;
+  e1.out_f16 = true;
+  rc = launch_gemm(pl.normed, B1, M, (int)inner, (int)H, e1, st);
+  if (rc) return rc;
+  GemmEpilogue e2 = {};
+  e2.bias = b2;
+  e2.residual = x;
+  e2.out = out;
+  e2.drop = drop;
+  e2.f16 = f16;
+  rc = launch_gemm(pl.inner, B2, M, (int)H, (int)inner, e2, st);
+  if (rc) return rc;
+  return check_launch("mlp_block");
 }
 
 }  // extern "C"

@@ -53,12 +53,43 @@ template <> struct Ld8<float> {
   }
 };
 
-// exp for the softmax: the fp32-storage build keeps the accurate library
-// routine (fewer fp16 rounding flips of P against the reference's np.exp);
-// the fp16-storage build uses the hardware exp2 path.
-template <typename T> __device__ __forceinline__ float softmax_exp(float x);
-template <> __device__ __forceinline__ float softmax_exp<float>(float x) { return expf(x); }
-template <> __device__ __forceinline__ float softmax_exp<_Float16>(float x) { return __expf(x); }
+// The softmax arithmetic, in two precisions.  ACC = false (fp16 storage): running max on the raw
+// scores, scale * log2(e) folded into one fused multiply-add in front of the hardware's exp2, a
+// reciprocal for the denominator -- the same real-number formula as the reference, two VALU
+// operations per score fewer.  ACC = true (fp32 storage, and the fp16 copies of q, k, v that the
+// block functions of fp32 models hand on): the reference's operation order, library exp and a true
+// division, so fewer fp16 rounding flips of P against the reference's np.exp.
+template <bool ACC>
+struct Softmax {
+  float c;  // ACC: scale; otherwise scale * log2(e)
+  __device__ __forceinline__ explicit Softmax(float scale)
+      : c(ACC ? scale : scale * 1.4426950408889634f) {}
+  // the multiple of the running max that weight() subtracts
+  __device__ __forceinline__ float base(float m) const { return m * c; }
+  // exp(scale * (s - m)) for base b = base(m)
+  __device__ __forceinline__ float weight(float s, float b) const {
+    if constexpr (ACC) {
+      float t = s * c;
+      asm("" : "+v"(t));  // rounded as the reference rounds it, not fused with the subtraction
+      return expf(t - b);
+    } else {
+      return __builtin_amdgcn_exp2f(fmaf(s, c, -b));
+    }
+  }
+  // exp(scale * (old - m)), the rescaling when the running max goes from `old` to m
+  __device__ __forceinline__ float rescale(float old, float m) const {
+    if constexpr (ACC) return expf(old * c - m * c);
+    else return __builtin_amdgcn_exp2f((old - m) * c);
+  }
+};
+
+// o / den for a whole row: ACC divides, otherwise the reciprocal (1 ulp of fp32) is taken once
+template <bool ACC>
+struct Normalise {
+  float d;
+  __device__ __forceinline__ explicit Normalise(float den) : d(ACC ? den : __builtin_amdgcn_rcpf(den)) {}
+  __device__ __forceinline__ float operator()(float o) const { return ACC ? o / d : o * d; }
+};
 
 __device__ __forceinline__ h8 zero_h8() {
   h8 z;
@@ -72,7 +103,7 @@ __device__ __forceinline__ h8 zero_h8() {
 // u ^ ((d>>1)&15)).  DG = head size of the tensors in memory: 16 and 32 run on the D = 64
 // staging layout (columns at or past DG are written as zeros, never read from memory) with
 // only DG / 16 k-steps of q . k and one 32-row block of O^T.
-template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D>
+template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
 __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
     T* __restrict__ O, int heads, int L, int Lk_arg, float scale, DropoutArgs drop) {
@@ -189,6 +220,7 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
   float mrun = -INFINITY, den = 0.f;
+  const Softmax<ACC> sm(scale);
 
   load_tile(0, stg[0]);
   if constexpr (!ONESET) {
@@ -235,51 +267,23 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
             s[kb][r] = key <= q ? s[kb][r] : -INFINITY;
           }
       }
-      float mult, psum = 0.f;
-      if constexpr (sizeof(T) == 2 && !DROP) {
-        // fp16 storage: running max on the raw scores, scale * log2(e) folded into one fused
-        // multiply-add in front of exp2 (as in the resident kernel below)
-        const float c = scale * 1.4426950408889634f;
-        float bmax = -INFINITY;
+      float bmax = -INFINITY, psum = 0.f;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-        const float mnew = bmax > mrun ? bmax : mrun;
-        mult = __builtin_amdgcn_exp2f((mrun - mnew) * c);
-        const float m2 = mnew * c;
+        for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+      const float mnew = bmax > mrun ? bmax : mrun;
+      const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][r], c, -m2));
-            s[kb][r] = p;
-            psum += p;
-          }
-        mrun = mnew;
-      } else {
-        float bmax = -INFINITY;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            s[kb][r] *= scale;
-            bmax = fmaxf(bmax, s[kb][r]);
-          }
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-        const float mnew = bmax > mrun ? bmax : mrun;
-        mult = softmax_exp<T>(mrun - mnew);
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float p = softmax_exp<T>(s[kb][r] - mnew);
-            s[kb][r] = p;
-            psum += p;
-          }
-        mrun = mnew;
-      }
+        for (int r = 0; r < 16; ++r) {
+          const float p = sm.weight(s[kb][r], mb);
+          s[kb][r] = p;
+          psum += p;
+        }
+      mrun = mnew;
       psum += __shfl_xor(psum, 32, kWave);
       den = den * mult + psum;
       if constexpr (DROP) {
@@ -376,7 +380,7 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
 // order from the most expensive one, which balances the triangle over the SIMDs
 // (L = 300: 8, 8, 7, 7 tiles).  The arithmetic per tile is that of the tiled kernel.
 // ---------------------------------------------------------------------------
-template <int D, typename T, bool BLND, int NW>
+template <int D, typename T, bool BLND, int NW, bool ACC = sizeof(T) == 4>
 __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_resident_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
     T* __restrict__ O, int heads, int L, float scale) {
@@ -443,6 +447,7 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
   __syncthreads();
 
   const int ql = lane & 31, g = lane >> 5;
+  const Softmax<ACC> sm(scale);
   const int nc = (L + 31) / 32;
   // snake deal over NW wavefronts: of every 2*NW positions (position i = chunk nc-1-i,
   // most expensive first) wavefront w takes w and 2*NW-1-w
@@ -494,53 +499,23 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
               s[kb][r] = key <= q ? s[kb][r] : -INFINITY;
             }
         }
-        float mult, psum = 0.f;
-        if constexpr (sizeof(T) == 2) {
-          // fp16 storage: the running max is kept on the raw scores and scale * log2(e) is
-          // folded into one fused multiply-add in front of exp2 -- the same real-number
-          // formula as the reference, two VALU operations per score fewer
-          const float c = scale * 1.4426950408889634f;
-          float bmax = -INFINITY;
+        float bmax = -INFINITY, psum = 0.f;
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-          bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-          const float mnew = bmax > mrun ? bmax : mrun;
-          mult = __builtin_amdgcn_exp2f((mrun - mnew) * c);
-          const float m2 = mnew * c;
+          for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+        const float mnew = bmax > mrun ? bmax : mrun;
+        const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][r], c, -m2));
-              s[kb][r] = p;
-              psum += p;
-            }
-          mrun = mnew;
-        } else {
-          // fp32 storage: the reference's operation order, library exp
-          float bmax = -INFINITY;
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              s[kb][r] *= scale;
-              bmax = fmaxf(bmax, s[kb][r]);
-            }
-          bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-          const float mnew = bmax > mrun ? bmax : mrun;
-          mult = softmax_exp<T>(mrun - mnew);
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const float p = softmax_exp<T>(s[kb][r] - mnew);
-              s[kb][r] = p;
-              psum += p;
-            }
-          mrun = mnew;
-        }
+          for (int r = 0; r < 16; ++r) {
+            const float p = sm.weight(s[kb][r], mb);
+            s[kb][r] = p;
+            psum += p;
+          }
+        mrun = mnew;
         psum += __shfl_xor(psum, 32, kWave);
         den = den * mult + psum;
 #pragma unroll
@@ -575,7 +550,7 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
         } else {
           row_off = base + (int64_t)q * D;
         }
-        const float inv = __builtin_amdgcn_rcpf(den);  // fp16 storage only (1 ulp of fp32)
+        const Normalise<ACC> norm(den);
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
@@ -584,12 +559,12 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
             if constexpr (sizeof(T) == 2) {
               h4 o;
 #pragma unroll
-              for (int j = 0; j < 4; ++j) o[j] = (_Float16)(oacc[b][4 * rg + j] * inv);
+              for (int j = 0; j < 4; ++j) o[j] = (_Float16)norm(oacc[b][4 * rg + j]);
               *reinterpret_cast<h4*>(O + row_off + d) = o;
             } else {
               f4 o;
 #pragma unroll
-              for (int j = 0; j < 4; ++j) o[j] = oacc[b][4 * rg + j] / den;
+              for (int j = 0; j < 4; ++j) o[j] = norm(oacc[b][4 * rg + j]);
               *reinterpret_cast<f4*>(O + row_off + d) = o;
             }
           }
@@ -654,7 +629,7 @@ __device__ __forceinline__ void attn_dma16(const void* base, unsigned lane_off, 
                : "memory", "m0");
 }
 
-template <bool BLND>
+template <bool BLND, bool ACC>
 __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, int num_bh,
@@ -725,7 +700,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     const int unit = 4 * i + 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1);
     v_off[i] = Lp * 128 + vrow * 128 + ((unit ^ (2 * (vrow & 3))) << 4) + (sl & 1) * 8;
   }
-  const float cexp = scale * 1.4426950408889634f;
+  const Softmax<ACC> sm(scale);
 
   // K fragments of the 64-key tile at row k0: [kb][ks]
   auto read_k = [&](const char* buf, int k0, h8 (&kf)[2][KS]) {
@@ -787,14 +762,13 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
     const float mnew = bmax > mrun ? bmax : mrun;
-    const float mult = __builtin_amdgcn_exp2f((mrun - mnew) * cexp);
-    const float m2 = mnew * cexp;
+    const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][r], cexp, -m2));
+        const float p = sm.weight(s[kb][r], mb);
         s[kb][r] = p;
         psum += p;
       }
@@ -855,7 +829,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     // half of the first operand against the lower half of the second), after which each owns 8
     // consecutive d of every other group: 4 stores of 16 bytes per lane instead of 8 of 8, and
     // 32 contiguous bytes per row and instruction.
-    const float inv = __builtin_amdgcn_rcpf(den);
+    const Normalise<ACC> norm(den);
     u4 out[DB][2];
 #pragma unroll
     for (int i = 0; i < DB; ++i)
@@ -864,8 +838,8 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
         h4 x, y;  // d = 32 i + 16 pr + 4 g + 0..3 and the same + 8
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          x[j] = (_Float16)(oacc[i][8 * pr + j] * inv);
-          y[j] = (_Float16)(oacc[i][8 * pr + 4 + j] * inv);
+          x[j] = (_Float16)norm(oacc[i][8 * pr + j]);
+          y[j] = (_Float16)norm(oacc[i][8 * pr + 4 + j]);
         }
         const u2 xd = __builtin_bit_cast(u2, x), yd = __builtin_bit_cast(u2, y);
         const auto r0 = __builtin_amdgcn_permlane32_swap(xd[0], yd[0], false, false);
@@ -957,7 +931,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 // odd 32-query chunk, one entirely visible block in front of it), later tiles are skipped -- as
 // in the streaming kernel, whose arithmetic per tile this is.
 // ---------------------------------------------------------------------------
-template <bool BLND>
+template <bool BLND, bool ACC>
 __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale) {
@@ -1024,7 +998,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     const int unit = 4 * i + 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1);
     v_off[i] = V_AT + vrow * 128 + ((unit ^ (2 * (vrow & 3))) << 4) + (sl & 1) * 8;
   }
-  const float cexp = scale * 1.4426950408889634f;
+  const Softmax<ACC> sm(scale);
 
   f16v oacc[DB];
 #pragma unroll
@@ -1085,8 +1059,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
     const float mnew = bmax > mrun ? bmax : mrun;
-    const float mult = __builtin_amdgcn_exp2f((mrun - mnew) * cexp);
-    const float m2 = mnew * cexp;
+    const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
@@ -1094,7 +1067,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * tt + j], cexp, -m2));
+          const float p = sm.weight(s[kb][8 * tt + j], mb);
           psum += p;
           pf[kb][tt][j] = (_Float16)p;
         }
@@ -1187,7 +1160,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
 
   // ---- output, as in the streaming kernel: the two lanes of a query trade halves through the
   // 32-lane swap and store 16 bytes each
-  const float inv = __builtin_amdgcn_rcpf(den);
+  const Normalise<ACC> norm(den);
   u4 out[DB][2];
 #pragma unroll
   for (int i = 0; i < DB; ++i)
@@ -1196,8 +1169,8 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
       h4 x, y;  // d = 32 i + 16 pr + 4 g + 0..3 and the same + 8
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        x[j] = (_Float16)(oacc[i][8 * pr + j] * inv);
-        y[j] = (_Float16)(oacc[i][8 * pr + 4 + j] * inv);
+        x[j] = (_Float16)norm(oacc[i][8 * pr + j]);
+        y[j] = (_Float16)norm(oacc[i][8 * pr + 4 + j]);
       }
       const u2 xd = __builtin_bit_cast(u2, x), yd = __builtin_bit_cast(u2, y);
       const auto r0 = __builtin_amdgcn_permlane32_swap(xd[0], yd[0], false, false);
@@ -1242,7 +1215,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
 // with vmcnt(0) in front of the next barrier.  Causal structure per wavefront as in the ring
 // kernel: tiles below qw0 / 64 entirely visible, tile qw0 / 64 with the block cut by the diagonal.
 // ---------------------------------------------------------------------------
-template <int D, bool BLND>
+template <int D, bool BLND, bool ACC>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale) {
@@ -1319,7 +1292,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
     const int unit = 4 * (i ^ (vrow & 3)) + 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1);
     v_off[i] = TILE + vrow * ROWB + (unit << 4) + (sl & 1) * 8;
   }
-  const float cexp = scale * 1.4426950408889634f;
+  const Softmax<ACC> sm(scale);
 
   f16v oacc[DB];
 #pragma unroll
@@ -1358,8 +1331,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
     bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
     const float mnew = bmax > mrun ? bmax : mrun;
-    const float mult = __builtin_amdgcn_exp2f((mrun - mnew) * cexp);
-    const float m2 = mnew * cexp;
+    const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
     h8 pf[NKB][2];
 #pragma unroll
@@ -1368,7 +1340,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * tt + j], cexp, -m2));
+          const float p = sm.weight(s[kb][8 * tt + j], mb);
           psum += p;
           pf[kb][tt][j] = (_Float16)p;
         }
@@ -1419,7 +1391,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
 
   // ---- output, as in the streaming kernel: the two lanes of a query trade halves through the
   // 32-lane swap and store 16 bytes each
-  const float inv = __builtin_amdgcn_rcpf(den);
+  const Normalise<ACC> norm(den);
   if (q < L) {
     int64_t row_off;
     if (BLND) {
@@ -1435,8 +1407,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
         h4 x, y;  // d = 32 i + 16 pr + 4 g + 0..3 and the same + 8
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          x[j] = (_Float16)(oacc[i][8 * pr + j] * inv);
-          y[j] = (_Float16)(oacc[i][8 * pr + 4 + j] * inv);
+          x[j] = (_Float16)norm(oacc[i][8 * pr + j]);
+          y[j] = (_Float16)norm(oacc[i][8 * pr + 4 + j]);
         }
         const u2 xd = __builtin_bit_cast(u2, x), yd = __builtin_bit_cast(u2, y);
         const auto r0 = __builtin_amdgcn_permlane32_swap(xd[0], yd[0], false, false);
@@ -1479,11 +1451,11 @@ inline size_t resident_lds_bytes(int L, int D) {
   return bytes <= 80 * 1024 ? bytes : 0;
 }
 
-template <int D, typename T, bool BLND>
+template <int D, typename T, bool BLND, bool ACC = sizeof(T) == 4>
 int launch_resident(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                     int L, float scale, size_t lds, hipStream_t st) {
   constexpr int NW = D == 64 ? RESIDENT_WAVES : 4;  // larger heads need > 128 registers
-  auto kern = flash_attn_resident_kernel<D, T, BLND, NW>;
+  auto kern = flash_attn_resident_kernel<D, T, BLND, NW, ACC>;
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1499,12 +1471,12 @@ int launch_resident(const void* q, const void* k, const void* v, void* out, int6
   return 0;
 }
 
-template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D>
+template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
 int launch_tiled_as(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                     int L, int Lk, float scale, DropoutArgs drop, hipStream_t st) {
   dim3 grid((unsigned)BN, (unsigned)((L + BQ - 1) / BQ));
   constexpr int lds = 2 * 2 * BKEY * D * 2;  // two stages of a K tile and a V^T tile
-  auto kern = flash_attn_kernel<D, T, BLND, DROP, UNEQ, DG>;
+  auto kern = flash_attn_kernel<D, T, BLND, DROP, UNEQ, DG, ACC>;
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done && lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1546,10 +1518,10 @@ inline int attn_cu_count() {
   return num_cus;
 }
 
-template <bool BLND>
+template <bool BLND, bool ACC = false>
 int launch_stream_attn(const void* q, const void* k, const void* v, void* out, int64_t BN,
                        int heads, int L, float scale, hipStream_t st) {
-  auto kern = flash_attn_stream_kernel<BLND>;
+  auto kern = flash_attn_stream_kernel<BLND, ACC>;
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1570,19 +1542,19 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   return 0;
 }
 
-template <bool BLND>
+template <bool BLND, bool ACC = false>
 int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                      int L, float scale, hipStream_t st) {
   dim3 grid((unsigned)BN, (unsigned)((L + BQ - 1) / BQ));
-  hipLaunchKernelGGL(flash_attn_ring_kernel<BLND>, grid, dim3(256), 0, st, (const _Float16*)q,
+  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), grid, dim3(256), 0, st, (const _Float16*)q,
                      (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale);
   return 0;
 }
 
-template <int D, bool BLND>
+template <int D, bool BLND, bool ACC = false>
 int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                      int L, float scale, hipStream_t st) {
-  auto kern = flash_attn_wide_kernel<D, BLND>;
+  auto kern = flash_attn_wide_kernel<D, BLND, ACC>;
   constexpr int lds = 2 * 2 * BKEY * D * 2;  // two stages of a K tile and a V tile
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -1674,7 +1646,58 @@ int launch_t(const void* q, const void* k, const void* v, void* out, int64_t BN,
   }
 }
 
+// fp32 arithmetic on fp16 q, k, v (equal lengths, merged-heads output in fp16): the values an fp32
+// model's kernels round their operands to anyway, see launch_flash_attn_operands.
+template <int D>
+int launch_operands_d(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
+                      int L, float scale, DropoutArgs da, hipStream_t st) {
+  typedef _Float16 T;
+  if (da.p > 0.f)
+    return launch_tiled_as<D, T, true, true, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+  if constexpr (D == 64) {
+    if (L <= 320 && BN >= 64) return launch_stream_attn<true, true>(q, k, v, out, BN, heads, L, scale, st);
+    if (resident_lds_bytes(L, D) == 0)
+      return launch_ring_attn<true, true>(q, k, v, out, BN, heads, L, scale, st);
+  }
+  if (const size_t lds = resident_lds_bytes(L, D))
+    return launch_resident<D, T, true, true>(q, k, v, out, BN, heads, L, scale, lds, st);
+  if constexpr (D >= 128) {
+    if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
+      return launch_wide_attn<D, true, true>(q, k, v, out, BN, heads, L, scale, st);
+  }
+  return launch_tiled_as<D, T, true, false, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+}
+
+template <int DG>
+int launch_operands_small(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
+                          int L, float scale, DropoutArgs da, hipStream_t st) {
+  typedef _Float16 T;
+  if (da.p > 0.f)
+    return launch_tiled_as<64, T, true, true, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+  return launch_tiled_as<64, T, true, false, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+}
+
 }  // namespace
+
+int launch_flash_attn_operands(const void* q, const void* k, const void* v, void* out, int64_t B,
+                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st) {
+  const int64_t BN = B * N;
+  if (BN > 0x7fffffffll || L > (1 << 24)) {
+    set_error("flash_attn: B*N=%lld or L=%lld beyond the grid limits", (long long)BN, (long long)L);
+    return -2;
+  }
+  const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
+  switch (d) {
+    case 16: return launch_operands_small<16>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    case 32: return launch_operands_small<32>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    case 64: return launch_operands_d<64>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    case 128: return launch_operands_d<128>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    case 256: return launch_operands_d<256>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    default:
+      set_error("flash_attn: head size %d not built (16, 32, 64, 128 and 256 are)", d);
+      return -2;
+  }
+}
 
 int launch_flash_attn(const void* q, const void* k, const void* v, void* out, int64_t B,
                       int64_t N, int64_t L, int64_t Lk, int d, float scale, Dropout drop,

@@ -320,7 +320,8 @@ __device__ __forceinline__ void store_wave_tile32(f4 (&acc)[2 * NB][2 * MB], con
   }
 }
 
-template <int WM, int WN, typename T, bool QKV>
+// T: type of the bias.  OT: type of the output (fp16, or T).
+template <int WM, int WN, typename T, typename OT, bool QKV>
 __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const _Float16* __restrict__ A, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep) {
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
   constexpr int A_IT = 4, B_IT = 4, LPT = A_IT + B_IT;  // 16-byte loads per thread per k-tile
   constexpr int STAGE = (BM + BN) * ROWB;               // 64 KB
   constexpr int SLABS = 2 * STAGE;                      // epilogue slabs start behind the stages
-  constexpr bool HALF_SLABS = sizeof(T) == 2;           // fp16 output: store_wave_tile_h
+  constexpr bool HALF_SLABS = sizeof(OT) == 2;          // fp16 output: store_wave_tile_h
   constexpr int EPI_STORES = HALF_SLABS ? MB * NB * 2 : MB * NB * 4;  // stores per lane per epilogue
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -578,8 +579,8 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
         if (ep.gelu) store_wave_tile_h<MB, NB, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
         else store_wave_tile_h<MB, NB, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
       } else {
-        if (ep.gelu) store_wave_tile32<MB, NB, T, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
-        else store_wave_tile32<MB, NB, T, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
+        if (ep.gelu) store_wave_tile32<MB, NB, OT, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
+        else store_wave_tile32<MB, NB, OT, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
       }
     }
     if (!has_next) break;
@@ -900,10 +901,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
   }
 }
 
-template <int WM, int WN, typename T, bool QKV>
+template <int WM, int WN, typename T, typename OT, bool QKV>
 int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                   hipStream_t st) {
-  auto kern = gemm_stream_kernel<WM, WN, T, QKV>;
+  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV>;
   constexpr int smem = 2 * 512 * 128 + 8 * 4096;  // 160 KB: two stages + the epilogue slabs
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -968,13 +969,13 @@ inline float stream_cost(int64_t tiles, int Kp, bool res, int cus) {
 // the cost model says is the fastest; the rows that are left follow in a launch of the tile kernel.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, no dropout.
-template <typename T, bool QKV>
+template <typename T, typename OT, bool QKV>
 int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                  hipStream_t st) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool persistent =
       M >= 256 && N >= 256 && N % 64 == 0 && Kp >= (res ? 192 : 128) && Kp <= (1 << 21) && ep.vec_ok &&
-      (sizeof(T) == 4 || ep.vec8_ok) && !(ep.drop.p > 0.f) &&
+      (sizeof(OT) == 4 || ep.vec8_ok) && !(ep.drop.p > 0.f) &&
       (!res || (sizeof(T) == 2 && (((uintptr_t)ep.residual) & 15) == 0));
   int64_t m_head = 0;
   if (persistent) {
@@ -998,19 +999,19 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
     int rc;
     if constexpr (sizeof(T) == 2 && !QKV)
       rc = res ? launch_stream_res(A, Bt, m_head, N, Kp, ep, st)
-               : launch_stream<2, 4, T, QKV>(A, Bt, m_head, N, Kp, ep, st);
+               : launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
     else
-      rc = launch_stream<2, 4, T, QKV>(A, Bt, m_head, N, Kp, ep, st);
+      rc = launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
     if (rc != 0 || m_head == M) return rc;
   }
   EpiDev tail = ep;
   if (QKV) tail.m_off = ep.m_off + (int)m_head;
   else {
-    tail.out = (T*)ep.out + m_head * N;
+    tail.out = (OT*)ep.out + m_head * N;
     if (res) tail.residual = (const T*)ep.residual + m_head * N;
   }
   return launch_gemm_tile((const _Float16*)A + m_head * Kp, Bt, M - m_head, N, Kp, tail, sizeof(T) == 2,
-                          QKV, st);
+                          sizeof(OT) == 2, QKV, st);
 }
 
 }  // namespace
@@ -1044,10 +1045,11 @@ static int make_epi(const GemmEpilogue& e, int64_t M, int N, EpiDev& ep) {
                    aligned(e.q) && aligned(e.k) && aligned(e.v);
   ep.vec_ok = vec ? 1 : 0;
   auto aligned16 = [&](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  const int cw = e.f16 ? 8 : 4;
+  const bool half_out = e.f16 || e.out_f16;
+  const int cw = half_out ? 8 : 4;
   ep.tile_vec = N % cw == 0 && (!e.qkv || e.d % cw == 0) && aligned16(e.bias) && aligned16(e.residual) &&
                 aligned16(e.out) && aligned16(e.q) && aligned16(e.k) && aligned16(e.v);
-  ep.vec8_ok = vec && e.f16 && (N % 8) == 0 && aligned16(e.out) && aligned16(e.q) &&
+  ep.vec8_ok = vec && half_out && (N % 8) == 0 && aligned16(e.out) && aligned16(e.q) &&
                aligned16(e.k) && aligned16(e.v) && (!e.qkv || (e.d % 8) == 0);
   return 0;
 }
@@ -1057,10 +1059,13 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp, const G
   EpiDev ep;
   if (const int rc = make_epi(e, M, N, ep)) return rc;
   if (e.f16)
-    return e.qkv ? launch_shape<_Float16, true>(A, Bt, M, N, Kp, ep, st)
-                 : launch_shape<_Float16, false>(A, Bt, M, N, Kp, ep, st);
-  return e.qkv ? launch_shape<float, true>(A, Bt, M, N, Kp, ep, st)
-               : launch_shape<float, false>(A, Bt, M, N, Kp, ep, st);
+    return e.qkv ? launch_shape<_Float16, _Float16, true>(A, Bt, M, N, Kp, ep, st)
+                 : launch_shape<_Float16, _Float16, false>(A, Bt, M, N, Kp, ep, st);
+  if (e.out_f16)
+    return e.qkv ? launch_shape<float, _Float16, true>(A, Bt, M, N, Kp, ep, st)
+                 : launch_shape<float, _Float16, false>(A, Bt, M, N, Kp, ep, st);
+  return e.qkv ? launch_shape<float, float, true>(A, Bt, M, N, Kp, ep, st)
+               : launch_shape<float, float, false>(A, Bt, M, N, Kp, ep, st);
 }
 
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,

@@ -190,7 +190,7 @@ inline int cu_count() {
 // One workgroup per output tile (gemm_tile.hip), every size, type and epilogue; the LayerNorm
 // prologue form of it; and what the cost model says a launch takes, in microseconds.
 int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
-                     bool f16, bool qkv, hipStream_t st);
+                     bool f16, bool out_f16, bool qkv, hipStream_t st);
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
                                const LnArgs& ln, bool qkv, hipStream_t st);
 float gemm_tile_cost(int64_t M, int N, int Kp, int cus);

@@ -135,9 +135,10 @@ struct Tile {
   static constexpr int THREADS = 64 * WM_ * WN_ * WK_;
 };
 
-// T: storage type of bias, residual and output (and of x with LNA).
+// T: storage type of bias and residual (and of x with LNA).  OT: type of the output: T, or fp16 for
+// fp32 storage where the output is the next product's operand (no residual then).
 // WIDE: rows of 2^22 elements and more (64-bit lane addresses).
-template <class C, typename T, bool QKV, bool LNA, bool DROP, bool WIDE>
+template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     const void* __restrict__ Av, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep, LnArgs ln) {
@@ -269,10 +270,11 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   // ---- bias and residual of the chunks this thread will store, requested behind the first k-steps
   // (the counted waits of the loop then wait for these too, once, and otherwise for no more than
   // they name; at the end of the loop they would cost a memory round trip of their own)
-  constexpr int CW = 16 / (int)sizeof(T);  // output columns per 16 bytes
+  constexpr int CW = 16 / (int)sizeof(OT);  // output columns per 16 bytes
   constexpr int CPR = BN / CW, CHUNKS = BM * CPR, IT = (CHUNKS + NT - 1) / NT;
   static_assert(NT % CPR == 0, "a thread keeps its columns");
   typedef T TV __attribute__((ext_vector_type(CW)));
+  typedef OT OV __attribute__((ext_vector_type(CW)));
   const int cc = tid % CPR, n = n0 + cc * CW, r_first = tid / CPR;
   constexpr int RSTEP = NT / CPR;
   const bool col_ok = n < N && (CHUNKS >= NT || tid < CHUNKS);
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
 #pragma unroll
   for (int e = 0; e < CW; ++e) bias_v[e] = (T)0.f;
   if (ep.bias && col_ok) bias_v = load_chunk((const T*)ep.bias + n);
-  const bool res = !QKV && ep.residual != nullptr;
+  const bool res = !QKV && sizeof(T) == sizeof(OT) && ep.residual != nullptr;
   if (res && col_ok) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
@@ -374,8 +376,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   __syncthreads();
   if (!col_ok) return;
 
-  T* col = nullptr;  // head-major scatter: row 0 of batch 0 at this thread's columns
-  if constexpr (QKV) col = qkv_column_base<T>(ep, n);
+  OT* col = nullptr;  // head-major scatter: row 0 of batch 0 at this thread's columns
+  if constexpr (QKV) col = qkv_column_base<OT>(ep, n);
   const int64_t batch_stride = (int64_t)ep.heads * ep.L * ep.d;
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -402,17 +404,17 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
       for (int e = 0; e < CW; ++e) off[e] = (unsigned)((uint64_t)m * (uint64_t)N + (uint64_t)(n + e));
       dropout_apply<CW>(ep.drop, off, z);
     }
-    TV o;
+    OV o;
 #pragma unroll
-    for (int e = 0; e < CW; ++e) o[e] = (T)(res ? z[e] + (float)res_v[it][e] : z[e]);
-    T* dst;
+    for (int e = 0; e < CW; ++e) o[e] = (OT)(res ? z[e] + (float)res_v[it][e] : z[e]);
+    OT* dst;
     if constexpr (QKV) {
       const unsigned mt = (unsigned)(m + ep.m_off), b = mt / (unsigned)ep.L, l = mt - b * (unsigned)ep.L;
       dst = col + ((int64_t)b * batch_stride + (int64_t)l * ep.d);
     } else {
-      dst = (T*)ep.out + ((int64_t)m * N + n);
+      dst = (OT*)ep.out + ((int64_t)m * N + n);
     }
-    if (vec) *reinterpret_cast<TV*>(dst) = o;
+    if (vec) *reinterpret_cast<OV*>(dst) = o;
     else {
 #pragma unroll
       for (int e = 0; e < CW; ++e)
@@ -421,10 +423,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   }
 }
 
-template <class C, typename T, bool QKV, bool LNA, bool DROP, bool WIDE = false>
+template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE = false>
 int launch_tile_cfg(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                     const LnArgs& ln, hipStream_t st) {
-  auto kern = gemm_tile_kernel<C, T, QKV, LNA, DROP, WIDE>;
+  auto kern = gemm_tile_kernel<C, T, OT, QKV, LNA, DROP, WIDE>;
   constexpr int stages = C::NST * ((LNA ? 0 : C::BM) + C::BN) * 128 * C::WK, sums = C::BM * C::BN * 4 * C::WK;
   static_assert(stages <= 160 * 1024 && sums <= 160 * 1024, "LDS");
   const size_t panel = LNA ? (size_t)C::BM * Kp * 2 : 0;
@@ -494,19 +496,19 @@ inline int pick_tile(int64_t M, int N, int Kp, int cus, float* cost) {
   return best;
 }
 
-template <typename T, bool QKV, bool DROP>
+template <typename T, typename OT, bool QKV, bool DROP>
 int launch_pick(int i, const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                 hipStream_t st) {
   const LnArgs ln = {};
   switch (i) {
-    case 0: return launch_tile_cfg<T32x16, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 1: return launch_tile_cfg<T32x32, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 2: return launch_tile_cfg<T64x32, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 3: return launch_tile_cfg<T64x64, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 4: return launch_tile_cfg<T64x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 5: return launch_tile_cfg<T128x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 6: return launch_tile_cfg<T192x128, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    default: return launch_tile_cfg<T128x256, T, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 0: return launch_tile_cfg<T32x16, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 1: return launch_tile_cfg<T32x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 2: return launch_tile_cfg<T64x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 3: return launch_tile_cfg<T64x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 4: return launch_tile_cfg<T64x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 5: return launch_tile_cfg<T128x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 6: return launch_tile_cfg<T192x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    default: return launch_tile_cfg<T128x256, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
   }
 }
 
@@ -521,7 +523,7 @@ float gemm_tile_cost(int64_t M, int N, int Kp, int cus) {
   return cost;
 }
 
-template <typename T, bool QKV>
+template <typename T, typename OT, bool QKV>
 static int launch_tile_t(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                          hipStream_t st) {
   const int cus = cu_count();
@@ -529,22 +531,25 @@ static int launch_tile_t(const void* A, const void* Bt, int64_t M, int N, int Kp
   if constexpr (!QKV) {
     if (ep.drop.p > 0.f) {
       if (Kp >= kWideK)
-        return launch_tile_cfg<T32x32, T, false, false, true, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
-      return launch_pick<T, false, true>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+        return launch_tile_cfg<T32x32, T, OT, false, false, true, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+      return launch_pick<T, OT, false, true>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
     }
   }
   if (Kp >= kWideK)
-    return launch_tile_cfg<T32x32, T, QKV, false, false, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
-  return launch_pick<T, QKV, false>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+    return launch_tile_cfg<T32x32, T, OT, QKV, false, false, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+  return launch_pick<T, OT, QKV, false>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
 }
 
 int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
-                     bool f16, bool qkv, hipStream_t st) {
+                     bool f16, bool out_f16, bool qkv, hipStream_t st) {
   if (f16)
-    return qkv ? launch_tile_t<_Float16, true>(A, Bt, M, N, Kp, ep, st)
-               : launch_tile_t<_Float16, false>(A, Bt, M, N, Kp, ep, st);
-  return qkv ? launch_tile_t<float, true>(A, Bt, M, N, Kp, ep, st)
-             : launch_tile_t<float, false>(A, Bt, M, N, Kp, ep, st);
+    return qkv ? launch_tile_t<_Float16, _Float16, true>(A, Bt, M, N, Kp, ep, st)
+               : launch_tile_t<_Float16, _Float16, false>(A, Bt, M, N, Kp, ep, st);
+  if (out_f16)
+    return qkv ? launch_tile_t<float, _Float16, true>(A, Bt, M, N, Kp, ep, st)
+               : launch_tile_t<float, _Float16, false>(A, Bt, M, N, Kp, ep, st);
+  return qkv ? launch_tile_t<float, float, true>(A, Bt, M, N, Kp, ep, st)
+             : launch_tile_t<float, float, false>(A, Bt, M, N, Kp, ep, st);
 }
 
 // ---- LayerNorm prologue ----------------------------------------------------------------------
@@ -563,9 +568,9 @@ int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiD
   const int cus = cu_count();
   if (cus < 0) return cus;
   switch (kTiles[pick_tile(M, N, K, cus, nullptr)].wk) {
-    case 4: return launch_tile_cfg<Ln32x32, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    case 2: return launch_tile_cfg<Ln32x64, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    default: return launch_tile_cfg<Ln32x128, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 4: return launch_tile_cfg<Ln32x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 2: return launch_tile_cfg<Ln32x64, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    default: return launch_tile_cfg<Ln32x128, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
   }
 }
 }  // namespace

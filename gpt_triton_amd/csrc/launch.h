@@ -17,8 +17,9 @@ int launch_embed(const int64_t* ids, const void* wte, const void* wpe, void* out
 bool launch_embed_layernorm(const int64_t* ids, const void* wte, const void* wpe, const void* w,
                             const void* b, void* emb, void* out, int64_t rows, int64_t L,
                             int64_t V, int H, float eps, bool f16, hipStream_t st);
+// out_f16 with fp32 rows: the result rounded to fp16, as the GEMM rounds its operands
 int launch_layernorm(const void* x, const void* w, const void* b, void* out,
-                     int64_t M, int H, float eps, bool f16, hipStream_t st);
+                     int64_t M, int H, float eps, bool f16, bool out_f16, hipStream_t st);
 int launch_softmax(const void* x, void* out, int64_t M, int H, bool f16,
                    hipStream_t st);
 void launch_pack_rows(const void* src, void* dst, int64_t R, int K, int Kp, bool f16,
@@ -42,6 +43,7 @@ struct GemmEpilogue {
   Dropout drop;   // after the GELU, before the residual (plain mode only)
   bool qkv;       // scatter mode
   bool f16;       // storage dtype of bias / residual / outputs
+  bool out_f16;   // fp32 storage: outputs rounded to fp16 all the same (the next product's operand)
 };
 
 // C[M][N] = A[M][Kp] . Bt[N][Kp]^T with fp16 operands (Kp % 64 == 0), fp32
@@ -63,5 +65,13 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
 int launch_flash_attn(const void* q, const void* k, const void* v, void* out,
                       int64_t B, int64_t N, int64_t L, int64_t Lk, int d, float scale,
                       Dropout drop, bool out_blnd, bool f16, hipStream_t st);
+
+
+// The attention of an fp32 model on fp16 copies of q, k, v: the fp32 kernels round q, k and v to fp16
+// as they read them, and the projection rounds its operand, so with the copies written by the product
+// in front and the output rounded here the values are the same and half the bytes move.  fp32 softmax
+// arithmetic as for fp32 storage; equal lengths; out [B][L][N][d] fp16.
+int launch_flash_attn_operands(const void* q, const void* k, const void* v, void* out, int64_t B,
+                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st);
 
 }  // namespace gptmi

@@ -96,11 +96,14 @@ __global__ __launch_bounds__(256) void embed_dropout_kernel(
 // quarter of them idle in the second pass -- and twice the rows are in flight per wavefront
 // (LayerNorm at the headline: 89 -> 74 us).  The launchers pick 32 when that wastes fewer lanes.
 // ---------------------------------------------------------------------------
-template <typename T, int CH, int LPR>
+// OT: type of the output.  fp32 rows may be emitted as fp16, the rounding of a GEMM operand (the
+// block functions of fp32 models: the operand is written at once instead of by a pack pass).
+template <typename T, int CH, int LPR, typename OT = T>
 __global__ __launch_bounds__(256) void layernorm_vec_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ b,
-    T* __restrict__ out, int64_t M, int H, float eps) {
+    OT* __restrict__ out, int64_t M, int H, float eps) {
   typedef typename Vec<T>::type V;
+  typedef OT OV __attribute__((ext_vector_type(Vec<T>::N)));
   constexpr int VN = Vec<T>::N;
   const int lane = threadIdx.x & (LPR - 1);
   const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
   }
   float mean, rstd;
   layernorm_stats<CH, VN, LPR>(v, s, lane, nchunks, H, eps, mean, rstd);
-  V* o = reinterpret_cast<V*>(out + row * H);
+  OV* o = reinterpret_cast<OV*>(out + row * H);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = lane + i * LPR;
@@ -142,10 +145,10 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
         tw[i] = wv[c];
         tb[i] = bv[c];
       }
-      V to;
+      OV to;
 #pragma unroll
       for (int j = 0; j < VN; ++j)
-        to[j] = (T)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+        to[j] = (OT)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
       // cached (not streaming) store: the [T, H] output is what the following GEMM reads, two
       // or three times over; it fits the 256 MB memory-side cache, and a GEMM fed from there
       // instead of HBM ran 12 % faster (its operand loads are only one k-tile ahead)
@@ -217,10 +220,10 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
 }
 
 // Any H (no alignment requirement): the row is re-read from cache per pass.
-template <typename T>
+template <typename T, typename OT = T>
 __global__ __launch_bounds__(256) void layernorm_scalar_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ b,
-    T* __restrict__ out, int64_t M, int H, float eps) {
+    OT* __restrict__ out, int64_t M, int H, float eps) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;
@@ -237,7 +240,7 @@ __global__ __launch_bounds__(256) void layernorm_scalar_kernel(
   const float rstd = 1.0f / sqrtf(var + eps);
   for (int c = lane; c < H; c += 64) {
     const float z = ((float)xr[c] - mean) * rstd;
-    out[row * H + c] = (T)(z * (float)w[c] + (float)b[c]);
+    out[row * H + c] = (OT)(z * (float)w[c] + (float)b[c]);
   }
 }
 
@@ -321,6 +324,33 @@ __global__ __launch_bounds__(256) void softmax_scalar_kernel(const T* __restrict
 //   pack_rows:      src[R][K]  -> dst[R][Kp]   (x, or a weight given as [N][K])
 //   pack_transpose: src[K][N]  -> dst[N][Kp]   (weight given as [K][N])
 // ---------------------------------------------------------------------------
+// Rows whose length is a multiple of 8 (so that a chunk of 8 never leaves its row) from a 16-byte
+// aligned source: a thread converts 8 elements, 16 bytes out (32 x 300 x 768 floats: 61 us with an
+// element and a 64-bit division per thread).
+template <typename T>
+__global__ __launch_bounds__(256) void pack_rows_vec_kernel(const T* __restrict__ src,
+                                                            _Float16* __restrict__ dst,
+                                                            int64_t R, unsigned K8, unsigned Kp8) {
+  typedef T V __attribute__((ext_vector_type(8)));
+  const unsigned rows_per = 256 / Kp8 ? 256 / Kp8 : 1;  // rows a workgroup turn covers
+  const unsigned lane_row = Kp8 <= 256 ? threadIdx.x / Kp8 : 0;
+  const unsigned c0 = Kp8 <= 256 ? threadIdx.x - lane_row * Kp8 : threadIdx.x;
+  if (lane_row >= rows_per) return;
+  for (int64_t r = (int64_t)blockIdx.x * rows_per + lane_row; r < R; r += (int64_t)gridDim.x * rows_per)
+    for (unsigned c = c0; c < Kp8; c += 256) {
+      h8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (_Float16)0.f;
+      if (c < K8) {
+        const V v = *reinterpret_cast<const V*>(src + (r * K8 + c) * 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = (_Float16)(float)v[j];
+      }
+      *reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8) = o;
+    }
+}
+
+// Any row length: an element per thread.
 template <typename T>
 __global__ __launch_bounds__(256) void pack_rows_kernel(const T* __restrict__ src,
                                                         _Float16* __restrict__ dst,
@@ -392,20 +422,20 @@ int launch_embed(const int64_t* ids, const void* wte, const void* wpe, void* out
              : launch_embed_t<float>(ids, wte, wpe, out, rows, L, V, H, drop, st);
 }
 
-template <typename T, int CH>
+template <typename T, typename OT, int CH>
 static void ln_go(const void* x, const void* w, const void* b, void* out, int64_t M,
                   int H, float eps, int lpr, hipStream_t st) {
   if (lpr == 32)
-    hipLaunchKernelGGL((layernorm_vec_kernel<T, CH, 32>), dim3((unsigned)((M + 7) / 8)),
+    hipLaunchKernelGGL((layernorm_vec_kernel<T, CH, 32, OT>), dim3((unsigned)((M + 7) / 8)),
                        dim3(256), 0, st, (const T*)x, (const T*)w, (const T*)b,
-                       (T*)out, M, H, eps);
+                       (OT*)out, M, H, eps);
   else
-    hipLaunchKernelGGL((layernorm_vec_kernel<T, CH, 64>), dim3((unsigned)((M + 3) / 4)),
+    hipLaunchKernelGGL((layernorm_vec_kernel<T, CH, 64, OT>), dim3((unsigned)((M + 3) / 4)),
                        dim3(256), 0, st, (const T*)x, (const T*)w, (const T*)b,
-                       (T*)out, M, H, eps);
+                       (OT*)out, M, H, eps);
 }
 
-template <typename T>
+template <typename T, typename OT>
 static int launch_layernorm_t(const void* x, const void* w, const void* b, void* out,
                               int64_t M, int H, float eps, hipStream_t st) {
   constexpr int VN = Vec<T>::N;
@@ -414,24 +444,25 @@ static int launch_layernorm_t(const void* x, const void* w, const void* b, void*
                        ((uintptr_t)out % 16) == 0;
   const int lpr = lanes_per_row(H / VN);
   const int need = aligned ? (H / VN + lpr - 1) / lpr : 1 << 30;
-  if (need <= 1) ln_go<T, 1>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 2) ln_go<T, 2>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 3) ln_go<T, 3>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 4) ln_go<T, 4>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 8) ln_go<T, 8>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 16) ln_go<T, 16>(x, w, b, out, M, H, eps, lpr, st);
-  else if (need <= 32) ln_go<T, 32>(x, w, b, out, M, H, eps, lpr, st);
+  if (need <= 1) ln_go<T, OT, 1>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 2) ln_go<T, OT, 2>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 3) ln_go<T, OT, 3>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 4) ln_go<T, OT, 4>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 8) ln_go<T, OT, 8>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 16) ln_go<T, OT, 16>(x, w, b, out, M, H, eps, lpr, st);
+  else if (need <= 32) ln_go<T, OT, 32>(x, w, b, out, M, H, eps, lpr, st);
   else
-    hipLaunchKernelGGL(layernorm_scalar_kernel<T>, dim3((unsigned)((M + 3) / 4)),
+    hipLaunchKernelGGL((layernorm_scalar_kernel<T, OT>), dim3((unsigned)((M + 3) / 4)),
                        dim3(256), 0, st, (const T*)x, (const T*)w, (const T*)b,
-                       (T*)out, M, H, eps);
+                       (OT*)out, M, H, eps);
   return 0;
 }
 
 int launch_layernorm(const void* x, const void* w, const void* b, void* out,
-                     int64_t M, int H, float eps, bool f16, hipStream_t st) {
-  return f16 ? launch_layernorm_t<_Float16>(x, w, b, out, M, H, eps, st)
-             : launch_layernorm_t<float>(x, w, b, out, M, H, eps, st);
+                     int64_t M, int H, float eps, bool f16, bool out_f16, hipStream_t st) {
+  if (f16) return launch_layernorm_t<_Float16, _Float16>(x, w, b, out, M, H, eps, st);
+  return out_f16 ? launch_layernorm_t<float, _Float16>(x, w, b, out, M, H, eps, st)
+                 : launch_layernorm_t<float, float>(x, w, b, out, M, H, eps, st);
 }
 
 template <typename T, int CH>
@@ -516,17 +547,25 @@ bool launch_embed_layernorm(const int64_t* ids, const void* wte, const void* wpe
                                                st);
 }
 
+template <typename T>
+static void launch_pack_rows_t(const T* src, _Float16* dst, int64_t R, int K, int Kp, hipStream_t st) {
+  if (K % 8 == 0 && ((uintptr_t)src & 15) == 0) {
+    const int64_t rows_per = 256 / (Kp / 8) ? 256 / (Kp / 8) : 1;
+    int64_t blocks = (R + rows_per - 1) / rows_per;
+    if (blocks > 16384) blocks = 16384;
+    hipLaunchKernelGGL(pack_rows_vec_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, dst, R,
+                       (unsigned)(K / 8), (unsigned)(Kp / 8));
+    return;
+  }
+  int64_t blocks = (R * (int64_t)Kp + 255) / 256;
+  if (blocks > 65536) blocks = 65536;
+  hipLaunchKernelGGL(pack_rows_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, dst, R, K, Kp);
+}
+
 void launch_pack_rows(const void* src, void* dst, int64_t R, int K, int Kp, bool f16,
                       hipStream_t st) {
-  const int64_t total = R * (int64_t)Kp;
-  int64_t blocks = (total + 255) / 256;
-  if (blocks > 65536) blocks = 65536;
-  if (f16)
-    hipLaunchKernelGGL(pack_rows_kernel<_Float16>, dim3((unsigned)blocks), dim3(256),
-                       0, st, (const _Float16*)src, (_Float16*)dst, R, K, Kp);
-  else
-    hipLaunchKernelGGL(pack_rows_kernel<float>, dim3((unsigned)blocks), dim3(256), 0,
-                       st, (const float*)src, (_Float16*)dst, R, K, Kp);
+  if (f16) launch_pack_rows_t((const _Float16*)src, (_Float16*)dst, R, K, Kp, st);
+  else launch_pack_rows_t((const float*)src, (_Float16*)dst, R, K, Kp, st);
 }
 
 void launch_pack_transpose(const void* src, void* dst, int K, int N, int Kp, bool f16,

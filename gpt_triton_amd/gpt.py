@@ -21,24 +21,37 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 
-from .kernels import (flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
+from .kernels import (HEAD_SIZES, attention_block, block_supported, flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
                       fused_layer_norm, layer_norm_ffn, layer_norm_linear_supported,
-                      layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, pack_lm_head,
-                      pack_weight)
+                      layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, mlp_block,
+                      pack_lm_head, pack_weight)
 
 # Up to this many token rows the blocks run their LayerNorm inside the following GEMM
-# (layer_norm_ffn, layer_norm_matmul_and_split_qkv: one launch instead of two, same bits): such
-# a forward is bound by its launches.  Above, the LayerNorm kernel and the big-tile GEMMs are
-# faster -- the fused form normalises a row block once per column tile and runs on small tiles --
-# and so are the two launches inside a captured graph, where a launch costs next to nothing.
-LN_PROLOGUE_MAX_ROWS = 1024
+# (layer_norm_ffn, layer_norm_in_gemm: one launch instead of two, same bits): such a forward is bound
+# by its launches.  Above, the LayerNorm kernel and the larger tiles are faster -- the fused form
+# normalises a row block once per column tile -- and so are the two launches inside a captured graph,
+# where a launch costs next to nothing.
+LN_PROLOGUE_MAX_ROWS = 128
 LN_PROLOGUE_UNDER_CAPTURE = False  # measurement switch (bench.py --ln-prologue-under-capture)
+
+# Up to this many token rows a block is one call of the library (attention_block, mlp_block) instead
+# of one per operator: below about 4000 rows of the 124M model the host, not the GPU, sets the pace of
+# an operator-by-operator forward (some 10 us per operator against 2 us per launch inside one call).
+# Above, the calls hide behind the GPU.  fp32 models take the block calls at every size: their
+# intermediate matrices are fp16 there (see gptmi_attention_block).
+BLOCK_MAX_ROWS = 8192
 
 
 def _ln_in_gemm(x, weight):
     return (x.numel() // x.shape[-1] <= LN_PROLOGUE_MAX_ROWS and
             layer_norm_linear_supported(x, weight) and
             (LN_PROLOGUE_UNDER_CAPTURE or not torch.cuda.is_current_stream_capturing()))
+
+
+def _as_block(x, width):
+    return ((x.dtype == torch.float32 or x.numel() // width <= BLOCK_MAX_ROWS) and
+            block_supported(x, width))
+
 
 # dense fp16/bf16 tensor throughput, FLOP/s
 GPU_TO_FLOPS = {
@@ -59,12 +72,12 @@ class _PackedWeights:
         self._entries = {}
 
     def get(self, name, param, pack=pack_weight):
-        key = (param.data_ptr(), param._version, param.dtype, tuple(param.shape))
         hit = self._entries.get(name)
-        if hit is None or hit[0] != key:
-            hit = (key, pack(param.data))
+        if (hit is None or hit[0] != param.data_ptr() or hit[1] != param._version or
+                hit[2] != param.dtype or hit[3] != param.shape):
+            hit = (param.data_ptr(), param._version, param.dtype, param.shape, pack(param.data))
             self._entries[name] = hit
-        return hit[1]
+        return hit[4]
 
     def clear(self):
         self._entries.clear()
@@ -97,7 +110,7 @@ class FusedAttention(nn.Module):
         self._packed = _PackedWeights()
 
     def _weight(self, name):
-        prm = getattr(self, name)
+        prm = self._parameters[name]
         if self.training or (self.hidden_size // self.num_heads) % 8 != 0:
             return prm.data
         return self._packed.get(name, prm)
@@ -110,21 +123,28 @@ class FusedAttention(nn.Module):
         """`normed`: LayerNorm(x) with this block's weights, if the caller already has it (the
         first block of FusedGPT gets it from the embedding kernel)."""
         p = self.dropout_prob if self.training else 0.0
+        prm = self._parameters
+        w_attn = self._weight("c_attn_weight")
+        in_gemm = normed is None and p == 0.0 and _ln_in_gemm(x, w_attn)
+        if _as_block(x, self.hidden_size) and self.hidden_size // self.num_heads in HEAD_SIZES:
+            return attention_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w_attn,
+                                   prm["c_attn_bias"], self._weight("c_proj_weight"),
+                                   prm["c_proj_bias"], self.num_heads, dropout_prob=p,
+                                   normed=normed, layer_norm_in_gemm=in_gemm)
         skip = x
         y = normed
-        w_attn = self._weight("c_attn_weight")
-        if y is None and p == 0.0 and _ln_in_gemm(x, w_attn):
-            q, k, v = layer_norm_matmul_and_split_qkv(x, self.layer_norm_weight.data,
-                                                      self.layer_norm_bias.data, w_attn,
-                                                      self.c_attn_bias.data, self.num_heads)
+        if in_gemm:
+            q, k, v = layer_norm_matmul_and_split_qkv(x, prm["layer_norm_weight"].data,
+                                                      prm["layer_norm_bias"].data, w_attn,
+                                                      prm["c_attn_bias"].data, self.num_heads)
         else:
             if y is None:
-                y = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)
-            q, k, v = matmul_and_split_qkv(y, w_attn, self.c_attn_bias.data, self.num_heads)
+                y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
+            q, k, v = matmul_and_split_qkv(y, w_attn, prm["c_attn_bias"].data, self.num_heads)
         # [B, N, L, d] values in a [B, L, N, d] buffer: the head merge below copies nothing
         y = flash_attention_v1(q, k, v, dropout_prob=p, merged_heads_layout=True)
         y = y.transpose(1, 2).contiguous().view(skip.shape)
-        return fused_ffn(y, self._weight("c_proj_weight"), bias=self.c_proj_bias.data,
+        return fused_ffn(y, self._weight("c_proj_weight"), bias=prm["c_proj_bias"].data,
                          residual=skip, add_gelu=False, dropout_prob=p)
 
     def get_fwd_flops(self, num_tokens):
@@ -151,7 +171,7 @@ class FusedMLP(nn.Module):
         self._packed = _PackedWeights()
 
     def _weight(self, name):
-        prm = getattr(self, name)
+        prm = self._parameters[name]
         return prm.data if self.training else self._packed.get(name, prm)
 
     def train(self, mode=True):
@@ -160,17 +180,20 @@ class FusedMLP(nn.Module):
 
     def forward(self, x):
         p = self.dropout_prob if self.training else 0.0
-        skip = x
-        w1 = self._weight("ffn1_weight")
+        prm = self._parameters
+        w1, w2 = self._weight("ffn1_weight"), self._weight("ffn2_weight")
         if p == 0.0 and _ln_in_gemm(x, w1):
-            y = layer_norm_ffn(x, self.layer_norm_weight.data, self.layer_norm_bias.data, w1,
-                               bias=self.ffn1_bias.data, add_gelu=True)
+            y = layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
+                               bias=prm["ffn1_bias"], add_gelu=True)
+        elif _as_block(x, self.hidden_size):
+            return mlp_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
+                             prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p)
         else:
-            y = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)
-            y = fused_ffn(y, w1, bias=self.ffn1_bias.data, residual=None, add_gelu=True,
+            y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
+            y = fused_ffn(y, w1, bias=prm["ffn1_bias"].data, residual=None, add_gelu=True,
                           dropout_prob=p)
-        return fused_ffn(y, self._weight("ffn2_weight"), bias=self.ffn2_bias.data, residual=skip,
-                         add_gelu=False, dropout_prob=p)
+        return fused_ffn(y, w2, bias=prm["ffn2_bias"].data, residual=x, add_gelu=False,
+                         dropout_prob=p)
 
     def get_fwd_flops(self, num_tokens):
         h, mid = self.hidden_size, self.intermediate_size
@@ -224,19 +247,20 @@ class FusedGPT(nn.Module):
     def forward(self, x, return_logits=False):
         # causal by construction; no attention or padding mask is taken
         p = self.config.dropout if self.training else 0.0
-        if p == 0.0 and len(self.blocks) > 0:
+        blocks = list(self.blocks)
+        if p == 0.0 and blocks:
             # eval mode: the first block's LayerNorm comes out of the embedding kernel.  The two
             # modules of blocks[0] are called one by one, so forward hooks registered on that
             # nn.Sequential container itself do not fire (hooks on its two modules do).
-            first = self.blocks[0]
+            first = blocks[0]
             x, y = fused_embeddings_layer_norm(x, self.wte_weight.data, self.wpe_weight.data,
                                                first[0].layer_norm_weight.data,
                                                first[0].layer_norm_bias.data)
             x = first[1](first[0](x, normed=y))
-            rest = self.blocks[1:]
+            rest = blocks[1:]
         else:
             x = fused_embeddings(x, self.wte_weight.data, self.wpe_weight.data, dropout_prob=p)
-            rest = self.blocks
+            rest = blocks
         for block in rest:
             x = block(x)
         x = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)

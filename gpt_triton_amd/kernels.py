@@ -37,50 +37,37 @@ def _dtype_code(t, what):
         raise TypeError(f"{what}: dtype {t.dtype} is not supported (float32 and float16 are)")
 
 
-def _on_gpu(*tensors):
-    dev = tensors[0].device
-    if dev.type != "cuda":
+def _on_gpu(first, *rest):
+    """Index of the GPU that all the tensors (None allowed behind the first) are on."""
+    index = first.get_device()  # -1 on the CPU
+    if index < 0:
         raise RuntimeError("gpt_triton_amd operators run on the GPU only; got a tensor on "
-                           f"{dev} (there is no CPU fallback)")
-    for t in tensors[1:]:
-        if t is not None and t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
-    return dev
+                           f"{first.device} (there is no CPU fallback)")
+    for t in rest:
+        if t is not None and t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} and {t.device}")
+    return index
 
 
-def _stream():
-    # torch's current stream on the current device as the raw hipStream_t; the direct binding
-    # costs a fraction of building a torch.cuda.Stream object per operator call
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-
-
-class _NoGuard:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_GUARD = _NoGuard()
-
-
-def _device(dev):
-    """Context in which `dev` is the current device: nothing to do (and nothing to pay per call)
-    when it already is, torch's guard otherwise."""
-    if dev.index is None or dev.index == torch._C._cuda_getDevice():
-        return _NO_GUARD
-    return torch.cuda.device(dev)
+def _call(index, what, fn, *args):
+    """One entry point of the library on torch's current stream of GPU `index`.  A forward of a few
+    tokens is bound by the host: no device guard where the GPU is the current one already, the raw
+    stream from torch's own binding instead of a torch.cuda.Stream object."""
+    if index == torch._C._cuda_getDevice():
+        rc = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(index):
+            rc = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    if rc != 0:
+        _lib.check(rc, what)
 
 
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-def _workspace(nbytes, device):
-    if nbytes == 0:
-        return None
-    return torch.empty(nbytes, dtype=torch.uint8, device=device)
+def _workspace(nbytes, like):
+    return like.new_empty(nbytes, dtype=torch.uint8) if nbytes else None
 
 
 class PackedWeight:
@@ -96,6 +83,9 @@ class PackedWeight:
     def is_contiguous(self):
         return True
 
+    def get_device(self):
+        return self.data.get_device()
+
     def data_ptr(self):
         return self.data.data_ptr()
 
@@ -108,11 +98,9 @@ def pack_weight(weight):
     dev = _on_gpu(weight)
     K_, N = weight.shape
     lib = _lib.load()
-    buf = torch.empty(lib.gptmi_packed_weight_bytes(N, K_), dtype=torch.uint8, device=dev)
-    with _device(dev):
-        rc = lib.gptmi_pack_weight(weight.data_ptr(), buf.data_ptr(), N, K_, _lib.GPTMI_W_KN,
-                                   _dtype_code(weight, "pack_weight"), _stream())
-    _lib.check(rc, "pack_weight")
+    buf = weight.new_empty(lib.gptmi_packed_weight_bytes(N, K_), dtype=torch.uint8)
+    _call(dev, "pack_weight", lib.gptmi_pack_weight, weight.data_ptr(), buf.data_ptr(), N, K_,
+          _lib.GPTMI_W_KN, _dtype_code(weight, "pack_weight"))
     return PackedWeight(buf, weight.shape, weight.dtype)
 
 
@@ -128,11 +116,9 @@ def pack_lm_head(wte):
     V, H = wte.shape
     Vp = -(-V // 64) * 64
     lib = _lib.load()
-    buf = torch.zeros(lib.gptmi_packed_weight_bytes(Vp, H), dtype=torch.uint8, device=dev)
-    with _device(dev):
-        rc = lib.gptmi_pack_weight(wte.data_ptr(), buf.data_ptr(), V, H, _lib.GPTMI_W_NK,
-                                   _dtype_code(wte, "pack_lm_head"), _stream())
-    _lib.check(rc, "pack_lm_head")
+    buf = wte.new_zeros(lib.gptmi_packed_weight_bytes(Vp, H), dtype=torch.uint8)
+    _call(dev, "pack_lm_head", lib.gptmi_pack_weight, wte.data_ptr(), buf.data_ptr(), V, H,
+          _lib.GPTMI_W_NK, _dtype_code(wte, "pack_lm_head"))
     return PackedWeight(buf, (H, Vp), wte.dtype, vocab=V)
 
 
@@ -155,7 +141,6 @@ def _wlayout(weight, default):
     return _lib.GPTMI_W_PACKED if isinstance(weight, PackedWeight) else default
 
 
-@torch.no_grad()
 def fused_embeddings(x, wte, wpe, dropout_prob=0.0):
     """dropout(wte[x] + wpe[position]) for token ids x [B, L] -> [B, L, H] in wte's dtype."""
     assert wte.shape[1] == wpe.shape[1]
@@ -171,17 +156,13 @@ def fused_embeddings(x, wte, wpe, dropout_prob=0.0):
         raise TypeError("fused_embeddings: wte and wpe must share a dtype")
     dev = _on_gpu(x, wte, wpe)
     _maybe_check_ids(x, V)
-    z = torch.empty((B * L, H), device=dev, dtype=wte.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_embed(x.data_ptr(), wte.data_ptr(), wpe.data_ptr(), z.data_ptr(), B, L, V,
-                             P, H, float(dropout_prob), 1337, _dtype_code(wte, "fused_embeddings"),
-                             _stream())
-    _lib.check(rc, "fused_embeddings")
-    return z.view((B, L, H))
+    z = wte.new_empty((B, L, H))
+    _call(dev, "fused_embeddings", _lib.load().gptmi_embed, x.data_ptr(), wte.data_ptr(),
+          wpe.data_ptr(), z.data_ptr(), B, L, V, P, H, float(dropout_prob), 1337,
+          _dtype_code(wte, "fused_embeddings"))
+    return z
 
 
-@torch.no_grad()
 def fused_embeddings_layer_norm(x, wte, wpe, weight, bias):
     """(fused_embeddings(x, wte, wpe), fused_layer_norm(of that, weight, bias)) from one kernel:
     the embedding row is normalised while it is still in registers.  Both results are
@@ -203,19 +184,14 @@ def fused_embeddings_layer_norm(x, wte, wpe, weight, bias):
         raise TypeError("fused_embeddings_layer_norm: wte, wpe, weight and bias must share a dtype")
     dev = _on_gpu(x, wte, wpe, weight, bias)
     _maybe_check_ids(x, V)
-    emb = torch.empty((B * L, H), device=dev, dtype=wte.dtype)
-    out = torch.empty((B * L, H), device=dev, dtype=wte.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_embed_layernorm(x.data_ptr(), wte.data_ptr(), wpe.data_ptr(),
-                                       weight.data_ptr(), bias.data_ptr(), emb.data_ptr(),
-                                       out.data_ptr(), B, L, V, P, H, 1e-5,
-                                       _dtype_code(wte, "fused_embeddings_layer_norm"), _stream())
-    _lib.check(rc, "fused_embeddings_layer_norm")
-    return emb.view((B, L, H)), out.view((B, L, H))
+    emb = wte.new_empty((B, L, H))
+    out = wte.new_empty((B, L, H))
+    _call(dev, "fused_embeddings_layer_norm", _lib.load().gptmi_embed_layernorm, x.data_ptr(),
+          wte.data_ptr(), wpe.data_ptr(), weight.data_ptr(), bias.data_ptr(), emb.data_ptr(),
+          out.data_ptr(), B, L, V, P, H, 1e-5, _dtype_code(wte, "fused_embeddings_layer_norm"))
+    return emb, out
 
 
-@torch.no_grad()
 def fused_layer_norm(x, weight, bias):
     """LayerNorm over the last dim (eps = 1e-5, biased variance), same shape and dtype as x."""
     assert x.is_contiguous()
@@ -228,98 +204,93 @@ def fused_layer_norm(x, weight, bias):
     dev = _on_gpu(x, weight, bias)
     H = x.shape[-1]
     M = x.numel() // H
-    z = torch.empty(x.shape, device=dev, dtype=x.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_layernorm(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), z.data_ptr(), M,
-                                 H, 1e-5, _dtype_code(x, "fused_layer_norm"), _stream())
-    _lib.check(rc, "fused_layer_norm")
+    z = torch.empty_like(x)
+    _call(dev, "fused_layer_norm", _lib.load().gptmi_layernorm, x.data_ptr(), weight.data_ptr(),
+          bias.data_ptr(), z.data_ptr(), M, H, 1e-5, _dtype_code(x, "fused_layer_norm"))
     return z
 
 
-@torch.no_grad()
 def fused_softmax(x):
     """softmax over the last dim with fp32 statistics, same shape and dtype as x."""
     assert x.is_contiguous()
     dev = _on_gpu(x)
     H = x.shape[-1]
     M = x.numel() // H
-    z = torch.empty(x.shape, device=dev, dtype=x.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_softmax(x.data_ptr(), z.data_ptr(), M, H, _dtype_code(x, "fused_softmax"),
-                               _stream())
-    _lib.check(rc, "fused_softmax")
+    z = torch.empty_like(x)
+    _call(dev, "fused_softmax", _lib.load().gptmi_softmax, x.data_ptr(), z.data_ptr(), M, H,
+          _dtype_code(x, "fused_softmax"))
     return z
 
 
-def _linear(x2d, weight, bias, residual, z, gelu, dropout_prob, wlayout, what):
-    M, K = x2d.shape
-    N = z.shape[1]
-    dev = x2d.device
-    code = _dtype_code(x2d, what)
-    for name, t in (("weight", weight), ("bias", bias), ("residual", residual)):
-        if t is not None and t.dtype != x2d.dtype:
-            raise TypeError(f"{what}: {name} is {t.dtype} but x is {x2d.dtype}")
+def _linear_workspace(lib, M, N, K, code, wlayout, like):
+    """(workspace or None, its bytes).  A packed image under fp16 rows that are whole 128-byte lines
+    needs none; that is every product of an eval-mode forward, and not worth a call to be told."""
+    if wlayout == _lib.GPTMI_W_PACKED and code == _lib.GPTMI_F16 and K % 64 == 0:
+        return None, 0
+    nbytes = lib.gptmi_linear_workspace_bytes(M, N, K, code, wlayout)
+    return _workspace(nbytes, like), nbytes
+
+
+def _linear(x, weight, bias, residual, z, gelu, dropout_prob, wlayout, what):
+    K, N = x.shape[-1], z.shape[-1]
+    M = x.numel() // K
+    dtype = x.dtype
+    code = _dtype_code(x, what)
+    if weight.dtype != dtype:
+        raise TypeError(f"{what}: weight is {weight.dtype} but x is {dtype}")
+    if bias is not None and bias.dtype != dtype:
+        raise TypeError(f"{what}: bias is {bias.dtype} but x is {dtype}")
+    if residual is not None and residual.dtype != dtype:
+        raise TypeError(f"{what}: residual is {residual.dtype} but x is {dtype}")
     lib = _lib.load()
-    ws_bytes = lib.gptmi_linear_workspace_bytes(M, N, K, code, wlayout)
-    ws = _workspace(ws_bytes, dev)
-    with _device(dev):
-        rc = lib.gptmi_linear(x2d.data_ptr(), weight.data_ptr(), _ptr(bias), _ptr(residual),
-                              z.data_ptr(), M, N, K, int(bool(gelu)), float(dropout_prob), 1337,
-                              wlayout, _ptr(ws), ws_bytes, code, _stream())
-    _lib.check(rc, what)
+    ws, ws_bytes = _linear_workspace(lib, M, N, K, code, wlayout, x)
+    _call(x.get_device(), what, lib.gptmi_linear, x.data_ptr(), weight.data_ptr(), _ptr(bias),
+          _ptr(residual), z.data_ptr(), M, N, K, 1 if gelu else 0, float(dropout_prob), 1337, wlayout,
+          _ptr(ws), ws_bytes, code)
     return z
 
 
-@torch.no_grad()
 def fused_ffn(x, weight, bias=None, residual=None, add_gelu=False, dropout_prob=0.0):
     """dropout(gelu?(x @ weight + bias)) + residual; weight is [K, N] (in x out)."""
-    out_shape_0 = x.shape[:-1]
-    x = x.view((-1, x.shape[-1]))
-    M, K = x.shape
+    shape = x.shape
+    K = shape[-1]
     N = weight.shape[1]
-    dev = _on_gpu(x, weight, bias, residual)
-    z = torch.empty((M, N), device=dev, dtype=x.dtype)
+    _on_gpu(x, weight, bias, residual)
+    z = x.new_empty((*shape[:-1], N))
 
     assert x.is_contiguous()
     assert weight.is_contiguous()
-    assert x.shape[1] == weight.shape[0]
+    assert K == weight.shape[0]
     if bias is not None:
         assert bias.is_contiguous()
-        assert weight.shape[1] == bias.shape[0]
+        assert N == bias.shape[0]
     if residual is not None:
-        residual = residual.view(z.shape)
+        assert residual.numel() == z.numel()
         assert residual.is_contiguous()
 
-    _linear(x, weight, bias, residual, z, add_gelu, dropout_prob,
-            _wlayout(weight, _lib.GPTMI_W_KN), "fused_ffn")
-    return z.view((*out_shape_0, N))
+    return _linear(x, weight, bias, residual, z, add_gelu, dropout_prob,
+                   _wlayout(weight, _lib.GPTMI_W_KN), "fused_ffn")
 
 
-@torch.no_grad()
 def lm_head(x, wte):
     """x @ wte^T: logits [*, V].  `wte` is the [V, H] embedding matrix itself (read in place, no
     transposed copy; the result is contiguous) or its `pack_lm_head` image (the result is then
     the [*, :V] view of a buffer whose rows are padded to a multiple of 64 logits)."""
-    out_shape_0 = x.shape[:-1]
-    x = x.view((-1, x.shape[-1]))
+    shape = x.shape
+    H = shape[-1]
     assert x.is_contiguous()
     assert wte.is_contiguous()
+    _on_gpu(x, wte)
     if isinstance(wte, PackedWeight):
-        assert wte.vocab is not None and x.shape[1] == wte.shape[0]
-        dev = _on_gpu(x, wte)
-        z = torch.empty((x.shape[0], wte.shape[1]), device=dev, dtype=x.dtype)
+        assert wte.vocab is not None and H == wte.shape[0]
+        z = x.new_empty((*shape[:-1], wte.shape[1]))
         _linear(x, wte, None, None, z, False, 0.0, _lib.GPTMI_W_PACKED, "lm_head")
-        return z.view((*out_shape_0, wte.shape[1]))[..., :wte.vocab]
-    assert x.shape[1] == wte.shape[1]
-    dev = _on_gpu(x, wte)
-    z = torch.empty((x.shape[0], wte.shape[0]), device=dev, dtype=x.dtype)
-    _linear(x, wte, None, None, z, False, 0.0, _lib.GPTMI_W_NK, "lm_head")
-    return z.view((*out_shape_0, wte.shape[0]))
+        return z[..., :wte.vocab]
+    assert H == wte.shape[1]
+    z = x.new_empty((*shape[:-1], wte.shape[0]))
+    return _linear(x, wte, None, None, z, False, 0.0, _lib.GPTMI_W_NK, "lm_head")
 
 
-@torch.no_grad()
 def matmul_and_split_qkv(x, weight, bias, num_heads):
     """x [B, L, h] @ weight [h, 3h] + bias, returned as q, k, v [B, num_heads, L, h/num_heads],
     each contiguous; the GEMM's store does the head split."""
@@ -348,19 +319,16 @@ def matmul_and_split_qkv(x, weight, bias, num_heads):
         return tuple(t.view(batch_size, seqlen, num_heads, head_size).transpose(1, 2).contiguous()
                      for t in (q, k, v))
     shape = (batch_size, num_heads, seqlen, head_size)
-    q = torch.empty(shape, device=dev, dtype=x.dtype)
-    k = torch.empty(shape, device=dev, dtype=x.dtype)
-    v = torch.empty(shape, device=dev, dtype=x.dtype)
+    q = x.new_empty(shape)
+    k = torch.empty_like(q)
+    v = torch.empty_like(q)
     lib = _lib.load()
     M, K, N = batch_size * seqlen, x.shape[2], 3 * hidden_size
     wl = _wlayout(weight, _lib.GPTMI_W_KN)
-    ws_bytes = lib.gptmi_linear_workspace_bytes(M, N, K, code, wl)
-    ws = _workspace(ws_bytes, dev)
-    with _device(dev):
-        rc = lib.gptmi_linear_qkv(x.data_ptr(), weight.data_ptr(), _ptr(bias), q.data_ptr(),
-                                  k.data_ptr(), v.data_ptr(), batch_size, seqlen, num_heads,
-                                  head_size, K, wl, _ptr(ws), ws_bytes, code, _stream())
-    _lib.check(rc, "matmul_and_split_qkv")
+    ws, ws_bytes = _linear_workspace(lib, M, N, K, code, wl, x)
+    _call(dev, "matmul_and_split_qkv", lib.gptmi_linear_qkv, x.data_ptr(), weight.data_ptr(),
+          _ptr(bias), q.data_ptr(), k.data_ptr(), v.data_ptr(), batch_size, seqlen, num_heads,
+          head_size, K, wl, _ptr(ws), ws_bytes, code)
     return q, k, v
 
 
@@ -388,7 +356,6 @@ def _check_layer_norm_linear(x, ln_weight, ln_bias, weight, bias, what):
     return _on_gpu(x, ln_weight, ln_bias, weight, bias)
 
 
-@torch.no_grad()
 def layer_norm_ffn(x, ln_weight, ln_bias, weight, bias=None, add_gelu=False):
     """gelu?(fused_layer_norm(x, ln_weight, ln_bias) @ weight + bias) in one launch: the
     LayerNorm runs in the GEMM's operand prologue (the fusion marked as to do in the reference,
@@ -398,17 +365,13 @@ def layer_norm_ffn(x, ln_weight, ln_bias, weight, bias=None, add_gelu=False):
     dev = _check_layer_norm_linear(x, ln_weight, ln_bias, weight, bias, "layer_norm_ffn")
     K, N = weight.shape
     M = x.numel() // K
-    z = torch.empty((*x.shape[:-1], N), device=dev, dtype=x.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_layernorm_linear(x.data_ptr(), ln_weight.data_ptr(), ln_bias.data_ptr(),
-                                        1e-5, weight.data_ptr(), _ptr(bias), z.data_ptr(), M, N, K,
-                                        int(bool(add_gelu)), _lib.GPTMI_F16, _stream())
-    _lib.check(rc, "layer_norm_ffn")
+    z = x.new_empty((*x.shape[:-1], N))
+    _call(dev, "layer_norm_ffn", _lib.load().gptmi_layernorm_linear, x.data_ptr(),
+          ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, weight.data_ptr(), _ptr(bias),
+          z.data_ptr(), M, N, K, 1 if add_gelu else 0, _lib.GPTMI_F16)
     return z
 
 
-@torch.no_grad()
 def layer_norm_matmul_and_split_qkv(x, ln_weight, ln_bias, weight, bias, num_heads):
     """matmul_and_split_qkv(fused_layer_norm(x, ln_weight, ln_bias), weight, bias, num_heads) in
     one launch, same bits; see `layer_norm_ffn`.  x [B, L, h]; head size a multiple of 8."""
@@ -419,20 +382,16 @@ def layer_norm_matmul_and_split_qkv(x, ln_weight, ln_bias, weight, bias, num_hea
     assert weight.shape[1] == 3 * hidden_size and hidden_size % num_heads == 0
     head_size = hidden_size // num_heads
     shape = (batch_size, num_heads, seqlen, head_size)
-    q = torch.empty(shape, device=dev, dtype=x.dtype)
-    k = torch.empty(shape, device=dev, dtype=x.dtype)
-    v = torch.empty(shape, device=dev, dtype=x.dtype)
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_layernorm_linear_qkv(x.data_ptr(), ln_weight.data_ptr(), ln_bias.data_ptr(),
-                                            1e-5, weight.data_ptr(), _ptr(bias), q.data_ptr(),
-                                            k.data_ptr(), v.data_ptr(), batch_size, seqlen,
-                                            num_heads, head_size, K, _lib.GPTMI_F16, _stream())
-    _lib.check(rc, "layer_norm_matmul_and_split_qkv")
+    q = x.new_empty(shape)
+    k = torch.empty_like(q)
+    v = torch.empty_like(q)
+    _call(dev, "layer_norm_matmul_and_split_qkv", _lib.load().gptmi_layernorm_linear_qkv,
+          x.data_ptr(), ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, weight.data_ptr(),
+          _ptr(bias), q.data_ptr(), k.data_ptr(), v.data_ptr(), batch_size, seqlen, num_heads,
+          head_size, K, _lib.GPTMI_F16)
     return q, k, v
 
 
-@torch.no_grad()
 def flash_attention_v1(q, k, v, dropout_prob=0.0, *, merged_heads_layout=False):
     """Causal softmax(q k^T / sqrt(d)) v for q, k, v [B, N, L, d] -> [B, N, L, d].
 
@@ -445,7 +404,7 @@ def flash_attention_v1(q, k, v, dropout_prob=0.0, *, merged_heads_layout=False):
     assert k.shape == v.shape
     B, N, Lq, H = q.shape
     Lk = k.shape[2]
-    assert H in {16, 32, 64, 128, 256}
+    assert H in HEAD_SIZES
     assert q.is_contiguous()
     assert k.is_contiguous()
     assert v.is_contiguous()
@@ -453,23 +412,88 @@ def flash_attention_v1(q, k, v, dropout_prob=0.0, *, merged_heads_layout=False):
         raise TypeError("flash_attention_v1: q, k and v must share a dtype")
     dev = _on_gpu(q, k, v)
     code = _dtype_code(q, "flash_attention_v1")
-    scale = 1 / math.sqrt(H)
-    return _flash(q, k, v, scale, dropout_prob, merged_heads_layout, dev, code)
-
-
-def _flash(q, k, v, scale, dropout_prob, merged_heads_layout, dev, code):
-    B, N, Lq, H = q.shape
-    Lk = k.shape[2]
     if merged_heads_layout:
-        buf = torch.empty((B, Lq, N, H), device=dev, dtype=q.dtype)
+        buf = q.new_empty((B, Lq, N, H))
         layout = _lib.GPTMI_O_BLND
     else:
-        buf = torch.empty((B, N, Lq, H), device=dev, dtype=q.dtype)
+        buf = torch.empty_like(q)
         layout = _lib.GPTMI_O_BNLD
-    lib = _lib.load()
-    with _device(dev):
-        rc = lib.gptmi_flash_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), buf.data_ptr(), B, N,
-                                  Lq, Lk, H, scale, float(dropout_prob), 1337, layout, code,
-                                  _stream())
-    _lib.check(rc, "flash_attention_v1")
+    _call(dev, "flash_attention_v1", _lib.load().gptmi_flash_attn, q.data_ptr(), k.data_ptr(),
+          v.data_ptr(), buf.data_ptr(), B, N, Lq, Lk, H, 1 / math.sqrt(H), float(dropout_prob), 1337,
+          layout, code)
     return buf.transpose(1, 2) if merged_heads_layout else buf
+
+
+# Head sizes of the attention kernels (the reference's set, kernels.py:490).
+HEAD_SIZES = frozenset((16, 32, 64, 128, 256))
+
+
+def block_supported(x, width):
+    """True where `attention_block` / `mlp_block` take rows of this width."""
+    return width % 64 == 0 and width <= 8192 and x.dtype in _DTYPES
+
+
+def _block_layout(first, second, what):
+    packed = isinstance(first, PackedWeight)
+    if packed != isinstance(second, PackedWeight):
+        raise TypeError(f"{what}: both weights packed or neither")
+    return _lib.GPTMI_W_PACKED if packed else _lib.GPTMI_W_KN
+
+
+def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, num_heads,
+                    dropout_prob=0.0, normed=None, layer_norm_in_gemm=False):
+    """x + dropout(proj(attention(qkv(LayerNorm(x))))) for x [B, L, h]: the operators of an attention
+    block (gpt.py:39-60) behind one call of the library, with their bits.  `normed`: LayerNorm(x), if
+    the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`."""
+    B, L, h = x.shape
+    dtype = x.dtype
+    dev = _on_gpu(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, normed)
+    assert x.is_contiguous() and (normed is None or normed.is_contiguous() and normed.shape == x.shape)
+    assert ln_weight.is_contiguous() and ln_bias.is_contiguous()
+    assert qkv_bias.is_contiguous() and proj_bias.is_contiguous()
+    assert qkv_weight.is_contiguous() and proj_weight.is_contiguous()
+    assert tuple(qkv_weight.shape) == (h, 3 * h) and tuple(proj_weight.shape) == (h, h)
+    assert h % num_heads == 0 and h // num_heads in HEAD_SIZES
+    if not (dtype == ln_weight.dtype == ln_bias.dtype == qkv_weight.dtype == qkv_bias.dtype ==
+            proj_weight.dtype == proj_bias.dtype and (normed is None or normed.dtype == dtype)):
+        raise TypeError("attention_block: x and the parameters must share a dtype")
+    code = _dtype_code(x, "attention_block")
+    layout = _block_layout(qkv_weight, proj_weight, "attention_block")
+    d = h // num_heads
+    lib = _lib.load()
+    nbytes = lib.gptmi_attention_block_workspace_bytes(B, L, num_heads, d, layout)
+    ws = _workspace(nbytes, x)
+    out = torch.empty_like(x)
+    _call(dev, "attention_block", lib.gptmi_attention_block, x.data_ptr(), _ptr(normed),
+          ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, qkv_weight.data_ptr(), qkv_bias.data_ptr(),
+          proj_weight.data_ptr(), proj_bias.data_ptr(), out.data_ptr(), B, L, num_heads, d,
+          float(dropout_prob), 1337, 1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
+    return out
+
+
+def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_prob=0.0):
+    """x + dropout(W2 . dropout(gelu(W1 . LayerNorm(x)))): the operators of an MLP block
+    (gpt.py:91-111) behind one call of the library, with their bits."""
+    h = x.shape[-1]
+    dtype = x.dtype
+    inner = weight1.shape[1]
+    dev = _on_gpu(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2)
+    assert x.is_contiguous() and ln_weight.is_contiguous() and ln_bias.is_contiguous()
+    assert weight1.is_contiguous() and weight2.is_contiguous()
+    assert bias1.is_contiguous() and bias2.is_contiguous()
+    assert weight1.shape[0] == h and tuple(weight2.shape) == (inner, h)
+    if not (dtype == ln_weight.dtype == ln_bias.dtype == weight1.dtype == bias1.dtype ==
+            weight2.dtype == bias2.dtype):
+        raise TypeError("mlp_block: x and the parameters must share a dtype")
+    code = _dtype_code(x, "mlp_block")
+    layout = _block_layout(weight1, weight2, "mlp_block")
+    M = x.numel() // h
+    lib = _lib.load()
+    nbytes = lib.gptmi_mlp_block_workspace_bytes(M, h, inner, layout)
+    ws = _workspace(nbytes, x)
+    out = torch.empty_like(x)
+    _call(dev, "mlp_block", lib.gptmi_mlp_block, x.data_ptr(), ln_weight.data_ptr(),
+          ln_bias.data_ptr(), 1e-5, weight1.data_ptr(), bias1.data_ptr(), weight2.data_ptr(),
+          bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337, layout,
+          ws.data_ptr(), nbytes, code)
+    return out

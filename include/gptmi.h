@@ -277,6 +277,35 @@ int gptmi_flash_attn(const void* q, const void* k, const void* v, void* out,
                      float scale, float p, uint64_t seed, int olayout, int dtype,
                      void* stream);
 
+/*
+ * A whole attention block, x + proj(attention(qkv(LayerNorm(x)))), and a whole MLP block,
+ * x + W2 . gelu(W1 . LayerNorm(x)), behind one call each: the launches of gptmi_layernorm (or the
+ * LayerNorm prologue, or `normed` = LayerNorm(x) from gptmi_embed_layernorm), gptmi_linear_qkv,
+ * gptmi_flash_attn and gptmi_linear, in that order, with the same bits.  What the calls save is host
+ * time (a few hundred tokens are bound by it) and, for fp32 storage, traffic: the intermediate
+ * matrices live in the workspace in fp16, the rounding that the next product applies to its operands.
+ *
+ * Replaces the bodies of FusedAttention.forward and FusedMLP.forward, gpt.py:39-60 and 91-111.
+ *   x, out [B*L][h] or [M][H]        normed: LayerNorm(x) in the storage type, or NULL
+ *   W_qkv [h][3h], W_proj [h][h], W1 [H][inner], W2 [inner][H]: all GPTMI_W_KN or all packed
+ *   h = heads*d and H and inner multiples of 64, h and H up to 8192; d as in gptmi_flash_attn
+ *   p, seed: dropout of the attention weights and of the projection's output (MLP: of both products)
+ *   fuse_layernorm: 1 = the LayerNorm prologue (see gptmi_layernorm_linear_supported)
+ * workspace: the given number of bytes, 256-byte aligned.
+ */
+size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d,
+                                             int wlayout);
+int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b,
+                          float eps, const void* W_qkv, const void* b_qkv, const void* W_proj,
+                          const void* b_proj, void* out, int64_t B, int64_t L, int64_t heads,
+                          int64_t d, float p, uint64_t seed, int fuse_layernorm, int wlayout,
+                          void* workspace, size_t workspace_bytes, int dtype, void* stream);
+size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int wlayout);
+int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
+                    const void* b1, const void* W2, const void* b2, void* out, int64_t M,
+                    int64_t H, int64_t inner, float p, uint64_t seed, int wlayout,
+                    void* workspace, size_t workspace_bytes, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

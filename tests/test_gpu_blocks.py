@@ -1,0 +1,98 @@
+"""attention_block and mlp_block: a block's operators behind one call of the library, against the same
+operators called one by one (fused_layer_norm, matmul_and_split_qkv, flash_attention_v1, fused_ffn),
+with packed and plain weights, with and without dropout.
+
+fp16 storage runs the very same launches on the same operands: equal bits.  fp32 storage hands fp16
+copies of q, k, v and of the operands on, which the operators round to anyway; only the attention may
+run another of its kernels, whose fp32 sums run in another order.  A last-bit difference there can turn
+the fp16 rounding of a weight P or of the attention output, so each of the h products of the
+projection may be off by 2^-11 of itself: |difference| <= 2^-11 * sum |attention| |W| is the bound; the
+MLP has no attention in it: equal bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(gpu_device):
+    from gpt_triton_amd import kernels
+
+    return kernels
+
+
+def params(h, dtype, device, seed):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    rn = lambda *s, std=1.0, mean=0.0: (mean + std * torch.randn(*s, generator=g)).to(dtype).to(device)
+    return dict(ln_w=rn(h, std=0.2, mean=1.0), ln_b=rn(h, std=0.1), qkv=rn(h, 3 * h, std=h**-0.5),
+                qkv_b=rn(3 * h, std=0.1), proj=rn(h, h, std=h**-0.5), proj_b=rn(h, std=0.1),
+                w1=rn(h, 4 * h, std=h**-0.5), b1=rn(4 * h, std=0.1), w2=rn(4 * h, h, std=0.5 * h**-0.5),
+                b2=rn(h, std=0.1)), rn
+
+
+CASES = [(1, 1, 64, 1), (2, 37, 128, 2), (3, 65, 192, 6), (2, 321, 128, 2), (6, 100, 768, 12),
+         (70, 40, 64, 1), (2, 130, 256, 2), (1, 300, 256, 1), (4, 50, 64, 4)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("B,L,h,heads", CASES)
+def test_attention_block(K, gpu_device, dtype, packed, p, B, L, h, heads):
+    P, rn = params(h, dtype, gpu_device, seed=L + h)
+    x = rn(B, L, h)
+    print(f"attention_block {dtype} B={B} L={L} h={h} heads={heads} packed={packed} p={p}", flush=True)
+    wq, wp = (K.pack_weight(P["qkv"]), K.pack_weight(P["proj"])) if packed else (P["qkv"], P["proj"])
+    y = K.fused_layer_norm(x, P["ln_w"], P["ln_b"])
+    q, k, v = K.matmul_and_split_qkv(y, wq, P["qkv_b"], heads)
+    a = K.flash_attention_v1(q, k, v, dropout_prob=p, merged_heads_layout=True)
+    a = a.transpose(1, 2).contiguous().view(x.shape)
+    want = K.fused_ffn(a, wp, bias=P["proj_b"], residual=x, dropout_prob=p)
+    for normed in (None, y):
+        got = K.attention_block(x, P["ln_w"], P["ln_b"], wq, P["qkv_b"], wp, P["proj_b"], heads,
+                                dropout_prob=p, normed=normed)
+        if dtype == torch.float16:
+            assert torch.equal(got, want)
+        else:
+            sums = a.abs().view(-1, h) @ P["proj"].abs()
+            bound = 2.0**-11 * sums.view_as(want) / (1.0 - p) + 1e-5 * want.abs().max()
+            assert float(((got - want).abs() - bound).max()) <= 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("M,h", [(1, 64), (33, 192), (600, 768), (2100, 256), (9000, 64)])
+def test_mlp_block(K, gpu_device, dtype, packed, p, M, h):
+    P, rn = params(h, dtype, gpu_device, seed=M + h)
+    x = rn(M, h)
+    print(f"mlp_block {dtype} M={M} h={h} packed={packed} p={p}", flush=True)
+    w1, w2 = (K.pack_weight(P["w1"]), K.pack_weight(P["w2"])) if packed else (P["w1"], P["w2"])
+    y = K.fused_ffn(K.fused_layer_norm(x, P["ln_w"], P["ln_b"]), w1, bias=P["b1"], add_gelu=True,
+                    dropout_prob=p)
+    want = K.fused_ffn(y, w2, bias=P["b2"], residual=x, dropout_prob=p)
+    got = K.mlp_block(x, P["ln_w"], P["ln_b"], w1, P["b1"], w2, P["b2"], dropout_prob=p)
+    assert torch.equal(got, want)
+
+
+def test_attention_block_layer_norm_in_gemm(K, gpu_device):
+    P, rn = params(768, torch.float16, gpu_device, seed=3)
+    x = rn(2, 50, 768)
+    wq, wp = K.pack_weight(P["qkv"]), K.pack_weight(P["proj"])
+    got, want = (K.attention_block(x, P["ln_w"], P["ln_b"], wq, P["qkv_b"], wp, P["proj_b"], 12,
+                                   layer_norm_in_gemm=flag) for flag in (True, False))
+    assert torch.equal(got, want)
+
+
+def test_blocks_turn_down_what_they_do_not_hold(K, gpu_device):
+    P, rn = params(96, torch.float16, gpu_device, seed=4)
+    x = rn(2, 5, 96)
+    assert not K.block_supported(x, 96)
+    with pytest.raises(NotImplementedError):
+        K.mlp_block(x, P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
+    P, rn = params(64, torch.float16, gpu_device, seed=5)
+    x = rn(2, 5, 64)
+    with pytest.raises(TypeError):
+        K.mlp_block(x, P["ln_w"], P["ln_b"], K.pack_weight(P["w1"]), P["b1"], P["w2"], P["b2"])
+    with pytest.raises(RuntimeError, match="GPU only"):
+        K.mlp_block(x.cpu(), P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
