@@ -16,29 +16,66 @@ typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
-// Sum / max over the 64 lanes of a wavefront; every lane gets the result.
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// Cross-lane steps without the LDS: an xor shuffle compiles to ds_bpermute, ~100 cycles of latency
+// per step of a reduction, and the reductions of a LayerNorm row (twelve steps) or of a softmax tile
+// sit on the critical path of their kernels.  The swaps and row rotations are VALU instructions.
+//   half_swap(v): v of lane ^ 32 and the lane's own, in some order (what a commutative step needs)
+struct LanePair {
+  float a, b;
+};
+__device__ __forceinline__ LanePair half_swap(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const unsigned x = r[0], y = r[1];
+  return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+__device__ __forceinline__ LanePair row_swap(float v) {  // lane ^ 16
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned x = r[0], y = r[1];
+  return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
 }
-// The same over aligned groups of G lanes (G = 64: the wavefront; G = 32: each half on its own).
+template <int N>
+__device__ __forceinline__ float row_rotate(float v) {  // within rows of 16 lanes
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 | N,
+                                                               0xf, 0xf, true));
+}
+// The other lane of xor-8, 4, 2, 1 steps taken in this order: behind the step of distance 2 N all
+// lanes that differ in the higher bits hold the same value, so rotating by N finds the value of lane ^ N.
+template <int G, typename Op>
+__device__ __forceinline__ float group_reduce(float v, Op op) {
+  static_assert(G == 64 || G == 32, "a wavefront or its halves");
+  if constexpr (G == 64) {
+    const LanePair p = half_swap(v);
+    v = op(p.a, p.b);
+  }
+  const LanePair p = row_swap(v);
+  v = op(p.a, p.b);
+  v = op(v, row_rotate<8>(v));
+  v = op(v, row_rotate<4>(v));
+  v = op(v, row_rotate<2>(v));
+  return op(v, row_rotate<1>(v));
+}
+// Sum / max over aligned groups of G lanes (G = 64: the wavefront; G = 32: each half on its own);
+// every lane gets the result.
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  return group_reduce<G>(v, [](float a, float b) { return a + b; });
 }
 template <int G>
 __device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+  return group_reduce<G>(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float wave_sum(float v) { return group_sum<kWave>(v); }
+__device__ __forceinline__ float wave_max(float v) { return group_max<kWave>(v); }
+// Sum / max of this lane's value and that of lane ^ 32.
+__device__ __forceinline__ float half_sum(float v) {
+  const LanePair p = half_swap(v);
+  return p.a + p.b;
+}
+__device__ __forceinline__ float half_max(float v) {
+  const LanePair p = half_swap(v);
+  return fmaxf(p.a, p.b);
 }
 
 // tanh-form GELU of the reference (kernels.py:15-26): 0.5 x (1 + tanh(u)) with

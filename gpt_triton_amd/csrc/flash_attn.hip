@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-      bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+      bmax = half_max(bmax);
       const float mnew = bmax > mrun ? bmax : mrun;
       const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
 #pragma unroll
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
           psum += p;
         }
       mrun = mnew;
-      psum += __shfl_xor(psum, 32, kWave);
+      psum = half_sum(psum);
       den = den * mult + psum;
       if constexpr (DROP) {
         // dropout of P after the denominator has summed it, before the fp16 rounding;
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+        bmax = half_max(bmax);
         const float mnew = bmax > mrun ? bmax : mrun;
         const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
 #pragma unroll
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
             psum += p;
           }
         mrun = mnew;
-        psum += __shfl_xor(psum, 32, kWave);
+        psum = half_sum(psum);
         den = den * mult + psum;
 #pragma unroll
         for (int b = 0; b < DB; ++b)
@@ -760,7 +760,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+    bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
@@ -773,7 +773,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
         psum += p;
       }
     mrun = mnew;
-    psum += __shfl_xor(psum, 32, kWave);
+    psum = half_sum(psum);
     den = den * mult + psum;
 #pragma unroll
     for (int i = 0; i < DB; ++i)
@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+    bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
@@ -1072,7 +1072,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
           pf[kb][tt][j] = (_Float16)p;
         }
     mrun = mnew;
-    psum += __shfl_xor(psum, 32, kWave);
+    psum = half_sum(psum);
     den = den * mult + psum;
 #pragma unroll
     for (int i = 0; i < DB; ++i)
@@ -1329,7 +1329,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+    bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
     float psum = 0.f;
@@ -1345,7 +1345,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
           pf[kb][tt][j] = (_Float16)p;
         }
     mrun = mnew;
-    psum += __shfl_xor(psum, 32, kWave);
+    psum = half_sum(psum);
     den = den * mult + psum;
 #pragma unroll
     for (int i = 0; i < DB; ++i)
