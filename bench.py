@@ -301,9 +301,6 @@ def main():
     ap.add_argument("--no-ln-prologue", action="store_true",
                     help="small batches: run every LayerNorm as a launch of its own instead of "
                          "inside the following GEMM (gpt.LN_PROLOGUE_MAX_ROWS = 0), for comparison")
-    ap.add_argument("--ln-prologue-under-capture", action="store_true",
-                    help="with --graph: keep the LayerNorm-in-GEMM form inside the captured graph "
-                         "(the model takes the two launches there), for comparison")
     ap.add_argument("--graph", action="store_true",
                     help="time replays of the forward captured into a HIP graph (gpt.GraphedForward)")
     ap.add_argument("--traffic-calibration", action="store_true",
@@ -361,8 +358,6 @@ def main():
         G.fused_layer_norm = skipped_ln
     if args.no_ln_prologue:
         G.LN_PROLOGUE_MAX_ROWS = 0
-    if args.ln_prologue_under_capture:
-        G.LN_PROLOGUE_UNDER_CAPTURE = True
     step = (lambda: model(ids, return_logits=True)) if args.lm_head else (lambda: model(ids))
     if args.graph:
         graphed = G.GraphedForward(model, ids, return_logits=args.lm_head)
@@ -435,9 +430,7 @@ def main():
         "config": {"workload": what + (", logits output (tied LM head)" if args.lm_head
                                        else ", hidden-state output (no LM head)") +
                                (", replays of a captured HIP graph" if args.graph else "") +
-                               (", LayerNorms as launches of their own" if args.no_ln_prologue else "") +
-                               (", LayerNorm-in-GEMM form kept under capture"
-                                if args.ln_prologue_under_capture else ""),
+                               (", LayerNorms as launches of their own" if args.no_ln_prologue else ""),
                    "tokens_per_step": tokens, "n_layer": arch["n_layer"], "n_embd": h,
                    "n_head": arch["n_head"]},
         # one ffn1 call = gemm_stream_kernel on the row tiles that fill whole rounds of the

@@ -645,8 +645,8 @@ size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int 
 
 int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
                     const void* b1, const void* W2, const void* b2, void* out, int64_t M, int64_t H,
-                    int64_t inner, float p, uint64_t seed, int wlayout, void* workspace,
-                    size_t workspace_bytes, int dtype, void* stream) {
+                    int64_t inner, float p, uint64_t seed, int fuse_layernorm, int wlayout,
+                    void* workspace, size_t workspace_bytes, int dtype, void* stream) {
   if (!x || !ln_w || !ln_b || !W1 || !W2 || !out || inner <= 0 || inner % 64 != 0 || inner > kMaxN) {
     set_error("mlp_block: invalid argument");
     return GPTMI_ERR_INVALID;
@@ -662,7 +662,6 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
     set_error("mlp_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
   }
-  launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)H, eps, f16, true, st);
   const Dropout drop = {p, seed};
   GemmEpilogue e1 = {};
   e1.bias = b1;
@@ -671,7 +670,17 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e1.drop = drop;
   e1.f16 = f16;
   e1.out_f16 = true;
-  rc = launch_gemm(pl.normed, B1, M, (int)inner, (int)H, e1, st);
+  if (fuse_layernorm) {
+    if (!f16 || p > 0.f || ((uintptr_t)x & 15) || !gemm_layernorm_supported(M, (int)H)) {
+      set_error("mlp_block: the LayerNorm prologue takes fp16 storage, no dropout and the row widths of "
+                "gptmi_layernorm_linear_supported");
+      return GPTMI_ERR_UNSUPPORTED;
+    }
+    rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
+  } else {
+    launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)H, eps, f16, true, st);
+    rc = launch_gemm(pl.normed, B1, M, (int)inner, (int)H, e1, st);
+  }
   if (rc) return rc;
   GemmEpilogue e2 = {};
   e2.bias = b2;

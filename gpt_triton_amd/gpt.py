@@ -26,13 +26,13 @@ from .kernels import (HEAD_SIZES, attention_block, block_supported, flash_attent
                       layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, mlp_block,
                       pack_lm_head, pack_weight)
 
-# Up to this many token rows the blocks run their LayerNorm inside the following GEMM
-# (layer_norm_ffn, layer_norm_in_gemm: one launch instead of two, same bits): such a forward is bound
-# by its launches.  Above, the LayerNorm kernel and the larger tiles are faster -- the fused form
-# normalises a row block once per column tile -- and so are the two launches inside a captured graph,
-# where a launch costs next to nothing.
-LN_PROLOGUE_MAX_ROWS = 128
-LN_PROLOGUE_UNDER_CAPTURE = False  # measurement switch (bench.py --ln-prologue-under-capture)
+# Up to this many token rows of up to this width the blocks run their LayerNorm inside the following
+# GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile and one
+# of its workgroups fills a CU, so it pays while all column tiles run at once: LayerNorm -> ffn1 at
+# 24 / 128 / 200 rows of 768 takes 6.6 / 8.5 / 13.5 us against 7.7 / 9.3 / 10.4 for the two launches, at
+# 24 rows of 1024 8.1 against 7.5, of 1600 13.0 against 11.9.
+LN_PROLOGUE_MAX_ROWS = 160
+LN_PROLOGUE_MAX_WIDTH = 768
 
 # Up to this many token rows a block is one call of the library (attention_block, mlp_block) instead
 # of one per operator: below about 4000 rows of the 124M model the host, not the GPU, sets the pace of
@@ -43,9 +43,9 @@ BLOCK_MAX_ROWS = 8192
 
 
 def _ln_in_gemm(x, weight):
-    return (x.numel() // x.shape[-1] <= LN_PROLOGUE_MAX_ROWS and
-            layer_norm_linear_supported(x, weight) and
-            (LN_PROLOGUE_UNDER_CAPTURE or not torch.cuda.is_current_stream_capturing()))
+    width = x.shape[-1]
+    return (width <= LN_PROLOGUE_MAX_WIDTH and x.numel() // width <= LN_PROLOGUE_MAX_ROWS and
+            layer_norm_linear_supported(x, weight))
 
 
 def _as_block(x, width):
@@ -183,15 +183,14 @@ class FusedMLP(nn.Module):
         prm = self._parameters
         w1, w2 = self._weight("ffn1_weight"), self._weight("ffn2_weight")
         if p == 0.0 and _ln_in_gemm(x, w1):
-            y = layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
-                               bias=prm["ffn1_bias"], add_gelu=True)
-        elif _as_block(x, self.hidden_size):
+            return layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
+                                  bias=prm["ffn1_bias"], add_gelu=True, then=(w2, prm["ffn2_bias"]))
+        if _as_block(x, self.hidden_size):
             return mlp_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                              prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p)
-        else:
-            y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
-            y = fused_ffn(y, w1, bias=prm["ffn1_bias"].data, residual=None, add_gelu=True,
-                          dropout_prob=p)
+        y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
+        y = fused_ffn(y, w1, bias=prm["ffn1_bias"].data, residual=None, add_gelu=True,
+                      dropout_prob=p)
         return fused_ffn(y, w2, bias=prm["ffn2_bias"].data, residual=x, add_gelu=False,
                          dropout_prob=p)
 

@@ -356,12 +356,18 @@ def _check_layer_norm_linear(x, ln_weight, ln_bias, weight, bias, what):
     return _on_gpu(x, ln_weight, ln_bias, weight, bias)
 
 
-def layer_norm_ffn(x, ln_weight, ln_bias, weight, bias=None, add_gelu=False):
+def layer_norm_ffn(x, ln_weight, ln_bias, weight, bias=None, add_gelu=False, then=None):
     """gelu?(fused_layer_norm(x, ln_weight, ln_bias) @ weight + bias) in one launch: the
     LayerNorm runs in the GEMM's operand prologue (the fusion marked as to do in the reference,
     kernels.py:132-133) and gives the bits of fused_layer_norm followed by fused_ffn.  Meant for
     few rows; `weight` is a `pack_weight` image, fp16 only (NotImplementedError otherwise, and
-    for row widths `layer_norm_linear_supported` turns down)."""
+    for row widths `layer_norm_linear_supported` turns down).
+
+    then=(weight2, bias2), with add_gelu and bias: the MLP's second product behind it in the same
+    call -- the result is x + that @ weight2 + bias2 (fused_ffn with x as the residual, same bits)."""
+    if then is not None:
+        assert add_gelu and bias is not None
+        return mlp_block(x, ln_weight, ln_bias, weight, bias, *then, layer_norm_in_gemm=True)
     dev = _check_layer_norm_linear(x, ln_weight, ln_bias, weight, bias, "layer_norm_ffn")
     K, N = weight.shape
     M = x.numel() // K
@@ -471,9 +477,11 @@ def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, pr
     return out
 
 
-def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_prob=0.0):
+def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_prob=0.0,
+              layer_norm_in_gemm=False):
     """x + dropout(W2 . dropout(gelu(W1 . LayerNorm(x)))): the operators of an MLP block
-    (gpt.py:91-111) behind one call of the library, with their bits."""
+    (gpt.py:91-111) behind one call of the library, with their bits; layer_norm_in_gemm: as in
+    `layer_norm_ffn`."""
     h = x.shape[-1]
     dtype = x.dtype
     inner = weight1.shape[1]
@@ -494,6 +502,6 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     out = torch.empty_like(x)
     _call(dev, "mlp_block", lib.gptmi_mlp_block, x.data_ptr(), ln_weight.data_ptr(),
           ln_bias.data_ptr(), 1e-5, weight1.data_ptr(), bias1.data_ptr(), weight2.data_ptr(),
-          bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337, layout,
-          ws.data_ptr(), nbytes, code)
+          bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337,
+          1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
     return out

@@ -303,8 +303,9 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
 size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int wlayout);
 int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
                     const void* b1, const void* W2, const void* b2, void* out, int64_t M,
-                    int64_t H, int64_t inner, float p, uint64_t seed, int wlayout,
-                    void* workspace, size_t workspace_bytes, int dtype, void* stream);
+                    int64_t H, int64_t inner, float p, uint64_t seed, int fuse_layernorm,
+                    int wlayout, void* workspace, size_t workspace_bytes, int dtype,
+                    void* stream);
 
 #ifdef __cplusplus
 }
