@@ -243,10 +243,14 @@ static MlpPlan plan_mlp(void* ws, int64_t M, int64_t h, int64_t inner, int wlayo
   return p;
 }
 
+// The generator's offsets are 32-bit numbers: a mask longer than that would repeat itself.
+constexpr int64_t kMaxMaskBits = 1ll << 32;
+
 // What the block functions take: row widths that are multiples of 64 (every operand is then read in
 // place), up to the LayerNorm kernel's 8192.
-static int check_block(const char* what, int64_t M, int64_t h, float p, int wlayout, int dtype,
-                       const void* ws, size_t ws_bytes, size_t need) {
+static int check_block(const char* what, int64_t M, int64_t h, float p, const void* keep,
+                       int64_t keep_bits, int64_t keep_need, int wlayout, int dtype, const void* ws,
+                       size_t ws_bytes, size_t need) {
   if (M <= 0 || h <= 0 || !dtype_ok(dtype) || (wlayout != GPTMI_W_KN && wlayout != GPTMI_W_PACKED)) {
     set_error("%s: invalid argument", what);
     return GPTMI_ERR_INVALID;
@@ -257,6 +261,11 @@ static int check_block(const char* what, int64_t M, int64_t h, float p, int wlay
   }
   if (!dropout_ok(p)) {
     set_error("%s: dropout probability %g outside [0, 1)", what, (double)p);
+    return GPTMI_ERR_INVALID;
+  }
+  if (keep != nullptr && (keep_bits < keep_need || keep_need > kMaxMaskBits || ((uintptr_t)keep & 3) != 0)) {
+    set_error("%s: a dropout mask of %lld bits (at most 2^32), 4-byte aligned, needed (%lld given)", what,
+              (long long)keep_need, (long long)keep_bits);
     return GPTMI_ERR_INVALID;
   }
   if (ws == nullptr || ws_bytes < need || ((uintptr_t)ws & 255) != 0) {
@@ -569,6 +578,19 @@ int gptmi_flash_attn(const void* q, const void* k, const void* v, void* out, int
   return check_launch("flash_attn");
 }
 
+size_t gptmi_dropout_mask_bytes(int64_t n) {
+  return n > 0 && n <= kMaxMaskBits ? (size_t)((n + 31) / 32 + 4) * 4 : 0;
+}
+
+int gptmi_dropout_mask(void* mask, int64_t n, float p, uint64_t seed, void* stream) {
+  if (!mask || n <= 0 || n > kMaxMaskBits || ((uintptr_t)mask & 3) != 0 || !dropout_ok(p)) {
+    set_error("dropout_mask: invalid argument");
+    return GPTMI_ERR_INVALID;
+  }
+  launch_dropout_mask(mask, (n + 31) / 32 + 4, Dropout{p, seed}, (hipStream_t)stream);
+  return check_launch("dropout_mask");
+}
+
 size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d,
                                              int wlayout) {
   if (B <= 0 || L <= 0 || heads <= 0 || d <= 0) return 0;
@@ -578,7 +600,7 @@ size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads
 int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
                           const void* W_qkv, const void* b_qkv, const void* W_proj, const void* b_proj,
                           void* out, int64_t B, int64_t L, int64_t heads, int64_t d, float p,
-                          uint64_t seed, int fuse_layernorm, int wlayout, void* workspace,
+                          uint64_t seed, const void* keep, int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace,
                           size_t workspace_bytes, int dtype, void* stream) {
   if (!x || !ln_w || !ln_b || !W_qkv || !W_proj || !out || B <= 0 || L <= 0 || heads <= 0 || d <= 0) {
     set_error("attention_block: invalid argument");
@@ -586,7 +608,8 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   }
   const int64_t M = B * L, h = heads * d;
   const AttentionPlan pl = plan_attention(workspace, M, h, wlayout);
-  int rc = check_block("attention_block", M, h, p, wlayout, dtype, workspace, workspace_bytes, pl.total);
+  int rc = check_block("attention_block", M, h, p, keep, keep_bits, M * h > L * L ? M * h : L * L, wlayout,
+                       dtype, workspace, workspace_bytes, pl.total);
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
@@ -622,7 +645,7 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     rc = launch_gemm(A, Bq, M, (int)(3 * h), (int)h, ep, st);
   }
   if (rc) return rc;
-  const Dropout drop = {p, seed};
+  const Dropout drop = {p, seed, keep};
   const float scale = (float)(1.0 / sqrt((double)d));
   rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
            : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
@@ -645,14 +668,15 @@ size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int 
 
 int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
                     const void* b1, const void* W2, const void* b2, void* out, int64_t M, int64_t H,
-                    int64_t inner, float p, uint64_t seed, int fuse_layernorm, int wlayout,
-                    void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+                    int64_t inner, float p, uint64_t seed, const void* keep, int64_t keep_bits,
+                    int fuse_layernorm, int wlayout, void* workspace, size_t workspace_bytes, int dtype, void* stream) {
   if (!x || !ln_w || !ln_b || !W1 || !W2 || !out || inner <= 0 || inner % 64 != 0 || inner > kMaxN) {
     set_error("mlp_block: invalid argument");
     return GPTMI_ERR_INVALID;
   }
   const MlpPlan pl = plan_mlp(workspace, M, H, inner, wlayout);
-  int rc = check_block("mlp_block", M, H, p, wlayout, dtype, workspace, workspace_bytes, pl.total);
+  int rc = check_block("mlp_block", M, H, p, keep, keep_bits, M * (inner > H ? inner : H), wlayout, dtype,
+                       workspace, workspace_bytes, pl.total);
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
@@ -662,7 +686,7 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
     set_error("mlp_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
   }
-  const Dropout drop = {p, seed};
+  const Dropout drop = {p, seed, keep};
   GemmEpilogue e1 = {};
   e1.bias = b1;
   e1.out = pl.inner;

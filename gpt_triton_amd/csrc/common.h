@@ -96,52 +96,100 @@ __device__ __forceinline__ float gelu_new(float x) {
 // the 64-bit seed as key; the first output word, read as int32 with negatives folded by
 // -x-1, times 4.6566127342e-10 gives the uniform in [0, 1).  NCH independent offsets share
 // one rolled round loop so that a call site stays a few dozen instructions.
+//
+// Bound by the 32 x 32 -> 64 bit products (quarter rate).  Of the 20 of the general form 17 are left,
+// one of them uniform: three counter words start as 0, so round 1 has one product and round 2's
+// second is the same for every offset, and of rounds 9 and 10 only what reaches the first word is
+// formed.
 // ---------------------------------------------------------------------------
 struct DropoutArgs {
   float p;
   unsigned seed_lo, seed_hi;
 };
 
+__device__ __forceinline__ unsigned xor3(unsigned a, unsigned b, unsigned c) {
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 template <int NCH>
 __device__ __forceinline__ void philox_uniform(const DropoutArgs& d, const unsigned (&offset)[NCH],
                                                float (&u)[NCH]) {
+  constexpr unsigned A = 0xD2511F53u, B = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
   unsigned c0[NCH], c1[NCH], c2[NCH], c3[NCH];
+  unsigned k0 = d.seed_lo, k1 = d.seed_hi;
+  const uint64_t seed_a = (uint64_t)A * k0;  // round 2's product of word 0, which round 1 makes k0
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    c0[i] = offset[i];
-    c1[i] = c2[i] = c3[i] = 0u;
+    const uint64_t a = (uint64_t)A * offset[i];
+    c2[i] = (unsigned)(a >> 32) ^ k1;
+    c3[i] = (unsigned)a;
   }
-  unsigned k0 = d.seed_lo, k1 = d.seed_hi;
+  k0 += W0;
+  k1 += W1;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const uint64_t b = (uint64_t)B * c2[i];
+    c0[i] = (unsigned)(b >> 32) ^ k0;
+    c1[i] = (unsigned)b;
+    c2[i] = xor3((unsigned)(seed_a >> 32), c3[i], k1);
+    c3[i] = (unsigned)seed_a;
+  }
 #pragma unroll 1
-  for (int r = 0; r < 10; ++r) {
+  for (int r = 0; r < 6; ++r) {
+    k0 += W0;
+    k1 += W1;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const unsigned hb = __umulhi(0xCD9E8D57u, c2[i]), lb = 0xCD9E8D57u * c2[i];
-      const unsigned ha = __umulhi(0xD2511F53u, c0[i]), la = 0xD2511F53u * c0[i];
-      c0[i] = hb ^ c1[i] ^ k0;
-      c2[i] = ha ^ c3[i] ^ k1;
-      c1[i] = lb;
-      c3[i] = la;
+      const uint64_t b = (uint64_t)B * c2[i], a = (uint64_t)A * c0[i];
+      c0[i] = xor3((unsigned)(b >> 32), c1[i], k0);
+      c2[i] = xor3((unsigned)(a >> 32), c3[i], k1);
+      c1[i] = (unsigned)b;
+      c3[i] = (unsigned)a;
     }
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
   }
+  k0 += W0;
+  k1 += W1;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    int x = (int)c0[i];
-    x = x < 0 ? -x - 1 : x;
-    u[i] = (float)x * 4.6566127342e-10f;
+    const unsigned n2 = xor3(__umulhi(A, c0[i]), c3[i], k1), n1 = B * c2[i];
+    const unsigned w = xor3(__umulhi(B, n2), n1, k0 + W0);
+    const int x = (int)w;
+    u[i] = (float)(x ^ (x >> 31)) * 4.6566127342e-10f;  // ~x = -x-1 for negative words
   }
 }
+
+// x / keep for the kept values.  Division by one number: its reciprocal is taken once, and the
+// remainder of the first quotient corrects it (correctly rounded for a correctly rounded reciprocal,
+// P. Markstein, IBM J. Res. Dev. 34, 1990); div_fixup passes infinities and NaN through.
+struct KeepScale {
+  float keep, inv;
+  __device__ __forceinline__ explicit KeepScale(float p) : keep(1.0f - p), inv(1.0f / (1.0f - p)) {}
+  __device__ __forceinline__ float operator()(float x) const {
+    const float q = x * inv;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, keep, x), inv, q), keep, x);
+  }
+  // for an x that is no infinity
+  __device__ __forceinline__ float finite(float x) const {
+    const float q = x * inv;
+    float r = fmaf(fmaf(-q, keep, x), inv, q);
+    asm("" : "+v"(r));  // rounded to fp32 before it is to fp16, not by one mixed-precision fma
+    return r;
+  }
+};
 
 template <int NCH>
 __device__ __forceinline__ void dropout_apply(const DropoutArgs& d, const unsigned (&offset)[NCH],
                                               float (&x)[NCH]) {
   float u[NCH];
   philox_uniform<NCH>(d, offset, u);
-  const float keep_scale = 1.0f - d.p;
+  const KeepScale scale(d.p);
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) x[i] = u[i] > d.p ? x[i] / keep_scale : 0.0f;
+  for (int i = 0; i < NCH; ++i) x[i] = u[i] > d.p ? scale(x[i]) : 0.0f;
+}
+
+// v where bit `b` of `bits` is set, +0 elsewhere (v's bits under a mask: one bit-field extract, one and).
+__device__ __forceinline__ float keep_if(unsigned bits, int b, float v) {
+  return __int_as_float(__builtin_amdgcn_sbfe((int)bits, (unsigned)b, 1u) & __float_as_int(v));
 }
 
 void set_error(const char* fmt, ...);

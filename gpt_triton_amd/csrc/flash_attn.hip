@@ -103,10 +103,14 @@ __device__ __forceinline__ h8 zero_h8() {
 // u ^ ((d>>1)&15)).  DG = head size of the tensors in memory: 16 and 32 run on the D = 64
 // staging layout (columns at or past DG are written as zeros, never read from memory) with
 // only DG / 16 k-steps of q . k and one 32-row block of O^T.
-template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
-__global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_kernel(
+//
+// DROP: 0 none; 1 the mask generated here, per weight; 2 its bits read from `keep` (offset
+// query * Lk + key: the same for every batch and head).
+template <int D, typename T, bool BLND, int DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
+__global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_attn_kernel(
     const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    T* __restrict__ O, int heads, int L, int Lk_arg, float scale, DropoutArgs drop) {
+    T* __restrict__ O, int heads, int L, int Lk_arg, float scale, DropoutArgs drop,
+    const unsigned* __restrict__ keep) {
   // L = query rows, Lk = key rows of every (batch, head); UNEQ = they may differ.  The mask is
   // "key <= query" alone and key rows at or past Lk count as zero rows, as in the reference
   // (kernels.py:421-436): with L > Lk the queries at or past Lk also see the zero rows that fill
@@ -221,6 +225,8 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
   float mrun = -INFINITY, den = 0.f;
   const Softmax<ACC> sm(scale);
+  const KeepScale keep_scale(DROP == 2 ? drop.p : 0.f);
+  const unsigned keep_row = (unsigned)(q < L ? q : L - 1) * (unsigned)Lk;
 
   load_tile(0, stg[0]);
   if constexpr (!ONESET) {
@@ -242,6 +248,13 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
     if (wave_active && k0 <= qw0 + 31) {
       const char* ks_ = smem + (t & 1) * STAGE;
       const char* vs_ = ks_ + K_BYTES;
+      // this query's 64 bits of the mask, from bit keep_at of three words on
+      unsigned kw[3] = {0, 0, 0};
+      const unsigned keep_at = keep_row + (unsigned)k0;
+      if constexpr (DROP == 2) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) kw[i] = keep[(keep_at >> 5) + i];
+      }
       // ---- S^T = K . Q^T ---------------------------------------------------
       f16v s[2];
 #pragma unroll
@@ -286,7 +299,17 @@ __global__ __launch_bounds__(256, (D == 64 && !DROP) ? 2 : 1) void flash_attn_ke
       mrun = mnew;
       psum = half_sum(psum);
       den = den * mult + psum;
-      if constexpr (DROP) {
+      if constexpr (DROP == 2) {
+        // the same, the mask read instead of generated
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const unsigned bits = __builtin_amdgcn_alignbit(kw[kb + 1], kw[kb], keep_at & 31) >> (4 * g);
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[kb][r] = keep_if(bits, 8 * (r >> 2) + (r & 3), keep_scale.finite(s[kb][r]));
+        }
+      }
+      if constexpr (DROP == 1) {
         // dropout of P after the denominator has summed it, before the fp16 rounding;
         // offset = query * Lk + key, the same for every batch and head (kernels.py:457-460)
 #pragma unroll
@@ -1471,9 +1494,10 @@ int launch_resident(const void* q, const void* k, const void* v, void* out, int6
   return 0;
 }
 
-template <int D, typename T, bool BLND, bool DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
+template <int D, typename T, bool BLND, int DROP, bool UNEQ, int DG = D, bool ACC = sizeof(T) == 4>
 int launch_tiled_as(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
-                    int L, int Lk, float scale, DropoutArgs drop, hipStream_t st) {
+                    int L, int Lk, float scale, DropoutArgs drop, hipStream_t st,
+                    const void* keep = nullptr) {
   dim3 grid((unsigned)BN, (unsigned)((L + BQ - 1) / BQ));
   constexpr int lds = 2 * 2 * BKEY * D * 2;  // two stages of a K tile and a V^T tile
   auto kern = flash_attn_kernel<D, T, BLND, DROP, UNEQ, DG, ACC>;
@@ -1488,13 +1512,13 @@ int launch_tiled_as(const void* q, const void* k, const void* v, void* out, int6
   }
   attr_done = true;
   hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const T*)q, (const T*)k, (const T*)v,
-                     (T*)out, heads, L, Lk, scale, drop);
+                     (T*)out, heads, L, Lk, scale, drop, (const unsigned*)keep);
   return 0;
 }
 
 // L query rows, Lk key rows per (batch, head); equal lengths take the variant without the
 // zero-row selects.
-template <int D, typename T, bool BLND, bool DROP>
+template <int D, typename T, bool BLND, int DROP>
 int launch_tiled(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                  int L, int Lk, float scale, DropoutArgs drop, hipStream_t st) {
   if (L != Lk)
@@ -1582,12 +1606,12 @@ int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
              int heads, int L, int Lk, float scale, Dropout drop, bool blnd, hipStream_t st) {
   const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
   if (drop.p > 0.f) {  // training-mode path: the tiled kernel carries the generator
-    return blnd ? launch_tiled<D, T, true, true>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
-                : launch_tiled<D, T, false, true>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
+    return blnd ? launch_tiled<D, T, true, 1>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
+                : launch_tiled<D, T, false, 1>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
   }
   if (L != Lk)  // query and key sequences of different lengths: the tiled kernel knows both
-    return blnd ? launch_tiled<D, T, true, false>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
-                : launch_tiled<D, T, false, false>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
+    return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
+                : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
   if constexpr (D == 64 && sizeof(T) == 2) {
     // fp16, head size 64, two (batch, head) pairs fit the LDS, enough pairs to keep every
     // persistent workgroup busy for a while: the streaming kernel
@@ -1610,8 +1634,8 @@ int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
       return blnd ? launch_wide_attn<D, true>(q, k, v, out, BN, heads, L, scale, st)
                   : launch_wide_attn<D, false>(q, k, v, out, BN, heads, L, scale, st);
   }
-  return blnd ? launch_tiled<D, T, true, false>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
-              : launch_tiled<D, T, false, false>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
+  return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
+              : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
 }
 
 // Head sizes 16 and 32: the tiled kernel on its 64-wide staging layout, reading the tensors at
@@ -1621,13 +1645,13 @@ int launch_small_head(const void* q, const void* k, const void* v, void* out, in
                       int L, int Lk, float scale, Dropout drop, bool blnd, hipStream_t st) {
   const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
   if (drop.p > 0.f)
-    return blnd ? launch_tiled_as<64, T, true, true, true, DG>(q, k, v, out, BN, heads, L, Lk,
+    return blnd ? launch_tiled_as<64, T, true, 1, true, DG>(q, k, v, out, BN, heads, L, Lk,
                                                                scale, da, st)
-                : launch_tiled_as<64, T, false, true, true, DG>(q, k, v, out, BN, heads, L, Lk,
+                : launch_tiled_as<64, T, false, 1, true, DG>(q, k, v, out, BN, heads, L, Lk,
                                                                 scale, da, st);
-  return blnd ? launch_tiled_as<64, T, true, false, true, DG>(q, k, v, out, BN, heads, L, Lk,
+  return blnd ? launch_tiled_as<64, T, true, 0, true, DG>(q, k, v, out, BN, heads, L, Lk,
                                                               scale, da, st)
-              : launch_tiled_as<64, T, false, false, true, DG>(q, k, v, out, BN, heads, L, Lk,
+              : launch_tiled_as<64, T, false, 0, true, DG>(q, k, v, out, BN, heads, L, Lk,
                                                                scale, da, st);
 }
 
@@ -1646,6 +1670,23 @@ int launch_t(const void* q, const void* k, const void* v, void* out, int64_t BN,
   }
 }
 
+// Dropout with the mask's bits at hand: fp16 q, k, v of equal lengths, merged-heads output.
+template <bool ACC>
+int launch_masked(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
+                  int d, float scale, DropoutArgs da, const void* keep, hipStream_t st) {
+  typedef _Float16 T;
+  switch (d) {
+    case 16: return launch_tiled_as<64, T, true, 2, true, 16, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    case 32: return launch_tiled_as<64, T, true, 2, true, 32, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    case 64: return launch_tiled_as<64, T, true, 2, false, 64, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    case 128: return launch_tiled_as<128, T, true, 2, false, 128, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    case 256: return launch_tiled_as<256, T, true, 2, false, 256, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    default:
+      set_error("flash_attn: head size %d not built (16, 32, 64, 128 and 256 are)", d);
+      return -2;
+  }
+}
+
 // fp32 arithmetic on fp16 q, k, v (equal lengths, merged-heads output in fp16): the values an fp32
 // model's kernels round their operands to anyway, see launch_flash_attn_operands.
 template <int D>
@@ -1653,7 +1694,7 @@ int launch_operands_d(const void* q, const void* k, const void* v, void* out, in
                       int L, float scale, DropoutArgs da, hipStream_t st) {
   typedef _Float16 T;
   if (da.p > 0.f)
-    return launch_tiled_as<D, T, true, true, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+    return launch_tiled_as<D, T, true, 1, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
   if constexpr (D == 64) {
     if (L <= 320 && BN >= 64) return launch_stream_attn<true, true>(q, k, v, out, BN, heads, L, scale, st);
     if (resident_lds_bytes(L, D) == 0)
@@ -1665,7 +1706,7 @@ int launch_operands_d(const void* q, const void* k, const void* v, void* out, in
     if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
       return launch_wide_attn<D, true, true>(q, k, v, out, BN, heads, L, scale, st);
   }
-  return launch_tiled_as<D, T, true, false, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+  return launch_tiled_as<D, T, true, 0, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
 }
 
 template <int DG>
@@ -1673,8 +1714,8 @@ int launch_operands_small(const void* q, const void* k, const void* v, void* out
                           int L, float scale, DropoutArgs da, hipStream_t st) {
   typedef _Float16 T;
   if (da.p > 0.f)
-    return launch_tiled_as<64, T, true, true, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
-  return launch_tiled_as<64, T, true, false, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+    return launch_tiled_as<64, T, true, 1, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
+  return launch_tiled_as<64, T, true, 0, true, DG, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
 }
 
 }  // namespace
@@ -1687,6 +1728,8 @@ int launch_flash_attn_operands(const void* q, const void* k, const void* v, void
     return -2;
   }
   const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
+  if (drop.p > 0.f && drop.keep)
+    return launch_masked<true>(q, k, v, out, BN, (int)N, (int)L, d, scale, da, drop.keep, st);
   switch (d) {
     case 16: return launch_operands_small<16>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
     case 32: return launch_operands_small<32>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
@@ -1707,6 +1750,10 @@ int launch_flash_attn(const void* q, const void* k, const void* v, void* out, in
     set_error("flash_attn: B*N=%lld, Lq=%lld or Lk=%lld beyond the grid limits", (long long)BN,
               (long long)L, (long long)Lk);
     return -2;
+  }
+  if (drop.p > 0.f && drop.keep && f16 && L == Lk && out_blnd) {
+    const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
+    return launch_masked<false>(q, k, v, out, BN, (int)N, (int)L, d, scale, da, drop.keep, st);
   }
   return f16 ? launch_t<_Float16>(q, k, v, out, BN, (int)N, (int)L, (int)Lk, d, scale, drop,
                                   out_blnd, st)

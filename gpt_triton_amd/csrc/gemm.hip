@@ -1039,6 +1039,7 @@ static int make_epi(const GemmEpilogue& e, int64_t M, int N, EpiDev& ep) {
   ep.gelu = e.gelu;
   ep.drop = DropoutArgs{e.qkv ? 0.f : e.drop.p, (unsigned)e.drop.seed,
                         (unsigned)(e.drop.seed >> 32)};
+  ep.keep = (const unsigned char*)e.drop.keep;
   const uintptr_t amask = e.f16 ? 7 : 15;
   auto aligned = [&](const void* p) { return p == nullptr || ((uintptr_t)p & amask) == 0; };
   const bool vec = (N % 4) == 0 && aligned(e.bias) && aligned(e.residual) && aligned(e.out) &&

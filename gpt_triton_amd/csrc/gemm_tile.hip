@@ -302,6 +302,21 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     }
   }
 
+  // the dropout mask of those chunks, where the caller has it: CW bits of one byte (N and n are
+  // multiples of CW then).  Generated in the epilogue, 17 wide products per element, it more than
+  // doubled the time of the launch (4800 x 768 x 3072: 85 us; 43 with the bits, 36 without dropout).
+  unsigned keep_v[DROP ? IT : 1];
+  if constexpr (DROP) {
+    if (ep.keep != nullptr && col_ok) {
+#pragma unroll
+      for (int it = 0; it < IT; ++it) {
+        const int m = m0 + r_first + it * RSTEP;
+        const uint64_t at = (uint64_t)m * (uint64_t)N + (uint64_t)n;
+        keep_v[it] = m < M ? (unsigned)ep.keep[at >> 3] >> (at & 7) : 0u;
+      }
+    }
+  }
+
   // One k-step: the MFMAs of its first half with the fragment reads of its second half dealt
   // between them; the barrier that publishes k-step t + 1 and frees this stage; the MFMAs of the
   // second half with the reads of the next k-step's first half and the refill of this stage
@@ -399,10 +414,16 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
       if (ep.gelu) z[e] = gelu_new(z[e]);
     }
     if constexpr (DROP) {
-      unsigned off[CW];
+      if (ep.keep != nullptr) {
+        const KeepScale scale(ep.drop.p);
 #pragma unroll
-      for (int e = 0; e < CW; ++e) off[e] = (unsigned)((uint64_t)m * (uint64_t)N + (uint64_t)(n + e));
-      dropout_apply<CW>(ep.drop, off, z);
+        for (int e = 0; e < CW; ++e) z[e] = keep_if(keep_v[it], e, scale(z[e]));
+      } else {
+        unsigned off[CW];
+#pragma unroll
+        for (int e = 0; e < CW; ++e) off[e] = (unsigned)((uint64_t)m * (uint64_t)N + (uint64_t)(n + e));
+        dropout_apply<CW>(ep.drop, off, z);
+      }
     }
     OV o;
 #pragma unroll

@@ -10,7 +10,11 @@ namespace gptmi {
 struct Dropout {
   float p;
   uint64_t seed;
+  const void* keep = nullptr;  // the mask's bits, if the caller has them (launch_dropout_mask)
 };
+
+// Bit o % 32 of word o / 32 of `mask`: whether offset o is kept, for all o below 32 * words.
+void launch_dropout_mask(void* mask, int64_t words, Dropout drop, hipStream_t st);
 
 int launch_embed(const int64_t* ids, const void* wte, const void* wpe, void* out,
                  int64_t rows, int64_t L, int64_t V, int H, Dropout drop, bool f16, hipStream_t st);

@@ -21,7 +21,8 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 
-from .kernels import (HEAD_SIZES, attention_block, block_supported, flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
+from .kernels import (HEAD_SIZES, attention_block, block_supported, dropout_mask,
+                      flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
                       fused_layer_norm, layer_norm_ffn, layer_norm_linear_supported,
                       layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, mlp_block,
                       pack_lm_head, pack_weight)
@@ -48,9 +49,9 @@ def _ln_in_gemm(x, weight):
             layer_norm_linear_supported(x, weight))
 
 
-def _as_block(x, width):
-    return ((x.dtype == torch.float32 or x.numel() // width <= BLOCK_MAX_ROWS) and
-            block_supported(x, width))
+def _as_block(x, width, keep=None):
+    return ((keep is not None or x.dtype == torch.float32 or
+             x.numel() // width <= BLOCK_MAX_ROWS) and block_supported(x, width))
 
 
 # dense fp16/bf16 tensor throughput, FLOP/s
@@ -60,6 +61,31 @@ GPU_TO_FLOPS = {
     "h100": 989 * 10**12,
     "mi355x": 2500 * 10**12,
 }
+
+
+def _keep_mask(x, width, layers, heads, p):
+    """The dropout mask of a training forward's blocks, or None where the kernels draw their own: sizes
+    the block calls do not take, and more offsets than the generator has.  The reference draws the
+    masks of all layers from one seed at offsets that count from 0, so they are all parts of the mask
+    of the widest matrix ([tokens, 4 * width]; attention weights: the first L * L offsets).  Drawn
+    once per forward instead of in every kernel that applies it: 16 x 300 tokens 124M, each of 12 ffn1
+    launches 85 -> 43 us, projections and ffn2 32 -> 22, attentions 72 -> 20, for one launch of 24."""
+    tokens, seqlen = x.numel() // width, x.shape[1]
+    bits = max(tokens * 4 * width, seqlen * seqlen)
+    if (layers == 0 or bits > 1 << 32 or not block_supported(x, width) or width % heads != 0 or
+            width // heads not in HEAD_SIZES):
+        return None
+    return dropout_mask(bits, p, x)
+
+
+class _Block(nn.Sequential):
+    """nn.Sequential(FusedAttention, FusedMLP) whose two modules may be handed a dropout mask.  Any
+    other module put in their place is called as nn.Sequential calls it."""
+
+    def forward(self, x, keep=None):
+        for module in self:
+            x = module(x, keep=keep) if type(module) in (FusedAttention, FusedMLP) else module(x)
+        return x
 
 
 class _PackedWeights:
@@ -119,18 +145,22 @@ class FusedAttention(nn.Module):
         self._packed.clear()
         return super().train(mode)
 
-    def forward(self, x, normed=None):
+    def forward(self, x, normed=None, keep=None):
         """`normed`: LayerNorm(x) with this block's weights, if the caller already has it (the
-        first block of FusedGPT gets it from the embedding kernel)."""
+        first block of FusedGPT gets it from the embedding kernel).  `keep`: a `dropout_mask`, used
+        if it is for this module's dropout and these sizes."""
         p = self.dropout_prob if self.training else 0.0
+        if keep is not None and not (p > 0.0 and keep.serves(x, max(x.numel(), x.shape[1] ** 2), p)):
+            keep = None
         prm = self._parameters
         w_attn = self._weight("c_attn_weight")
         in_gemm = normed is None and p == 0.0 and _ln_in_gemm(x, w_attn)
-        if _as_block(x, self.hidden_size) and self.hidden_size // self.num_heads in HEAD_SIZES:
+        if (_as_block(x, self.hidden_size, keep) and
+                self.hidden_size // self.num_heads in HEAD_SIZES):
             return attention_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w_attn,
                                    prm["c_attn_bias"], self._weight("c_proj_weight"),
                                    prm["c_proj_bias"], self.num_heads, dropout_prob=p,
-                                   normed=normed, layer_norm_in_gemm=in_gemm)
+                                   normed=normed, layer_norm_in_gemm=in_gemm, keep=keep)
         skip = x
         y = normed
         if in_gemm:
@@ -178,16 +208,19 @@ class FusedMLP(nn.Module):
         self._packed.clear()
         return super().train(mode)
 
-    def forward(self, x):
+    def forward(self, x, keep=None):
+        """`keep`: as in FusedAttention.forward."""
         p = self.dropout_prob if self.training else 0.0
+        if keep is not None and not (p > 0.0 and keep.serves(x, 4 * x.numel(), p)):
+            keep = None
         prm = self._parameters
         w1, w2 = self._weight("ffn1_weight"), self._weight("ffn2_weight")
         if p == 0.0 and _ln_in_gemm(x, w1):
             return layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                                   bias=prm["ffn1_bias"], add_gelu=True, then=(w2, prm["ffn2_bias"]))
-        if _as_block(x, self.hidden_size):
+        if _as_block(x, self.hidden_size, keep):
             return mlp_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
-                             prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p)
+                             prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p, keep=keep)
         y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
         y = fused_ffn(y, w1, bias=prm["ffn1_bias"].data, residual=None, add_gelu=True,
                       dropout_prob=p)
@@ -221,8 +254,8 @@ class FusedGPT(nn.Module):
         self.wte_weight = nn.Parameter(torch.rand(config.vocab_size, h))
         self.wpe_weight = nn.Parameter(torch.rand(config.block_size, h))
         self.blocks = nn.ModuleList([
-            nn.Sequential(FusedAttention(h, config.n_head, dropout_prob=config.dropout),
-                          FusedMLP(h, dropout_prob=config.dropout))
+            _Block(FusedAttention(h, config.n_head, dropout_prob=config.dropout),
+                   FusedMLP(h, dropout_prob=config.dropout))
             for _ in range(config.n_layer)
         ])
         self.layer_norm_weight = nn.Parameter(torch.ones((h,)))
@@ -260,8 +293,9 @@ class FusedGPT(nn.Module):
         else:
             x = fused_embeddings(x, self.wte_weight.data, self.wpe_weight.data, dropout_prob=p)
             rest = blocks
+        keep = _keep_mask(x, self.config.n_embd, len(rest), self.config.n_head, p) if p > 0.0 else None
         for block in rest:
-            x = block(x)
+            x = block(x, keep=keep) if keep is not None and type(block) is _Block else block(x)
         x = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)
         if return_logits:
             return x, lm_head(x, self._lm_head_weight())

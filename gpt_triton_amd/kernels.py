@@ -430,6 +430,37 @@ def flash_attention_v1(q, k, v, dropout_prob=0.0, *, merged_heads_layout=False):
     return buf.transpose(1, 2) if merged_heads_layout else buf
 
 
+class DropoutMask:
+    """Bits of the dropout mask that `fused_ffn` (offset m * N + n) and `flash_attention_v1` (offset
+    query * Lk + key) draw for probability p: both count flat indices from 0 under one seed, so the
+    mask of the largest matrix serves all of them.  `bits` offsets are held."""
+
+    __slots__ = ("data", "bits", "p", "device")
+
+    def __init__(self, data, bits, p):
+        self.data, self.bits, self.p, self.device = data, bits, p, data.device
+
+    def serves(self, x, bits, p):
+        return self.p == p and bits <= self.bits and self.data.get_device() == x.get_device()
+
+
+def dropout_mask(bits, p, like):
+    """DropoutMask of `bits` offsets (at most 2^32) for 0 < p < 1 on the GPU of `like`."""
+    dev = _on_gpu(like)
+    lib = _lib.load()
+    buf = like.new_empty(lib.gptmi_dropout_mask_bytes(bits), dtype=torch.uint8)
+    _call(dev, "dropout_mask", lib.gptmi_dropout_mask, buf.data_ptr(), bits, float(p), 1337)
+    return DropoutMask(buf, bits, p)
+
+
+def _keep_args(keep, x, dropout_prob, what):
+    if keep is None:
+        return None, 0
+    if dropout_prob != keep.p or keep.data.get_device() != x.get_device():
+        raise ValueError(f"{what}: the dropout mask is for p = {keep.p} on {keep.device}")
+    return keep.data.data_ptr(), keep.bits
+
+
 # Head sizes of the attention kernels (the reference's set, kernels.py:490).
 HEAD_SIZES = frozenset((16, 32, 64, 128, 256))
 
@@ -447,10 +478,12 @@ def _block_layout(first, second, what):
 
 
 def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, num_heads,
-                    dropout_prob=0.0, normed=None, layer_norm_in_gemm=False):
+                    dropout_prob=0.0, normed=None, layer_norm_in_gemm=False, keep=None):
     """x + dropout(proj(attention(qkv(LayerNorm(x))))) for x [B, L, h]: the operators of an attention
     block (gpt.py:39-60) behind one call of the library, with their bits.  `normed`: LayerNorm(x), if
-    the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`."""
+    the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`; keep: a
+    `dropout_mask` for dropout_prob of at least max(x.numel(), L * L) offsets, read instead of
+    generating the masks here."""
     B, L, h = x.shape
     dtype = x.dtype
     dev = _on_gpu(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, normed)
@@ -473,15 +506,16 @@ def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, pr
     _call(dev, "attention_block", lib.gptmi_attention_block, x.data_ptr(), _ptr(normed),
           ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, qkv_weight.data_ptr(), qkv_bias.data_ptr(),
           proj_weight.data_ptr(), proj_bias.data_ptr(), out.data_ptr(), B, L, num_heads, d,
-          float(dropout_prob), 1337, 1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
+          float(dropout_prob), 1337, *_keep_args(keep, x, dropout_prob, "attention_block"),
+          1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
     return out
 
 
 def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_prob=0.0,
-              layer_norm_in_gemm=False):
+              layer_norm_in_gemm=False, keep=None):
     """x + dropout(W2 . dropout(gelu(W1 . LayerNorm(x)))): the operators of an MLP block
     (gpt.py:91-111) behind one call of the library, with their bits; layer_norm_in_gemm: as in
-    `layer_norm_ffn`."""
+    `layer_norm_ffn`; keep: as in `attention_block`, of at least (rows of x) * max(inner, h) offsets."""
     h = x.shape[-1]
     dtype = x.dtype
     inner = weight1.shape[1]
@@ -503,5 +537,5 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     _call(dev, "mlp_block", lib.gptmi_mlp_block, x.data_ptr(), ln_weight.data_ptr(),
           ln_bias.data_ptr(), 1e-5, weight1.data_ptr(), bias1.data_ptr(), weight2.data_ptr(),
           bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337,
-          1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
+          *_keep_args(keep, x, dropout_prob, "mlp_block"), 1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
     return out

@@ -278,6 +278,15 @@ int gptmi_flash_attn(const void* q, const void* k, const void* v, void* out,
                      void* stream);
 
 /*
+ * The dropout mask of gptmi_linear and gptmi_flash_attn as bits: bit o % 32 of 32-bit word o / 32 is set
+ * iff offset o < n is kept, rand(seed, o) > p.  Both count flat indices from 0, so one mask of the
+ * largest matrix serves all the layers of a forward; 1 <= n <= 2^32.  gptmi_dropout_mask_bytes(n) is what
+ * the array needs (it reads as a few words longer than n bits).
+ */
+size_t gptmi_dropout_mask_bytes(int64_t n);
+int gptmi_dropout_mask(void* mask, int64_t n, float p, uint64_t seed, void* stream);
+
+/*
  * A whole attention block, x + proj(attention(qkv(LayerNorm(x)))), and a whole MLP block,
  * x + W2 . gelu(W1 . LayerNorm(x)), behind one call each: the launches of gptmi_layernorm (or the
  * LayerNorm prologue, or `normed` = LayerNorm(x) from gptmi_embed_layernorm), gptmi_linear_qkv,
@@ -290,6 +299,9 @@ int gptmi_flash_attn(const void* q, const void* k, const void* v, void* out,
  *   W_qkv [h][3h], W_proj [h][h], W1 [H][inner], W2 [inner][H]: all GPTMI_W_KN or all packed
  *   h = heads*d and H and inner multiples of 64, h and H up to 8192; d as in gptmi_flash_attn
  *   p, seed: dropout of the attention weights and of the projection's output (MLP: of both products)
+ *   keep, keep_bits: gptmi_dropout_mask's result for this p and seed and its n, at least
+ *                   max(B*L*h, L*L) (MLP: M * max(inner, H)) and at most 2^32, or NULL, 0: the
+ *                   kernels generate the mask themselves
  *   fuse_layernorm: 1 = the LayerNorm prologue (see gptmi_layernorm_linear_supported)
  * workspace: the given number of bytes, 256-byte aligned.
  */
@@ -298,13 +310,14 @@ size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads
 int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b,
                           float eps, const void* W_qkv, const void* b_qkv, const void* W_proj,
                           const void* b_proj, void* out, int64_t B, int64_t L, int64_t heads,
-                          int64_t d, float p, uint64_t seed, int fuse_layernorm, int wlayout,
-                          void* workspace, size_t workspace_bytes, int dtype, void* stream);
+                          int64_t d, float p, uint64_t seed, const void* keep,
+                          int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace,
+                          size_t workspace_bytes, int dtype, void* stream);
 size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int wlayout);
 int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps, const void* W1,
                     const void* b1, const void* W2, const void* b2, void* out, int64_t M,
-                    int64_t H, int64_t inner, float p, uint64_t seed, int fuse_layernorm,
-                    int wlayout, void* workspace, size_t workspace_bytes, int dtype,
+                    int64_t H, int64_t inner, float p, uint64_t seed, const void* keep,
+                    int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace, size_t workspace_bytes, int dtype,
                     void* stream);
 
 #ifdef __cplusplus

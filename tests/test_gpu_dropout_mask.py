@@ -1,0 +1,82 @@
+"""dropout_mask (the generator's decisions as bits) against the oracle's generator, and the block
+functions and the model reading it against the same kernels drawing the masks themselves: the same
+decisions and the same arithmetic on what is kept, so equal bits."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import gpt2_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(gpu_device):
+    from gpt_triton_amd import kernels
+
+    return kernels
+
+
+@pytest.mark.parametrize("bits", [1, 31, 32, 33, 8191, 8192 * 32 + 5, 1 << 20])
+@pytest.mark.parametrize("p", [0.1, 0.5, 0.999])
+def test_mask_bits(K, gpu_device, bits, p):
+    print(f"dropout_mask {bits} p={p}", flush=True)
+    like = torch.empty(1, device=gpu_device)
+    words = K.dropout_mask(bits, p, like).data.cpu().numpy().view(np.uint8)
+    got = np.unpackbits(words, bitorder="little")[:bits].astype(bool)
+    u = O.tl_rand(1337, np.arange(bits, dtype=np.uint32))
+    assert np.array_equal(got, u > np.float32(p))
+
+
+def block_params(h, dtype, device, seed):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    rn = lambda *s, std=1.0, mean=0.0: (mean + std * torch.randn(*s, generator=g)).to(dtype).to(device)
+    ln = (rn(h, std=0.2, mean=1.0), rn(h, std=0.1))
+    att = (rn(h, 3 * h, std=h**-0.5), rn(3 * h, std=0.1), rn(h, h, std=h**-0.5), rn(h, std=0.1))
+    mlp = (rn(h, 4 * h, std=h**-0.5), rn(4 * h, std=0.1), rn(4 * h, h, std=0.5 * h**-0.5),
+           rn(h, std=0.1))
+    return ln, att, mlp, rn
+
+
+# head sizes 16 to 256; one row, ragged tiles, sequences whose rows of the attention mask start at
+# every bit of a word, and L * L beyond the matrices' offsets
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,L,h,heads", [(1, 1, 64, 1), (3, 65, 192, 6), (2, 37, 128, 8), (2, 321, 128, 2),
+                                         (6, 100, 768, 12), (1, 300, 256, 2), (2, 130, 256, 1),
+                                         (16, 300, 128, 2), (1, 1023, 64, 1)])
+def test_blocks_with_the_mask(K, gpu_device, dtype, B, L, h, heads):
+    print(f"blocks with a dropout mask {dtype} B={B} L={L} h={h} heads={heads}", flush=True)
+    ln, att, mlp, rn = block_params(h, dtype, gpu_device, seed=L + h)
+    x, p = rn(B, L, h), 0.1
+    keep = K.dropout_mask(max(4 * x.numel(), L * L), p, x)
+    want = K.attention_block(x, *ln, *att, heads, dropout_prob=p)
+    got = K.attention_block(x, *ln, *att, heads, dropout_prob=p, keep=keep)
+    assert torch.equal(got, want)
+    want = K.mlp_block(x, *ln, *mlp, dropout_prob=p)
+    assert torch.equal(K.mlp_block(x, *ln, *mlp, dropout_prob=p, keep=keep), want)
+    with pytest.raises(ValueError):
+        K.mlp_block(x, *ln, *mlp, dropout_prob=0.2, keep=keep)
+    with pytest.raises(RuntimeError, match="mask"):
+        K.mlp_block(x, *ln, *mlp, dropout_prob=p, keep=K.dropout_mask(4 * x.numel() - 1, p, x))
+
+
+def test_training_forward_module_by_module(K, gpu_device):
+    """FusedGPT draws one mask; its modules called one by one draw their own.  A module with another
+    dropout probability, and another module in an MLP's place, do not take the model's mask."""
+    from gpt_triton_amd.gpt import FusedGPT, GPTConfig
+
+    cfg = GPTConfig(vocab_size=512, block_size=128, n_layer=3, n_head=2, n_embd=128, dropout=0.1)
+    model = FusedGPT(cfg).init_synthetic_().to(gpu_device).half().train()
+    model.blocks[1][0].dropout_prob = 0.3
+    model.blocks[2][1] = torch.nn.Identity()
+    seen = []
+    model.blocks[0].register_forward_hook(lambda *_: seen.append(1))
+    ids = torch.randint(0, 512, (3, 77), device=gpu_device)
+    with torch.no_grad():
+        got = model(ids)
+        x = K.fused_embeddings(ids, model.wte_weight.data, model.wpe_weight.data, dropout_prob=0.1)
+        for block in model.blocks:
+            for module in block:
+                x = module(x)
+        want = K.fused_layer_norm(x, model.layer_norm_weight.data, model.layer_norm_bias.data)
+    assert torch.equal(got, want) and seen == [1]
