@@ -198,12 +198,16 @@ struct Carver {
   }
 };
 
-// The weight image a product reads: the caller's (packed), or one built into `ws`.
-static const void* weight_image(const void* W, void* ws, int64_t N, int64_t K, int wlayout, bool f16,
-                                hipStream_t st) {
-  if (wlayout == GPTMI_W_PACKED) return W;
-  launch_pack_transpose(W, ws, (int)K, (int)N, (int)round_up(K, 64), f16, st);
-  return ws;
+// The weight images that a block's two products read: the caller's (packed), or built into ws1 and ws2.
+// K1 and K2 are multiples of 64.
+struct WeightImages {
+  const void *first, *second;
+};
+static WeightImages weight_images(const void* W1, void* ws1, int64_t K1, int64_t N1, const void* W2,
+                                  void* ws2, int64_t K2, int64_t N2, int wlayout, bool f16, hipStream_t st) {
+  if (wlayout == GPTMI_W_PACKED) return {W1, W2};
+  launch_pack_transpose_pair(W1, ws1, (int)K1, (int)N1, W2, ws2, (int)K2, (int)N2, f16, st);
+  return {ws1, ws2};
 }
 static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
   return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
@@ -613,8 +617,7 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const void* Bq = weight_image(W_qkv, pl.w_qkv, 3 * h, h, wlayout, f16, st);
-  const void* Bp = weight_image(W_proj, pl.w_proj, h, h, wlayout, f16, st);
+  const auto [Bq, Bp] = weight_images(W_qkv, pl.w_qkv, h, 3 * h, W_proj, pl.w_proj, h, h, wlayout, f16, st);
   if (((uintptr_t)x & 15) || ((uintptr_t)normed & 15) || ((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
     set_error("attention_block: x and the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
@@ -680,8 +683,7 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const void* B1 = weight_image(W1, pl.w1, inner, H, wlayout, f16, st);
-  const void* B2 = weight_image(W2, pl.w2, H, inner, wlayout, f16, st);
+  const auto [B1, B2] = weight_images(W1, pl.w1, H, inner, W2, pl.w2, inner, H, wlayout, f16, st);
   if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
     set_error("mlp_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;

@@ -30,6 +30,9 @@ void launch_pack_rows(const void* src, void* dst, int64_t R, int K, int Kp, bool
                       hipStream_t st);
 void launch_pack_transpose(const void* src, void* dst, int K, int N, int Kp, bool f16,
                            hipStream_t st);
+// two weights, K1 and K2 multiples of 64
+void launch_pack_transpose_pair(const void* s1, void* d1, int K1, int N1, const void* s2, void* d2, int K2,
+                                int N2, bool f16, hipStream_t st);
 
 // Epilogue description of one GEMM launch: out = gelu?(acc + bias) + residual,
 // stored either as a plain [M][N] matrix or scattered into q/k/v [B][heads][L][d].
