@@ -80,3 +80,18 @@ def test_training_forward_module_by_module(K, gpu_device):
                 x = module(x)
         want = K.fused_layer_norm(x, model.layer_norm_weight.data, model.layer_norm_bias.data)
     assert torch.equal(got, want) and seen == [1]
+
+
+# one chunk of columns, workgroups of several rows with idle threads, exactly 256 and just past 256
+# chunks, rows that are no whole chunks; fewer rows than a workgroup takes and many
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,L,H", [(1, 1, 8), (2, 5, 768), (3, 700, 96), (1, 9, 2048), (2, 3, 2056), (1, 7, 100),
+                                   (1, 7, 1024), (1, 7, 1028)])
+def test_embedding_dropout(K, gpu_device, dtype, B, L, H):
+    print(f"embedding dropout {dtype} B={B} L={L} H={H}", flush=True)
+    r = np.random.default_rng(H + L)
+    npdt = np.float16 if dtype == torch.float16 else np.float32
+    wte, wpe = r.standard_normal((50, H)).astype(npdt), r.standard_normal((L, H)).astype(npdt)
+    ids = r.integers(0, 50, (B, L))
+    got = K.fused_embeddings(*(torch.from_numpy(t).to(gpu_device) for t in (ids, wte, wpe)), dropout_prob=0.1)
+    assert np.array_equal(got.cpu().numpy(), O.fused_embeddings(ids, wte, wpe, dropout_prob=0.1))
