@@ -618,8 +618,8 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
   const auto [Bq, Bp] = weight_images(W_qkv, pl.w_qkv, h, 3 * h, W_proj, pl.w_proj, h, h, wlayout, f16, st);
-  if (((uintptr_t)x & 15) || ((uintptr_t)normed & 15) || ((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
-    set_error("attention_block: x and the weights must be 16-byte aligned");
+  if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
+    set_error("attention_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
   }
   GemmEpilogue ep = {};
@@ -643,8 +643,8 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   } else {
     const void* A = pl.normed;
     if (!normed) launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)h, eps, f16, true, st);
-    else if (f16) A = normed;
-    else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, false, st);
+    else if (f16 && ((uintptr_t)normed & 15) == 0) A = normed;
+    else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, f16, st);
     rc = launch_gemm(A, Bq, M, (int)(3 * h), (int)h, ep, st);
   }
   if (rc) return rc;

@@ -275,8 +275,13 @@ __global__ __launch_bounds__(256) void layernorm_scalar_kernel(
   const float var = wave_sum(q) / (float)H;
   const float rstd = 1.0f / sqrtf(var + eps);
   for (int c = lane; c < H; c += 64) {
-    const float z = ((float)xr[c] - mean) * rstd;
-    out[row * H + c] = (OT)(z * (float)w[c] + (float)b[c]);
+    if constexpr (sizeof(T) != sizeof(OT)) {
+      // fp32 rows with an fp16 output stand for the fp32 LayerNorm and a conversion: two roundings
+      out[row * H + c] = (OT)layernorm_apply((float)xr[c], mean, rstd, (float)w[c], (float)b[c]);
+    } else {
+      const float z = ((float)xr[c] - mean) * rstd;
+      out[row * H + c] = (OT)(z * (float)w[c] + (float)b[c]);
+    }
   }
 }
 

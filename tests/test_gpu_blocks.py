@@ -96,3 +96,28 @@ def test_blocks_turn_down_what_they_do_not_hold(K, gpu_device):
         K.mlp_block(x, P["ln_w"], P["ln_b"], K.pack_weight(P["w1"]), P["b1"], P["w2"], P["b2"])
     with pytest.raises(RuntimeError, match="GPU only"):
         K.mlp_block(x.cpu(), P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
+
+
+# x (and LayerNorm(x)) on storage that is aligned to its element only: the operators take it
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,L,h,heads", [(2, 37, 128, 2), (3, 300, 64, 1)])
+def test_blocks_on_unaligned_rows(K, gpu_device, dtype, B, L, h, heads):
+    print(f"blocks, unaligned rows {dtype} B={B} L={L} h={h}", flush=True)
+    P, rn = params(h, dtype, gpu_device, seed=L)
+    shift = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    x = shift(rn(B, L, h))
+    assert x.data_ptr() % 16 == x.element_size()
+    y = K.fused_layer_norm(x, P["ln_w"], P["ln_b"])
+    q, k, v = K.matmul_and_split_qkv(y, P["qkv"], P["qkv_b"], heads)
+    a = K.flash_attention_v1(q, k, v).transpose(1, 2).contiguous().view(x.shape)
+    want = K.fused_ffn(a, P["proj"], bias=P["proj_b"], residual=x)
+    # equal bits in fp16; in fp32 the bound at the head of this file
+    sums = (a.abs().float().view(-1, h) @ P["proj"].abs().float()).view_as(want)
+    bound = 0 if dtype == torch.float16 else 2.0**-11 * sums + 1e-5 * want.abs().max()
+    for normed in (None, y, shift(y)):
+        got = K.attention_block(x, P["ln_w"], P["ln_b"], P["qkv"], P["qkv_b"], P["proj"], P["proj_b"],
+                                heads, normed=normed)
+        assert float(((got - want).abs() - bound).max()) <= 0
+    got = K.mlp_block(x, P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
+    y = K.fused_ffn(y, P["w1"], bias=P["b1"], add_gelu=True)
+    assert torch.equal(got, K.fused_ffn(y, P["w2"], bias=P["b2"], residual=x))
