@@ -118,6 +118,15 @@ def _norm_flops(tokens, width):
     return 2 * tokens * width
 
 
+def _tensors(module, names):
+    """The tensors of a module by name: its dictionary of parameters where that has them all (an
+    attribute of an nn.Module takes a failed lookup of its class and instance first, and a forward of
+    few tokens waits for the host), else its attributes, which is where pruning, parametrisations
+    and replicas put what stands in a parameter's place."""
+    prm = module._parameters
+    return prm if names <= prm.keys() else {name: getattr(module, name) for name in names}
+
+
 class FusedAttention(nn.Module):
     """Pre-LN causal self-attention block: x + proj(attention(qkv(LN(x))))."""
 
@@ -135,9 +144,15 @@ class FusedAttention(nn.Module):
         self.c_proj_bias = nn.Parameter(torch.rand(h))
         self._packed = _PackedWeights()
 
-    def _weight(self, name):
-        prm = self._parameters[name]
-        if self.training or (self.hidden_size // self.num_heads) % 8 != 0:
+    _NAMES = frozenset(("layer_norm_weight", "layer_norm_bias", "c_attn_weight", "c_attn_bias",
+                        "c_proj_weight", "c_proj_bias"))
+
+    def _weight(self, name, tensors=None):
+        # an image is kept for a parameter only: what stands in for one is another tensor every time
+        tensors = tensors or _tensors(self, self._NAMES)
+        prm = tensors[name]
+        if (self.training or tensors is not self._parameters or
+                (self.hidden_size // self.num_heads) % 8 != 0):
             return prm.data
         return self._packed.get(name, prm)
 
@@ -152,13 +167,13 @@ class FusedAttention(nn.Module):
         p = self.dropout_prob if self.training else 0.0
         if keep is not None and not (p > 0.0 and keep.serves(x, max(x.numel(), x.shape[1] ** 2), p)):
             keep = None
-        prm = self._parameters
-        w_attn = self._weight("c_attn_weight")
+        prm = _tensors(self, self._NAMES)
+        w_attn = self._weight("c_attn_weight", prm)
         in_gemm = normed is None and p == 0.0 and _ln_in_gemm(x, w_attn)
         if (_as_block(x, self.hidden_size, keep) and
                 self.hidden_size // self.num_heads in HEAD_SIZES):
             return attention_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w_attn,
-                                   prm["c_attn_bias"], self._weight("c_proj_weight"),
+                                   prm["c_attn_bias"], self._weight("c_proj_weight", prm),
                                    prm["c_proj_bias"], self.num_heads, dropout_prob=p,
                                    normed=normed, layer_norm_in_gemm=in_gemm, keep=keep)
         skip = x
@@ -174,7 +189,7 @@ class FusedAttention(nn.Module):
         # [B, N, L, d] values in a [B, L, N, d] buffer: the head merge below copies nothing
         y = flash_attention_v1(q, k, v, dropout_prob=p, merged_heads_layout=True)
         y = y.transpose(1, 2).contiguous().view(skip.shape)
-        return fused_ffn(y, self._weight("c_proj_weight"), bias=prm["c_proj_bias"].data,
+        return fused_ffn(y, self._weight("c_proj_weight", prm), bias=prm["c_proj_bias"].data,
                          residual=skip, add_gelu=False, dropout_prob=p)
 
     def get_fwd_flops(self, num_tokens):
@@ -200,9 +215,16 @@ class FusedMLP(nn.Module):
         self.ffn2_bias = nn.Parameter(torch.rand(h))
         self._packed = _PackedWeights()
 
-    def _weight(self, name):
-        prm = self._parameters[name]
-        return prm.data if self.training else self._packed.get(name, prm)
+    _NAMES = frozenset(("layer_norm_weight", "layer_norm_bias", "ffn1_weight", "ffn1_bias",
+                        "ffn2_weight", "ffn2_bias"))
+
+    def _weight(self, name, tensors=None):
+        # as in FusedAttention
+        tensors = tensors or _tensors(self, self._NAMES)
+        prm = tensors[name]
+        if self.training or tensors is not self._parameters:
+            return prm.data
+        return self._packed.get(name, prm)
 
     def train(self, mode=True):
         self._packed.clear()
@@ -213,8 +235,8 @@ class FusedMLP(nn.Module):
         p = self.dropout_prob if self.training else 0.0
         if keep is not None and not (p > 0.0 and keep.serves(x, 4 * x.numel(), p)):
             keep = None
-        prm = self._parameters
-        w1, w2 = self._weight("ffn1_weight"), self._weight("ffn2_weight")
+        prm = _tensors(self, self._NAMES)
+        w1, w2 = self._weight("ffn1_weight", prm), self._weight("ffn2_weight", prm)
         if p == 0.0 and _ln_in_gemm(x, w1):
             return layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                                   bias=prm["ffn1_bias"], add_gelu=True, then=(w2, prm["ffn2_bias"]))

@@ -121,3 +121,32 @@ def test_blocks_on_unaligned_rows(K, gpu_device, dtype, B, L, h, heads):
     got = K.mlp_block(x, P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
     y = K.fused_ffn(y, P["w1"], bias=P["b1"], add_gelu=True)
     assert torch.equal(got, K.fused_ffn(y, P["w2"], bias=P["b2"], residual=x))
+
+
+# where something else stands in a parameter's place the modules read it through the attribute, and
+# follow it when it changes
+@pytest.mark.parametrize("how", ["prune", "parametrize"])
+def test_modules_with_replaced_parameters(K, gpu_device, how):
+    from torch.nn.utils import parametrize, prune
+
+    from gpt_triton_amd.gpt import FusedAttention, FusedMLP
+
+    torch.manual_seed(2)
+    x = torch.randn(2, 70, 128, device=gpu_device, dtype=torch.float16)
+    for module, name in ((FusedAttention(128, 2), "c_attn_weight"), (FusedMLP(128), "ffn1_weight")):
+        for prm in module.parameters():
+            prm.data.normal_(0.0, 0.05)
+        module = module.to(gpu_device).half().eval()
+        want = module(x)
+        if how == "prune":
+            prune.identity(module, name)
+            source = getattr(module, name + "_orig")
+        else:
+            parametrize.register_parametrization(module, name, torch.nn.Identity())
+            source = getattr(module.parametrizations, name).original
+        assert torch.equal(module(x), want)
+        with torch.no_grad():
+            source.mul_(2)
+        changed = module(x)
+        (prune.remove if how == "prune" else parametrize.remove_parametrizations)(module, name)
+        assert torch.equal(changed, module(x)) and not torch.equal(changed, want)
