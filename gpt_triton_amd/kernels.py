@@ -486,6 +486,8 @@ def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, pr
     generating the masks here."""
     B, L, h = x.shape
     dtype = x.dtype
+    assert ln_weight.shape[0] == ln_bias.shape[0] == proj_bias.shape[0] == h
+    assert qkv_bias.shape[0] == 3 * h
     dev = _on_gpu(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, normed)
     assert x.is_contiguous() and (normed is None or normed.is_contiguous() and normed.shape == x.shape)
     assert ln_weight.is_contiguous() and ln_bias.is_contiguous()
@@ -519,6 +521,7 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     h = x.shape[-1]
     dtype = x.dtype
     inner = weight1.shape[1]
+    assert ln_weight.shape[0] == ln_bias.shape[0] == bias2.shape[0] == h and bias1.shape[0] == inner
     dev = _on_gpu(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2)
     assert x.is_contiguous() and ln_weight.is_contiguous() and ln_bias.is_contiguous()
     assert weight1.is_contiguous() and weight2.is_contiguous()

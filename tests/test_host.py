@@ -156,6 +156,27 @@ def test_cpu_tensors_are_refused_not_emulated(lib):
         K.flash_attention_v1(q, q, q)
 
 
+@pytest.mark.parametrize("name", ["layer_norm_weight", "layer_norm_bias", "c_attn_bias", "c_proj_bias",
+                                  "ffn1_bias", "ffn2_bias"])
+def test_blocks_check_the_sizes_of_their_vectors(lib, name):
+    """A vector shorter than the kernels read is refused as by the single operators, before the
+    library is called."""
+    from gpt_triton_amd import kernels
+
+    h = 64
+    vec = {"layer_norm_weight": h, "layer_norm_bias": h, "c_attn_bias": 3 * h, "c_proj_bias": h,
+           "ffn1_bias": 4 * h, "ffn2_bias": h}
+    vec = {k: torch.zeros(n - 1 if k == name else n) for k, n in vec.items()}
+    x, ln = torch.zeros(1, 2, h), (vec["layer_norm_weight"], vec["layer_norm_bias"])
+    attention = lambda: kernels.attention_block(x, *ln, torch.zeros(h, 3 * h), vec["c_attn_bias"],
+                                                torch.zeros(h, h), vec["c_proj_bias"], 1)
+    mlp = lambda: kernels.mlp_block(x, *ln, torch.zeros(h, 4 * h), vec["ffn1_bias"],
+                                    torch.zeros(4 * h, h), vec["ffn2_bias"])
+    for block, takes in ((attention, not name.startswith("ffn")), (mlp, not name.startswith("c_"))):
+        with pytest.raises(AssertionError if takes else RuntimeError):
+            block()
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys
