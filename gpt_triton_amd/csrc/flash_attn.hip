@@ -57,28 +57,29 @@ template <> struct Ld8<float> {
 // scores, scale * log2(e) folded into one fused multiply-add in front of the hardware's exp2, a
 // reciprocal for the denominator -- the same real-number formula as the reference, two VALU
 // operations per score fewer.  ACC = true (fp32 storage, and the fp16 copies of q, k, v that the
-// block functions of fp32 models hand on): the reference's operation order, library exp and a true
-// division, so fewer fp16 rounding flips of P against the reference's np.exp.
+// block functions of fp32 models hand on): the running max is that of the scaled scores, as in the
+// reference, with library exp and a true division, so fewer fp16 rounding flips of P against the
+// reference's np.exp.  Where a tile leaves the max in place its difference is 0 and the rescaling
+// exactly 1: formed from the products instead (old * c - m * c), the compiler fuses one of the two
+// and every key tile multiplies by exp of a rounding error (d = 128, scaled scores of 700, 16 tiles:
+// up to 5.2e-4 of the output).
 template <bool ACC>
 struct Softmax {
   float c;  // ACC: scale; otherwise scale * log2(e)
   __device__ __forceinline__ explicit Softmax(float scale)
       : c(ACC ? scale : scale * 1.4426950408889634f) {}
-  // the multiple of the running max that weight() subtracts
-  __device__ __forceinline__ float base(float m) const { return m * c; }
-  // exp(scale * (s - m)) for base b = base(m)
+  // what the running max is taken of
+  __device__ __forceinline__ float score(float s) const { return ACC ? s * c : s; }
+  // what weight() subtracts for the running max m
+  __device__ __forceinline__ float base(float m) const { return ACC ? m : m * c; }
+  // the weight of score s = score(.) for base b = base(m)
   __device__ __forceinline__ float weight(float s, float b) const {
-    if constexpr (ACC) {
-      float t = s * c;
-      asm("" : "+v"(t));  // rounded as the reference rounds it, not fused with the subtraction
-      return expf(t - b);
-    } else {
-      return __builtin_amdgcn_exp2f(fmaf(s, c, -b));
-    }
+    if constexpr (ACC) return expf(s - b);
+    else return __builtin_amdgcn_exp2f(fmaf(s, c, -b));
   }
-  // exp(scale * (old - m)), the rescaling when the running max goes from `old` to m
+  // the rescaling when the running max goes from `old` to m
   __device__ __forceinline__ float rescale(float old, float m) const {
-    if constexpr (ACC) return expf(old * c - m * c);
+    if constexpr (ACC) return expf(old - m);
     else return __builtin_amdgcn_exp2f((old - m) * c);
   }
 };
@@ -284,7 +285,10 @@ __global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_att
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+        for (int r = 0; r < 16; ++r) {
+          s[kb][r] = sm.score(s[kb][r]);
+          bmax = fmaxf(bmax, s[kb][r]);
+        }
       bmax = half_max(bmax);
       const float mnew = bmax > mrun ? bmax : mrun;
       const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
@@ -526,7 +530,10 @@ __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : NW / 2) void flash_attn_res
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+          for (int r = 0; r < 16; ++r) {
+            s[kb][r] = sm.score(s[kb][r]);
+            bmax = fmaxf(bmax, s[kb][r]);
+          }
         bmax = half_max(bmax);
         const float mnew = bmax > mrun ? bmax : mrun;
         const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
@@ -782,7 +789,10 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+      for (int r = 0; r < 16; ++r) {
+        s[kb][r] = sm.score(s[kb][r]);
+        bmax = fmaxf(bmax, s[kb][r]);
+      }
     bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
@@ -1079,7 +1089,10 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+      for (int r = 0; r < 16; ++r) {
+        s[kb][r] = sm.score(s[kb][r]);
+        bmax = fmaxf(bmax, s[kb][r]);
+      }
     bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
@@ -1351,7 +1364,10 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[kb][r]);
+      for (int r = 0; r < 16; ++r) {
+        s[kb][r] = sm.score(s[kb][r]);
+        bmax = fmaxf(bmax, s[kb][r]);
+      }
     bmax = half_max(bmax);
     const float mnew = bmax > mrun ? bmax : mrun;
     const float mult = sm.rescale(mrun, mnew), mb = sm.base(mnew);
