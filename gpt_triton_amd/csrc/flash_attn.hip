@@ -53,33 +53,38 @@ template <> struct Ld8<float> {
   }
 };
 
-// The softmax arithmetic, in two precisions.  ACC = false (fp16 storage): running max on the raw
-// scores, scale * log2(e) folded into one fused multiply-add in front of the hardware's exp2, a
-// reciprocal for the denominator -- the same real-number formula as the reference, two VALU
-// operations per score fewer.  ACC = true (fp32 storage, and the fp16 copies of q, k, v that the
-// block functions of fp32 models hand on): the running max is that of the scaled scores, as in the
-// reference, with library exp and a true division, so fewer fp16 rounding flips of P against the
-// reference's np.exp.  Where a tile leaves the max in place its difference is 0 and the rescaling
-// exactly 1: formed from the products instead (old * c - m * c), the compiler fuses one of the two
-// and every key tile multiplies by exp of a rounding error (d = 128, scaled scores of 700, 16 tiles:
-// up to 5.2e-4 of the output).
-template <bool ACC>
+// The softmax arithmetic, in three forms.
+// ACC = false, SCALED = false (fp16 storage): running max on the raw scores, scale * log2(e) folded
+// into one fused multiply-add in front of the hardware's exp2, a reciprocal for the denominator -- the
+// same real-number formula as the reference, two VALU operations per score fewer.
+// SCALED = true: the running max is that of the scaled scores, as in the reference, so that what the
+// weights subtract and what the rescaling divides are the same number.  Where a tile leaves the max
+// in place its difference is 0 and the rescaling exactly 1.  Formed from the products instead
+// (old * c - m * c), the compiler fuses one of the two and every key tile multiplies by exp of a
+// rounding error (fp32, d = 128, scaled scores of 700, 16 tiles: up to 5.2e-4 of the output); with the
+// product rounded per max, tiles of different max disagree by that rounding (fp16, scaled scores of
+// 500000: 3.6e-3).
+//   ACC = true (fp32 storage, and the fp16 copies of q, k, v that the block functions of fp32 models
+//   hand on): library exp and a true division, so fewer fp16 rounding flips of P against the
+//   reference's np.exp.
+//   ACC = false (fp16 storage with dropout): the hardware's exp2.
+template <bool ACC, bool SCALED = ACC>
 struct Softmax {
-  float c;  // ACC: scale; otherwise scale * log2(e)
+  float c;  // SCALED: scale; otherwise scale * log2(e)
   __device__ __forceinline__ explicit Softmax(float scale)
-      : c(ACC ? scale : scale * 1.4426950408889634f) {}
+      : c(SCALED ? scale : scale * 1.4426950408889634f) {}
   // what the running max is taken of
-  __device__ __forceinline__ float score(float s) const { return ACC ? s * c : s; }
+  __device__ __forceinline__ float score(float s) const { return SCALED ? s * c : s; }
   // what weight() subtracts for the running max m
-  __device__ __forceinline__ float base(float m) const { return ACC ? m : m * c; }
+  __device__ __forceinline__ float base(float m) const { return SCALED ? m : m * c; }
   // the weight of score s = score(.) for base b = base(m)
   __device__ __forceinline__ float weight(float s, float b) const {
-    if constexpr (ACC) return expf(s - b);
+    if constexpr (SCALED) return ACC ? expf(s - b) : __expf(s - b);
     else return __builtin_amdgcn_exp2f(fmaf(s, c, -b));
   }
   // the rescaling when the running max goes from `old` to m
   __device__ __forceinline__ float rescale(float old, float m) const {
-    if constexpr (ACC) return expf(old - m);
+    if constexpr (SCALED) return ACC ? expf(old - m) : __expf(old - m);
     else return __builtin_amdgcn_exp2f((old - m) * c);
   }
 };
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_att
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
   float mrun = -INFINITY, den = 0.f;
-  const Softmax<ACC> sm(scale);
+  const Softmax<ACC, ACC || DROP != 0> sm(scale);
   const KeepScale keep_scale(DROP == 2 ? drop.p : 0.f);
   const unsigned keep_row = (unsigned)(q < L ? q : L - 1) * (unsigned)Lk;
 

@@ -54,3 +54,23 @@ def test_equal_scores_fp32(K, gpu_device, d, L):
     bound = (m + 33 + tiles + 8) * 2.0**-24
     rel = float(((got - want).abs() / want).max())
     assert rel <= bound, f"relative error {rel:.2e}, bound {bound:.2e}"
+
+
+def test_large_scores_dropout_fp16(K, gpu_device):
+    """fp16 storage with dropout: the second key tile's scores are 1 above the first's, at scaled scores
+    around 504000 (scale = 1/8 and the scores, whole numbers below 2^24, are exact).  What is left is the
+    rounding of P / (1 - p) and of the output to fp16, half a unit each, and exp: 3 * 2^-11."""
+    L, d, p = 128, 64, 0.1
+    for b in (246, 247, 249, 250):
+        q = np.full((1, 1, L, d), 256, np.float16)
+        k = np.full((1, 1, L, d), b, np.float16)
+        q[..., -1] = 1
+        k[..., -1] = 0
+        k[:, :, 64:, -1] = 8
+        v = np.zeros((1, 1, L, d), np.float16)
+        v[:, :, :64] = 1
+        print(f"fp16 attention with dropout, scaled scores {256 * 63 * b / 8:.0f}", flush=True)
+        got = K.flash_attention_v1(*(torch.from_numpy(t).to(gpu_device) for t in (q, k, v)), dropout_prob=p)
+        want = O.flash_attention_v1(q, k, v, dropout_prob=p).astype(np.float64)
+        rel = np.abs(got.cpu().numpy().astype(np.float64) - want) / np.maximum(np.abs(want), 2.0**-10)
+        assert rel.max() <= 3 * 2.0**-11, f"relative error {rel.max():.2e}"
