@@ -280,6 +280,12 @@ static int check_block(const char* what, int64_t M, int64_t h, float p, const vo
   return GPTMI_OK;
 }
 
+// The LayerNorm prologue reads rows and parameters in 16-byte units; the block functions run the
+// LayerNorm kernel in front of the product where one of them lies otherwise.
+static bool prologue_aligned(const void* x, const void* ln_w, const void* ln_b) {
+  return (((uintptr_t)x | (uintptr_t)ln_w | (uintptr_t)ln_b) & 15) == 0;
+}
+
 }  // namespace gptmi
 
 using namespace gptmi;
@@ -633,12 +639,16 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   ep.qkv = true;
   ep.f16 = f16;
   ep.out_f16 = true;
-  if (fuse_layernorm && !normed) {
+  bool prologue = fuse_layernorm && !normed;
+  if (prologue) {
     if (!f16 || !gemm_layernorm_supported(M, (int)h)) {
       set_error("attention_block: the LayerNorm prologue takes fp16 storage and the row widths of "
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
+    prologue = prologue_aligned(x, ln_w, ln_b);
+  }
+  if (prologue) {
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
   } else {
     const void* A = pl.normed;
@@ -696,12 +706,16 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e1.drop = drop;
   e1.f16 = f16;
   e1.out_f16 = true;
-  if (fuse_layernorm) {
-    if (!f16 || p > 0.f || ((uintptr_t)x & 15) || !gemm_layernorm_supported(M, (int)H)) {
+  bool prologue = fuse_layernorm != 0;
+  if (prologue) {
+    if (!f16 || p > 0.f || !gemm_layernorm_supported(M, (int)H)) {
       set_error("mlp_block: the LayerNorm prologue takes fp16 storage, no dropout and the row widths of "
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
+    prologue = prologue_aligned(x, ln_w, ln_b);
+  }
+  if (prologue) {
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
   } else {
     launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)H, eps, f16, true, st);

@@ -150,3 +150,32 @@ def test_modules_with_replaced_parameters(K, gpu_device, how):
         changed = module(x)
         (prune.remove if how == "prune" else parametrize.remove_parametrizations)(module, name)
         assert torch.equal(changed, module(x)) and not torch.equal(changed, want)
+
+
+# the modules in eval mode at row counts where the blocks run their LayerNorm inside the GEMM: rows or
+# LayerNorm parameters aligned to their element only take the LayerNorm kernel
+@pytest.mark.parametrize("which", ["x", "layer_norm_weight", "layer_norm_bias"])
+def test_modules_on_unaligned_rows(K, gpu_device, which):
+    from gpt_triton_amd.gpt import FusedAttention, FusedMLP
+
+    print(f"FusedAttention, FusedMLP in eval mode, {which} unaligned", flush=True)
+    P, rn = params(128, torch.float16, gpu_device, seed=6)
+    shift = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    x = rn(2, 37, 128)
+    attn, mlp = FusedAttention(128, 2), FusedMLP(128)
+    for module, keys in ((attn, ("ln_w", "ln_b", "qkv", "qkv_b", "proj", "proj_b")),
+                         (mlp, ("ln_w", "ln_b", "w1", "b1", "w2", "b2"))):
+        module.to(gpu_device).half().eval()
+        for prm, key in zip(module.parameters(), keys):
+            prm.data = P[key]
+        if which != "x":
+            getattr(module, which).data = shift(P["ln_w" if which.endswith("weight") else "ln_b"])
+    if which == "x":
+        x = shift(x)
+    lw, lb = attn.layer_norm_weight.data, attn.layer_norm_bias.data
+    y = K.fused_layer_norm(x, lw, lb)
+    q, k, v = K.matmul_and_split_qkv(y, P["qkv"], P["qkv_b"], 2)
+    a = K.flash_attention_v1(q, k, v).transpose(1, 2).contiguous().view(x.shape)
+    assert torch.equal(attn(x), K.fused_ffn(a, P["proj"], bias=P["proj_b"], residual=x))
+    y = K.fused_ffn(y, P["w1"], bias=P["b1"], add_gelu=True)
+    assert torch.equal(mlp(x), K.fused_ffn(y, P["w2"], bias=P["b2"], residual=x))
