@@ -969,32 +969,53 @@ inline float stream_cost(int64_t tiles, int Kp, bool res, int cus) {
 // the cost model says is the fastest; the rows that are left follow in a launch of the tile kernel.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, no dropout.
+// Sets *head to the number of rows for the persistent kernel.
 template <typename T, typename OT, bool QKV>
-int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
-                 hipStream_t st) {
+int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool persistent =
       M >= 256 && N >= 256 && N % 64 == 0 && Kp >= (res ? 192 : 128) && Kp <= (1 << 21) && ep.vec_ok &&
       (sizeof(OT) == 4 || ep.vec8_ok) && !(ep.drop.p > 0.f) &&
       (!res || (sizeof(T) == 2 && (((uintptr_t)ep.residual) & 15) == 0));
-  int64_t m_head = 0;
-  if (persistent) {
-    const int cus = cu_count();
-    if (cus < 0) return cus;
-    const int64_t tiles_m = M / 256, tiles_n = (N + 255) / 256;
-    const int64_t whole = tiles_m * tiles_n / cus * cus / tiles_n;  // row tiles that fill whole rounds
-    // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
-    // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
-    // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
-    // 20480 x 1024 x 4096, is the other way round, 196 against 183).
-    float least = tiles_m * tiles_n >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
-    for (const int64_t tm : {tiles_m, whole}) {
-      if (tm == 0) continue;
-      float c = stream_cost(tm * tiles_n, Kp, res, cus);
-      if (tm * 256 < M) c += 1.0f + gemm_tile_cost(M - tm * 256, N, Kp, cus);
-      if (c < least) least = c, m_head = tm * 256;
-    }
+  *head = 0;
+  if (!persistent) return 0;
+  const int cus = cu_count();
+  if (cus < 0) return cus;
+  const int64_t tiles_m = M / 256, tiles_n = (N + 255) / 256;
+  const int64_t whole = tiles_m * tiles_n / cus * cus / tiles_n;  // row tiles that fill whole rounds
+  // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
+  // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
+  // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
+  // 20480 x 1024 x 4096, is the other way round, 196 against 183).
+  float least = tiles_m * tiles_n >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
+  for (const int64_t tm : {tiles_m, whole}) {
+    if (tm == 0) continue;
+    float c = stream_cost(tm * tiles_n, Kp, res, cus);
+    if (tm * 256 < M) c += 1.0f + gemm_tile_cost(M - tm * 256, N, Kp, cus);
+    if (c < least) least = c, *head = tm * 256;
   }
+  return 0;
+}
+
+// The epilogue of the rows from `head` on.
+template <typename T, typename OT, bool QKV>
+EpiDev tail_epi(const EpiDev& ep, int64_t head, int N) {
+  EpiDev tail = ep;
+  if (QKV) {
+    tail.m_off = ep.m_off + (int)head;
+  } else {
+    tail.out = (OT*)ep.out + head * N;
+    if (ep.residual) tail.residual = (const T*)ep.residual + head * N;
+  }
+  return tail;
+}
+
+template <typename T, typename OT, bool QKV>
+int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
+                 hipStream_t st) {
+  const bool res = !QKV && ep.residual != nullptr;
+  int64_t m_head;
+  if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head)) return rc;
   if (m_head > 0) {
     int rc;
     if constexpr (sizeof(T) == 2 && !QKV)
@@ -1004,14 +1025,23 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
       rc = launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
     if (rc != 0 || m_head == M) return rc;
   }
-  EpiDev tail = ep;
-  if (QKV) tail.m_off = ep.m_off + (int)m_head;
-  else {
-    tail.out = (OT*)ep.out + m_head * N;
-    if (res) tail.residual = (const T*)ep.residual + m_head * N;
+  return launch_gemm_tile((const _Float16*)A + m_head * Kp, Bt, M - m_head, N, Kp,
+                          tail_epi<T, OT, QKV>(ep, m_head, N), sizeof(T) == 2, sizeof(OT) == 2, QKV, st);
+}
+
+// The rows divided as the plain launch divides them, so that every row's sum is formed in the same
+// order: those of the persistent kernel by the form that does not split K.
+template <bool QKV>
+int launch_shape_layernorm(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
+                           const LnArgs& ln, hipStream_t st) {
+  int64_t m_head;
+  if (const int rc = persistent_rows<_Float16, _Float16, QKV>(M, N, H, ep, &m_head)) return rc;
+  if (m_head > 0) {
+    const int rc = launch_gemm_layernorm_tile(x, Bt, m_head, N, H, ep, ln, QKV, false, st);
+    if (rc != 0 || m_head == M) return rc;
   }
-  return launch_gemm_tile((const _Float16*)A + m_head * Kp, Bt, M - m_head, N, Kp, tail, sizeof(T) == 2,
-                          sizeof(OT) == 2, QKV, st);
+  return launch_gemm_layernorm_tile((const _Float16*)x + m_head * H, Bt, M - m_head, N, H,
+                                    tail_epi<_Float16, _Float16, QKV>(ep, m_head, N), ln, QKV, true, st);
 }
 
 }  // namespace
@@ -1084,7 +1114,8 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
   EpiDev ep;
   if (const int rc = make_epi(e, M, N, ep)) return rc;
   const LnArgs ln = {ln_w, ln_b, eps, lanes_per_row(H / 8)};
-  return launch_gemm_layernorm_tile(x, Bt, M, N, H, ep, ln, e.qkv, st);
+  return e.qkv ? launch_shape_layernorm<true>(x, Bt, M, N, H, ep, ln, st)
+               : launch_shape_layernorm<false>(x, Bt, M, N, H, ep, ln, st);
 }
 
 }  // namespace gptmi

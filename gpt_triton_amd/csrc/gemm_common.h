@@ -189,11 +189,12 @@ inline int cu_count() {
 }
 
 // One workgroup per output tile (gemm_tile.hip), every size, type and epilogue; the LayerNorm
-// prologue form of it; and what the cost model says a launch takes, in microseconds.
+// prologue form of it (split: K over as many groups as the cost model takes for these rows, otherwise
+// one); and what the cost model says a launch takes, in microseconds.
 int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                      bool f16, bool out_f16, bool qkv, hipStream_t st);
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
-                               const LnArgs& ln, bool qkv, hipStream_t st);
+                               const LnArgs& ln, bool qkv, bool split, hipStream_t st);
 float gemm_tile_cost(int64_t M, int N, int Kp, int cus);
 
 }  // namespace gptmi

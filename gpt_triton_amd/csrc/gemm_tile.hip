@@ -576,8 +576,9 @@ int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, co
 // ---- LayerNorm prologue ----------------------------------------------------------------------
 // 32-row tiles on 8 wavefronts: the LDS panel of the normalised rows takes 64 * K bytes (100 KB at
 // GPT-2 XL's 1600), three stages of weight rows 48 KB beside it -- up to K = 1024 also 96 KB, and then
-// the four-way split has a 64-wide tile.  K is split over as many groups as the plain launch of these
-// sizes splits it, so that the sums, too, are formed in the same order.  One workgroup fills a CU's
+// the four-way split has a 64-wide tile.  K is split over as many groups as the plain launch splits
+// it (split = false: not at all, the rows that launch gives to the persistent kernel), so that the
+// sums, too, are formed in the same order.  One workgroup fills a CU's
 // LDS, so more workgroups than CUs take a second round: one launch of 128 rows x 768 x 3072 as 384
 // tiles of 32 x 32 took 13.4 us against 9.6 for the LayerNorm launch and the plain one, as 192 of
 // 32 x 64 8.9; 24 rows (96 tiles) 6.9 against 8.0.
@@ -589,8 +590,8 @@ typedef Tile<32, 128, 1, 8, 1, 3> Ln32x128;
 constexpr int kLnStages = 3 * 128 * 128;
 
 // Index and column width of the form that serves these sizes.
-inline int pick_ln(int64_t M, int N, int K, int cus, int* bn) {
-  const int wk = kTiles[pick_tile(M, N, K, cus, nullptr)].wk;
+inline int pick_ln(int64_t M, int N, int K, bool split, int cus, int* bn) {
+  const int wk = split ? kTiles[pick_tile(M, N, K, cus, nullptr)].wk : 1;
   const int64_t rows = (M + 31) / 32;
   const bool wide = wk == 4 && K <= 1024 && rows * ((N + 31) / 32) > cus;
   *bn = wk == 1 ? 128 : wk == 2 || wide ? 64 : 32;
@@ -599,11 +600,11 @@ inline int pick_ln(int64_t M, int N, int K, int cus, int* bn) {
 
 template <bool QKV>
 int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiDev& ep, const LnArgs& ln,
-              hipStream_t st) {
+              bool split, hipStream_t st) {
   const int cus = cu_count();
   if (cus < 0) return cus;
   int bn;
-  switch (pick_ln(M, N, K, cus, &bn)) {
+  switch (pick_ln(M, N, K, split, cus, &bn)) {
     case 0: return launch_tile_cfg<Ln32x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 1: return launch_tile_cfg<Ln32x64w, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 2: return launch_tile_cfg<Ln32x64, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
@@ -619,8 +620,9 @@ bool gemm_layernorm_supported(int64_t M, int H) {
 }
 
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
-                               const LnArgs& ln, bool qkv, hipStream_t st) {
-  return qkv ? launch_ln<true>(x, Bt, M, N, H, ep, ln, st) : launch_ln<false>(x, Bt, M, N, H, ep, ln, st);
+                               const LnArgs& ln, bool qkv, bool split, hipStream_t st) {
+  return qkv ? launch_ln<true>(x, Bt, M, N, H, ep, ln, split, st)
+             : launch_ln<false>(x, Bt, M, N, H, ep, ln, split, st);
 }
 
 }  // namespace gptmi

@@ -176,3 +176,23 @@ def test_model_same_bits_with_and_without_the_prologue(gpu_device, monkeypatch):
     diff = np.abs(host(hid_a).astype(np.float64) - want.astype(np.float64)).max()
     print(f"2 x 64 forward, fp16: max|diff| to the oracle {diff:.3e}", flush=True)
     assert diff <= 2e-2
+
+
+# row counts where the plain launch divides the rows between two kernels (the persistent one takes whole
+# 256-row tiles, and a tile split over K other than for all the rows takes the rest), and one row less
+@pytest.mark.parametrize("M,H,N", [(5376, 768, 3072), (5377, 768, 3072), (5416, 768, 3072),
+                                   (4097, 1024, 4096), (2561, 1600, 6400)])
+def test_layer_norm_linear_where_the_plain_launch_divides_its_rows(K, gpu_device, M, H, N):
+    x, ln_w, ln_b, w, b = operands(M, H, N, seed=M)
+    print(f"layer_norm_ffn, layer_norm_matmul_and_split_qkv: M={M} H={H} N={N}", flush=True)
+    xd, lwd, lbd, wd, bd = (dev(a, gpu_device) for a in (x, ln_w, ln_b, w, b))
+    wp = K.pack_weight(wd)
+    y = K.fused_layer_norm(xd, lwd, lbd)
+    assert torch.equal(K.layer_norm_ffn(xd, lwd, lbd, wp, bias=bd, add_gelu=True),
+                       K.fused_ffn(y, wp, bias=bd, add_gelu=True))
+    heads = H // 64
+    wq, bq = K.pack_weight(wd[:, :N // 4 * 3].contiguous()), bd[:N // 4 * 3].contiguous()
+    got = K.layer_norm_matmul_and_split_qkv(xd.view(1, M, H), lwd, lbd, wq, bq, heads)
+    two = K.matmul_and_split_qkv(y.view(1, M, H), wq, bq, heads)
+    for name, g, t in zip("qkv", got, two):
+        assert torch.equal(g, t), name
