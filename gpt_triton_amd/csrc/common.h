@@ -160,15 +160,31 @@ __device__ __forceinline__ void philox_uniform(const DropoutArgs& d, const unsig
 
 // x / keep for the kept values.  Division by one number: its reciprocal is taken once, and the
 // remainder of the first quotient corrects it (correctly rounded for a correctly rounded reciprocal,
-// P. Markstein, IBM J. Res. Dev. 34, 1990); div_fixup passes infinities and NaN through.
+// P. Markstein, IBM J. Res. Dev. 34, 1990).  That takes a quotient that is finite and a remainder
+// that is no subnormal number, 24 bits below x: |x| from 2^-100 to 2^127 keep.  Values among which
+// there are others (infinities, NaN and 0 count) are divided; asked once for the N values of a thread
+// (MLP block of 4800 x 768 with the mask at hand: 77.1 us; 79.3 asked per value, 76.3 never).
 struct KeepScale {
   float keep, inv;
   __device__ __forceinline__ explicit KeepScale(float p) : keep(1.0f - p), inv(1.0f / (1.0f - p)) {}
-  __device__ __forceinline__ float operator()(float x) const {
-    const float q = x * inv;
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, keep, x), inv, q), keep, x);
+  template <int N>
+  __device__ __forceinline__ void apply(float (&x)[N]) const {
+    float lo = __builtin_fabsf(x[0]), hi = lo;
+#pragma unroll
+    for (int i = 1; i < N; ++i) {
+      lo = fminf(lo, __builtin_fabsf(x[i]));
+      hi = fmaxf(hi, __builtin_fabsf(x[i]));
+    }
+    if (__builtin_expect(lo >= 0x1p-100f && hi <= 0x1p127f * keep, 1)) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] = finite(x[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] = x[i] / keep;
+    }
   }
-  // for an x that is no infinity
+  // for an x that is rounded to fp16 afterwards and no infinity (the quotients that `finite` would
+  // round otherwise are far below fp16's smallest)
   __device__ __forceinline__ float finite(float x) const {
     const float q = x * inv;
     float r = fmaf(fmaf(-q, keep, x), inv, q);
@@ -182,9 +198,9 @@ __device__ __forceinline__ void dropout_apply(const DropoutArgs& d, const unsign
                                               float (&x)[NCH]) {
   float u[NCH];
   philox_uniform<NCH>(d, offset, u);
-  const KeepScale scale(d.p);
+  KeepScale(d.p).apply(x);
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) x[i] = u[i] > d.p ? scale(x[i]) : 0.0f;
+  for (int i = 0; i < NCH; ++i) x[i] = u[i] > d.p ? x[i] : 0.0f;
 }
 
 // v where bit `b` of `bits` is set, +0 elsewhere (v's bits under a mask: one bit-field extract, one and).

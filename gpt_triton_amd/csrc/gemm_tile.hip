@@ -415,9 +415,9 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     }
     if constexpr (DROP) {
       if (ep.keep != nullptr) {
-        const KeepScale scale(ep.drop.p);
+        KeepScale(ep.drop.p).apply(z);
 #pragma unroll
-        for (int e = 0; e < CW; ++e) z[e] = keep_if(keep_v[it], e, scale(z[e]));
+        for (int e = 0; e < CW; ++e) z[e] = keep_if(keep_v[it], e, z[e]);
       } else {
         unsigned off[CW];
 #pragma unroll

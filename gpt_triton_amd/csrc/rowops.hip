@@ -90,12 +90,13 @@ __global__ __launch_bounds__(256) void embed_dropout_vec_kernel(
     const bool known = (uint64_t)tok < (uint64_t)V_;
     const V va = reinterpret_cast<const V*>(wte + (known ? tok : 0) * H)[c];
     const V vb = reinterpret_cast<const V*>(wpe + row % L * H)[c];
+    float sum[VN];
+#pragma unroll
+    for (int j = 0; j < VN; ++j) sum[j] = (float)(T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
+    scale.apply(sum);
     V vo;
 #pragma unroll
-    for (int j = 0; j < VN; ++j) {
-      const T sum = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-      vo[j] = (T)(u[j] > drop.p ? scale((float)sum) : 0.f);
-    }
+    for (int j = 0; j < VN; ++j) vo[j] = (T)(u[j] > drop.p ? sum[j] : 0.f);
     reinterpret_cast<V*>(out + row * H)[c] = vo;
   }
 }

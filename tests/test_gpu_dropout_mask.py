@@ -95,3 +95,32 @@ def test_embedding_dropout(K, gpu_device, dtype, B, L, H):
     ids = r.integers(0, 50, (B, L))
     got = K.fused_embeddings(*(torch.from_numpy(t).to(gpu_device) for t in (ids, wte, wpe)), dropout_prob=0.1)
     assert np.array_equal(got.cpu().numpy(), O.fused_embeddings(ids, wte, wpe, dropout_prob=0.1))
+
+
+# x / (1 - p) in fp32 from the smallest subnormal to the largest finite value, infinities and NaN: the
+# correctly rounded quotient, as a true division gives it
+@pytest.mark.parametrize("p", [0.1, 0.5, 0.9])
+def test_division_over_the_whole_range(K, gpu_device, p):
+    print(f"dropout of fp32 values of every magnitude, p={p}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(9)
+    bits = torch.arange(0, 255 << 23, 1 << 19, dtype=torch.int64)  # 16 values an octave, subnormals too
+    bits = bits + torch.randint(0, 1 << 19, bits.shape, generator=g)
+    special = torch.tensor([0, 1, 2, 3, 0x7fffff, 0x800000, 0x7f7fffff, 0x7f800000, 0x7fc00000])
+    bits = torch.cat([bits, special, torch.arange(0x0c000000, 0x0d000000, 0x3331)])
+    x = bits.to(torch.int32).view(torch.float32)
+    x = torch.cat([x, -x])
+    x = torch.cat([x, x.new_zeros(-len(x) % 64)])
+    N = len(x)
+    with np.errstate(all="ignore"):
+        want = torch.from_numpy(x.numpy() / (np.float32(1) - np.float32(p)))
+    keep = torch.from_numpy(O.tl_rand(O.SEED, np.arange(N)) > np.float32(p))
+    want = torch.where(keep, want, torch.zeros(()))
+    same = lambda a, b: bool(((a == b) | (a.isnan() & b.isnan())).all())
+    xd = x.to(gpu_device)
+    got = K.fused_embeddings(torch.zeros((1, 1), dtype=torch.int64, device=gpu_device), xd[None],
+                             torch.zeros((1, N), device=gpu_device), dropout_prob=p)[0, 0].cpu()
+    assert same(got, want), "embedding"
+    # a zero product and the values as the bias; offsets m * N + n: the columns of row 0
+    z = torch.zeros((1, 64), device=gpu_device)
+    got = K.fused_ffn(z, torch.zeros((64, N), device=gpu_device), bias=xd, dropout_prob=p)[0].cpu()
+    assert same(got, want), "fused_ffn"
