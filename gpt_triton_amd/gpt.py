@@ -84,8 +84,16 @@ class _Block(nn.Sequential):
 
     def forward(self, x, keep=None):
         for module in self:
-            x = module(x, keep=keep) if type(module) in (FusedAttention, FusedMLP) else module(x)
+            x = _call_with_mask(module, x, keep)
         return x
+
+
+def _call_with_mask(module, x, keep):
+    """module(x), with the mask where the forward that the call will run is one of this file's: one
+    replaced on the instance, in its class or by a subclass takes what nn.Sequential hands it."""
+    if keep is not None and getattr(module.forward, "__func__", None) in _TAKE_MASK:
+        return module(x, keep=keep)
+    return module(x)
 
 
 class _PackedWeights:
@@ -255,6 +263,9 @@ class FusedMLP(nn.Module):
                 _linear_flops(num_tokens, mid, h))
 
 
+_TAKE_MASK = (_Block.forward, FusedAttention.forward, FusedMLP.forward)
+
+
 @dataclass
 class GPTConfig:
     vocab_size: int = 50304
@@ -317,7 +328,7 @@ class FusedGPT(nn.Module):
             rest = blocks
         keep = _keep_mask(x, self.config.n_embd, len(rest), self.config.n_head, p) if p > 0.0 else None
         for block in rest:
-            x = block(x, keep=keep) if keep is not None and type(block) is _Block else block(x)
+            x = _call_with_mask(block, x, keep)
         x = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)
         if return_logits:
             return x, lm_head(x, self._lm_head_weight())

@@ -184,3 +184,38 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True)
     assert r.returncode != 0 and "--gpus must be 1" in r.stderr
+
+
+def test_replaced_forwards_are_called_with_x_alone(monkeypatch):
+    # a forward wrapped to time or record it takes what nn.Sequential hands it, with dropout too
+    from gpt_triton_amd import gpt
+
+    monkeypatch.setattr(gpt, "fused_embeddings", lambda ids, *a, **k: torch.zeros(*ids.shape, 64))
+    monkeypatch.setattr(gpt, "fused_layer_norm", lambda x, w, b: x)
+    monkeypatch.setattr(gpt, "dropout_mask", lambda bits, p, like: "mask")
+    ids = torch.zeros((1, 4), dtype=torch.int64)
+    # on the instances of a block's two modules, on the block, on the class
+    model = gpt.FusedGPT(gpt.GPTConfig(n_layer=2, n_head=1, n_embd=64)).train()
+    for block in model.blocks:
+        block[0].forward = lambda x: x + 1
+        block[1].forward = lambda x: x * 2
+    assert torch.equal(model(ids), torch.full((1, 4, 64), 6.0))
+    model.blocks[1].forward = lambda x: x - 1
+    assert torch.equal(model(ids), torch.full((1, 4, 64), 1.0))
+    model = gpt.FusedGPT(gpt.GPTConfig(n_layer=2, n_head=1, n_embd=64)).train()
+    monkeypatch.setattr(gpt.FusedAttention, "forward", lambda self, x: x + 1)
+    monkeypatch.setattr(gpt.FusedMLP, "forward", lambda self, x: x * 2)
+    assert torch.equal(model(ids), torch.full((1, 4, 64), 6.0))
+    # what takes the mask gets it, in a subclass too
+    class Attention(gpt.FusedAttention):
+        pass
+
+    monkeypatch.undo()
+    seen = []
+    monkeypatch.setattr(gpt, "attention_block", lambda x, *a, keep=None, **k: seen.append(keep))
+
+    class Mask:
+        serves = staticmethod(lambda x, bits, p: True)
+
+    gpt._Block(Attention(64, 1, dropout_prob=0.1), torch.nn.Identity()).train()(torch.zeros(1, 4, 64), keep=Mask)
+    assert seen == [Mask]
