@@ -135,6 +135,14 @@ def _tensors(module, names):
     return prm if names <= prm.keys() else {name: getattr(module, name) for name in names}
 
 
+def _are_parameters(module, tensors, first, second):
+    """Whether a module's two weights are parameters: images are kept for those only, and for both or
+    neither.  What stands in for one is another tensor every time, in the dictionary of parameters too
+    (torch.func.functional_call puts plain tensors there)."""
+    return (tensors is module._parameters and isinstance(tensors[first], nn.Parameter) and
+            isinstance(tensors[second], nn.Parameter))
+
+
 class FusedAttention(nn.Module):
     """Pre-LN causal self-attention block: x + proj(attention(qkv(LN(x))))."""
 
@@ -156,11 +164,10 @@ class FusedAttention(nn.Module):
                         "c_proj_weight", "c_proj_bias"))
 
     def _weight(self, name, tensors=None):
-        # an image is kept for a parameter only: what stands in for one is another tensor every time
         tensors = tensors or _tensors(self, self._NAMES)
         prm = tensors[name]
-        if (self.training or tensors is not self._parameters or
-                (self.hidden_size // self.num_heads) % 8 != 0):
+        if (self.training or (self.hidden_size // self.num_heads) % 8 != 0 or
+                not _are_parameters(self, tensors, "c_attn_weight", "c_proj_weight")):
             return prm.data
         return self._packed.get(name, prm)
 
@@ -227,10 +234,9 @@ class FusedMLP(nn.Module):
                         "ffn2_weight", "ffn2_bias"))
 
     def _weight(self, name, tensors=None):
-        # as in FusedAttention
         tensors = tensors or _tensors(self, self._NAMES)
         prm = tensors[name]
-        if self.training or tensors is not self._parameters:
+        if self.training or not _are_parameters(self, tensors, "ffn1_weight", "ffn2_weight"):
             return prm.data
         return self._packed.get(name, prm)
 
@@ -305,7 +311,7 @@ class FusedGPT(nn.Module):
         # whole 128-byte lines and the product runs on the persistent GEMM kernel, and the image
         # is built once instead of on every call; see kernels.pack_lm_head.
         w = self.wte_weight
-        if self.training:
+        if self.training or not isinstance(w, nn.Parameter):
             return w.data
         return self._packed.get("lm_head", w, pack_lm_head)
 

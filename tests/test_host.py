@@ -219,3 +219,38 @@ def test_replaced_forwards_are_called_with_x_alone(monkeypatch):
 
     gpt._Block(Attention(64, 1, dropout_prob=0.1), torch.nn.Identity()).train()(torch.zeros(1, 4, 64), keep=Mask)
     assert seen == [Mask]
+
+
+def test_weight_images_are_kept_for_parameters_only(monkeypatch):
+    # torch.func.functional_call puts plain tensors in the place of the parameters: another tensor on
+    # every call, whose address and version say nothing about its values
+    from torch.func import functional_call
+
+    from gpt_triton_amd import gpt
+
+    class Probe(torch.nn.Module):
+        def __init__(self, module, names):
+            super().__init__()
+            self.module, self.names = module, names
+
+        def forward(self):
+            return [self.module._weight(n) if n else self.module._lm_head_weight() for n in self.names]
+
+    model = gpt.FusedGPT(gpt.GPTConfig(n_layer=1, n_head=1, n_embd=64, vocab_size=64)).eval()
+    for module, names in ((gpt.FusedAttention(64, 1).eval(), ["c_attn_weight", "c_proj_weight"]),
+                          (gpt.FusedMLP(64).eval(), ["ffn1_weight", "ffn2_weight"]), (model, [None])):
+        kept = []
+        module._packed.get = lambda name, prm, pack=None: kept.append(name)
+        probe = Probe(module, names)
+        probe()
+        assert kept == [n or "lm_head" for n in names]
+        kept.clear()
+        plain = {n: p.detach().clone() for n, p in probe.named_parameters()}
+        got = functional_call(probe, plain)
+        assert not kept
+        for n, t in zip(names, got):
+            assert t.data_ptr() == plain[f"module.{n or 'wte_weight'}"].data_ptr()
+        # one of the two replaced: the block calls take both weights packed or neither
+        name = f"module.{names[0] or 'wte_weight'}"
+        functional_call(probe, {name: plain[name]})
+        assert not kept
