@@ -49,7 +49,8 @@ def _ln_in_gemm(x, weight):
             layer_norm_linear_supported(x, weight))
 
 
-def _as_block(x, width, keep=None):
+def _as_block(x, keep=None):
+    width = x.shape[-1]
     return ((keep is not None or x.dtype == torch.float32 or
              x.numel() // width <= BLOCK_MAX_ROWS) and block_supported(x, width))
 
@@ -185,8 +186,7 @@ class FusedAttention(nn.Module):
         prm = _tensors(self, self._NAMES)
         w_attn = self._weight("c_attn_weight", prm)
         in_gemm = normed is None and p == 0.0 and _ln_in_gemm(x, w_attn)
-        if (_as_block(x, self.hidden_size, keep) and
-                self.hidden_size // self.num_heads in HEAD_SIZES):
+        if _as_block(x, keep) and x.shape[-1] // self.num_heads in HEAD_SIZES:
             return attention_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w_attn,
                                    prm["c_attn_bias"], self._weight("c_proj_weight", prm),
                                    prm["c_proj_bias"], self.num_heads, dropout_prob=p,
@@ -247,14 +247,18 @@ class FusedMLP(nn.Module):
     def forward(self, x, keep=None):
         """`keep`: as in FusedAttention.forward."""
         p = self.dropout_prob if self.training else 0.0
-        if keep is not None and not (p > 0.0 and keep.serves(x, 4 * x.numel(), p)):
-            keep = None
         prm = _tensors(self, self._NAMES)
         w1, w2 = self._weight("ffn1_weight", prm), self._weight("ffn2_weight", prm)
-        if p == 0.0 and _ln_in_gemm(x, w1):
+        # the weights, and x with them, may have other widths than h and 4h (pruned, exchanged)
+        width, inner = x.shape[-1], w1.shape[1]
+        if keep is not None and not (
+                p > 0.0 and keep.serves(x, x.numel() // width * max(inner, width), p)):
+            keep = None
+        as_block = inner % 64 == 0
+        if as_block and p == 0.0 and _ln_in_gemm(x, w1):
             return layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                                   bias=prm["ffn1_bias"], add_gelu=True, then=(w2, prm["ffn2_bias"]))
-        if _as_block(x, self.hidden_size, keep):
+        if as_block and _as_block(x, keep):
             return mlp_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                              prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p, keep=keep)
         y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)

@@ -179,3 +179,44 @@ def test_modules_on_unaligned_rows(K, gpu_device, which):
     assert torch.equal(attn(x), K.fused_ffn(a, P["proj"], bias=P["proj_b"], residual=x))
     y = K.fused_ffn(y, P["w1"], bias=P["b1"], add_gelu=True)
     assert torch.equal(mlp(x), K.fused_ffn(y, P["w2"], bias=P["b2"], residual=x))
+
+
+# modules whose weights were exchanged for others: an inner width that is not a multiple of 64 (the
+# operators take it, the block call does not), one above 4h (a forward's dropout mask is too short for
+# it), rows of another width than the module was built for
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows", [70, 700])
+@pytest.mark.parametrize("h,inner", [(128, 100), (128, 640), (96, 512), (192, 512)])
+@pytest.mark.parametrize("p", [0.0, 0.1])
+def test_mlp_of_other_widths(K, gpu_device, dtype, rows, h, inner, p):
+    from gpt_triton_amd.gpt import FusedMLP
+
+    print(f"FusedMLP {dtype} rows={rows} h={h} inner={inner} p={p}", flush=True)
+    P, rn = params(h, dtype, gpu_device, seed=inner)
+    x = rn(rows, h)
+    mlp = FusedMLP(128, dropout_prob=p).to(gpu_device).to(dtype).train(p > 0)
+    w1, b1, w2 = rn(h, inner, std=0.1), rn(inner), rn(inner, h, std=0.1)
+    for prm, t in zip(mlp.parameters(), (P["ln_w"], P["ln_b"], w1, b1, w2, P["b2"])):
+        prm.data = t
+    y = K.fused_layer_norm(x, P["ln_w"], P["ln_b"])
+    y = K.fused_ffn(y, w1, bias=b1, add_gelu=True, dropout_prob=p)
+    want = K.fused_ffn(y, w2, bias=P["b2"], residual=x, dropout_prob=p)
+    keeps = [None] if p == 0 else [None, K.dropout_mask(4 * x.numel(), p, x)]
+    for keep in keeps:
+        assert torch.equal(mlp(x, keep=keep), want)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+def test_attention_of_another_width(K, gpu_device, p):
+    from gpt_triton_amd.gpt import FusedAttention
+
+    print(f"FusedAttention of 96-wide rows p={p}", flush=True)
+    P, rn = params(96, torch.float16, gpu_device, seed=8)
+    x = rn(2, 35, 96)
+    attn = FusedAttention(192, 3, dropout_prob=p).to(gpu_device).half().train(p > 0)
+    for prm, key in zip(attn.parameters(), ("ln_w", "ln_b", "qkv", "qkv_b", "proj", "proj_b")):
+        prm.data = P[key]
+    q, k, v = K.matmul_and_split_qkv(K.fused_layer_norm(x, P["ln_w"], P["ln_b"]), P["qkv"], P["qkv_b"], 3)
+    a = K.flash_attention_v1(q, k, v, dropout_prob=p).transpose(1, 2).contiguous().view(x.shape)
+    want = K.fused_ffn(a, P["proj"], bias=P["proj_b"], residual=x, dropout_prob=p)
+    assert torch.equal(attn(x), want)
