@@ -509,7 +509,7 @@ def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, pr
           ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, qkv_weight.data_ptr(), qkv_bias.data_ptr(),
           proj_weight.data_ptr(), proj_bias.data_ptr(), out.data_ptr(), B, L, num_heads, d,
           float(dropout_prob), 1337, *_keep_args(keep, x, dropout_prob, "attention_block"),
-          1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
+          1 if layer_norm_in_gemm else 0, layout, _ptr(ws), nbytes, code)
     return out
 
 
@@ -540,5 +540,6 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     _call(dev, "mlp_block", lib.gptmi_mlp_block, x.data_ptr(), ln_weight.data_ptr(),
           ln_bias.data_ptr(), 1e-5, weight1.data_ptr(), bias1.data_ptr(), weight2.data_ptr(),
           bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337,
-          *_keep_args(keep, x, dropout_prob, "mlp_block"), 1 if layer_norm_in_gemm else 0, layout, ws.data_ptr(), nbytes, code)
+          *_keep_args(keep, x, dropout_prob, "mlp_block"), 1 if layer_norm_in_gemm else 0, layout,
+          _ptr(ws), nbytes, code)
     return out

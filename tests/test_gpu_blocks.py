@@ -220,3 +220,14 @@ def test_attention_of_another_width(K, gpu_device, p):
     a = K.flash_attention_v1(q, k, v, dropout_prob=p).transpose(1, 2).contiguous().view(x.shape)
     want = K.fused_ffn(a, P["proj"], bias=P["proj_b"], residual=x, dropout_prob=p)
     assert torch.equal(attn(x), want)
+
+
+def test_no_rows_are_refused_as_the_operators_refuse_them(K, gpu_device):
+    P, rn = params(64, torch.float16, gpu_device, seed=7)
+    x = rn(0, 5, 64)
+    with pytest.raises(RuntimeError, match="status -1"):
+        K.fused_layer_norm(x, P["ln_w"], P["ln_b"])
+    with pytest.raises(RuntimeError, match="status -1"):
+        K.attention_block(x, P["ln_w"], P["ln_b"], P["qkv"], P["qkv_b"], P["proj"], P["proj_b"], 1)
+    with pytest.raises(RuntimeError, match="status -1"):
+        K.mlp_block(x, P["ln_w"], P["ln_b"], P["w1"], P["b1"], P["w2"], P["b2"])
