@@ -616,6 +616,11 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     set_error("attention_block: invalid argument");
     return GPTMI_ERR_INVALID;
   }
+  // before the product, whose scatter stores 8 columns of a head at a time
+  if (d != 16 && d != 32 && d != 64 && d != 128 && d != 256) {
+    set_error("attention_block: head size %lld not built (16, 32, 64, 128 and 256 are)", (long long)d);
+    return GPTMI_ERR_UNSUPPORTED;
+  }
   const int64_t M = B * L, h = heads * d;
   const AttentionPlan pl = plan_attention(workspace, M, h, wlayout);
   int rc = check_block("attention_block", M, h, p, keep, keep_bits, M * h > L * L ? M * h : L * L, wlayout,

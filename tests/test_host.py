@@ -254,3 +254,12 @@ def test_weight_images_are_kept_for_parameters_only(monkeypatch):
         name = f"module.{names[0] or 'wte_weight'}"
         functional_call(probe, {name: plain[name]})
         assert not kept
+
+
+def test_attention_block_checks_the_head_size_before_any_launch(lib):
+    fake = ctypes.c_void_p(256)
+    for heads, d in ((16, 4), (8, 24), (2, 96), (1, 512)):
+        need = lib.gptmi_attention_block_workspace_bytes(1, 8, heads, d, 2)
+        rc = lib.gptmi_attention_block(fake, None, fake, fake, 1e-5, fake, fake, fake, fake, fake, 1, 8, heads, d,
+                                       0.0, 1337, None, 0, 0, 2, fake, need, 1, None)
+        assert rc == -2 and b"head size" in lib.gptmi_last_error()
