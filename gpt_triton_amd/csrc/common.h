@@ -183,6 +183,11 @@ struct KeepScale {
       for (int i = 0; i < N; ++i) x[i] = x[i] / keep;
     }
   }
+  // for an x that is an fp16 number: no range to ask for, div_fixup passes infinities, NaN and 0 through
+  __device__ __forceinline__ float of_half(float x) const {
+    const float q = x * inv;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, keep, x), inv, q), keep, x);
+  }
   // for an x that is rounded to fp16 afterwards and no infinity (the quotients that `finite` would
   // round otherwise are far below fp16's smallest)
   __device__ __forceinline__ float finite(float x) const {

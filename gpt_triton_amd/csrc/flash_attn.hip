@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_att
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
   float mrun = -INFINITY, den = 0.f;
   const Softmax<ACC, ACC || DROP != 0> sm(scale);
-  const KeepScale keep_scale(DROP == 2 ? drop.p : 0.f);
+  const KeepScale keep_scale(DROP != 0 ? drop.p : 0.f);
   const unsigned keep_row = (unsigned)(q < L ? q : L - 1) * (unsigned)Lk;
 
   load_tile(0, stg[0]);
@@ -328,10 +328,11 @@ __global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_att
             const unsigned key0 = (unsigned)(k0 + kb * 32 + 8 * rg + 4 * g);
             const unsigned base_off = (unsigned)q * (unsigned)Lk + key0;
             unsigned off[4] = {base_off, base_off + 1u, base_off + 2u, base_off + 3u};
-            float pv[4] = {s[kb][4 * rg], s[kb][4 * rg + 1], s[kb][4 * rg + 2], s[kb][4 * rg + 3]};
-            dropout_apply<4>(drop, off, pv);
+            float u[4];
+            philox_uniform<4>(drop, off, u);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) s[kb][4 * rg + e] = pv[e];
+            for (int e = 0; e < 4; ++e)
+              s[kb][4 * rg + e] = u[e] > drop.p ? keep_scale.finite(s[kb][4 * rg + e]) : 0.f;
           }
       }
 #pragma unroll

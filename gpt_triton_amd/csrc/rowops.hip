@@ -93,7 +93,12 @@ __global__ __launch_bounds__(256) void embed_dropout_vec_kernel(
     float sum[VN];
 #pragma unroll
     for (int j = 0; j < VN; ++j) sum[j] = (float)(T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-    scale.apply(sum);
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int j = 0; j < VN; ++j) sum[j] = scale.of_half(sum[j]);
+    } else {
+      scale.apply(sum);
+    }
     V vo;
 #pragma unroll
     for (int j = 0; j < VN; ++j) vo[j] = (T)(u[j] > drop.p ? sum[j] : 0.f);
