@@ -11,7 +11,9 @@
 //   * WK groups of wavefronts split K inside the workgroup: group g multiplies the 64-wide
 //     k-slices g, g + WK, ..., so a "k-step" of the workgroup is WK slices wide and the number of
 //     barriers and round trips falls by WK.  The groups' partial sums meet in LDS at the end and are
-//     added in group order (deterministic, and the same whichever tile a row falls into);
+//     added in group order: deterministic, but the order depends on the tile that the row count picks,
+//     so a row's last bit may differ between batches (four sums of K / 4 terms are nearer to the exact
+//     one: 128 x 768 x 3072 in fp32 1.8e-7 rms against 3.5e-7 for one running sum);
 //   * the fragments of the whole next k-step are read from LDS (into a second register set) while the
 //     current one is multiplied, one read behind every MFMA or two, so an LDS round trip has the time
 //     of a k-step, not of one slice;
@@ -34,24 +36,19 @@ namespace {
 // goes to k-slice k / 64, row r's 128 bytes there, 16-byte unit (k % 64) / 8 ^ key(r).  A row is
 // spread over LPR lanes as in layernorm_vec_kernel (same sums, same bits); rows past the end
 // repeat the last row.
-template <int BM, int NT, typename T, int LPR, int CH>
-__device__ __forceinline__ void normalise_rows(const T* __restrict__ x, int M, int H, int m0,
+template <int BM, int NT, int LPR, int CH>
+__device__ __forceinline__ void normalise_rows(const _Float16* __restrict__ x, int M, int H, int m0,
                                                const LnArgs& ln, char* panel, int tid) {
-  constexpr int VN = 16 / sizeof(T);
-  typedef T V __attribute__((ext_vector_type(VN)));
-  typedef _Float16 HV __attribute__((ext_vector_type(VN)));
   constexpr int RPP = NT / LPR;  // rows per pass
   constexpr int PASSES = BM / RPP;
   static_assert(PASSES >= 1 && BM % RPP == 0, "row passes");
-  const int nchunks = H / VN, ll = tid & (LPR - 1), rsub = tid / LPR;
-  const V* wv = reinterpret_cast<const V*>(ln.w);
-  const V* bv = reinterpret_cast<const V*>(ln.b);
-  // the rows of G passes are requested together: one memory round trip for them (long rows: two
-  // passes at a time, and the parameters per row from L1, or the registers do not hold them)
-  constexpr bool LONG = CH > 4;
-  constexpr int G = LONG && PASSES > 2 ? 2 : PASSES;
-  static_assert(PASSES % G == 0, "pass groups");
-  V tw[CH], tb[CH];
+  const int nchunks = H / 8, ll = tid & (LPR - 1), rsub = tid / LPR;
+  const h8* wv = reinterpret_cast<const h8*>(ln.w);
+  const h8* bv = reinterpret_cast<const h8*>(ln.b);
+  // the rows of all passes and the parameters are requested together: one memory round trip
+  h8 tw[CH], tb[CH], t[PASSES][CH];
+  // as a lambda the parameters stay packed halves until they are used (135 registers instead of 158;
+  // LayerNorm -> ffn1 at 24 x 768 6.5 against 6.8 us)
   auto params = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
@@ -62,65 +59,59 @@ __device__ __forceinline__ void normalise_rows(const T* __restrict__ x, int M, i
       }
     }
   };
-  if constexpr (!LONG) params();
-#pragma unroll(LONG ? 1 : 2)
-  for (int p0 = 0; p0 < PASSES; p0 += G) {
-    V t[G][CH];
+  params();
 #pragma unroll
-    for (int p = 0; p < G; ++p) {
-      int row = m0 + (p0 + p) * RPP + rsub;
-      row = row < M ? row : M - 1;
-      const V* xr = reinterpret_cast<const V*>(x + (size_t)row * H);
+  for (int p = 0; p < PASSES; ++p) {
+    int row = m0 + p * RPP + rsub;
+    row = row < M ? row : M - 1;
+    const h8* xr = reinterpret_cast<const h8*>(x + (size_t)row * H);
 #pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int c = ll + i * LPR;
-        if (c < nchunks) t[p][i] = xr[c];
+    for (int i = 0; i < CH; ++i) {
+      const int c = ll + i * LPR;
+      if (c < nchunks) t[p][i] = xr[c];
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int r = p * RPP + rsub;
+    float v[CH][8], sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const bool in = ll + i * LPR < nchunks;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[i][j] = in ? (float)t[p][i][j] : 0.f;
+        if (in) sum += v[i][j];
       }
     }
+    float mean, rstd;
+    layernorm_stats<CH, 8, LPR>(v, sum, ll, nchunks, H, ln.eps, mean, rstd);
 #pragma unroll
-    for (int p = 0; p < G; ++p) {
-      const int r = (p0 + p) * RPP + rsub;
-      float v[CH][VN], sum = 0.f;
+    for (int i = 0; i < CH; ++i) {
+      const int c = ll + i * LPR;
+      if (c < nchunks) {
+        h8 o;
 #pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const bool in = ll + i * LPR < nchunks;
-#pragma unroll
-        for (int j = 0; j < VN; ++j) {
-          v[i][j] = in ? (float)t[p][i][j] : 0.f;
-          if (in) sum += v[i][j];
-        }
-      }
-      float mean, rstd;
-      layernorm_stats<CH, VN, LPR>(v, sum, ll, nchunks, H, ln.eps, mean, rstd);
-      if constexpr (LONG) params();
-#pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int c = ll + i * LPR;
-        if (c < nchunks) {
-          HV o;
-#pragma unroll
-          for (int j = 0; j < VN; ++j)
-            o[j] = (_Float16)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
-          const int k = c * VN, unit = (k & 63) >> 3;
-          *reinterpret_cast<HV*>(panel + (k >> 6) * (BM * 128) + r * 128 +
-                                 ((unit ^ ((r >> 1) & 7)) << 4) + (k & 7) * 2) = o;
-        }
+        for (int j = 0; j < 8; ++j)
+          o[j] = (_Float16)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+        *reinterpret_cast<h8*>(panel + (c >> 3) * (BM * 128) + r * 128 +
+                               (((c & 7) ^ ((r >> 1) & 7)) << 4)) = o;
       }
     }
   }
 }
 
-template <int BM, int NT, typename T>
-__device__ __forceinline__ void normalise_panel(const T* x, int M, int H, int m0, const LnArgs& ln,
+// At most 4 chunks per lane: rows of up to 224 chunks (gemm_layernorm_supported), 64 lanes beyond 128.
+template <int BM, int NT>
+__device__ __forceinline__ void normalise_panel(const _Float16* x, int M, int H, int m0, const LnArgs& ln,
                                                 char* panel, int tid) {
-  const int need = (H / (16 / (int)sizeof(T)) + ln.lpr - 1) / ln.lpr;  // chunks per lane
+  const int need = (H / 8 + ln.lpr - 1) / ln.lpr;  // chunks per lane
 #define GPTMI_LN_ROWS(L)                                                       \
   do {                                                                         \
-    if (need <= 1) normalise_rows<BM, NT, T, L, 1>(x, M, H, m0, ln, panel, tid);      \
-    else if (need <= 2) normalise_rows<BM, NT, T, L, 2>(x, M, H, m0, ln, panel, tid); \
-    else if (need <= 3) normalise_rows<BM, NT, T, L, 3>(x, M, H, m0, ln, panel, tid); \
-    else if (need <= 4) normalise_rows<BM, NT, T, L, 4>(x, M, H, m0, ln, panel, tid); \
-    else normalise_rows<BM, NT, T, L, 8>(x, M, H, m0, ln, panel, tid);                \
+    if (need <= 1) normalise_rows<BM, NT, L, 1>(x, M, H, m0, ln, panel, tid);      \
+    else if (need <= 2) normalise_rows<BM, NT, L, 2>(x, M, H, m0, ln, panel, tid); \
+    else if (need <= 3) normalise_rows<BM, NT, L, 3>(x, M, H, m0, ln, panel, tid); \
+    else normalise_rows<BM, NT, L, 4>(x, M, H, m0, ln, panel, tid);                \
   } while (0)
   if (ln.lpr == 32) GPTMI_LN_ROWS(32);
   else GPTMI_LN_ROWS(64);
@@ -135,7 +126,7 @@ struct Tile {
   static constexpr int THREADS = 64 * WM_ * WN_ * WK_;
 };
 
-// T: storage type of bias and residual (and of x with LNA).  OT: type of the output: T, or fp16 for
+// T: storage type of bias and residual (fp16 with LNA).  OT: type of the output: T, or fp16 for
 // fp32 storage where the output is the next product's operand (no residual then).
 // WIDE: rows of 2^22 elements and more (64-bit lane addresses).
 template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE>
@@ -255,7 +246,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   };
 
   if constexpr (LNA) {
-    normalise_panel<BM, NT, T>((const T*)Av, M, Kp, m0, ln, smem + NST * STAGE, tid);
+    normalise_panel<BM, NT>((const _Float16*)Av, M, Kp, m0, ln, smem + NST * STAGE, tid);
     wait_vmcnt<0>();
     __syncthreads();
   } else {
@@ -589,12 +580,11 @@ typedef Tile<32,  64, 1, 4, 2, 3> Ln32x64;
 typedef Tile<32, 128, 1, 8, 1, 3> Ln32x128;
 constexpr int kLnStages = 3 * 128 * 128;
 
-// Index and column width of the form that serves these sizes.
-inline int pick_ln(int64_t M, int N, int K, bool split, int cus, int* bn) {
+// Index of the form that serves these sizes.
+inline int pick_ln(int64_t M, int N, int K, bool split, int cus) {
   const int wk = split ? kTiles[pick_tile(M, N, K, cus, nullptr)].wk : 1;
   const int64_t rows = (M + 31) / 32;
   const bool wide = wk == 4 && K <= 1024 && rows * ((N + 31) / 32) > cus;
-  *bn = wk == 1 ? 128 : wk == 2 || wide ? 64 : 32;
   return wk == 1 ? 3 : wk == 2 ? 2 : wide ? 1 : 0;
 }
 
@@ -603,8 +593,7 @@ int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiD
               bool split, hipStream_t st) {
   const int cus = cu_count();
   if (cus < 0) return cus;
-  int bn;
-  switch (pick_ln(M, N, K, split, cus, &bn)) {
+  switch (pick_ln(M, N, K, split, cus)) {
     case 0: return launch_tile_cfg<Ln32x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 1: return launch_tile_cfg<Ln32x64w, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 2: return launch_tile_cfg<Ln32x64, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
@@ -616,7 +605,7 @@ int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiD
 bool gemm_layernorm_supported(int64_t M, int H) {
   if (H <= 0 || H % 64 != 0 || M <= 0) return false;
   const int nchunks = H / 8, lpr = lanes_per_row(nchunks);
-  return (nchunks + lpr - 1) / lpr <= 8 && (size_t)kLnStages + 64 * (size_t)H <= 160 * 1024;
+  return (nchunks + lpr - 1) / lpr <= 4 && (size_t)kLnStages + 64 * (size_t)H <= 160 * 1024;
 }
 
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
