@@ -185,7 +185,7 @@ static int check_linear_args(const void* x, const void* W, const void* out, int6
 // workspace, all of them fp16: for fp16 storage that is the storage type, for fp32 storage it is the
 // rounding that the next product (or the attention) applies to its operands anyway -- LayerNorm, q, k,
 // v, the attention's output and the GELU's output are each written once in fp16 instead of in fp32 and
-// again by a pack pass, with the same bits at the end.
+// again by a pack pass.
 
 // Carves 256-byte aligned pieces out of a workspace.
 struct Carver {

@@ -28,17 +28,21 @@ from .kernels import (HEAD_SIZES, attention_block, block_supported, dropout_mask
                       pack_lm_head, pack_weight)
 
 # Up to this many token rows of up to this width the blocks run their LayerNorm inside the following
-# GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile and one
-# of its workgroups fills a CU, so it pays while all column tiles run at once: LayerNorm -> ffn1 at
-# 24 / 128 / 200 rows of 768 takes 6.6 / 8.5 / 13.5 us against 7.7 / 9.3 / 10.4 for the two launches, at
-# 24 rows of 1024 8.1 against 7.5, of 1600 13.0 against 11.9.
+# GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile, in front
+# of its first product, and one of its workgroups fills a CU.  So it pays while all column tiles run at
+# once and while normalising 32 rows costs less than a launch, up to 768: LayerNorm -> ffn1 at 24 / 128 /
+# 160 / 192 rows of 768 takes 6.5 / 8.3 / 8.5 / 13.3 us against 7.7 / 9.3 / 9.9 / 9.9 for the two
+# launches, 24 and 64 rows of 1024 8.0 and 9.3 against 7.5 and 8.6, 24 of 1600 13.1 against 12.2.
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
 
 # Up to this many token rows a block is one call of the library (attention_block, mlp_block) instead
-# of one per operator: below about 4000 rows of the 124M model the host, not the GPU, sets the pace of
-# an operator-by-operator forward (some 10 us per operator against 2 us per launch inside one call).
-# Above, the calls hide behind the GPU.  fp32 models take the block calls at every size: their
+# of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one the host
+# sets the pace of an operator-by-operator forward (some 10 us per operator against 2 us per launch
+# inside one call: 512 rows 898 against 566 us, 2048 rows 887 against 819; 1024-wide 512 rows 1759
+# against 1386).  From there to 24576 rows the two are within 1 % (6144 rows of 124M: 1814 against 1716);
+# the line lies where that holds for any model, and beyond it the operators give each intermediate
+# matrix back before they take the next.  fp32 models take the block calls at every size: their
 # intermediate matrices are fp16 there (see gptmi_attention_block).
 BLOCK_MAX_ROWS = 8192
 
@@ -411,9 +415,9 @@ def convert_hf_and_load_model(model_id, device):
 
 class GraphedForward:
     """The forward of an eval-mode FusedGPT for one input shape, captured once into a HIP graph
-    and replayed per call: the ~110 launches of a forward become one graph launch, which is what
-    a small batch is bound by (2 x 64 tokens, 124M: 1.76 -> 1.06 ms).  Nothing in the library
-    allocates or synchronises, so capture needs no special path; the operators' output tensors
+    and replayed per call: the 63 launches of a forward become one graph launch and their host work
+    goes (2 x 64 tokens, 124M: 0.50 -> 0.42 ms).  Nothing in the library allocates or
+    synchronises, so capture needs no special path; the operators' output tensors
     come from the graph's private pool.  The result of a call is overwritten by the next call --
     clone it to keep it.  No counterpart in the reference (Triton launches kernel by kernel)."""
 

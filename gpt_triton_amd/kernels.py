@@ -480,8 +480,8 @@ def _block_layout(first, second, what):
 def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, num_heads,
                     dropout_prob=0.0, normed=None, layer_norm_in_gemm=False, keep=None):
     """x + dropout(proj(attention(qkv(LayerNorm(x))))) for x [B, L, h]: the operators of an attention
-    block (gpt.py:39-60) behind one call of the library, with their bits.  `normed`: LayerNorm(x), if
-    the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`; keep: a
+    block (gpt.py:39-60) behind one call of the library, with their bits in fp16 (fp32: up to the fp16
+    rounding of the projection's operands).  `normed`: LayerNorm(x), if the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`; keep: a
     `dropout_mask` for dropout_prob of at least max(x.numel(), L * L) offsets, read instead of
     generating the masks here."""
     B, L, h = x.shape

@@ -290,9 +290,12 @@ int gptmi_dropout_mask(void* mask, int64_t n, float p, uint64_t seed, void* stre
  * A whole attention block, x + proj(attention(qkv(LayerNorm(x)))), and a whole MLP block,
  * x + W2 . gelu(W1 . LayerNorm(x)), behind one call each: the launches of gptmi_layernorm (or the
  * LayerNorm prologue, or `normed` = LayerNorm(x) from gptmi_embed_layernorm), gptmi_linear_qkv,
- * gptmi_flash_attn and gptmi_linear, in that order, with the same bits.  What the calls save is host
- * time (a few hundred tokens are bound by it) and, for fp32 storage, traffic: the intermediate
- * matrices live in the workspace in fp16, the rounding that the next product applies to its operands.
+ * gptmi_flash_attn and gptmi_linear, in that order; for fp16 storage with the same bits.  What the
+ * calls save is host time (a few hundred tokens are bound by it) and, for fp32 storage, traffic: the
+ * intermediate matrices live in the workspace in fp16, the rounding that the next product applies to
+ * its operands.  The MLP block has the operators' bits there too; the attention may run another of its
+ * kernels, whose fp32 sums run in another order, and a last-bit difference can turn the fp16 rounding of
+ * one of the projection's operands.
  *
  * Replaces the bodies of FusedAttention.forward and FusedMLP.forward, gpt.py:39-60 and 91-111.
  *   x, out [B*L][h] or [M][H]        normed: LayerNorm(x) in the storage type, or NULL

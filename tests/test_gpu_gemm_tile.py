@@ -1,7 +1,8 @@
 """The GEMM with one workgroup per output tile (gemm_tile.hip) at the sizes where it can go wrong:
-fewer k-slices than groups that split K, k-steps fewer than, equal to and one more than the stages,
-a last k-step that not every group has a slice of, one row and one column past a tile, columns that do
-not fill a 16-byte chunk, and a shape each that the cost model sends to every tile of the menu.
+fewer k-slices than groups that split K (two groups; a four-way split is never picked below four slices),
+k-steps fewer than, equal to and one more than the stages, a last k-step that not every group has a slice
+of, one row and one column past a tile, columns that do not fill a 16-byte chunk, and a shape each that
+the cost model sends to every tile of the menu (test_host.py holds the list to that).
 Reference: an fp32 product of the fp16-rounded operands (the operands of the kernel), epilogue in fp32.
 
 Tolerance: the fp32 sums of K products differ by at most K * 2^-24 of the sum of their absolute values,
@@ -49,7 +50,7 @@ def check(got, want, sums, Kd, what):
 # (M, N, K): tiles 32x16 and 32x32 split K four ways with four stages of 256, 64x32 with three,
 # 64x64 two ways with four of 128, 64x128 with three, the others walk 64 at a time
 SHAPES = [
-    (1, 16, 64), (24, 768, 64), (31, 48, 192), (32, 32, 256), (33, 40, 320),   # 1, 1, 3, 4, 5 slices
+    (1, 16, 64), (24, 768, 64), (31, 48, 192), (32, 32, 256), (33, 40, 320),   # 1, 1, 3; 4, 5 slices
     (24, 768, 1024), (24, 768, 1088), (24, 768, 1344),   # stages full, one slice and one step more
     (128, 768, 3072), (129, 776, 448),
     (200, 3072, 128), (300, 2304, 832), (65, 6400, 576),
@@ -57,6 +58,8 @@ SHAPES = [
     (1477, 768, 576), (1500, 1544, 320),
     (1024, 3072, 768), (3073, 768, 832), (2049, 2304, 256), (2500, 3080, 192),
     (37, 50, 128), (130, 33, 70), (1100, 1001, 200),     # columns and k that fill no chunk
+    (127, 2311, 448), (128, 2304, 768), (127, 2312, 832),      # 64x32: 2, 3 and 4 k-steps of three stages
+    (4700, 3001, 200), (4800, 3072, 768), (4801, 3080, 832),   # 128x256
 ]
 
 

@@ -65,8 +65,8 @@ def operands(M, H, N, seed):
     (70, 128, 256, False, True),     # one chunk per lane, 32 lanes per row
     (300, 256, 520, True, True),
     (64, 1024, 4096, True, True),    # GPT-2 medium's width: 64 lanes per row, two chunks each
-    (40, 1280, 1280, False, True),   # large: five chunks per lane (the eight-chunk variant)
-    (32, 1600, 6400, True, True),    # XL: seven chunks per lane, the widest panel that fits
+    (40, 1280, 1280, False, True),   # large: 64 lanes per row, three chunks each
+    (32, 1600, 6400, True, True),    # XL: four chunks per lane, a panel of 100 KB
     (5, 64, 64, False, False),
     (5000, 768, 768, False, True),   # 157 row tiles, the last with 8 rows (far beyond where the model uses it)
 ])

@@ -263,3 +263,30 @@ def test_attention_block_checks_the_head_size_before_any_launch(lib):
         rc = lib.gptmi_attention_block(fake, None, fake, fake, 1e-5, fake, fake, fake, fake, fake, 1, 8, heads, d,
                                        0.0, 1337, None, 0, 0, 2, fake, need, 1, None)
         assert rc == -2 and b"head size" in lib.gptmi_last_error()
+
+
+def test_the_tile_gemm_cases_reach_every_tile():
+    # the cost model of gemm_tile.hip, its numbers read from there, on 256 CUs
+    import test_gpu_gemm_tile
+
+    source = open(os.path.join(ROOT, "gpt_triton_amd", "csrc", "gemm_tile.hip")).read()
+    menu = re.search(r"TileCost kTiles\[\] = \{(.*?)\};", source, re.S).group(1)
+    tiles = [[float(v.rstrip("f")) for v in row.split(",")] for row in re.findall(r"\{([^{}]*)\}", menu)]
+    assert len(tiles) == 8
+
+    def pick(M, N, slices):
+        def cost(tile):
+            bm, bn, _, launch, fixed, per_slice = tile
+            rounds = -(-(-(-M // int(bm)) * -(-N // int(bn))) // 256)
+            return launch + rounds * (fixed + slices * per_slice)
+        return min(range(len(tiles)), key=lambda i: cost(tiles[i]))
+
+    picked = {(pick(M, N, -(-K // 64)), -(-K // 64)) for M, N, K in test_gpu_gemm_tile.SHAPES}
+    assert {i for i, _ in picked} == set(range(len(tiles)))
+    # k-slices: fewer than the groups; as many and more, with groups that have none in the last k-step
+    groups = [int(tile[2]) for tile in tiles]
+    assert any(slices < groups[i] for i, slices in picked)
+    for i in range(3):  # the four-way splits
+        assert groups[i] == 4 and {s % 4 == 0 for j, s in picked if j == i} == {True, False}
+    sizes = [(M, N) for M in (1, 8, 24, 64, 128, 200, 513, 1477, 4800) for N in (16, 40, 768, 2304, 6400)]
+    assert all(groups[pick(M, N, slices)] < 4 for M, N in sizes for slices in (1, 2, 3))
