@@ -401,7 +401,7 @@ def main():
         # no ffn1 launch of its own was seen: the LayerNorm-prologue form (few rows) or a graph
         # replay; time the call by itself
         xs = torch.randn(tokens, h, device=dev).half()
-        w1 = model.blocks[0][1]._weight("ffn1_weight")
+        w1 = model.blocks[0][1]._packed.get("ffn1_weight", model.blocks[0][1].ffn1_weight)
         b1 = model.blocks[0][1].ffn1_bias.data
         ffn1_ms = time_op(lambda: inner(xs, w1, b1, None, True, 0.0), min_ms=20.0, warm_ms=5.0)[0]
     achieved = ffn1_flops / (ffn1_ms * 1e-3) / 1e12

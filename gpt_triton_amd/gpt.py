@@ -89,14 +89,14 @@ class _Block(nn.Sequential):
 
     def forward(self, x, keep=None):
         for module in self:
-            x = _call_with_mask(module, x, keep)
+            x = module(x) if keep is None else _call_with_mask(module, x, keep)
         return x
 
 
 def _call_with_mask(module, x, keep):
     """module(x), with the mask where the forward that the call will run is one of this file's: one
     replaced on the instance, in its class or by a subclass takes what nn.Sequential hands it."""
-    if keep is not None and getattr(module.forward, "__func__", None) in _TAKE_MASK:
+    if getattr(module.forward, "__func__", None) in _TAKE_MASK:
         return module(x, keep=keep)
     return module(x)
 
@@ -140,12 +140,15 @@ def _tensors(module, names):
     return prm if names <= prm.keys() else {name: getattr(module, name) for name in names}
 
 
-def _are_parameters(module, tensors, first, second):
-    """Whether a module's two weights are parameters: images are kept for those only, and for both or
-    neither.  What stands in for one is another tensor every time, in the dictionary of parameters too
-    (torch.func.functional_call puts plain tensors there)."""
-    return (tensors is module._parameters and isinstance(tensors[first], nn.Parameter) and
-            isinstance(tensors[second], nn.Parameter))
+def _weights(module, tensors, first, second):
+    """A module's two weights as the products take them: images in eval mode, kept for parameters only,
+    and for both or neither.  What stands in for one is another tensor every time, in the dictionary of
+    parameters too (torch.func.functional_call puts plain tensors there)."""
+    a, b = tensors[first], tensors[second]
+    if (module.training or tensors is not module._parameters or not isinstance(a, nn.Parameter) or
+            not isinstance(b, nn.Parameter)):
+        return a.data, b.data
+    return module._packed.get(first, a), module._packed.get(second, b)
 
 
 class FusedAttention(nn.Module):
@@ -168,13 +171,10 @@ class FusedAttention(nn.Module):
     _NAMES = frozenset(("layer_norm_weight", "layer_norm_bias", "c_attn_weight", "c_attn_bias",
                         "c_proj_weight", "c_proj_bias"))
 
-    def _weight(self, name, tensors=None):
-        tensors = tensors or _tensors(self, self._NAMES)
-        prm = tensors[name]
-        if (self.training or (self.hidden_size // self.num_heads) % 8 != 0 or
-                not _are_parameters(self, tensors, "c_attn_weight", "c_proj_weight")):
-            return prm.data
-        return self._packed.get(name, prm)
+    def _weights(self, tensors):
+        if (self.hidden_size // self.num_heads) % 8 != 0:
+            return tensors["c_attn_weight"].data, tensors["c_proj_weight"].data
+        return _weights(self, tensors, "c_attn_weight", "c_proj_weight")
 
     def train(self, mode=True):
         self._packed.clear()
@@ -188,13 +188,13 @@ class FusedAttention(nn.Module):
         if keep is not None and not (p > 0.0 and keep.serves(x, max(x.numel(), x.shape[1] ** 2), p)):
             keep = None
         prm = _tensors(self, self._NAMES)
-        w_attn = self._weight("c_attn_weight", prm)
+        w_attn, w_proj = self._weights(prm)
         in_gemm = normed is None and p == 0.0 and _ln_in_gemm(x, w_attn)
         if _as_block(x, keep) and x.shape[-1] // self.num_heads in HEAD_SIZES:
             return attention_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w_attn,
-                                   prm["c_attn_bias"], self._weight("c_proj_weight", prm),
-                                   prm["c_proj_bias"], self.num_heads, dropout_prob=p,
-                                   normed=normed, layer_norm_in_gemm=in_gemm, keep=keep)
+                                   prm["c_attn_bias"], w_proj, prm["c_proj_bias"], self.num_heads,
+                                   dropout_prob=p, normed=normed, layer_norm_in_gemm=in_gemm,
+                                   keep=keep)
         skip = x
         y = normed
         if in_gemm:
@@ -208,8 +208,8 @@ class FusedAttention(nn.Module):
         # [B, N, L, d] values in a [B, L, N, d] buffer: the head merge below copies nothing
         y = flash_attention_v1(q, k, v, dropout_prob=p, merged_heads_layout=True)
         y = y.transpose(1, 2).contiguous().view(skip.shape)
-        return fused_ffn(y, self._weight("c_proj_weight", prm), bias=prm["c_proj_bias"].data,
-                         residual=skip, add_gelu=False, dropout_prob=p)
+        return fused_ffn(y, w_proj, bias=prm["c_proj_bias"].data, residual=skip, add_gelu=False,
+                         dropout_prob=p)
 
     def get_fwd_flops(self, num_tokens):
         h = self.hidden_size
@@ -237,12 +237,8 @@ class FusedMLP(nn.Module):
     _NAMES = frozenset(("layer_norm_weight", "layer_norm_bias", "ffn1_weight", "ffn1_bias",
                         "ffn2_weight", "ffn2_bias"))
 
-    def _weight(self, name, tensors=None):
-        tensors = tensors or _tensors(self, self._NAMES)
-        prm = tensors[name]
-        if self.training or not _are_parameters(self, tensors, "ffn1_weight", "ffn2_weight"):
-            return prm.data
-        return self._packed.get(name, prm)
+    def _weights(self, tensors):
+        return _weights(self, tensors, "ffn1_weight", "ffn2_weight")
 
     def train(self, mode=True):
         self._packed.clear()
@@ -252,9 +248,9 @@ class FusedMLP(nn.Module):
         """`keep`: as in FusedAttention.forward."""
         p = self.dropout_prob if self.training else 0.0
         prm = _tensors(self, self._NAMES)
-        w1, w2 = self._weight("ffn1_weight", prm), self._weight("ffn2_weight", prm)
+        w1, w2 = self._weights(prm)
         # the weights, and x with them, may have other widths than h and 4h (pruned, exchanged)
-        width, inner = x.shape[-1], w1.shape[1]
+        width, inner = w1.shape
         if keep is not None and not (
                 p > 0.0 and keep.serves(x, x.numel() // width * max(inner, width), p)):
             keep = None
@@ -342,7 +338,7 @@ class FusedGPT(nn.Module):
             rest = blocks
         keep = _keep_mask(x, self.config.n_embd, len(rest), self.config.n_head, p) if p > 0.0 else None
         for block in rest:
-            x = _call_with_mask(block, x, keep)
+            x = block(x) if keep is None else _call_with_mask(block, x, keep)
         x = fused_layer_norm(x, self.layer_norm_weight.data, self.layer_norm_bias.data)
         if return_logits:
             return x, lm_head(x, self._lm_head_weight())
