@@ -571,8 +571,8 @@ int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, co
 // it (split = false: not at all, the rows that launch gives to the persistent kernel), so that the
 // sums, too, are formed in the same order.  One workgroup fills a CU's
 // LDS, so more workgroups than CUs take a second round: one launch of 128 rows x 768 x 3072 as 384
-// tiles of 32 x 32 took 13.4 us against 9.6 for the LayerNorm launch and the plain one, as 192 of
-// 32 x 64 8.9; 24 rows (96 tiles) 6.9 against 8.0.
+// tiles of 32 x 32 took 13.4 us against 9.3 for the LayerNorm launch and the plain one, as 192 of
+// 32 x 64 8.3; 24 rows (96 tiles) 6.5 against 7.7.
 namespace {
 typedef Tile<32,  32, 1, 2, 4, 3> Ln32x32;
 typedef Tile<32,  64, 1, 2, 4, 3> Ln32x64w;

@@ -40,9 +40,9 @@ LN_PROLOGUE_MAX_WIDTH = 768
 # of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one the host
 # sets the pace of an operator-by-operator forward (some 10 us per operator against 2 us per launch
 # inside one call: 512 rows 898 against 566 us, 2048 rows 887 against 819; 1024-wide 512 rows 1759
-# against 1386).  From there to 24576 rows the two are within 1 % (6144 rows of 124M: 1814 against 1716);
-# the line lies where that holds for any model, and beyond it the operators give each intermediate
-# matrix back before they take the next.  fp32 models take the block calls at every size: their
+# against 1386).  From there to 24576 rows the two are within 2 %, but for 5 % at 6144 rows of 124M (1814
+# against 1716); the line lies beyond that, where only the memory differs: the operators give each
+# intermediate matrix back before they take the next.  fp32 models take the block calls at every size: their
 # intermediate matrices are fp16 there (see gptmi_attention_block).
 BLOCK_MAX_ROWS = 8192
 
@@ -74,7 +74,7 @@ def _keep_mask(x, width, layers, heads, p):
     masks of all layers from one seed at offsets that count from 0, so they are all parts of the mask
     of the widest matrix ([tokens, 4 * width]; attention weights: the first L * L offsets).  Drawn
     once per forward instead of in every kernel that applies it: 16 x 300 tokens 124M, each of 12 ffn1
-    launches 85 -> 43 us, projections and ffn2 32 -> 22, attentions 72 -> 20, for one launch of 24."""
+    launches 85 -> 44 us, projections and ffn2 32 -> 23, attentions 72 -> 21, for one launch of 24."""
     tokens, seqlen = x.numel() // width, x.shape[1]
     bits = max(tokens * 4 * width, seqlen * seqlen)
     if (layers == 0 or bits > 1 << 32 or not block_supported(x, width) or width % heads != 0 or
