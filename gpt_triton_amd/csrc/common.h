@@ -16,6 +16,23 @@ typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
+// Stores that write through: the line goes to memory at once instead of staying dirty in the XCD's L2
+// until the kernel ends, when the write-back of all of it stands between this launch and the next
+// (behind 29 MB of plain stores 3.0 us from the last wavefront to the first of the next launch, 1.1
+// without).  The memory-side cache keeps the line for the next kernel; non-temporal stores, which are as
+// fast by themselves, send it to HBM (124M forward, 16 x 300 tokens: plain 1907, non-temporal 1858,
+// these 1813 us; 2 x 64 tokens captured: 412, 424, 410).  In assembly, since no builtin stores 16
+// bytes this way: the trailing s_nop keeps the next VALU instruction from overwriting data registers
+// that a store of more than 64 bits reads a little after issue.
+template <typename V>
+__device__ __forceinline__ void store_through(V* p, V v) {
+  static_assert(sizeof(V) == 8 || sizeof(V) == 16, "8 or 16 bytes");
+  if constexpr (sizeof(V) == 16)
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+  else
+    asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
+}
+
 // Cross-lane steps without the LDS: an xor shuffle compiles to ds_bpermute, ~100 cycles of latency
 // per step of a reduction, and the reductions of a LayerNorm row (twelve steps) or of a softmax tile
 // sit on the critical path of their kernels.  The swaps and row rotations are VALU instructions.

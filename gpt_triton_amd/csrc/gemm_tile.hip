@@ -426,7 +426,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     } else {
       dst = (OT*)ep.out + ((int64_t)m * N + n);
     }
-    if (vec) *reinterpret_cast<OV*>(dst) = o;
+    if (vec) store_through(reinterpret_cast<OV*>(dst), o);
     else {
 #pragma unroll
       for (int e = 0; e < CW; ++e)

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void embed_vec_kernel(
     V va = a[c], vb = b[c], vo;
 #pragma unroll
     for (int j = 0; j < VN; ++j) vo[j] = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-    __builtin_nontemporal_store(vo, o + c);
+    store_through(o + c, vo);
   }
 }
 
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void embed_dropout_vec_kernel(
     V vo;
 #pragma unroll
     for (int j = 0; j < VN; ++j) vo[j] = (T)(u[j] > drop.p ? sum[j] : 0.f);
-    reinterpret_cast<V*>(out + row * H)[c] = vo;
+    store_through(reinterpret_cast<V*>(out + row * H) + c, vo);
   }
 }
 
@@ -191,10 +191,10 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
 #pragma unroll
       for (int j = 0; j < VN; ++j)
         to[j] = (OT)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
-      // cached (not streaming) store: the [T, H] output is what the following GEMM reads, two
+      // not a streaming store: the [T, H] output is what the following GEMM reads, two
       // or three times over; it fits the 256 MB memory-side cache, and a GEMM fed from there
       // instead of HBM ran 12 % faster (its operand loads are only one k-tile ahead)
-      o[c] = to;
+      store_through(o + c, to);
     }
   }
 }
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
         v[i][j] = (float)e[j];
         s += v[i][j];
       }
-      __builtin_nontemporal_store(e, eo + c);  // the residual stream; next read by a GEMM epilogue
+      store_through(eo + c, e);  // the residual stream; next read by a GEMM epilogue
     } else {
 #pragma unroll
       for (int j = 0; j < VN; ++j) v[i][j] = 0.f;
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
 #pragma unroll
       for (int j = 0; j < VN; ++j)
         to[j] = (T)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
-      o[c] = to;  // cached store, as in layernorm_vec_kernel: the following GEMM reads it
+      store_through(o + c, to);  // as in layernorm_vec_kernel: the following GEMM reads it
     }
   }
 }
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256) void pack_rows_vec_kernel(const T* __restrict_
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = (_Float16)(float)v[j];
       }
-      *reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8) = o;
+      store_through(reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8), o);
     }
 }
 
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(256) void pack_transpose_vec_kernel(PackArgs<T> fir
     h8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j) o[j] = tile[(kg * 8 + j) * PITCH + n];
-    if (n0 + n < N) *reinterpret_cast<h8*>(dst + (int64_t)(n0 + n) * Kp + k0 + kg * 8) = o;
+    if (n0 + n < N) store_through(reinterpret_cast<h8*>(dst + (int64_t)(n0 + n) * Kp + k0 + kg * 8), o);
   }
 }
 
