@@ -19,6 +19,9 @@ SOURCES = ["rowops.hip", "gemm.hip", "gemm_tile.hip", "flash_attn.hip", "capi.cp
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first kernel arguments (pointers and sizes) come in scalar registers instead of by a load that
+    # every workgroup waits for first: 0.2 us of each launch (128 rows x 768 x 768: 3.68 -> 3.44)
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument", "-Wno-inline-asm",
 ]
 

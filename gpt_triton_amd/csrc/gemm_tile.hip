@@ -36,7 +36,7 @@ namespace {
 // goes to k-slice k / 64, row r's 128 bytes there, 16-byte unit (k % 64) / 8 ^ key(r).  A row is
 // spread over LPR lanes as in layernorm_vec_kernel (same sums, same bits); rows past the end
 // repeat the last row.
-template <int BM, int NT, int LPR, int CH>
+template <int BM, int NT, int LPR, int CH, bool FULL>
 __device__ __forceinline__ void normalise_rows(const _Float16* __restrict__ x, int M, int H, int m0,
                                                const LnArgs& ln, char* panel, int tid) {
   constexpr int RPP = NT / LPR;  // rows per pass
@@ -47,19 +47,6 @@ __device__ __forceinline__ void normalise_rows(const _Float16* __restrict__ x, i
   const h8* bv = reinterpret_cast<const h8*>(ln.b);
   // the rows of all passes and the parameters are requested together: one memory round trip
   h8 tw[CH], tb[CH], t[PASSES][CH];
-  // as a lambda the parameters stay packed halves until they are used (135 registers instead of 158;
-  // LayerNorm -> ffn1 at 24 x 768 6.5 against 6.8 us)
-  auto params = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c = ll + i * LPR;
-      if (c < nchunks) {
-        tw[i] = wv[c];
-        tb[i] = bv[c];
-      }
-    }
-  };
-  params();
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
     int row = m0 + p * RPP + rsub;
@@ -68,32 +55,34 @@ __device__ __forceinline__ void normalise_rows(const _Float16* __restrict__ x, i
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int c = ll + i * LPR;
-      if (c < nchunks) t[p][i] = xr[c];
+      if (FULL || c < nchunks) t[p][i] = xr[c];
+      else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[p][i][j] = (_Float16)0.f;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = ll + i * LPR;
+    if (FULL || c < nchunks) {
+      tw[i] = wv[c];
+      tb[i] = bv[c];
     }
   }
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
     const int r = p * RPP + rsub;
-    float v[CH][8], sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const bool in = ll + i * LPR < nchunks;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v[i][j] = in ? (float)t[p][i][j] : 0.f;
-        if (in) sum += v[i][j];
-      }
-    }
-    float mean, rstd;
-    layernorm_stats<CH, 8, LPR>(v, sum, ll, nchunks, H, ln.eps, mean, rstd);
+    float d[CH][8], rstd;
+    layernorm_stats<CH, 8, LPR, FULL>(t[p], ll, nchunks, H, ln.eps, d, rstd);
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int c = ll + i * LPR;
-      if (c < nchunks) {
+      if (FULL || c < nchunks) {
         h8 o;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          o[j] = (_Float16)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+          o[j] = (_Float16)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
         *reinterpret_cast<h8*>(panel + (c >> 3) * (BM * 128) + r * 128 +
                                (((c & 7) ^ ((r >> 1) & 7)) << 4)) = o;
       }
@@ -106,15 +95,16 @@ template <int BM, int NT>
 __device__ __forceinline__ void normalise_panel(const _Float16* x, int M, int H, int m0, const LnArgs& ln,
                                                 char* panel, int tid) {
   const int need = (H / 8 + ln.lpr - 1) / ln.lpr;  // chunks per lane
-#define GPTMI_LN_ROWS(L)                                                       \
-  do {                                                                         \
-    if (need <= 1) normalise_rows<BM, NT, L, 1>(x, M, H, m0, ln, panel, tid);      \
-    else if (need <= 2) normalise_rows<BM, NT, L, 2>(x, M, H, m0, ln, panel, tid); \
-    else if (need <= 3) normalise_rows<BM, NT, L, 3>(x, M, H, m0, ln, panel, tid); \
-    else normalise_rows<BM, NT, L, 4>(x, M, H, m0, ln, panel, tid);                \
+#define GPTMI_LN_ROWS(L, FULL)                                                       \
+  do {                                                                               \
+    if (need <= 1) normalise_rows<BM, NT, L, 1, FULL>(x, M, H, m0, ln, panel, tid);      \
+    else if (need <= 2) normalise_rows<BM, NT, L, 2, FULL>(x, M, H, m0, ln, panel, tid); \
+    else if (need <= 3) normalise_rows<BM, NT, L, 3, FULL>(x, M, H, m0, ln, panel, tid); \
+    else normalise_rows<BM, NT, L, 4, FULL>(x, M, H, m0, ln, panel, tid);                \
   } while (0)
-  if (ln.lpr == 32) GPTMI_LN_ROWS(32);
-  else GPTMI_LN_ROWS(64);
+  if (H / 8 == need * 32 && ln.lpr == 32) GPTMI_LN_ROWS(32, true);
+  else if (ln.lpr == 32) GPTMI_LN_ROWS(32, false);
+  else GPTMI_LN_ROWS(64, false);
 #undef GPTMI_LN_ROWS
 }
 
@@ -572,8 +562,11 @@ int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, co
 // sums, too, are formed in the same order.  One workgroup fills a CU's
 // LDS, so more workgroups than CUs take a second round: one launch of 128 rows x 768 x 3072 as 384
 // tiles of 32 x 32 took 13.4 us against 9.3 for the LayerNorm launch and the plain one, as 192 of
-// 32 x 64 8.3; 24 rows (96 tiles) 6.5 against 7.7.
+// 32 x 64 8.3 (7.3 with the arithmetic of layernorm.h as it stands).  Normalising is a third of the
+// launch, so while tiles of 16 rows still run at once, they do (24 rows x 768 x 2304: 5.6 us as 72 tiles
+// of 32 x 32, 5.0 as 144 of 16 x 32).
 namespace {
+typedef Tile<16,  32, 1, 2, 4, 3> Ln16x32;
 typedef Tile<32,  32, 1, 2, 4, 3> Ln32x32;
 typedef Tile<32,  64, 1, 2, 4, 3> Ln32x64w;
 typedef Tile<32,  64, 1, 4, 2, 3> Ln32x64;
@@ -583,9 +576,10 @@ constexpr int kLnStages = 3 * 128 * 128;
 // Index of the form that serves these sizes.
 inline int pick_ln(int64_t M, int N, int K, bool split, int cus) {
   const int wk = split ? kTiles[pick_tile(M, N, K, cus, nullptr)].wk : 1;
-  const int64_t rows = (M + 31) / 32;
-  const bool wide = wk == 4 && K <= 1024 && rows * ((N + 31) / 32) > cus;
-  return wk == 1 ? 3 : wk == 2 ? 2 : wide ? 1 : 0;
+  if (wk < 4) return wk == 1 ? 3 : 2;
+  const int64_t cols = (N + 31) / 32;
+  if ((M + 15) / 16 * cols <= cus) return 4;
+  return K <= 1024 && (M + 31) / 32 * cols > cus ? 1 : 0;
 }
 
 template <bool QKV>
@@ -597,6 +591,7 @@ int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiD
     case 0: return launch_tile_cfg<Ln32x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 1: return launch_tile_cfg<Ln32x64w, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 2: return launch_tile_cfg<Ln32x64, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 4: return launch_tile_cfg<Ln16x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     default: return launch_tile_cfg<Ln32x128, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
   }
 }

@@ -154,30 +154,23 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
   const V* xr = reinterpret_cast<const V*>(x + row * H);
   const V* wv = reinterpret_cast<const V*>(w);
   const V* bv = reinterpret_cast<const V*>(b);
-  float v[CH][VN];
-  V tw[CH], tb[CH];  // weight and bias chunks, requested with the row: off the tail of the row
-  float s = 0.f;
+  V t[CH], tw[CH], tb[CH];  // weight and bias chunks, requested with the row: off the tail of the row
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = lane + i * LPR;
     if (c < nchunks) {
-      V t = __builtin_nontemporal_load(xr + c);
+      t[i] = __builtin_nontemporal_load(xr + c);
       if (CH <= 4) {
         tw[i] = wv[c];
         tb[i] = bv[c];
       }
-#pragma unroll
-      for (int j = 0; j < VN; ++j) {
-        v[i][j] = (float)t[j];
-        s += v[i][j];
-      }
     } else {
 #pragma unroll
-      for (int j = 0; j < VN; ++j) v[i][j] = 0.f;
+      for (int j = 0; j < VN; ++j) t[i][j] = (T)0.f;
     }
   }
-  float mean, rstd;
-  layernorm_stats<CH, VN, LPR>(v, s, lane, nchunks, H, eps, mean, rstd);
+  float d[CH][VN], rstd;
+  layernorm_stats<CH, VN, LPR, false>(t, lane, nchunks, H, eps, d, rstd);
   OV* o = reinterpret_cast<OV*>(out + row * H);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
@@ -190,7 +183,7 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
       OV to;
 #pragma unroll
       for (int j = 0; j < VN; ++j)
-        to[j] = (OT)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+        to[j] = (OT)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
       // not a streaming store: the [T, H] output is what the following GEMM reads, two
       // or three times over; it fits the 256 MB memory-side cache, and a GEMM fed from there
       // instead of HBM ran 12 % faster (its operand loads are only one k-tile ahead)
@@ -222,9 +215,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
   const V* wv = reinterpret_cast<const V*>(w);
   const V* bv = reinterpret_cast<const V*>(b);
   V* eo = reinterpret_cast<V*>(emb + row * H);
-  float v[CH][VN];
-  V tw[CH], tb[CH];
-  float s = 0.f;
+  V e[CH], tw[CH], tb[CH];
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = lane + i * LPR;
@@ -232,21 +223,16 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
       const V va = ar[c], vb = pr[c];
       tw[i] = wv[c];
       tb[i] = bv[c];
-      V e;
 #pragma unroll
-      for (int j = 0; j < VN; ++j) {
-        e[j] = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-        v[i][j] = (float)e[j];
-        s += v[i][j];
-      }
-      store_through(eo + c, e);  // the residual stream; next read by a GEMM epilogue
+      for (int j = 0; j < VN; ++j) e[i][j] = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
+      store_through(eo + c, e[i]);  // the residual stream; next read by a GEMM epilogue
     } else {
 #pragma unroll
-      for (int j = 0; j < VN; ++j) v[i][j] = 0.f;
+      for (int j = 0; j < VN; ++j) e[i][j] = (T)0.f;
     }
   }
-  float mean, rstd;
-  layernorm_stats<CH, VN, LPR>(v, s, lane, nchunks, H, eps, mean, rstd);
+  float d[CH][VN], rstd;
+  layernorm_stats<CH, VN, LPR, false>(e, lane, nchunks, H, eps, d, rstd);
   V* o = reinterpret_cast<V*>(out + row * H);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
@@ -255,7 +241,7 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
       V to;
 #pragma unroll
       for (int j = 0; j < VN; ++j)
-        to[j] = (T)layernorm_apply(v[i][j], mean, rstd, (float)tw[i][j], (float)tb[i][j]);
+        to[j] = (T)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
       store_through(o + c, to);  // as in layernorm_vec_kernel: the following GEMM reads it
     }
   }
@@ -283,7 +269,7 @@ __global__ __launch_bounds__(256) void layernorm_scalar_kernel(
   for (int c = lane; c < H; c += 64) {
     if constexpr (sizeof(T) != sizeof(OT)) {
       // fp32 rows with an fp16 output stand for the fp32 LayerNorm and a conversion: two roundings
-      out[row * H + c] = (OT)layernorm_apply((float)xr[c], mean, rstd, (float)w[c], (float)b[c]);
+      out[row * H + c] = (OT)layernorm_apply((float)xr[c] - mean, rstd, (float)w[c], (float)b[c]);
     } else {
       const float z = ((float)xr[c] - mean) * rstd;
       out[row * H + c] = (OT)(z * (float)w[c] + (float)b[c]);
