@@ -147,14 +147,14 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
             l = m - b * Lu;
           }
           _Float16* dst = qkv_col[i2] + ((int64_t)b * batch_stride + (int64_t)l * ep.d);
-          __builtin_nontemporal_store(v, reinterpret_cast<h8*>(dst));
+          store_at(ep.through, reinterpret_cast<h8*>(dst), v);
         } else {
           // wavefront-uniform 64-bit part in scalar registers + one 32-bit lane offset.  mw0 and
           // nw0 derive from a wavefront index the kernel made provably uniform, so this is
           // scalar arithmetic: a base produced by v_readfirstlane right in front of the store
           // would need five wait states the compiler does not insert for assembly, and the
           // store would now and then go out with the previous base.
-          store_nt_base(reinterpret_cast<char*>(ep.out) +
+          store_base(ep.through, reinterpret_cast<char*>(ep.out) +
                             ((mw0 + j * 32 + rr * 8) * (int64_t)N + nw0 + i2 * 64) * 2,
                         lane_byte_off, v);
         }
@@ -223,7 +223,7 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
                                             ((runit ^ rkey ^ ((rr & 1) * 4)) << 4));
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr)
-      store_nt_base(reinterpret_cast<char*>(ep.out) +
+      store_base(ep.through, reinterpret_cast<char*>(ep.out) +
                         ((mw0 + j * 32 + rr * 8) * (int64_t)N + nw0) * 2,
                     lane_byte_off, vv[rr]);
   }
@@ -246,7 +246,8 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
 // loads of the next tile's k-tile 1 are issued BEFORE the epilogue's stores, so waiting for them
 // with vmcnt(EPI_STORES) -- the epilogue issues exactly 16 (fp16) or 32 (fp32) stores per lane --
 // does not wait for the stores' acknowledgements.  The bias is fetched, and waited for, before those loads are issued, so
-// that no compiler-placed wait inside the epilogue falls behind them.  Only whole tiles, no
+// that no compiler-placed wait inside the epilogue falls behind them.  Only whole row tiles (the last one
+// starts at row M - 256, see persistent_rows), no
 // residual, no dropout: the launcher sends everything else to gemm_tile.hip.
 // ---------------------------------------------------------------------------
 template <int MB, int NB, typename T, bool QKV, bool GELU>
@@ -307,10 +308,10 @@ __device__ __forceinline__ void store_wave_tile32(f4 (&acc)[2 * NB][2 * MB], con
             l = m - b * Lu;
           }
           T* dst = qkv_col[i] + ((int64_t)b * batch_stride + (int64_t)l * ep.d);
-          __builtin_nontemporal_store(o, reinterpret_cast<P4*>(dst));
+          store_at(ep.through, reinterpret_cast<P4*>(dst), o);
         } else {
           // wavefront-uniform 64-bit part in scalar registers + one 32-bit lane offset
-          store_nt_base(reinterpret_cast<char*>(ep.out) +
+          store_base(ep.through, reinterpret_cast<char*>(ep.out) +
                             ((mw0 + j * 32 + rr * 8) * (int64_t)N + (nw0 + i * 32)) *
                                 (int64_t)sizeof(T),
                         lane_byte_off, o);
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 
   // Operand-tile slot s = it * 512 + tid: row it * 64 + tid / 8, 16-byte position tid % 8,
   // which holds source chunk (tid % 8) ^ ((row >> 1) & 7) -- the key does not depend on `it`.
-  // M and N are multiples of 256 here (the launcher sends other rows to gemm_tile.hip), so no
+  // M is 256 or more, the last row tile starts at M - 256 and N is a multiple of 64, so no
   // row is clamped: a load address is a per-tile scalar base (first row of the tile, k-tile
   // offset) plus one of four per-thread 32-bit offsets shared by A and B.
   const int r0 = tid >> 3;
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const int grp = tile / (tiles_m * group_w);
     const int in_grp = tile - grp * tiles_m * group_w;
     const int grp_w = min(group_w, tiles_n - grp * group_w);
-    m0 = (in_grp / grp_w) * BM;
+    m0 = min((in_grp / grp_w) * BM, M - BM);
     n0 = (grp * group_w + in_grp % grp_w) * BN;
   };
   // A k-tile is eight 16-byte loads per lane: four for the A rows, four for the B rows.  The
@@ -594,7 +595,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Streaming kernel WITH a residual (fp16 row-major output, whole 256 x 256 tiles): the
+// Streaming kernel WITH a residual (fp16 row-major output, 256 rows or more): the
 // persistent pipeline of gemm_stream_kernel, and the residual brought through LDS as in
 // store_wave_tile_rs says.  The residual of a tile (128 KB) has no place of its own in LDS, so it
 // takes the operand stages as they fall free at the end of the tile, and the next tile's first two
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 // A barrier stands in front of every refill because a wavefront's loads write stripes of every
 // wavefront's part of a stage.  What this buys over one workgroup per tile: no pipeline fill per
 // tile beyond what the epilogue's second half hides, and no idle CU between two workgroups while
-// the stores of the one that ended drain.  Whole tiles only; the launcher sends row tiles that
+// the stores of the one that ended drain.  The launcher sends row tiles that
 // do not fill a round of the persistent workgroups to gemm_tile.hip.
 // ---------------------------------------------------------------------------
 template <int WM, int WN>
@@ -649,7 +650,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
     const int grp = tile / (tiles_m * group_w);
     const int in_grp = tile - grp * tiles_m * group_w;
     const int grp_w = min(group_w, tiles_n - grp * group_w);
-    m0 = (in_grp / grp_w) * BM;
+    m0 = min((in_grp / grp_w) * BM, M - BM);
     n0 = (grp * group_w + in_grp % grp_w) * BN;
   };
   // the halves of a k-tile (four loads per lane each) and their scalar sources, as in
@@ -943,7 +944,7 @@ int launch_stream_res(const void* A, const void* Bt, int64_t M, int N, int Kp, c
   }
   const int num_cus = cu_count();
   if (num_cus < 0) return num_cus;
-  const int tiles_m = (int)(M / 256), tiles_n = (N + 255) / 256;
+  const int tiles_m = (int)((M + 255) / 256), tiles_n = (N + 255) / 256;
   const int num_tiles = tiles_m * tiles_n;
   const int group_w = column_group(tiles_n, 256, Kp);
   const int grid = num_tiles < num_cus ? num_tiles : num_cus;
@@ -953,20 +954,30 @@ int launch_stream_res(const void* A, const void* Bt, int64_t M, int N, int Kp, c
 }
 
 // Cost in microseconds of a persistent launch over `tiles` 256 x 256 tiles, in the terms of the
-// cost model of gemm_tile.hip: every workgroup walks ceil(tiles / CUs) of them, and a k-slice takes
-// longer the more of the chip works (L2 and clock).  Fitted to the products of four GPT-2 widths at 12
-// row counts from 2048 to 65536 (11 % off at worst, 6 % at the 10th and 90th percentile).
+// cost model of gemm_tile.hip: every workgroup walks ceil(tiles / CUs) of them, and tile and k-slice take
+// longer the more of the chip works (L2 and clock).  Fitted to the same products from 256 rows on.
 inline float stream_cost(int64_t tiles, int Kp, bool res, int cus) {
   const float rounds = (float)((tiles + cus - 1) / cus), fill = (float)tiles / (float)cus, k = (float)(Kp / 64);
-  return res ? rounds * 6.1f + k * (1.018f * rounds + 0.602f * fill)
-             : 3.25f + rounds * 3.33f + k * (0.965f * rounds + 0.656f * fill);
+  return res ? rounds * 7.42f + k * (0.787f * rounds + 0.780f * fill)
+             : 1.67f + rounds * 4.70f + fill * 1.63f + k * (0.917f * rounds + 0.659f * fill);
+}
+
+// Whether the two matrices of M x N elements share an address.
+inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem) {
+  const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+  return (p < q ? q - p : p - q) < (uintptr_t)M * (uintptr_t)N * elem;
 }
 
 // Divides the rows between the persistent kernel and the tile kernel.  The persistent kernel takes
-// whole 256-row tiles: all of them, as many as fill whole rounds of the CUs (every workgroup walks
+// 256-row tiles: all rows, as many tiles as fill whole rounds of the CUs (every workgroup walks
 // ceil(tiles / CUs) tiles, so a few tiles beyond a whole number of rounds cost a full round: the
 // headline's ffn1 has 7200 tiles = 28 rounds + 32, 597 of its 600 row tiles stay), or none, whichever
 // the cost model says is the fastest; the rows that are left follow in a launch of the tile kernel.
+// All rows also where they are no multiple of 256: the last row tile starts at row M - 256, and the rows
+// that it shares with the tile in front of it are formed twice, from the same operands in the same order,
+// so both store the same bits (4800 x 768 x 3072 with GELU: 27.0 us, 35.4 on the tile kernel; 3885 x 1024 x
+// 4096 35.2, 43.6; a second launch for the rows beyond a multiple costs 6 us and more).  Not with an output
+// over its own residual, which the second pass would read changed: whole row tiles and a launch behind them.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, no dropout.
 // Sets *head to the number of rows for the persistent kernel.
@@ -981,18 +992,20 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   if (!persistent) return 0;
   const int cus = cu_count();
   if (cus < 0) return cus;
-  const int64_t tiles_m = M / 256, tiles_n = (N + 255) / 256;
-  const int64_t whole = tiles_m * tiles_n / cus * cus / tiles_n;  // row tiles that fill whole rounds
+  const int64_t tiles_n = (N + 255) / 256;
+  const int64_t all = res && overlap(ep.out, ep.residual, M, N, sizeof(OT)) ? M / 256 * 256 : M;
+  const int64_t tiles = (all + 255) / 256 * tiles_n;
+  const int64_t whole = tiles / cus * cus / tiles_n * 256;  // rows of the row tiles that fill whole rounds
   // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
   // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
   // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
   // 20480 x 1024 x 4096, is the other way round, 196 against 183).
-  float least = tiles_m * tiles_n >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
-  for (const int64_t tm : {tiles_m, whole}) {
-    if (tm == 0) continue;
-    float c = stream_cost(tm * tiles_n, Kp, res, cus);
-    if (tm * 256 < M) c += 1.0f + gemm_tile_cost(M - tm * 256, N, Kp, cus);
-    if (c < least) least = c, *head = tm * 256;
+  float least = tiles >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
+  for (const int64_t rows : {all, whole < all ? whole : all}) {
+    if (rows == 0) continue;
+    float c = stream_cost((rows + 255) / 256 * tiles_n, Kp, res, cus);
+    if (rows < M) c += 1.0f + gemm_tile_cost(M - rows, N, Kp, cus);
+    if (c < least) least = c, *head = rows;
   }
   return 0;
 }
@@ -1077,6 +1090,11 @@ static int make_epi(const GemmEpilogue& e, int64_t M, int N, EpiDev& ep) {
   ep.vec_ok = vec ? 1 : 0;
   auto aligned16 = [&](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool half_out = e.f16 || e.out_f16;
+  // What the next kernel finds in the 256 MB memory-side cache it need not fetch from HBM; beyond half of
+  // that, non-temporal stores, which leave the cache to the operands (forwards, all non-temporal / all through:
+  // medium 5 x 777 3686 / 3461 us, 16 x 300 with logits 1720 / 1697 (1686 with the line), 512 x 300
+  // 28.57 / 30.16 ms; lines from 40 to 160 MB are equal).
+  ep.through = M * (int64_t)N * (half_out ? 2 : 4) <= (128ll << 20);
   const int cw = half_out ? 8 : 4;
   ep.tile_vec = N % cw == 0 && (!e.qkv || e.d % cw == 0) && aligned16(e.bias) && aligned16(e.residual) &&
                 aligned16(e.out) && aligned16(e.q) && aligned16(e.k) && aligned16(e.v);

@@ -22,6 +22,7 @@ struct EpiDev {
   int vec_ok;  // pointers and N allow 4-element vector accesses
   int tile_vec; // gemm_tile_kernel: N, head size and every pointer allow 16-byte accesses
   int vec8_ok; // fp16 output: N, head size and the output pointers also allow 16-byte stores
+  int through; // outputs written through (store_through), not non-temporal: make_epi
   int m_off;   // head-major scatter: row 0 of this launch is row m_off of the [B*L] token rows
   DropoutArgs drop;  // p > 0: dropout between GELU and residual (gemm_tile_kernel only)
   const unsigned char* keep;  // its mask by flat index, or nullptr: generated in the epilogue
@@ -62,8 +63,9 @@ __device__ __forceinline__ void lds_dma16_base(const void* base, unsigned lane_o
                : "memory", "m0");
 }
 
-// Streaming store of 4 or 8 output elements at (wavefront-uniform 64-bit base) + (32-bit lane
-// offset).  Written as assembly because the compiler otherwise materialises one 64-bit address
+// Store of 4 or 8 output elements at (wavefront-uniform 64-bit base) + (32-bit lane
+// offset), written through (see store_through) or non-temporal as ep.through says (make_epi).
+// Written as assembly because the compiler otherwise materialises one 64-bit address
 // pair per store of an unrolled epilogue and spills.  Two hazards the compiler handles for its
 // own instructions and cannot see inside assembly:
 //   * a scalar register written by a VALU instruction (v_readfirstlane) must not be read by a
@@ -71,23 +73,30 @@ __device__ __forceinline__ void lds_dma16_base(const void* base, unsigned lane_o
 //     that the compiler had to move out of a vector register;
 //   * a store of more than 64 bits reads its data registers a little after issue -- the
 //     trailing s_nop 1 keeps the next VALU instruction from overwriting them.
-__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, h4 v) {
-  asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2 nt"
-               :
-               : "v"(lane_off), "v"(v), "s"(base)
-               : "memory");
+template <typename V>
+__device__ __forceinline__ void store_base(int through, void* base, unsigned lane_off, V v) {
+  static_assert(sizeof(V) == 8 || sizeof(V) == 16, "8 or 16 bytes");
+  if constexpr (sizeof(V) == 8) {
+    if (through)
+      asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2 sc0 sc1"
+                   : : "v"(lane_off), "v"(v), "s"(base) : "memory");
+    else
+      asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2 nt"
+                   : : "v"(lane_off), "v"(v), "s"(base) : "memory");
+  } else {
+    if (through)
+      asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1"
+                   : : "v"(lane_off), "v"(v), "s"(base) : "memory");
+    else
+      asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
+                   : : "v"(lane_off), "v"(v), "s"(base) : "memory");
+  }
 }
-__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, f4 v) {
-  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
-               :
-               : "v"(lane_off), "v"(v), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void store_nt_base(void* base, unsigned lane_off, h8 v) {
-  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
-               :
-               : "v"(lane_off), "v"(v), "s"(base)
-               : "memory");
+// The same at a pointer of each lane's own.
+template <typename V>
+__device__ __forceinline__ void store_at(int through, V* p, V v) {
+  if (through) store_through(p, v);
+  else __builtin_nontemporal_store(v, p);
 }
 
 // Workgroup barrier that does not drain the vector-memory counter: the

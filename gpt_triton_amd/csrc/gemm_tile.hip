@@ -378,7 +378,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
     const int r = r_first + it * RSTEP, m = m0 + r;
-    if (m >= M) break;
+    if (m >= M || (CHUNKS % NT != 0 && r >= BM)) break;  // the last turn may be one of some threads only
     float z[CW];
 #pragma unroll
     for (int u = 0; u < CW / 4; ++u) {
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     } else {
       dst = (OT*)ep.out + ((int64_t)m * N + n);
     }
-    if (vec) store_through(reinterpret_cast<OV*>(dst), o);
+    if (vec) store_at(ep.through, reinterpret_cast<OV*>(dst), o);
     else {
 #pragma unroll
       for (int e = 0; e < CW; ++e)
@@ -454,12 +454,14 @@ int launch_tile_cfg(const void* A, const void* Bt, int64_t M, int N, int Kp, con
   return 0;
 }
 
-// The menu, with the two numbers of the cost model: a launch of ceil(tiles / CUs) = R rounds takes
-// about launch + R (fixed + k_slices * slice) microseconds.  Fitted to 16 products of the four GPT-2
-// widths at 19 row counts from 8 to 20000 (weights from HBM, activations warm), where the model's
-// choice is 0.5 % slower than the best of the menu on average and 13 % at worst.  What the numbers
-// say: a workgroup takes in 40 to 48 bytes per clock whatever its shape, so a tile costs its
-// operand bytes -- small tiles win while they fill the 256 CUs once, large ones as soon as they do.
+// The menu, with the numbers of the cost model: a launch of ceil(tiles / CUs) = R rounds takes about
+// launch + R (fixed + k_slices * slice) microseconds.  Fitted to the products of a layer of the four GPT-2
+// widths (GELU and residual epilogues, weights from HBM, outputs written through) at 23 row counts from 8 to
+// 20000: 8 % off on average, and the model's choice among these tiles and the persistent kernels is 0.9 %
+// slower than the fastest of 17 shapes.  What the numbers say: a workgroup takes in 36 to 48 bytes per
+// clock whatever its shape (4800 x 3072 x 768: the loads alone take 18 of the 22 us of the k-loop, 14.5 of
+// them if every line is in the L2), so a tile costs its operand bytes -- small tiles win while they
+// fill the 256 CUs once, large ones as soon as they do.
 //                    BM   BN  WM WN WK NST
 typedef Tile< 32,  16, 1, 1, 4, 4> T32x16;
 typedef Tile< 32,  32, 1, 1, 4, 4> T32x32;
@@ -474,12 +476,28 @@ struct TileCost {
   float launch, fixed, slice;
 };
 constexpr TileCost kTiles[] = {
-    {32, 16, 4, 2.18f, 1.36f, 0.057f},  {32, 32, 4, 1.98f, 1.34f, 0.086f},
-    {64, 32, 4, 1.82f, 1.45f, 0.131f},  {64, 64, 2, 1.55f, 1.37f, 0.189f},
-    {64, 128, 2, 0.99f, 2.09f, 0.305f}, {128, 128, 1, 0.f, 3.89f, 0.435f},
-    {192, 128, 1, 0.f, 5.01f, 0.556f},  {128, 256, 1, 0.f, 5.77f, 0.655f},
+    {32, 16, 4, 0.92f, 2.50f, 0.049f},  {32, 32, 4, 1.26f, 1.76f, 0.086f},
+    {64, 32, 4, 1.09f, 2.17f, 0.129f},  {64, 64, 2, 1.00f, 1.65f, 0.180f},
+    {64, 128, 2, 0.85f, 3.23f, 0.283f}, {128, 128, 1, 0.f, 4.21f, 0.476f},
+    {192, 128, 1, 0.f, 5.35f, 0.664f},  {128, 256, 1, 0.f, 6.91f, 0.740f},
 };
-constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+// Shapes between those: for row and column counts that leave the ones above a last round with few tiles
+// (products at 24 to 4800 rows, before -> after: 48 x 1280 x 5120 8.4 -> 7.0 us, 1477 x 768 x 3072 15.7 -> 14.0,
+// 3072 x 768 x 3072 24.1 -> 22.0, 4800 x 1600 x 6400 111 -> 91; 1.6 % over all of them).
+typedef Tile< 16,  16, 1, 1, 4, 4> T16x16;
+typedef Tile< 48,  32, 1, 1, 4, 3> T48x32;
+typedef Tile< 96,  64, 2, 2, 2, 3> T96x64;
+typedef Tile<192,  64, 4, 2, 1, 4> T192x64;
+typedef Tile<256, 128, 4, 2, 1, 3> T256x128;
+constexpr TileCost kTilesBetween[] = {
+    {16, 16, 4, 2.70f, 0.72f, 0.033f},  {48, 32, 4, 1.28f, 1.91f, 0.108f},
+    {96, 64, 2, 1.04f, 2.58f, 0.236f},  {192, 64, 1, 0.28f, 3.52f, 0.403f},
+    {256, 128, 1, 0.f, 6.84f, 0.753f},
+};
+constexpr int kNumFirst = sizeof(kTiles) / sizeof(kTiles[0]);
+constexpr int kNumTiles = kNumFirst + sizeof(kTilesBetween) / sizeof(kTilesBetween[0]);
+
+inline const TileCost& tile_cost(int i) { return i < kNumFirst ? kTiles[i] : kTilesBetween[i - kNumFirst]; }
 
 inline float cost_of(const TileCost& c, int64_t M, int N, int Kp, int cus) {
   const int64_t tiles = ((M + c.bm - 1) / c.bm) * (((int64_t)N + c.bn - 1) / c.bn);
@@ -489,9 +507,9 @@ inline float cost_of(const TileCost& c, int64_t M, int N, int Kp, int cus) {
 
 inline int pick_tile(int64_t M, int N, int Kp, int cus, float* cost) {
   int best = 0;
-  float least = cost_of(kTiles[0], M, N, Kp, cus);
+  float least = cost_of(tile_cost(0), M, N, Kp, cus);
   for (int i = 1; i < kNumTiles; ++i) {
-    const float c = cost_of(kTiles[i], M, N, Kp, cus);
+    const float c = cost_of(tile_cost(i), M, N, Kp, cus);
     if (c < least) least = c, best = i;
   }
   if (cost) *cost = least;
@@ -510,7 +528,12 @@ int launch_pick(int i, const void* A, const void* Bt, int64_t M, int N, int Kp, 
     case 4: return launch_tile_cfg<T64x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
     case 5: return launch_tile_cfg<T128x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
     case 6: return launch_tile_cfg<T192x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    default: return launch_tile_cfg<T128x256, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 7: return launch_tile_cfg<T128x256, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 8: return launch_tile_cfg<T16x16, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 9: return launch_tile_cfg<T48x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 10: return launch_tile_cfg<T96x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 11: return launch_tile_cfg<T192x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    default: return launch_tile_cfg<T256x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
   }
 }
 
@@ -575,7 +598,7 @@ constexpr int kLnStages = 3 * 128 * 128;
 
 // Index of the form that serves these sizes.
 inline int pick_ln(int64_t M, int N, int K, bool split, int cus) {
-  const int wk = split ? kTiles[pick_tile(M, N, K, cus, nullptr)].wk : 1;
+  const int wk = split ? tile_cost(pick_tile(M, N, K, cus, nullptr)).wk : 1;
   if (wk < 4) return wk == 1 ? 3 : 2;
   const int64_t cols = (N + 31) / 32;
   if ((M + 15) / 16 * cols <= cus) return 4;
