@@ -45,6 +45,9 @@ SIGNATURES = {
     "gptmi_mlp_block_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "gptmi_mlp_block": (_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _f32,
                                _u64, _vp, _i64, _int, _int, _vp, _sz, _int, _vp]),
+    "gptmi_blocks_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _int]),
+    "gptmi_blocks": (_int, [_vp, _vp, _vp, _i64, _f32, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _sz,
+                            _int, _vp]),
     "gptmi_dropout_mask_bytes": (_sz, [_i64]),
     "gptmi_dropout_mask": (_int, [_vp, _i64, _f32, _u64, _vp]),
     "gptmi_flash_attn": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _f32, _f32,

@@ -738,4 +738,49 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   return check_launch("mlp_block");
 }
 
+// Two matrices of the residual stream in front of the larger block's workspace.
+size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner, int dtype) {
+  if (B <= 0 || L <= 0 || heads <= 0 || d <= 0 || inner <= 0 || !dtype_ok(dtype)) return 0;
+  const int64_t M = B * L, h = heads * d;
+  const size_t a = plan_attention(nullptr, M, h, GPTMI_W_PACKED).total;
+  const size_t m = plan_mlp(nullptr, M, h, inner, GPTMI_W_PACKED).total;
+  return 2 * (size_t)round_up(M * h * (dtype == GPTMI_F16 ? 2 : 4), 256) + (a > m ? a : m);
+}
+
+int gptmi_blocks(const void* x, const void* normed, const void* const* params, int64_t n, float eps,
+                 void* out, int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner,
+                 int fuse_layernorm, void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+  if (!x || !params || !out || n <= 0 || B <= 0 || L <= 0 || heads <= 0 || d <= 0 || inner <= 0 ||
+      !dtype_ok(dtype)) {
+    set_error("blocks: invalid argument");
+    return GPTMI_ERR_INVALID;
+  }
+  const size_t need = gptmi_blocks_workspace_bytes(B, L, heads, d, inner, dtype);
+  if (workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0) {
+    set_error("blocks: workspace of %zu bytes, 256-byte aligned, needed (%zu given)", need,
+              workspace ? workspace_bytes : (size_t)0);
+    return GPTMI_ERR_WORKSPACE;
+  }
+  const int64_t M = B * L, h = heads * d;
+  Carver c = {(char*)workspace, 0};
+  const size_t mat = (size_t)(M * h * (dtype == GPTMI_F16 ? 2 : 4));
+  void *mid = c.take(mat), *next = c.take(mat);
+  char* ws = (char*)workspace + c.used;
+  const size_t ws_bytes = workspace_bytes - c.used;
+  for (int64_t i = 0; i < n; ++i) {
+    const void* const* p = params + 12 * i;
+    int rc = gptmi_attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B,
+                                   L, heads, d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws,
+                                   ws_bytes, dtype, stream);
+    if (rc) return rc;
+    // x is not read again: the layer's output may take its place
+    void* y = i + 1 == n ? out : next;
+    rc = gptmi_mlp_block(mid, p[6], p[7], eps, p[8], p[9], p[10], p[11], y, M, h, inner, 0.0f, 1337, nullptr, 0,
+                         fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream);
+    if (rc) return rc;
+    x = y;
+  }
+  return GPTMI_OK;
+}
+
 }  // extern "C"

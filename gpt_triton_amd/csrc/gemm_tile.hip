@@ -497,21 +497,26 @@ constexpr TileCost kTilesBetween[] = {
 constexpr int kNumFirst = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kNumTiles = kNumFirst + sizeof(kTilesBetween) / sizeof(kTilesBetween[0]);
 
-inline const TileCost& tile_cost(int i) { return i < kNumFirst ? kTiles[i] : kTilesBetween[i - kNumFirst]; }
+constexpr const TileCost& tile_cost(int i) { return i < kNumFirst ? kTiles[i] : kTilesBetween[i - kNumFirst]; }
 
-inline float cost_of(const TileCost& c, int64_t M, int N, int Kp, int cus) {
-  const int64_t tiles = ((M + c.bm - 1) / c.bm) * (((int64_t)N + c.bn - 1) / c.bn);
-  const int64_t rounds = (tiles + cus - 1) / cus;
-  return c.launch + (float)rounds * (c.fixed + (float)(Kp / 64) * c.slice);
+// Unrolled, with the table's numbers as constants: a forward of few tokens asks four times a layer, and
+// the host sets its pace.
+template <int I>
+inline void pick_from(int64_t M, int N, float k, int cus, int& best, float& least) {
+  if constexpr (I < kNumTiles) {
+    constexpr TileCost c = tile_cost(I);
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + (c.bn - 1)) / c.bn);
+    const int64_t rounds = tiles <= cus ? 1 : (tiles + cus - 1) / cus;
+    const float cost = c.launch + (float)rounds * (c.fixed + k * c.slice);
+    if (cost < least) least = cost, best = I;
+    pick_from<I + 1>(M, N, k, cus, best, least);
+  }
 }
 
 inline int pick_tile(int64_t M, int N, int Kp, int cus, float* cost) {
   int best = 0;
-  float least = cost_of(tile_cost(0), M, N, Kp, cus);
-  for (int i = 1; i < kNumTiles; ++i) {
-    const float c = cost_of(tile_cost(i), M, N, Kp, cus);
-    if (c < least) least = c, best = i;
-  }
+  float least = INFINITY;
+  pick_from<0>(M, N, (float)(Kp / 64), cus, best, least);
   if (cost) *cost = least;
   return best;
 }

@@ -324,6 +324,20 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
                     int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace, size_t workspace_bytes, int dtype,
                     void* stream);
 
+/*
+ * The attention and MLP blocks of n layers one after the other in one call: gptmi_attention_block and
+ * gptmi_mlp_block for each, packed weights, no dropout, with their launches, order and bits.  A forward of
+ * a few hundred tokens is bound by the host otherwise.  Replaces the loop over the blocks, gpt.py:171.
+ *   params: n * 12 device pointers (a host array, read during the call): for each layer ln_w, ln_b, W_qkv,
+ *           b_qkv, W_proj, b_proj of the attention block, then ln_w, ln_b, W1, b1, W2, b2 of the MLP
+ *   x, out [B*L][h]   normed: LayerNorm(x) of the first layer, or NULL
+ *   inner, fuse_layernorm, workspace: as for those two calls, for every layer
+ */
+size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner, int dtype);
+int gptmi_blocks(const void* x, const void* normed, const void* const* params, int64_t n, float eps,
+                 void* out, int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner,
+                 int fuse_layernorm, void* workspace, size_t workspace_bytes, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
