@@ -198,17 +198,26 @@ struct Carver {
   }
 };
 
-// The weight images that a block's two products read: the caller's (packed), or built into ws1 and ws2.
+// The weight images that a block's two products read: the caller's (packed), or built into its workspace.
 // K1 and K2 are multiples of 64.
-struct WeightImages {
-  const void *first, *second;
+struct BlockWeights {
+  const void *W1, *W2;
+  void *ws1, *ws2;
+  int K1, N1, K2, N2;
+  bool packed, f16;
+  const void* first() const { return packed ? W1 : ws1; }
+  const void* second() const { return packed ? W2 : ws2; }
+  void build(hipStream_t st) const {
+    if (!packed) launch_pack_transpose_pair(W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
+  }
+  // together with the block's LayerNorm, to fp16
+  void build_and_normalise(const void* x, const void* ln_w, const void* ln_b, void* normed, int64_t M, int h,
+                           float eps, hipStream_t st) const {
+    if (packed) launch_layernorm(x, ln_w, ln_b, normed, M, h, eps, f16, true, st);
+    else
+      launch_layernorm_pack_pair(x, ln_w, ln_b, normed, M, h, eps, W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
+  }
 };
-static WeightImages weight_images(const void* W1, void* ws1, int64_t K1, int64_t N1, const void* W2,
-                                  void* ws2, int64_t K2, int64_t N2, int wlayout, bool f16, hipStream_t st) {
-  if (wlayout == GPTMI_W_PACKED) return {W1, W2};
-  launch_pack_transpose_pair(W1, ws1, (int)K1, (int)N1, W2, ws2, (int)K2, (int)N2, f16, st);
-  return {ws1, ws2};
-}
 static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
   return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
 }
@@ -628,7 +637,9 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const auto [Bq, Bp] = weight_images(W_qkv, pl.w_qkv, h, 3 * h, W_proj, pl.w_proj, h, h, wlayout, f16, st);
+  const BlockWeights bw = {W_qkv, W_proj, pl.w_qkv, pl.w_proj, (int)h, (int)(3 * h), (int)h, (int)h,
+                           wlayout == GPTMI_W_PACKED, f16};
+  const void *Bq = bw.first(), *Bp = bw.second();
   if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
     set_error("attention_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
@@ -654,12 +665,17 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     prologue = prologue_aligned(x, ln_w, ln_b);
   }
   if (prologue) {
+    bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
   } else {
     const void* A = pl.normed;
-    if (!normed) launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)h, eps, f16, true, st);
-    else if (f16 && ((uintptr_t)normed & 15) == 0) A = normed;
-    else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, f16, st);
+    if (!normed) {
+      bw.build_and_normalise(x, ln_w, ln_b, pl.normed, M, (int)h, eps, st);
+    } else {
+      bw.build(st);
+      if (f16 && ((uintptr_t)normed & 15) == 0) A = normed;
+      else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, f16, st);
+    }
     rc = launch_gemm(A, Bq, M, (int)(3 * h), (int)h, ep, st);
   }
   if (rc) return rc;
@@ -698,7 +714,9 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const auto [B1, B2] = weight_images(W1, pl.w1, H, inner, W2, pl.w2, inner, H, wlayout, f16, st);
+  const BlockWeights bw = {W1, W2, pl.w1, pl.w2, (int)H, (int)inner, (int)inner, (int)H,
+                           wlayout == GPTMI_W_PACKED, f16};
+  const void *B1 = bw.first(), *B2 = bw.second();
   if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
     set_error("mlp_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
@@ -721,9 +739,10 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
     prologue = prologue_aligned(x, ln_w, ln_b);
   }
   if (prologue) {
+    bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
   } else {
-    launch_layernorm(x, ln_w, ln_b, pl.normed, M, (int)H, eps, f16, true, st);
+    bw.build_and_normalise(x, ln_w, ln_b, pl.normed, M, (int)H, eps, st);
     rc = launch_gemm(pl.normed, B1, M, (int)inner, (int)H, e1, st);
   }
   if (rc) return rc;

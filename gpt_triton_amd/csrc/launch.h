@@ -34,6 +34,12 @@ void launch_pack_transpose(const void* src, void* dst, int K, int N, int Kp, boo
 void launch_pack_transpose_pair(const void* s1, void* d1, int K1, int N1, const void* s2, void* d2, int K2,
                                 int N2, bool f16, hipStream_t st);
 
+// launch_layernorm to fp16 and launch_pack_transpose_pair, which do not depend on each other, in one launch
+// where their sizes and alignments allow it.
+void launch_layernorm_pack_pair(const void* x, const void* w, const void* b, void* out, int64_t M, int H,
+                                float eps, const void* s1, void* d1, int K1, int N1, const void* s2, void* d2,
+                                int K2, int N2, bool f16, hipStream_t st);
+
 // Epilogue description of one GEMM launch: out = gelu?(acc + bias) + residual,
 // stored either as a plain [M][N] matrix or scattered into q/k/v [B][heads][L][d].
 struct GemmEpilogue {
