@@ -68,6 +68,29 @@ __device__ __forceinline__ void bias_to_f32_16(const P4 (&raw)[NB][2], f4 (&bias
       for (int e = 0; e < 4; ++e) bias_r[i][nh][e] = (float)raw[i][nh][e];
 }
 
+// The dropout mask of a wavefront's 128 x 64 sub-tile: a lane takes the word of row 32 j + lane / 2 and the
+// 32 columns from 32 (lane % 2) on.  N and nw0 are multiples of 64, so the words are aligned.
+template <int MB>
+__device__ __forceinline__ void load_keep(const EpiDev& ep, int64_t mw0, int nw0, int N, int lane,
+                                          unsigned (&w)[MB]) {
+#pragma unroll
+  for (int j = 0; j < MB; ++j) {
+    const uint64_t at = (uint64_t)(mw0 + 32 * j + (lane >> 1)) * (uint64_t)N + (uint64_t)(nw0 + 32 * (lane & 1));
+    w[j] = *reinterpret_cast<const unsigned*>(ep.keep + (at >> 3));
+  }
+}
+// v where its bit of the low 8 of `bits` is set, +0 elsewhere
+__device__ __forceinline__ h8 keep_halves(unsigned bits, h8 v) {
+  u4 d = __builtin_bit_cast(u4, v);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_sbfe((int)bits, 2 * e, 1);
+    const unsigned hi = (unsigned)__builtin_amdgcn_sbfe((int)bits, 2 * e + 1, 1);
+    d[e] &= (lo & 0xffffu) | (hi & 0xffff0000u);
+  }
+  return __builtin_bit_cast(h8, d);
+}
+
 // fp16 output without residual, whole tile, vector accesses allowed (and head size % 8 == 0 for
 // the head-major scatter): bias (+GELU) and the rounding to fp16 happen in the accumulator
 // layout, the transposition through the wavefront's slab moves halves (32 rows x 64 columns x
@@ -78,10 +101,17 @@ __device__ __forceinline__ void bias_to_f32_16(const P4 (&raw)[NB][2], f4 (&bias
 // (NB / 2) * MB * 4 stores per lane.  acc[2 NB][2 MB]: of the 32 x 32 block (i, j) a lane holds the
 // quads (mh, nh) = acc[2 i + nh][2 j + mh]: row 16 mh + lane % 16, columns 16 nh + 4 (lane / 16) +
 // 0..3, bias_r[i][nh] (see load_bias16).
-template <int MB, int NB, bool QKV, bool GELU>
+//
+// DROP: dropout behind the GELU, its mask at hand (ep.keep).  The division by 1 - p happens in fp32 in
+// the accumulator layout; what is dropped is cleared in the halves on their way out, 8 columns = one byte
+// of the mask.  keep_w[j]: the mask word of row 32 j + lane / 2, columns 32 (lane % 2).. (load_keep),
+// which a lane takes from the lane that has it.  ffn1 of a training forward of 4800 rows x 768 on this
+// kernel instead of 456 tiles of 128 x 256 with the mask (40.5 us a launch): the forward 1724 -> 1542 us.
+template <int MB, int NB, bool QKV, bool GELU, bool DROP>
 __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
                                                   const f4 (&bias_r)[NB][2], const EpiDev& ep, int64_t mw0, int nw0, int N,
-                                                  char* slab, int lane) {
+                                                  char* slab, int lane, const unsigned (&keep_w)[DROP ? MB : 1]) {
+  static_assert(!DROP || NB == 2, "a mask word of 32 of the 64 columns per lane");
   static_assert(NB % 2 == 0, "wave tile must be a multiple of 64 columns");
   // key (row >> 1) & 7: the 32 rows x 2 lanes of one 8-byte write then cover 16 distinct
   // 16-byte slots of the 256-byte bank window twice -- the minimum for 512 bytes
@@ -103,6 +133,7 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
     l0 = m_first - b0 * Lu;
   }
   const int64_t batch_stride = (int64_t)ep.heads * ep.L * ep.d;
+  const KeepScale scale(DROP ? ep.drop.p : 0.f);
   const unsigned lane_byte_off = ((unsigned)rrow * (unsigned)N + runit * 8) * 2u;
 #pragma unroll
   for (int j = 0; j < MB; ++j) {
@@ -111,19 +142,24 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
 #pragma unroll
       for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
+        for (int mh = 0; mh < 2; ++mh) {
           const int i = i2 * 2 + ii;
-          const int mh = g >> 1, nh = g & 1;
-          h4 o;
+          float z[8];  // both quads of the row
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float z = acc[2 * i + nh][2 * j + mh][e] + bias_r[i][nh][e];
-            if (GELU) z = gelu_new(z);
-            o[e] = (_Float16)z;
+          for (int e = 0; e < 8; ++e) {
+            z[e] = acc[2 * i + e / 4][2 * j + mh][e % 4] + bias_r[i][e / 4][e % 4];
+            if (GELU) z[e] = gelu_new(z[e]);
           }
-          const int row = 16 * mh + frow;
-          const int grp = 2 * nh + (lq >> 1);  // 8-column group of the quad
-          *reinterpret_cast<h4*>(slab + row * 128 + (((ii * 4 + grp) ^ fkey) << 4) + fhalf * 8) = o;
+          if constexpr (DROP) scale.apply(z);
+#pragma unroll
+          for (int nh = 0; nh < 2; ++nh) {
+            h4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (_Float16)z[4 * nh + e];
+            const int row = 16 * mh + frow;
+            const int grp = 2 * nh + (lq >> 1);  // 8-column group of the quad
+            *reinterpret_cast<h4*>(slab + row * 128 + (((ii * 4 + grp) ^ fkey) << 4) + fhalf * 8) = o;
+          }
         }
       // all four reads first: the stores are assembly with a memory clobber, which no LDS
       // read may cross, so reading inside the store loop would expose one LDS latency per store
@@ -134,7 +170,12 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
                                               ((runit ^ rkey ^ ((rr & 1) * 4)) << 4));
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const h8 v = vv[rr];
+        h8 v = vv[rr];
+        if constexpr (DROP) {
+          const unsigned word =
+              __builtin_amdgcn_ds_bpermute((2 * (rr * 8 + rrow) + (runit >> 2)) * 4, (int)keep_w[j]);
+          v = keep_halves(word >> ((runit & 3) * 8), v);
+        }
         if constexpr (QKV) {
           unsigned b, l;
           if (step_rows) {
@@ -321,13 +362,14 @@ __device__ __forceinline__ void store_wave_tile32(f4 (&acc)[2 * NB][2 * MB], con
   }
 }
 
-// T: type of the bias.  OT: type of the output (fp16, or T).
-template <int WM, int WN, typename T, typename OT, bool QKV>
+// T: type of the bias.  OT: type of the output (fp16, or T).  DROP: fp16 output, plain, the mask at hand.
+template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP>
 __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const _Float16* __restrict__ A, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep) {
   constexpr int BM = 256, BN = 256, ROWB = 128, T_ = 512, KS = 4;
   static_assert(WM * WN == 8, "8 wavefronts");
+  static_assert(!DROP || (!QKV && sizeof(OT) == 2), "dropout with a plain fp16 output");
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int MB = TM / 32, NB = TN / 32;
   constexpr int A_IT = 4, B_IT = 4, LPT = A_IT + B_IT;  // 16-byte loads per thread per k-tile
@@ -545,17 +587,26 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     // stage is free for a refill then); the bias is requested in front of the k-tile and waited
     // for BEFORE the next tile's second k-tile is requested, so that no wait inside the epilogue
     // falls behind those loads.  The next tile's first fragments are read after the epilogue.
-    // fp16: requested a whole k-tile before it is needed; fp32 (twice the registers): in front
-    // of the last slice
+    // fp16: requested a whole k-tile before it is needed; fp32 (twice the registers) and with the words
+    // of a dropout mask: in front of the last slice
     typename Pack4<T>::type bias_raw[NB][2];
-    if constexpr (sizeof(T) == 2) {
+    constexpr bool EARLY_BIAS = sizeof(T) == 2 && !DROP;
+    if constexpr (EARLY_BIAS) {
       if (wave_stores) load_bias16<T, NB>(ep, nw0, lq, bias_raw);
     }
     __builtin_amdgcn_sched_barrier(0);
     first_slices(with_b_half);
     if (has_next) publish_next(false);
-    if constexpr (sizeof(T) == 4) {
-      if (wave_stores) load_bias16<T, NB>(ep, nw0, lq, bias_raw);
+    unsigned keep_w[DROP ? MB : 1] = {};
+    if constexpr (!EARLY_BIAS) {
+      if (wave_stores) {
+        load_bias16<T, NB>(ep, nw0, lq, bias_raw);
+        if constexpr (DROP) {
+          int lane_k = lane;  // as lane_e below
+          asm volatile("" : "+v"(lane_k));
+          load_keep(ep, mw0, nw0, N, lane_k, keep_w);
+        }
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     slice(1, false, 0, 0, nothing);
@@ -565,6 +616,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int g = 0; g < 2; ++g) asm volatile("" : "+v"(bias_r[i][g]));
+    if constexpr (DROP) {
+#pragma unroll
+      for (int j = 0; j < MB; ++j) asm volatile("" : "+v"(keep_w[j]));
+    }
     if (has_next) issue(stage, m0_n, n0_n, 1);
     stage ^= 1;
 
@@ -577,8 +632,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
       int lane_e = lane;
       asm volatile("" : "+v"(lane_e));
       if constexpr (HALF_SLABS) {
-        if (ep.gelu) store_wave_tile_h<MB, NB, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
-        else store_wave_tile_h<MB, NB, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
+        if (ep.gelu)
+          store_wave_tile_h<MB, NB, QKV, true, DROP>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e, keep_w);
+        else
+          store_wave_tile_h<MB, NB, QKV, false, DROP>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e, keep_w);
       } else {
         if (ep.gelu) store_wave_tile32<MB, NB, OT, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
         else store_wave_tile32<MB, NB, OT, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
@@ -902,10 +959,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
   }
 }
 
-template <int WM, int WN, typename T, typename OT, bool QKV>
+template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP = false>
 int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                   hipStream_t st) {
-  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV>;
+  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV, DROP>;
   constexpr int smem = 2 * 512 * 128 + 8 * 4096;  // 160 KB: two stages + the epilogue slabs
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -979,14 +1036,17 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // 4096 35.2, 43.6; a second launch for the rows beyond a multiple costs 6 us and more).  Not with an output
 // over its own residual, which the second pass would read changed: whole row tiles and a launch behind them.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
-// edge store nothing), two k-tiles (three with a residual), vector epilogues, no dropout.
+// edge store nothing), two k-tiles (three with a residual), vector epilogues, and dropout only with its
+// mask at hand, an fp16 output and no residual.
 // Sets *head to the number of rows for the persistent kernel.
 template <typename T, typename OT, bool QKV>
 int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const bool res = !QKV && ep.residual != nullptr;
+  const bool drop = ep.drop.p > 0.f;
+  const bool drop_ok = !QKV && !res && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0;
   const bool persistent =
       M >= 256 && N >= 256 && N % 64 == 0 && Kp >= (res ? 192 : 128) && Kp <= (1 << 21) && ep.vec_ok &&
-      (sizeof(OT) == 4 || ep.vec8_ok) && !(ep.drop.p > 0.f) &&
+      (sizeof(OT) == 4 || ep.vec8_ok) && (!drop || drop_ok) &&
       (!res || (sizeof(T) == 2 && (((uintptr_t)ep.residual) & 15) == 0));
   *head = 0;
   if (!persistent) return 0;
@@ -995,7 +1055,8 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const int64_t tiles_n = (N + 255) / 256;
   const int64_t all = res && overlap(ep.out, ep.residual, M, N, sizeof(OT)) ? M / 256 * 256 : M;
   const int64_t tiles = (all + 255) / 256 * tiles_n;
-  const int64_t whole = tiles / cus * cus / tiles_n * 256;  // rows of the row tiles that fill whole rounds
+  // rows of the row tiles that fill whole rounds (with dropout all or none: the mask counts from row 0)
+  const int64_t whole = drop ? all : tiles / cus * cus / tiles_n * 256;
   // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
   // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
   // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
@@ -1031,6 +1092,9 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
   if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head)) return rc;
   if (m_head > 0) {
     int rc;
+    if constexpr (sizeof(OT) == 2 && !QKV) {
+      if (ep.drop.p > 0.f) return launch_stream<2, 4, T, OT, QKV, true>(A, Bt, M, N, Kp, ep, st);
+    }
     if constexpr (sizeof(T) == 2 && !QKV)
       rc = res ? launch_stream_res(A, Bt, m_head, N, Kp, ep, st)
                : launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);

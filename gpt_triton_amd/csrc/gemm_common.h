@@ -24,8 +24,8 @@ struct EpiDev {
   int vec8_ok; // fp16 output: N, head size and the output pointers also allow 16-byte stores
   int through; // outputs written through (store_through), not non-temporal: make_epi
   int m_off;   // head-major scatter: row 0 of this launch is row m_off of the [B*L] token rows
-  DropoutArgs drop;  // p > 0: dropout between GELU and residual (gemm_tile_kernel only)
-  const unsigned char* keep;  // its mask by flat index, or nullptr: generated in the epilogue
+  DropoutArgs drop;  // p > 0: dropout between GELU and residual
+  const unsigned char* keep;  // its mask by flat index, or nullptr: generated in the epilogue (gemm_tile_kernel)
 };
 
 // LayerNorm in the operand prologue (gemm_tile_kernel<..., LNA = true>): weight, bias, epsilon and
