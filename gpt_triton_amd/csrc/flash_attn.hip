@@ -400,8 +400,8 @@ __global__ __launch_bounds__(256, (D == 64 && DROP != 1) ? 2 : 1) void flash_att
 }
 
 // ---------------------------------------------------------------------------
-// Resident-K/V variant for short sequences (L*D small enough that K and V^T of
-// one (batch, head) fit in half a CU's LDS, e.g. L <= 320 at D = 64).
+// Resident-K/V variant for short sequences (L*D small enough that K and V^T of one (batch, head) fit in
+// half a CU's LDS, e.g. L <= 312 at D = 64): fp32 storage, and head sizes 128 and 256.
 //
 // One workgroup = 8 wavefronts (4 for head sizes above 64, which need more than 128
 // registers) = one (batch, head).  K ([L][D], 16-byte chunks
@@ -994,7 +994,8 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Ring variant for sequences too long for the streaming kernel: fp16 storage, head size 64,
+// Ring variant for sequences too long for the streaming kernel, and for few pairs of one tile: fp16
+// storage, head size 64,
 // equal query and key lengths, no dropout.  One workgroup = 4 wavefronts = one (batch, head) x
 // 128 queries, as in the tiled kernel, but the 64-key tiles of K and V travel the way the
 // streaming kernel moves them: by direct global->LDS loads (no staging registers, no LDS store
@@ -1666,6 +1667,21 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
   return 0;
 }
 
+// fp16 q, k, v of equal lengths at head size 64, no dropout.  Up to 320 rows two (batch, head) pairs fit
+// the LDS: the streaming kernel.  Longer ones take their key tiles through the ring, and so does a single
+// tile of up to 512 pairs, where nothing is left to overlap and the ring's workgroup, with half the
+// wavefronts, is through sooner.  Microseconds, streaming / ring (the resident kernel): 12 x 24 rows
+// 3.6 / 3.1 (3.7), 24 x 64 3.9 / 3.5 (4.0), 192 x 64 4.2 / 3.7 (4.3), 768 x 64 7.9 / 8.0 (9.3), 12 x 128
+// 4.7 / 4.6 (5.0), 12 x 211 5.9 / 6.2 (6.9), 36 x 300 8.0 / 7.8 (9.6), 192 x 300 11.4 / 12.8 (13.1), 1536 x
+// 300 55 / 76 (66).
+template <bool BLND, bool ACC = false>
+int launch_d64(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
+               float scale, hipStream_t st) {
+  if (L <= 320 && !(L <= BKEY && BN <= 512))
+    return launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
+  return launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
+}
+
 template <int D, typename T>
 int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
              int heads, int L, int Lk, float scale, Dropout drop, bool blnd, hipStream_t st) {
@@ -1678,29 +1694,22 @@ int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
     return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
                 : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
   if constexpr (D == 64 && sizeof(T) == 2) {
-    // fp16, head size 64, two (batch, head) pairs fit the LDS, enough pairs to keep every
-    // persistent workgroup busy for a while: the streaming kernel
-    if (L <= 320 && BN >= 64)
-      return blnd ? launch_stream_attn<true>(q, k, v, out, BN, heads, L, scale, st)
-                  : launch_stream_attn<false>(q, k, v, out, BN, heads, L, scale, st);
-    // sequences that do not fit the resident variant either: key tiles through the ring
-    if (resident_lds_bytes(L, D) == 0)
-      return blnd ? launch_ring_attn<true>(q, k, v, out, BN, heads, L, scale, st)
-                  : launch_ring_attn<false>(q, k, v, out, BN, heads, L, scale, st);
+    return blnd ? launch_d64<true>(q, k, v, out, BN, heads, L, scale, st)
+                : launch_d64<false>(q, k, v, out, BN, heads, L, scale, st);
+  } else {
+    if (const size_t lds = resident_lds_bytes(L, D))
+      return blnd ? launch_resident<D, T, true>(q, k, v, out, BN, heads, L, scale, lds, st)
+                  : launch_resident<D, T, false>(q, k, v, out, BN, heads, L, scale, lds, st);
+    if constexpr (D >= 128 && sizeof(T) == 2) {
+      // fp16, head sizes 128 and 256, longer sequences: tiles by direct loads, no staging registers
+      // (pairs in the grid's second dimension; 32-bit byte offsets inside a pair)
+      if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
+        return blnd ? launch_wide_attn<D, true>(q, k, v, out, BN, heads, L, scale, st)
+                    : launch_wide_attn<D, false>(q, k, v, out, BN, heads, L, scale, st);
+    }
+    return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
+                : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
   }
-  if (const size_t lds = resident_lds_bytes(L, D)) {
-    return blnd ? launch_resident<D, T, true>(q, k, v, out, BN, heads, L, scale, lds, st)
-                : launch_resident<D, T, false>(q, k, v, out, BN, heads, L, scale, lds, st);
-  }
-  if constexpr (D >= 128 && sizeof(T) == 2) {
-    // fp16, head sizes 128 and 256, longer sequences: tiles by direct loads, no staging registers
-    // (pairs in the grid's second dimension; 32-bit byte offsets inside a pair)
-    if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
-      return blnd ? launch_wide_attn<D, true>(q, k, v, out, BN, heads, L, scale, st)
-                  : launch_wide_attn<D, false>(q, k, v, out, BN, heads, L, scale, st);
-  }
-  return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
-              : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
 }
 
 // Head sizes 16 and 32: the tiled kernel on its 64-wide staging layout, reading the tensors at
@@ -1764,17 +1773,14 @@ int launch_operands_d(const void* q, const void* k, const void* v, void* out, in
   if (da.p > 0.f)
     return launch_tiled_as<D, T, true, 1, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
   if constexpr (D == 64) {
-    if (L <= 320 && BN >= 64) return launch_stream_attn<true, true>(q, k, v, out, BN, heads, L, scale, st);
-    if (resident_lds_bytes(L, D) == 0)
-      return launch_ring_attn<true, true>(q, k, v, out, BN, heads, L, scale, st);
-  }
-  if (const size_t lds = resident_lds_bytes(L, D))
-    return launch_resident<D, T, true, true>(q, k, v, out, BN, heads, L, scale, lds, st);
-  if constexpr (D >= 128) {
+    return launch_d64<true, true>(q, k, v, out, BN, heads, L, scale, st);
+  } else {
+    if (const size_t lds = resident_lds_bytes(L, D))
+      return launch_resident<D, T, true, true>(q, k, v, out, BN, heads, L, scale, lds, st);
     if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
       return launch_wide_attn<D, true, true>(q, k, v, out, BN, heads, L, scale, st);
+    return launch_tiled_as<D, T, true, 0, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
   }
-  return launch_tiled_as<D, T, true, 0, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
 }
 
 template <int DG>
