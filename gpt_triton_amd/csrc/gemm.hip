@@ -213,17 +213,22 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
 // is free again (the kernel refills it there).  Younger than the first half's loads when band 0
 // starts: the second half's 8 loads.  Younger than the second half's loads when band 2 starts: the
 // 8 stores of bands 0 and 1 and, if `refilled`, the 8 operand loads `mid` issued.
-template <int MB, int NB, bool GELU, typename Mid>
+// DROP: as in store_wave_tile_h, but cleared in the accumulator layout, in front of the residual.  Training
+// forwards of 16800 rows x 768, projection and ffn2 on this kernel instead of one workgroup per tile: 4660 ->
+// 4330 us.
+template <int MB, int NB, bool GELU, bool DROP, typename Mid>
 __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], const f4 (&bias_r)[NB][2],
                                                    const EpiDev& ep, int64_t mw0, int nw0, int N,
                                                    const char* res_lo, const char* res_hi,
-                                                   char* slab, int lane, bool refilled, Mid&& mid) {
+                                                   char* slab, int lane, bool refilled, Mid&& mid,
+                                                   const unsigned (&keep_w)[DROP ? MB : 1]) {
   static_assert(MB == 4 && NB == 2, "128 x 64 sub-tile");
   // accumulators of v_mfma_f32_16x16x32: quad (mh, nh) of the 32 x 32 block (i, j), see
   // store_wave_tile_h<L16>
   const int frow = lane & 15, lq = lane >> 4, fhalf = lq & 1, fkey = (frow >> 1) & 7;
   const int rrow = lane >> 3, runit = lane & 7, rkey = rrow >> 1;
   const unsigned lane_byte_off = ((unsigned)rrow * (unsigned)N + runit * 8) * 2u;
+  const KeepScale scale(DROP ? ep.drop.p : 0.f);
 #pragma unroll
   for (int j = 0; j < MB; ++j) {
     if (j == 0) wait_vmcnt<8>();
@@ -245,17 +250,28 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int mh = g >> 1, nh = g & 1;
-        h4 o;
+      for (int mh = 0; mh < 2; ++mh) {
+        float z[8];  // both quads of the row
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float z = acc[2 * i + nh][2 * j + mh][e] + bias_r[i][nh][e];
-          if (GELU) z = gelu_new(z);
-          o[e] = (_Float16)(z + (float)r[i][g][e]);
+        for (int e = 0; e < 8; ++e) {
+          z[e] = acc[2 * i + e / 4][2 * j + mh][e % 4] + bias_r[i][e / 4][e % 4];
+          if (GELU) z[e] = gelu_new(z[e]);
         }
-        *reinterpret_cast<h4*>(slab + (16 * mh + frow) * 128 +
-                               (((i * 4 + 2 * nh + (lq >> 1)) ^ fkey) << 4) + fhalf * 8) = o;
+        if constexpr (DROP) {
+          const unsigned word =
+              (unsigned)__builtin_amdgcn_ds_bpermute((2 * (16 * mh + frow) + i) * 4, (int)keep_w[j]) >> (4 * lq);
+          scale.apply(z);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) z[e] = keep_if(word, 16 * (e / 4) + e % 4, z[e]);
+        }
+#pragma unroll
+        for (int nh = 0; nh < 2; ++nh) {
+          h4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (_Float16)(z[4 * nh + e] + (float)r[i][2 * mh + nh][e]);
+          *reinterpret_cast<h4*>(slab + (16 * mh + frow) * 128 +
+                                 (((i * 4 + 2 * nh + (lq >> 1)) ^ fkey) << 4) + fhalf * 8) = o;
+        }
       }
     h8 vv[4];
 #pragma unroll
@@ -674,7 +690,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 // the stores of the one that ended drain.  The launcher sends row tiles that
 // do not fill a round of the persistent workgroups to gemm_tile.hip.
 // ---------------------------------------------------------------------------
-template <int WM, int WN>
+template <int WM, int WN, bool DROP>
 __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
     const _Float16* __restrict__ A, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep) {
@@ -907,6 +923,12 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
     h4 bias_raw[NB][2];
     // all 4 loads in flight under the last slice
     if (wave_stores) load_bias16<_Float16, NB>(ep, nw0, lq, bias_raw);
+    unsigned keep_w[DROP ? MB : 1] = {};
+    if constexpr (DROP) {
+      int lane_k = lane;  // addresses made here, not kept through the tile loop
+      asm volatile("" : "+v"(lane_k));
+      if (wave_stores) load_keep(ep, mw0, nw0, N, lane_k, keep_w);
+    }
     __builtin_amdgcn_sched_barrier(0);
     slice(1, false, 0, 0, nothing);
     f4 bias_r[NB][2];
@@ -915,6 +937,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int g = 0; g < 2; ++g) asm volatile("" : "+v"(bias_r[i][g]));
+    if constexpr (DROP) {
+#pragma unroll
+      for (int j = 0; j < MB; ++j) asm volatile("" : "+v"(keep_w[j]));
+    }
     barrier_lds();  // every wavefront has read the last k-tile's fragments
     if (wave_stores) {
       const char* res1 = res_src(m0, n0, 1);
@@ -935,11 +961,11 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
         }
       };
       if (ep.gelu)
-        store_wave_tile_rs<MB, NB, true>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
-                                         has_next, mid);
+        store_wave_tile_rs<MB, NB, true, DROP>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
+                                               has_next, mid, keep_w);
       else
-        store_wave_tile_rs<MB, NB, false>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
-                                          has_next, mid);
+        store_wave_tile_rs<MB, NB, false, DROP>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
+                                                has_next, mid, keep_w);
     } else if (has_next) {
       barrier_lds();  // the barrier and the refill of `mid`
       issue(stage, m0_n, n0_n, 0);
@@ -985,9 +1011,10 @@ int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const
   return 0;
 }
 
+template <bool DROP>
 int launch_stream_res(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                       hipStream_t st) {
-  auto kern = gemm_stream_res_kernel<2, 4>;
+  auto kern = gemm_stream_res_kernel<2, 4, DROP>;
   constexpr int smem = 2 * 512 * 128 + 8 * 4096;  // 160 KB: two stages + the epilogue slabs
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -1037,13 +1064,13 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // over its own residual, which the second pass would read changed: whole row tiles and a launch behind them.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, and dropout only with its
-// mask at hand, an fp16 output and no residual.
+// mask at hand and an fp16 output.
 // Sets *head to the number of rows for the persistent kernel.
 template <typename T, typename OT, bool QKV>
 int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool drop = ep.drop.p > 0.f;
-  const bool drop_ok = !QKV && !res && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0;
+  const bool drop_ok = !QKV && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0;
   const bool persistent =
       M >= 256 && N >= 256 && N % 64 == 0 && Kp >= (res ? 192 : 128) && Kp <= (1 << 21) && ep.vec_ok &&
       (sizeof(OT) == 4 || ep.vec8_ok) && (!drop || drop_ok) &&
@@ -1054,8 +1081,9 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   if (cus < 0) return cus;
   const int64_t tiles_n = (N + 255) / 256;
   const int64_t all = res && overlap(ep.out, ep.residual, M, N, sizeof(OT)) ? M / 256 * 256 : M;
+  if (drop && all != M) return 0;  // all or none: the mask counts from row 0
   const int64_t tiles = (all + 255) / 256 * tiles_n;
-  // rows of the row tiles that fill whole rounds (with dropout all or none: the mask counts from row 0)
+  // rows of the row tiles that fill whole rounds
   const int64_t whole = drop ? all : tiles / cus * cus / tiles_n * 256;
   // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
   // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
@@ -1093,10 +1121,14 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
   if (m_head > 0) {
     int rc;
     if constexpr (sizeof(OT) == 2 && !QKV) {
-      if (ep.drop.p > 0.f) return launch_stream<2, 4, T, OT, QKV, true>(A, Bt, M, N, Kp, ep, st);
+      if (ep.drop.p > 0.f) {  // m_head == M
+        if constexpr (sizeof(T) == 2)
+          if (res) return launch_stream_res<true>(A, Bt, M, N, Kp, ep, st);
+        return launch_stream<2, 4, T, OT, QKV, true>(A, Bt, M, N, Kp, ep, st);
+      }
     }
     if constexpr (sizeof(T) == 2 && !QKV)
-      rc = res ? launch_stream_res(A, Bt, m_head, N, Kp, ep, st)
+      rc = res ? launch_stream_res<false>(A, Bt, m_head, N, Kp, ep, st)
                : launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
     else
       rc = launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
