@@ -74,7 +74,7 @@ def _keep_mask(x, width, layers, heads, p):
     masks of all layers from one seed at offsets that count from 0, so they are all parts of the mask
     of the widest matrix ([tokens, 4 * width]; attention weights: the first L * L offsets).  Drawn
     once per forward instead of in every kernel that applies it: 16 x 300 tokens 124M, each of 12 ffn1
-    launches 85 -> 44 us, projections and ffn2 32 -> 23, attentions 72 -> 21, for one launch of 24."""
+    launches 85 -> 31 us, projections and ffn2 32 -> 22, attentions 72 -> 18, for one launch of 25."""
     tokens, seqlen = x.numel() // width, x.shape[1]
     bits = max(tokens * 4 * width, seqlen * seqlen)
     if (layers == 0 or bits > 1 << 32 or not block_supported(x, width) or width % heads != 0 or
@@ -500,7 +500,7 @@ def convert_hf_and_load_model(model_id, device):
 class GraphedForward:
     """The forward of an eval-mode FusedGPT for one input shape, captured once into a HIP graph
     and replayed per call: the 63 launches of a forward become one graph launch and their host work
-    goes (2 x 64 tokens, 124M: 0.50 -> 0.42 ms).  Nothing in the library allocates or
+    goes (2 x 64 tokens, 124M, a pass that is waited for: 0.54 -> 0.40 ms).  Nothing in the library allocates or
     synchronises, so capture needs no special path; the operators' output tensors
     come from the graph's private pool.  The result of a call is overwritten by the next call --
     clone it to keep it.  No counterpart in the reference (Triton launches kernel by kernel)."""
