@@ -16,10 +16,12 @@ Differences, all additive: GPU_TO_FLOPS knows "mi355x"; FusedGPT.forward takes
 dataclass does not have, gpt.py:165, and so only works in eval mode).
 """
 import re
+import weakref
 from dataclasses import dataclass
 
 import torch
 import torch.nn as nn
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_supported, blocks_forward, dropout_mask,
                       flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
@@ -101,11 +103,17 @@ def _call_with_mask(module, x, keep):
     return module(x)
 
 
+_storage_expired = torch.UntypedStorage._expired  # of a StorageWeakRef's cdata
+
+
 class _PackedWeights:
-    """Per-module cache of the GEMM's packed weight images, used in eval mode only.  An entry
-    is rebuilt when the parameter's storage, dtype or version counter changes (optimizer steps,
-    load_state_dict, .to()); in-place edits made through `param.data` bypass the version
-    counter -- call `clear()` (or `model.train()`) after those."""
+    """Per-module cache of the GEMM's packed weight images, used in eval mode only.  An entry is that of one
+    Parameter object while it has the storage, address, dtype, shape and version counter that it was
+    packed with (optimizer steps, load_state_dict, .to() and assignments change one of them), and is
+    rebuilt otherwise.  Parameter and storage are referred to weakly: nothing is kept alive by its image,
+    and an address that was freed and handed out again is not taken for the weight that lay there before.
+    In-place edits made through `param.data` bypass the version counter -- call `clear()` (or
+    `model.train()`) after those.  Copies and pickles of a module start without images."""
 
     def __init__(self):
         self._entries = {}
@@ -114,19 +122,31 @@ class _PackedWeights:
         hit = self.held(name, param)
         if hit is None:
             hit = pack(param.data)
-            self._entries[name] = (param.data_ptr(), param._version, param.dtype, param.shape, hit)
+            self._entries[name] = (weakref.ref(param), StorageWeakRef(param.untyped_storage()),
+                                   param.data_ptr(), param._version, param.dtype, param.shape, hit)
         return hit
 
     def held(self, name, param):
         """The image of this parameter as it is now, or None where there is none yet."""
-        hit = self._entries.get(name)
-        if (hit is None or hit[0] != param.data_ptr() or hit[1] != param._version or
-                hit[2] != param.dtype or hit[3] != param.shape):
+        entry = self._entries.get(name)
+        if entry is None:
             return None
-        return hit[4]
+        owner, storage, address, version, dtype, shape, hit = entry
+        # an address inside a storage that is still there is that storage's: no other has it
+        if (owner() is not param or param._version != version or param.data_ptr() != address or
+                param.dtype != dtype or param.shape != shape or not param.is_contiguous() or
+                _storage_expired(storage.cdata)):
+            return None
+        return hit
 
     def clear(self):
         self._entries.clear()
+
+    def __reduce__(self):
+        return _PackedWeights, ()
+
+    def __setstate__(self, state):  # of a pickle that holds entries
+        self._entries = {}
 
 
 def _linear_flops(tokens, fan_in, fan_out):
@@ -323,8 +343,7 @@ def _stack(blocks, x):
 
     def image(module, name, shape):
         t = module._parameters[name]
-        if (type(t) is not nn.Parameter or t.dtype != dtype or t.shape != shape or t.get_device() != index or
-                not t.is_contiguous()):
+        if type(t) is not nn.Parameter or t.dtype != dtype or t.shape != shape or t.get_device() != index:
             return False
         packed = module._packed.held(name, t)
         if type(packed) is not PackedWeight or packed.dtype != dtype:
