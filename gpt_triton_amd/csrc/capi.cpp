@@ -757,6 +757,38 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   return check_launch("mlp_block");
 }
 
+// What the calls of the layers would refuse one by one, with the layers in front of them launched.
+static int check_blocks(const void* const* params, int64_t n, int64_t B, int64_t L, int64_t heads, int64_t h,
+                        int64_t inner, int fuse_layernorm, int dtype) {
+  if (inner % 64 != 0 || inner > kMaxN) {
+    set_error("blocks: inner width %lld is not a multiple of 64 up to %d", (long long)inner, kMaxN);
+    return GPTMI_ERR_INVALID;
+  }
+  for (int64_t i = 0; i < n; ++i) {
+    const void* const* p = params + 12 * i;
+    for (const int j : {0, 1, 2, 4, 6, 7, 8, 10})
+      if (p[j] == nullptr) {
+        set_error("blocks: pointer %d of layer %lld is NULL", j, (long long)i);
+        return GPTMI_ERR_INVALID;
+      }
+    if (((uintptr_t)p[2] | (uintptr_t)p[4] | (uintptr_t)p[8] | (uintptr_t)p[10]) & 15) {
+      set_error("blocks: the weights of layer %lld must be 16-byte aligned", (long long)i);
+      return GPTMI_ERR_INVALID;
+    }
+  }
+  if (fuse_layernorm && (dtype != GPTMI_F16 || !gemm_layernorm_supported(B * L, (int)h))) {
+    set_error("blocks: the LayerNorm prologue takes fp16 storage and the row widths of "
+              "gptmi_layernorm_linear_supported");
+    return GPTMI_ERR_UNSUPPORTED;
+  }
+  if (B * heads > 0x7fffffffll || L > (1 << 24) || B * L >= (1ll << 31) - 512) {
+    set_error("blocks: B*heads=%lld, L=%lld or B*L=%lld beyond the grid limits", (long long)(B * heads),
+              (long long)L, (long long)(B * L));
+    return GPTMI_ERR_UNSUPPORTED;
+  }
+  return GPTMI_OK;
+}
+
 // Two matrices of the residual stream in front of the larger block's workspace.
 size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner, int dtype) {
   if (B <= 0 || L <= 0 || heads <= 0 || d <= 0 || inner <= 0 || !dtype_ok(dtype)) return 0;
@@ -781,6 +813,7 @@ int gptmi_blocks(const void* x, const void* normed, const void* const* params, i
     return GPTMI_ERR_WORKSPACE;
   }
   const int64_t M = B * L, h = heads * d;
+  if (const int rc = check_blocks(params, n, B, L, heads, h, inner, fuse_layernorm, dtype)) return rc;
   Carver c = {(char*)workspace, 0};
   const size_t mat = (size_t)(M * h * (dtype == GPTMI_F16 ? 2 : 4));
   void *mid = c.take(mat), *next = c.take(mat);

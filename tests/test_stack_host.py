@@ -60,3 +60,35 @@ def test_a_replaced_function_runs(name, monkeypatch):
     model, x = build()
     monkeypatch.setattr(gpt, name, lambda *a, **k: None)
     assert not taken(model, x)
+
+
+def refusals():
+    """(what, changed arguments, changed pointers of the last layer, status)"""
+    yield "inner", {"inner": 100}, {}, -1
+    yield "inner", {"inner": 1 << 27}, {}, -1
+    for i in (0, 1, 2, 4, 6, 7, 8, 10):
+        yield f"pointer {i}", {}, {i: None}, -1
+    for i in (2, 4, 8, 10):
+        yield f"image {i}", {}, {i: 256 + 8}, -1
+    yield "LayerNorm in the product in fp32", {"dtype": 0, "fuse": 1}, {}, -2
+    yield "LayerNorm in the product, behind rows normalised already", {"dtype": 0, "fuse": 1, "normed": 256}, {}, -2
+    yield "rows beyond the attention's", {"L": (1 << 24) + 1}, {}, -2
+    yield "pairs beyond the grid", {"B": 1 << 31, "L": 1, "heads": 1}, {}, -2
+
+
+@pytest.mark.parametrize("what,args,pointers,status", refusals())
+@pytest.mark.parametrize("layers", [1, 3])
+def test_blocks_refuse_before_any_launch(what, args, pointers, status, layers):
+    import ctypes
+
+    from gpt_triton_amd import _lib
+    lib = _lib.load()
+    a = {"normed": None, "B": 1, "L": 8, "heads": 2, "inner": 512, "fuse": 0, "dtype": 1, **args}
+    table = [256] * 12 * layers
+    for i, p in pointers.items():
+        table[12 * (layers - 1) + i] = p
+    need = lib.gptmi_blocks_workspace_bytes(a["B"], a["L"], a["heads"], 64, a["inner"], a["dtype"])
+    fake = ctypes.c_void_p(256)
+    rc = lib.gptmi_blocks(fake, a["normed"], (ctypes.c_void_p * len(table))(*table), layers, 1e-5, fake, a["B"],
+                          a["L"], a["heads"], 64, a["inner"], a["fuse"], fake, need, a["dtype"], None)
+    assert rc == status and lib.gptmi_last_error().startswith(b"blocks:")
