@@ -289,6 +289,16 @@ static int check_block(const char* what, int64_t M, int64_t h, float p, const vo
   return GPTMI_OK;
 }
 
+// The limits of the product's row index and of the attention's grid.
+static int check_grid(const char* what, int64_t B, int64_t L, int64_t heads) {
+  if (B * heads > 0x7fffffffll || L > (1 << 24) || B * L >= (1ll << 31) - 512) {
+    set_error("%s: B*heads=%lld, L=%lld or B*L=%lld beyond the grid limits", what, (long long)(B * heads),
+              (long long)L, (long long)(B * L));
+    return GPTMI_ERR_UNSUPPORTED;
+  }
+  return GPTMI_OK;
+}
+
 // The LayerNorm prologue reads rows and parameters in 16-byte units; the block functions run the
 // LayerNorm kernel in front of the product where one of them lies otherwise.
 static bool prologue_aligned(const void* x, const void* ln_w, const void* ln_b) {
@@ -634,6 +644,7 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   const AttentionPlan pl = plan_attention(workspace, M, h, wlayout);
   int rc = check_block("attention_block", M, h, p, keep, keep_bits, M * h > L * L ? M * h : L * L, wlayout,
                        dtype, workspace, workspace_bytes, pl.total);
+  if (!rc) rc = check_grid("attention_block", B, L, heads);
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
@@ -781,12 +792,7 @@ static int check_blocks(const void* const* params, int64_t n, int64_t B, int64_t
               "gptmi_layernorm_linear_supported");
     return GPTMI_ERR_UNSUPPORTED;
   }
-  if (B * heads > 0x7fffffffll || L > (1 << 24) || B * L >= (1ll << 31) - 512) {
-    set_error("blocks: B*heads=%lld, L=%lld or B*L=%lld beyond the grid limits", (long long)(B * heads),
-              (long long)L, (long long)(B * L));
-    return GPTMI_ERR_UNSUPPORTED;
-  }
-  return GPTMI_OK;
+  return check_grid("blocks", B, L, heads);
 }
 
 // Two matrices of the residual stream in front of the larger block's workspace.

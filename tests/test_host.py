@@ -292,3 +292,12 @@ def test_the_tile_gemm_cases_reach_every_tile():
         assert groups[i] == 4 and {s % 4 == 0 for j, s in picked if j == i} == {True, False}
     sizes = [(M, N) for M in (1, 8, 24, 64, 128, 200, 513, 1477, 4800) for N in (16, 40, 768, 2304, 6400)]
     assert all(groups[pick(M, N, slices)] < 4 for M, N in sizes for slices in (1, 2, 3))
+
+
+@pytest.mark.parametrize("B,L,heads", [(1, (1 << 24) + 1, 1), (1 << 31, 1, 1)])
+def test_attention_block_checks_the_grid_before_any_launch(lib, B, L, heads):
+    fake = ctypes.c_void_p(256)
+    need = lib.gptmi_attention_block_workspace_bytes(B, L, heads, 64, 2)
+    rc = lib.gptmi_attention_block(fake, None, fake, fake, 1e-5, fake, fake, fake, fake, fake, B, L, heads, 64,
+                                   0.0, 1337, None, 0, 0, 2, fake, need, 1, None)
+    assert rc == -2 and lib.gptmi_last_error().startswith(b"attention_block:")
