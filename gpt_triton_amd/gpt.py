@@ -23,7 +23,8 @@ import torch
 import torch.nn as nn
 from torch.multiprocessing.reductions import StorageWeakRef
 
-from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_supported, blocks_forward, dropout_mask,
+from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, block_supported, blocks_forward,
+                      dropout_mask,
                       flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
                       fused_layer_norm, layer_norm_ffn, layer_norm_linear_supported,
                       layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, mlp_block,
@@ -313,74 +314,130 @@ def _parts():
 
 
 _OWN = _parts()
-_METHODS = frozenset(("forward", "_weights", "_call_impl", "_wrapped_call_impl"))
 _GLOBAL_HOOKS = tuple(getattr(nn.modules.module, name) for name in (
     "_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
     "_global_backward_pre_hooks"))
 
 
 def _untouched(module, kind):
-    return (type(module) is kind and not module.training and module.__dict__.keys().isdisjoint(_METHODS) and
-            not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
-                 module._backward_pre_hooks) and module._compiled_call_impl is None)
+    own = module.__dict__
+    return (type(module) is kind and not own["training"] and "forward" not in own and "_weights" not in own and
+            "_call_impl" not in own and "_wrapped_call_impl" not in own and
+            not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
+                 own["_backward_pre_hooks"]) and module._compiled_call_impl is None)
 
 
-def _stack(blocks, x):
-    """(device addresses for `blocks_forward`, heads, inner width, LayerNorm in the GEMM, what must outlive
-    the call) where all the blocks of an eval-mode forward can go to the library in one call; None where a
-    module, an operator or a parameter is not what this file makes it, or a size is not the block calls',
-    and on a first forward, which builds the weight images between its launches: the modules are called
-    one by one then.  All of it is asked on every forward, 95 us of host
-    work for 12 layers, where the modules and 24 calls take 240: 2 x 64 tokens 498 -> 343 us."""
-    if _parts() != _OWN or any(_GLOBAL_HOOKS) or torch._C._get_tracing_state() is not None:
-        return None
-    h, dtype, index = x.shape[-1], x.dtype, x.get_device()
-    if not _as_block(x) or not block_supported(x, h):
-        return None
-    heads = inner = None
-    pointers, keep = [], []
+class _Layers:
+    """What the layers that go to the library together have in common: the sizes, type and device of the
+    first one, under x.  `pointers` gives a block's 12 device addresses for `block_layers`, or None where a
+    module or a parameter is not what this file makes it, or has another size: the modules are called one
+    by one from that block on.  Weight images that are not held (a first forward, a weight edited in
+    place) are built there as the modules build them."""
 
-    def vector(t, n):
-        if (type(t) is not nn.Parameter or t.dtype != dtype or t.shape != (n,) or t.get_device() != index or
-                not t.is_contiguous()):
-            return False
-        pointers.append(t.data_ptr())
-        return True
+    def __init__(self, block, x):
+        attention, mlp = block
+        h = x.shape[-1]
+        self.h, self.heads, self.inner = h, attention.num_heads, mlp.ffn1_weight.shape[-1]
+        self.dtype, self.index = x.dtype, x.get_device()
+        self.alive = []  # the images, until they are launched
+        self.built = 0  # blocks whose images were built
+        row, wide, inner = torch.Size((h,)), torch.Size((3 * h,)), torch.Size((self.inner,))
+        self.vectors = ((("layer_norm_weight", row), ("layer_norm_bias", row), ("c_attn_bias", wide),
+                         ("c_proj_bias", row)),
+                        (("layer_norm_weight", row), ("layer_norm_bias", row), ("ffn1_bias", inner),
+                         ("ffn2_bias", row)))
+        self.weights = ((("c_attn_weight", (h, 3 * h)), ("c_proj_weight", (h, h))),
+                        (("ffn1_weight", (h, self.inner)), ("ffn2_weight", (self.inner, h))))
 
-    def image(module, name, shape):
-        t = module._parameters[name]
-        if type(t) is not nn.Parameter or t.dtype != dtype or t.shape != shape or t.get_device() != index:
-            return False
-        packed = module._packed.held(name, t)
-        if type(packed) is not PackedWeight or packed.dtype != dtype:
-            return False
-        keep.append(packed)
-        pointers.append(packed.data_ptr())
-        return True
-
-    for block in blocks:
+    def pointers(self, block):
         if not _untouched(block, _Block) or len(block._modules) != 2:
             return None
         attention, mlp = block._modules.values()
-        if not _untouched(attention, FusedAttention) or not _untouched(mlp, FusedMLP):
+        if (not _untouched(attention, FusedAttention) or not _untouched(mlp, FusedMLP) or
+                attention.num_heads != self.heads or attention.hidden_size != self.h):
             return None
-        a, m = attention._parameters, mlp._parameters
-        if not (FusedAttention._NAMES <= a.keys() and FusedMLP._NAMES <= m.keys()):
-            return None
-        w1 = m["ffn1_weight"]
-        if heads is None:
-            heads, inner = attention.num_heads, w1.shape[-1]
-            if h % heads != 0 or h // heads not in HEAD_SIZES or inner % 64 != 0:
+        first = self._half(attention._parameters, attention._packed, 0)
+        second = first and self._half(mlp._parameters, mlp._packed, 1)
+        return second and first + second
+
+    def _half(self, own, packed, which):
+        dtype, index, kind, found = self.dtype, self.index, nn.Parameter, []
+        for name, shape in self.vectors[which]:
+            t = own.get(name)
+            if (type(t) is not kind or t.dtype is not dtype or t.get_device() != index or t.shape != shape or
+                    not t.is_contiguous()):
                 return None
-        if not (attention.num_heads == heads and attention.hidden_size == h and
-                vector(a["layer_norm_weight"], h) and vector(a["layer_norm_bias"], h) and
-                image(attention, "c_attn_weight", (h, 3 * h)) and vector(a["c_attn_bias"], 3 * h) and
-                image(attention, "c_proj_weight", (h, h)) and vector(a["c_proj_bias"], h) and
-                vector(m["layer_norm_weight"], h) and vector(m["layer_norm_bias"], h) and
-                image(mlp, "ffn1_weight", (h, inner)) and vector(m["ffn1_bias"], inner) and
-                image(mlp, "ffn2_weight", (inner, h)) and vector(m["ffn2_bias"], h)):
-            return None
-    return pointers, heads, inner, _ln_in_gemm(x, keep[0]), keep
+            found.append(t.data_ptr())
+        images = []
+        for name, shape in self.weights[which]:
+            t = own.get(name)
+            if type(t) is not kind or t.get_device() != index:
+                return None
+            image = packed.held(name, t)  # of these values, in this type and shape
+            if image is None:
+                if t.dtype is not dtype or t.shape != shape or not t.is_contiguous():
+                    return None
+            elif type(image) is not PackedWeight or image.dtype is not dtype or image.shape != shape:
+                return None
+            images.append(image)
+        if None in images:  # both weights are fit to be packed: what the module would do now
+            self.built += 1
+            images = [image or packed.get(name, own[name]) for image, (name, _) in
+                      zip(images, self.weights[which])]
+        self.alive += images
+        norm_w, norm_b, first, second = found
+        return [norm_w, norm_b, images[0].data.data_ptr(), first, images[1].data.data_ptr(), second]
+
+
+def _stack(blocks, x):
+    """(the `_Layers` of an eval-mode forward, the first block's addresses) where its blocks, or the first
+    of them, can go to the library together; None where the first block or an operator is not what this
+    file makes it, or a size is not the block calls'."""
+    h = x.shape[-1]
+    if (_parts() != _OWN or any(_GLOBAL_HOOKS) or torch._C._get_tracing_state() is not None or not _as_block(x) or
+            not _untouched(blocks[0], _Block) or len(blocks[0]._modules) != 2):
+        return None
+    attention, mlp = blocks[0]
+    if type(attention) is not FusedAttention or type(mlp) is not FusedMLP:
+        return None
+    heads, inner = attention.num_heads, mlp._parameters.get("ffn1_weight")
+    if (h % heads != 0 or h // heads not in HEAD_SIZES or inner is None or inner.dim() != 2 or
+            inner.shape[1] % 64 != 0):
+        return None
+    layers = _Layers(blocks[0], x)
+    first = layers.pointers(blocks[0])
+    return None if first is None else (layers, first)
+
+
+def _through(stack, blocks, x, normed):
+    """(x behind the blocks that went to the library together, the blocks that are left).  Every block is
+    looked over on every forward, 8 to 10 us of host work each, so they go in calls of 1, 2, 4, ... layers: the
+    GPU works on those launched while the next are looked over.  Microseconds of a forward that is waited for /
+    of one among others, modules called one by one, all blocks looked over before one call, and this: 1 x 24
+    tokens 124M 571 / 499, 438 / 315, 395 / 330; 2 x 64 570 / 500, 516 / 344, 428 / 339; 7 x 211 721 / 665, 864 /
+    687, 723 / 666; 2 x 300 tokens of the 48-layer model 4230 / 4183, 4824 / 4279, 4242 / 4188.  A weight of the
+    last layer edited in place before each forward of 2 x 64: 560, 680, 425."""
+    layers, found = stack
+    in_gemm = _ln_in_gemm(x, layers.alive[0])
+    sent, seen, size = 0, 1, 1
+    while True:
+        more, built = found, layers.built
+        while more is not None and seen < min(sent + size, len(blocks)):
+            more = layers.pointers(blocks[seen])
+            if more is not None:
+                found += more
+                seen += 1
+        if seen == len(blocks) and not layers.built:
+            return blocks_forward(x, found, layers.heads, layers.inner, normed=normed,
+                                  layer_norm_in_gemm=in_gemm), []
+        if found:
+            # in place behind the first call, whose x is the caller's
+            x = block_layers(x, found, layers.heads, layers.inner, normed=normed, layer_norm_in_gemm=in_gemm,
+                             out=x if sent else None)
+        if more is None or seen == len(blocks):
+            return x, blocks[seen:]
+        # packing two weights takes the host as long as a layer takes the GPU
+        normed, sent, size, found = None, seen, 1 if layers.built > built else 2 * size, []
 
 
 @dataclass
@@ -440,9 +497,7 @@ class FusedGPT(nn.Module):
                                                first[0].layer_norm_bias.data)
             stack = _stack(blocks, x)
             if stack is not None:
-                pointers, heads, inner, in_gemm, _alive = stack
-                x = blocks_forward(x, pointers, heads, inner, normed=y, layer_norm_in_gemm=in_gemm)
-                rest = []
+                x, rest = _through(stack, blocks, x, y)
             else:
                 x = first[1](first[0](x, normed=y))
                 rest = blocks[1:]

@@ -20,46 +20,119 @@ def build(layers=3):
     return model, torch.zeros(1, 4, 128)
 
 
-def taken(model, x):
-    return gpt._stack(list(model.blocks), x) is not None
+@pytest.fixture
+def through(monkeypatch):
+    """(layers of each call of the library, layers left to the modules) of a forward of these blocks."""
+    def run(model, x):
+        calls = []
+
+        def call(x, pointers, heads, inner, normed=None, layer_norm_in_gemm=False, out=None):
+            assert (heads, inner, layer_norm_in_gemm) == (2, 512, False) and (normed is None) == bool(calls)
+            calls.append(pointers)
+            return x
+
+        monkeypatch.setattr(gpt, "block_layers", call)
+        monkeypatch.setattr(gpt, "blocks_forward", call)
+        blocks = list(model.blocks)
+        stack = gpt._stack(blocks, x)
+        rest = blocks if stack is None else gpt._through(stack, blocks, x, x)[1]
+        assert rest == blocks[len(blocks) - len(rest):]
+        assert sum(calls, []) == addresses(blocks[:len(blocks) - len(rest)])
+        return [len(c) // 12 for c in calls], len(rest)
+    return run
 
 
-def test_untouched_blocks_are_taken():
-    model, x = build()
-    pointers, heads, inner, in_gemm, _ = gpt._stack(list(model.blocks), x)
-    assert len(pointers) == 36 and (heads, inner, in_gemm) == (2, 512, False)
-    mlp = model.blocks[2][1]
-    assert pointers[-6:] == [mlp.layer_norm_weight.data_ptr(), mlp.layer_norm_bias.data_ptr(),
-                             mlp._packed.held("ffn1_weight", mlp.ffn1_weight).data_ptr(), mlp.ffn1_bias.data_ptr(),
-                             mlp._packed.held("ffn2_weight", mlp.ffn2_weight).data_ptr(), mlp.ffn2_bias.data_ptr()]
+def addresses(blocks):
+    found = []
+    for attention, mlp in blocks:
+        for module, names in ((attention, ("layer_norm_weight", "layer_norm_bias", "c_attn_weight", "c_attn_bias",
+                                           "c_proj_weight", "c_proj_bias")),
+                              (mlp, ("layer_norm_weight", "layer_norm_bias", "ffn1_weight", "ffn1_bias",
+                                     "ffn2_weight", "ffn2_bias"))):
+            for name in names:
+                t = module._parameters[name]
+                found.append((t if t.dim() == 1 else module._packed.held(name, t)).data_ptr())
+    return found
+
+
+@pytest.mark.parametrize("layers,calls", [(1, [1]), (2, [1, 1]), (3, [1, 2]), (4, [1, 2, 1]), (12, [1, 2, 4, 5])])
+def test_untouched_blocks_are_taken(layers, calls, through):
+    assert through(*build(layers)) == (calls, 0)
 
 
 @pytest.mark.parametrize("name", ["__call__", "_call_impl"])
 @pytest.mark.parametrize("kind", ["_Block", "FusedAttention", "FusedMLP"])
-def test_a_call_of_the_class_runs(kind, name, monkeypatch):
+def test_a_call_of_the_class_runs(kind, name, through, monkeypatch):
     model, x = build()
-    monkeypatch.setattr(getattr(gpt, kind), name, lambda self, *a, **k: None, raising=False)
-    assert not taken(model, x)
-    monkeypatch.undo()
-    assert taken(model, x)
+    with monkeypatch.context() as m:
+        m.setattr(getattr(gpt, kind), name, lambda self, *a, **k: None, raising=False)
+        assert through(model, x) == ([], 3)
+    assert through(model, x) == ([1, 2], 0)
 
 
 @pytest.mark.parametrize("name", ["forward", "_weights", "_call_impl", "_wrapped_call_impl"])
 @pytest.mark.parametrize("which", [0, 1])
-def test_what_an_instance_has_in_the_place_of_a_method_runs(name, which):
+def test_what_an_instance_has_in_the_place_of_a_method_runs(name, which, through):
     model, x = build()
-    module = model.blocks[1][which]
-    setattr(module, name, lambda *a, **k: None)
-    assert not taken(model, x)
-    delattr(module, name)
-    assert taken(model, x)
+    for block, want in ((0, ([], 3)), (1, ([1], 2)), (2, ([1, 1], 1))):
+        module = model.blocks[block][which]
+        setattr(module, name, lambda *a, **k: None)
+        assert through(model, x) == want
+        delattr(module, name)
+    assert through(model, x) == ([1, 2], 0)
 
 
 @pytest.mark.parametrize("name", ["attention_block", "mlp_block", "layer_norm_ffn", "_weights", "_tensors"])
-def test_a_replaced_function_runs(name, monkeypatch):
+def test_a_replaced_function_runs(name, through, monkeypatch):
     model, x = build()
     monkeypatch.setattr(gpt, name, lambda *a, **k: None)
-    assert not taken(model, x)
+    assert through(model, x) == ([], 3)
+
+
+def test_the_layers_in_front_of_another_one_are_taken(through):
+    changes = [lambda block: setattr(block[1].ffn2_weight, "data", torch.zeros(1024, 64)), lambda block: block[0].train(),
+               lambda block: block.append(torch.nn.Identity()), lambda block: block.__setattr__("extra", block[0]),
+               lambda block: block[0].register_forward_hook(lambda *a: None),
+               lambda block: block[1].register_forward_pre_hook(lambda *a: None),
+               lambda block: block.register_forward_hook(lambda *a: None),
+               lambda block: setattr(block[0], "hidden_size", 64),
+               lambda block: setattr(block[0].c_attn_bias, "data", block[0].c_attn_bias.data.half()),
+               lambda block: setattr(block[0].c_attn_bias, "data", torch.zeros(768)[::2]),
+               lambda block: setattr(block[1].layer_norm_bias, "data", torch.zeros(1, 128)),
+               lambda block: block[1]._parameters.pop("ffn1_bias"),
+               lambda block: block[1]._parameters.__setitem__("ffn1_bias", torch.zeros(512)),
+               lambda block: block[0]._parameters.__setitem__("c_proj_weight", torch.zeros(128, 128)),
+               lambda block: block[0]._packed._entries.clear() or block[0]._parameters.pop("c_proj_weight"),
+               lambda block: setattr(block[0].c_attn_weight, "data", torch.zeros(384, 128).t())]
+    with torch.no_grad():
+        for change in changes:
+            for block, want in ((0, ([], 5)), (1, ([1], 4)), (2, ([1, 1], 3)), (4, ([1, 2, 1], 1))):
+                model, x = build(5)
+                change(model.blocks[block])
+                if change is changes[0]:
+                    model.blocks[block][1]._packed.get("ffn2_weight", model.blocks[block][1].ffn2_weight, pack)
+                calls, left = through(model, x)
+                assert (calls, left) == want, (changes.index(change), block)
+
+
+@pytest.mark.parametrize("edit", [lambda block: block[0].c_proj_weight.add_(1), lambda block: block[1]._packed.clear(),
+                                  lambda block: setattr(block[1], "ffn2_weight", torch.nn.Parameter(torch.zeros(512, 128)))])
+def test_images_that_are_not_held_are_built(edit, through, monkeypatch):
+    packed = []
+    monkeypatch.setattr(gpt._PackedWeights.get, "__defaults__", (lambda w: packed.append(w) or pack(w),))
+    with torch.no_grad():
+        for block, calls in ((0, [1, 2, 2]), (1, [1, 2, 1, 1]), (4, [1, 2, 2])):
+            model, x = build(5)
+            edit(model.blocks[block])
+            packed.clear()
+            assert through(model, x) == (calls, 0) and 1 <= len(packed) <= 2
+            packed.clear()
+            assert through(model, x) == ([1, 2, 2], 0) and not packed
+    # none built for a module whose other weight cannot be packed
+    model, x = build(2)
+    model.blocks[1][0].train().eval()
+    model.blocks[1][0]._parameters["c_proj_weight"] = torch.zeros(128, 128)
+    assert through(model, x) == ([1], 1) and not packed
 
 
 def refusals():
