@@ -88,7 +88,7 @@ def test_what_a_program_changed_still_runs(G, gpu_device, monkeypatch):
         del model.blocks[1][2]
         # weights edited in place, and others in the place of the parameters
         model.blocks[0][0].c_proj_weight.mul_(1.5)
-        edited = model(ids)  # through the modules: a weight image has to be built again
+        edited = model(ids)  # not whole from images at hand: one has to be built again
         assert not calls and not torch.equal(edited, plain)
         assert torch.equal(model(ids), edited) and calls.pop() == 1
         assert torch.equal(edited, one_by_one(G, model, ids, monkeypatch))
