@@ -1744,6 +1744,24 @@ int launch_t(const void* q, const void* k, const void* v, void* out, int64_t BN,
   }
 }
 
+// Head size 64 with the mask's bits at hand: whether the streaming kernel (8 wavefronts and one workgroup a
+// pair, at most one a CU) or the tiled one (4 wavefronts for each 128 rows of a pair) is through sooner.  Blocks
+// of 12 heads in fp16, microseconds, tiled / streaming; in fp32, the fp16 operands' sums in fp32, alike:
+//   one round of pairs: 60 x 64 rows 23.9 / 23.7, 96 x 128 30.3 / 29.0, 96 x 256 37.3 / 36.3, 192 x 300 59.2 / 56.2;
+//     beyond 288 rows the last of 10 chunks sets the pace, and while the tiled kernel's three workgroups a pair
+//     find CUs of their own it wins: 12 x 300 30.9 / 32.1, 96 x 300 39.8 / 41.7, 120 x 320 44.9 / 46.9, 132 x 320
+//     49.0 / 48.1; at 257 to 288 rows the two are equal (96 x 257 38.4 / 38.5);
+//   a second round that leaves most CUs without a pair: 264 x 300 74.5 / 77.3, 336 x 320 91.8 / 94.2, 384 x 300 101.4 /
+//     97.7; up to 256 rows the streaming kernel's halved work a pair outweighs it (264 x 160 50.0 / 46.4);
+//   up to 128 rows, one workgroup a pair in both, more rounds are the tiled kernel's: 264 x 32 27.1 / 28.4, 504 x
+//     128 54.8 / 55.2 (fp32 576 x 128 71.9 / 74.1), 1536 x 64 80.2 / 80.8; three chunks, which leave one of its four
+//     wavefronts idle, excepted beyond two rounds (288 x 96 36.0 / 36.3, 672 x 96 58.5 / 56.0).
+inline bool masked_streams(int64_t BN, int L, int cus) {
+  if (L > 320) return false;
+  if (L > 288) return BN > cus + cus / 3 || (BN > cus / 2 && BN <= cus);
+  return L > 128 || BN <= cus || (L > 64 && L <= 96 && BN > 2 * cus);
+}
+
 // Dropout with the mask's bits at hand: fp16 q, k, v of equal lengths, merged-heads output.
 template <bool ACC>
 int launch_masked(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
@@ -1752,10 +1770,13 @@ int launch_masked(const void* q, const void* k, const void* v, void* out, int64_
   switch (d) {
     case 16: return launch_tiled_as<64, T, true, 2, true, 16, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
     case 32: return launch_tiled_as<64, T, true, 2, true, 32, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
-    case 64:
-      if (L <= 320 && BN <= 0x7fffffff)
+    case 64: {
+      const int cus = attn_cu_count();
+      if (cus < 0) return cus;
+      if (masked_streams(BN, L, cus))
         return launch_stream_attn<true, ACC, true>(q, k, v, out, BN, heads, L, scale, st, da.p, keep);
       return launch_tiled_as<64, T, true, 2, false, 64, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
+    }
     case 128: return launch_tiled_as<128, T, true, 2, false, 128, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
     case 256: return launch_tiled_as<256, T, true, 2, false, 256, ACC>(q, k, v, out, BN, heads, L, L, scale, da, st, keep);
     default:

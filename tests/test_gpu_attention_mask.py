@@ -1,6 +1,7 @@
-"""Attention dropout with the mask's bits at hand in the streaming kernel (head size 64, up to 320 rows),
-against the tiled kernel that draws them: the same sums in the same order, so equal bits.  More (batch, head)
-pairs than CUs, so that workgroups go on to a second pair; chunk counts from one to ten, mask rows that start
+"""Attention dropout with the mask's bits at hand in the streaming kernel and, where that has the pairs and rows
+for it, in the tiled one (head size 64, up to 320 rows; masked_streams in flash_attn.hip), against the tiled
+kernel that draws them: the same sums in the same order, so equal bits.  Fewer and more (batch, head) pairs
+than the 256 CUs, so that workgroups go on to a second pair; chunk counts from one to ten, mask rows that start
 at every bit of a word."""
 import pytest
 import torch
@@ -16,7 +17,12 @@ def K(gpu_device):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("B,L", [(1, 1), (1, 320), (90, 17), (90, 32), (90, 33), (90, 64), (90, 127), (90, 211),
-                                 (90, 257), (90, 319), (180, 320)])
+                                 (90, 257), (90, 319), (180, 320),
+                                 # streaming, one round of pairs: one to four chunks, nine and ten
+                                 (30, 17), (30, 32), (85, 33), (30, 64), (85, 127), (30, 288), (43, 289), (85, 320),
+                                 # streaming, more rounds: three chunks, five, ten; the tiled kernel beside them
+                                 (171, 65), (171, 96), (170, 96), (171, 97), (90, 129), (90, 288), (114, 319),
+                                 (113, 319), (42, 320)])
 def test_bits(K, gpu_device, B, L, dtype):
     heads, h, p = 3, 192, 0.1
     print(f"attention block with a dropout mask: B={B} L={L} {dtype}", flush=True)
