@@ -1670,16 +1670,19 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
 // fp16 q, k, v of equal lengths at head size 64, no dropout.  Up to 320 rows two (batch, head) pairs fit
 // the LDS: the streaming kernel.  Longer ones take their key tiles through the ring, and so does a single
 // tile of up to 512 pairs, where nothing is left to overlap and the ring's workgroup, with half the
-// wavefronts, is through sooner.  Microseconds, streaming / ring (the resident kernel): 12 x 24 rows
-// 3.6 / 3.1 (3.7), 24 x 64 3.9 / 3.5 (4.0), 192 x 64 4.2 / 3.7 (4.3), 768 x 64 7.9 / 8.0 (9.3), 12 x 128
-// 4.7 / 4.6 (5.0), 12 x 211 5.9 / 6.2 (6.9), 36 x 300 8.0 / 7.8 (9.6), 192 x 300 11.4 / 12.8 (13.1), 1536 x
-// 300 55 / 76 (66).
+// wavefronts, is through sooner, and more than 288 rows (the last of ten chunks sets the streaming kernel's
+// pace) while the ring's three workgroups a pair find CUs of their own.  Microseconds, streaming / ring (the
+// resident kernel): 12 x 24 rows 3.6 / 3.1 (3.7), 24 x 64 3.9 / 3.5 (4.0), 192 x 64 4.2 / 3.7 (4.3), 768 x 64
+// 7.9 / 8.0 (9.3), 12 x 128 4.7 / 4.6 (5.0), 12 x 211 5.9 / 6.2 (6.9), 24 x 288 7.4 / 7.4, 12 x 300 8.1 / 7.7 (9.6),
+// 60 x 320 8.5 / 8.1, 96 x 320 8.6 / 8.7, 192 x 300 11.4 / 12.8 (13.1), 1536 x 300 55 / 76 (66).
 template <bool BLND, bool ACC = false>
 int launch_d64(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
                float scale, hipStream_t st) {
-  if (L <= 320 && !(L <= BKEY && BN <= 512))
-    return launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
-  return launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
+  const int cus = attn_cu_count();
+  if (cus < 0) return cus;
+  const bool ring = L > 320 || (L > 288 && 3 * BN <= cus) || (L <= BKEY && BN <= 512);
+  return ring ? launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st)
+              : launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
 }
 
 template <int D, typename T>
