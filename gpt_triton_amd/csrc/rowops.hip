@@ -386,7 +386,9 @@ __global__ __launch_bounds__(256) void pack_rows_vec_kernel(const T* __restrict_
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = (_Float16)(float)v[j];
       }
-      store_through(reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8), o);
+      // not written through: one store a thread and turn, with nothing behind it to hide the longer way
+      // (2048 x 1280 floats and the product with 1280 columns 20.2 us, 24.7; 4800 x 1280 alone 13.3, 16.6)
+      *reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8) = o;
     }
 }
 
