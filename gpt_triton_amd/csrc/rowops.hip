@@ -1,6 +1,8 @@
 // Bandwidth-bound row kernels: embedding gather, LayerNorm, row softmax and the
 // operand packers of the GEMM.  One wavefront owns one row; a row is held in
 // registers between its passes so HBM sees one read and one write per element.
+#include <type_traits>
+
 #include "common.h"
 #include "layernorm.h"
 #include "launch.h"
@@ -17,6 +19,35 @@ template <> struct Vec<float> {
   typedef f4 type;
 };
 
+// The row kernels write through (store_through): a line is on its way while the kernel still runs.  All stores
+// of a thread come behind all its loads and arithmetic, kept there by `pin`, with one wait in front of them
+// (`loads_done`): a wait for a load between two stores, which the compiler puts in front of every value that a
+// branch may have left in flight, would be a wait for the first store's way to memory.  LayerNorm, us, plain
+// stores / through with such waits / through without: halves 128 x 768 3.3 / 3.4 / 2.9, 128 x 1600 3.8 / 4.0 / 3.2,
+// 4800 x 768 4.7 / 4.2 / 3.8, 4800 x 1600 8.2 / 7.0 / 6.2; captured forwards of 1 x 24 tokens, 1600-wide, 48 layers,
+// 1820 / 1890 / 1770.
+// What an embedding writes beyond half of the memory-side cache is non-temporal, as make_epi does it: a GEMM's
+// epilogue reads it a block later (through / non-temporal: 65536 x 1024 halves 39 / 39, 65536 x 1600 79 / 61,
+// 153600 x 768 75 / 67; with the LayerNorm, whose output counts too, 65536 x 768 51 / 44, 65536 x 1024 86 / 58).  A
+// LayerNorm's output is the next kernel's operand and stays at any size (all non-temporal, the forward of 512 x
+// 300 tokens takes 29.49 ms, 28.42).
+constexpr int64_t kStreamBytes = 128 << 20;
+
+template <typename V>
+__device__ __forceinline__ void pin(V& v) {
+  typedef std::conditional_t<sizeof(V) == 16, u4, u2> U;
+  U u = __builtin_bit_cast(U, v);
+  asm volatile("" : "+v"(u));
+  v = __builtin_bit_cast(V, u);
+}
+__device__ __forceinline__ void loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+
+template <typename V>
+__device__ __forceinline__ void store_row(bool stream, V* p, V v) {
+  if (stream) __builtin_nontemporal_store(v, p);
+  else store_through(p, v);
+}
+
 // ---------------------------------------------------------------------------
 // Embedding gather: out[row,:] = wte[ids[row],:] + wpe[row % L,:]
 // (reference: fused_embeddings_kernel, kernels.py:37-72).  The add is done in
@@ -27,7 +58,7 @@ template <> struct Vec<float> {
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void embed_vec_kernel(
     const int64_t* __restrict__ ids, const T* __restrict__ wte,
-    const T* __restrict__ wpe, T* __restrict__ out, int64_t rows, int64_t L, int64_t V_, int H) {
+    const T* __restrict__ wpe, T* __restrict__ out, int64_t rows, int64_t L, int64_t V_, int H, int stream) {
   typedef typename Vec<T>::type V;
   constexpr int VN = Vec<T>::N;
   const int lane = threadIdx.x & (LPR - 1);  // LPR lanes per token, as in the LayerNorm kernel
@@ -40,11 +71,25 @@ __global__ __launch_bounds__(256) void embed_vec_kernel(
   const V* b = reinterpret_cast<const V*>(wpe + pos * H);
   V* o = reinterpret_cast<V*>(out + row * H);
   const int nchunks = H / VN;
-  for (int c = lane; c < nchunks; c += LPR) {
-    V va = a[c], vb = b[c], vo;
+  for (int c0 = lane; c0 < nchunks; c0 += 4 * LPR) {
+    V va[4], vb[4];
 #pragma unroll
-    for (int j = 0; j < VN; ++j) vo[j] = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-    store_through(o + c, vo);
+    for (int i = 0; i < 4; ++i)
+      if (c0 + i * LPR < nchunks) {
+        va[i] = a[c0 + i * LPR];
+        vb[i] = b[c0 + i * LPR];
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c0 + i * LPR < nchunks) {
+#pragma unroll
+        for (int j = 0; j < VN; ++j) va[i][j] = (T)((known ? (float)va[i][j] : 0.f) + (float)vb[i][j]);
+        pin(va[i]);
+      }
+    loads_done();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c0 + i * LPR < nchunks) store_row(stream, o + c0 + i * LPR, va[i]);
   }
 }
 
@@ -67,7 +112,7 @@ __global__ __launch_bounds__(256) void embed_scalar_kernel(
 // token sees the same mask.  Rows of whole 16-byte chunks: a thread owns one chunk of columns, draws
 // its mask once and walks the rows of its workgroup's share (4800 x 768 halves: 10.2 us, 16.1 with an evaluation
 // per element).
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(256) void embed_dropout_vec_kernel(
     const int64_t* __restrict__ ids, const T* __restrict__ wte,
     const T* __restrict__ wpe, T* __restrict__ out, int64_t rows, int64_t L, int64_t V_, int H,
@@ -102,7 +147,7 @@ __global__ __launch_bounds__(256) void embed_dropout_vec_kernel(
     V vo;
 #pragma unroll
     for (int j = 0; j < VN; ++j) vo[j] = (T)(u[j] > drop.p ? sum[j] : 0.f);
-    store_through(reinterpret_cast<V*>(out + row * H) + c, vo);
+    store_row(STREAM, reinterpret_cast<V*>(out + row * H) + c, vo);
   }
 }
 
@@ -172,24 +217,28 @@ __device__ __forceinline__ void layernorm_rows(
   float d[CH][VN], rstd;
   layernorm_stats<CH, VN, LPR, false>(t, lane, nchunks, H, eps, d, rstd);
   OV* o = reinterpret_cast<OV*>(out + row * H);
+  // not a streaming store: the [T, H] output is what the following GEMM reads, two
+  // or three times over; it fits the 256 MB memory-side cache, and a GEMM fed from there
+  // instead of HBM ran 12 % faster (its operand loads are only one k-tile ahead)
+  OV to[CH];
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = lane + i * LPR;
     if (c < nchunks) {
-      if (CH > 4) {  // long rows: too many registers to hold them from the start
+      if (CH > 4) {
         tw[i] = wv[c];
         tb[i] = bv[c];
       }
-      OV to;
 #pragma unroll
       for (int j = 0; j < VN; ++j)
-        to[j] = (OT)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
-      // not a streaming store: the [T, H] output is what the following GEMM reads, two
-      // or three times over; it fits the 256 MB memory-side cache, and a GEMM fed from there
-      // instead of HBM ran 12 % faster (its operand loads are only one k-tile ahead)
-      store_through(o + c, to);
+        to[i][j] = (OT)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
+      pin(to[i]);
     }
   }
+  loads_done();
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+    if (lane + i * LPR < nchunks) store_through(o + lane + i * LPR, to[i]);
 }
 
 template <typename T, int CH, int LPR, typename OT = T>
@@ -208,7 +257,7 @@ template <typename T, int CH, int LPR>
 __global__ __launch_bounds__(256) void embed_layernorm_kernel(
     const int64_t* __restrict__ ids, const T* __restrict__ wte, const T* __restrict__ wpe,
     const T* __restrict__ w, const T* __restrict__ b, T* __restrict__ emb, T* __restrict__ out,
-    int64_t rows, int64_t L, int64_t V_, int H, float eps) {
+    int64_t rows, int64_t L, int64_t V_, int H, float eps, int stream) {
   typedef typename Vec<T>::type V;
   constexpr int VN = Vec<T>::N;
   const int lane = threadIdx.x & (LPR - 1);
@@ -232,26 +281,31 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(
       tb[i] = bv[c];
 #pragma unroll
       for (int j = 0; j < VN; ++j) e[i][j] = (T)((known ? (float)va[j] : 0.f) + (float)vb[j]);
-      store_through(eo + c, e[i]);  // the residual stream; next read by a GEMM epilogue
+      pin(e[i]);
     } else {
 #pragma unroll
       for (int j = 0; j < VN; ++j) e[i][j] = (T)0.f;
     }
   }
+  // (no loads_done: the parameters may still be on their way, and in front of the second stores it would be
+  // a wait for these)
+#pragma unroll
+  for (int i = 0; i < CH; ++i)
+    if (lane + i * LPR < nchunks) store_row(stream, eo + lane + i * LPR, e[i]);  // next read by a GEMM epilogue
   float d[CH][VN], rstd;
   layernorm_stats<CH, VN, LPR, false>(e, lane, nchunks, H, eps, d, rstd);
   V* o = reinterpret_cast<V*>(out + row * H);
 #pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int c = lane + i * LPR;
-    if (c < nchunks) {
-      V to;
+  for (int i = 0; i < CH; ++i)
+    if (lane + i * LPR < nchunks) {
 #pragma unroll
       for (int j = 0; j < VN; ++j)
-        to[j] = (T)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
-      store_through(o + c, to);  // as in layernorm_vec_kernel: the following GEMM reads it
+        e[i][j] = (T)layernorm_apply(d[i][j], rstd, (float)tw[i][j], (float)tb[i][j]);
+      pin(e[i]);
     }
-  }
+#pragma unroll
+  for (int i = 0; i < CH; ++i)  // as in layernorm_rows: the following GEMM reads it
+    if (lane + i * LPR < nchunks) store_through(o + lane + i * LPR, e[i]);
 }
 
 // Any H (no alignment requirement): the row is re-read from cache per pass.
@@ -541,6 +595,8 @@ static int launch_embed_t(const int64_t* ids, const void* wte, const void* wpe,
   const bool aligned = (H % Vec<T>::N) == 0 && ((uintptr_t)wte % 16) == 0 &&
                        ((uintptr_t)wpe % 16) == 0 && ((uintptr_t)out % 16) == 0;
   const unsigned grid = (unsigned)((rows + 3) / 4);
+  const int64_t bytes = rows * H * (int64_t)sizeof(T);
+  const int stream = bytes > kStreamBytes;
   // The reference runs the dropout even at p = 0 (kernels.py:70), where it is the identity
   // unless a column's uniform is exactly 0; for the default seed no column below 2^20 has
   // that, so only other seeds or wider rows need the generator at p = 0.
@@ -550,8 +606,15 @@ static int launch_embed_t(const int64_t* ids, const void* wte, const void* wpe,
       const int nchunks = H / Vec<T>::N, rows_per = nchunks < 256 ? 256 / nchunks : 1;
       const int64_t groups = (rows + rows_per - 1) / rows_per;
       const dim3 vgrid((unsigned)(groups < 768 ? groups : 768), (unsigned)((nchunks + 255) / 256));
-      hipLaunchKernelGGL(embed_dropout_vec_kernel<T>, vgrid, dim3(256), 0, st, ids, (const T*)wte,
-                         (const T*)wpe, (T*)out, rows, L, V, H, d);
+      // a thread's rows follow one another, so stores written through hold up the loads of the next: only
+      // where it has one or two (7 x 211 x 768 halves non-temporal 5.3, through 5.1 us; 16 x 300 7.2, 7.6; 512 x 300
+      // 101, 128)
+      if (bytes > (4 << 20))
+        hipLaunchKernelGGL((embed_dropout_vec_kernel<T, true>), vgrid, dim3(256), 0, st, ids, (const T*)wte,
+                           (const T*)wpe, (T*)out, rows, L, V, H, d);
+      else
+        hipLaunchKernelGGL((embed_dropout_vec_kernel<T, false>), vgrid, dim3(256), 0, st, ids, (const T*)wte,
+                           (const T*)wpe, (T*)out, rows, L, V, H, d);
       return 0;
     }
     hipLaunchKernelGGL(embed_dropout_kernel<T>, dim3(grid), dim3(256), 0, st, ids,
@@ -561,10 +624,10 @@ static int launch_embed_t(const int64_t* ids, const void* wte, const void* wpe,
   if (aligned)
     if (lanes_per_row(H / Vec<T>::N) == 32)
       hipLaunchKernelGGL((embed_vec_kernel<T, 32>), dim3((unsigned)((rows + 7) / 8)), dim3(256), 0,
-                         st, ids, (const T*)wte, (const T*)wpe, (T*)out, rows, L, V, H);
+                         st, ids, (const T*)wte, (const T*)wpe, (T*)out, rows, L, V, H, stream);
     else
       hipLaunchKernelGGL((embed_vec_kernel<T, 64>), dim3(grid), dim3(256), 0, st, ids,
-                         (const T*)wte, (const T*)wpe, (T*)out, rows, L, V, H);
+                         (const T*)wte, (const T*)wpe, (T*)out, rows, L, V, H, stream);
   else
     hipLaunchKernelGGL(embed_scalar_kernel<T>, dim3(grid), dim3(256), 0, st, ids,
                        (const T*)wte, (const T*)wpe, (T*)out, rows, L, V, H);
@@ -662,14 +725,15 @@ template <typename T, int CH>
 static void eln_go(const int64_t* ids, const void* wte, const void* wpe, const void* w,
                    const void* b, void* emb, void* out, int64_t rows, int64_t L, int64_t V, int H,
                    float eps, int lpr, hipStream_t st) {
+  const int stream = 2 * rows * H * (int64_t)sizeof(T) > kStreamBytes;  // both outputs
   if (lpr == 32)
     hipLaunchKernelGGL((embed_layernorm_kernel<T, CH, 32>), dim3((unsigned)((rows + 7) / 8)),
                        dim3(256), 0, st, ids, (const T*)wte, (const T*)wpe, (const T*)w,
-                       (const T*)b, (T*)emb, (T*)out, rows, L, V, H, eps);
+                       (const T*)b, (T*)emb, (T*)out, rows, L, V, H, eps, stream);
   else
     hipLaunchKernelGGL((embed_layernorm_kernel<T, CH, 64>), dim3((unsigned)((rows + 3) / 4)),
                        dim3(256), 0, st, ids, (const T*)wte, (const T*)wpe, (const T*)w,
-                       (const T*)b, (T*)emb, (T*)out, rows, L, V, H, eps);
+                       (const T*)b, (T*)emb, (T*)out, rows, L, V, H, eps, stream);
 }
 
 template <typename T>
