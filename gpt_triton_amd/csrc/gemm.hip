@@ -1186,11 +1186,13 @@ static int make_epi(const GemmEpilogue& e, int64_t M, int N, EpiDev& ep) {
   ep.vec_ok = vec ? 1 : 0;
   auto aligned16 = [&](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool half_out = e.f16 || e.out_f16;
-  // What the next kernel finds in the 256 MB memory-side cache it need not fetch from HBM; beyond half of
-  // that, non-temporal stores, which leave the cache to the operands (forwards, all non-temporal / all through:
+  // What the next kernel finds in the 256 MB memory-side cache it need not fetch from HBM; beyond a good third
+  // of that, non-temporal stores, which leave the cache to the operands (forwards, all non-temporal / all through:
   // medium 5 x 777 3686 / 3461 us, 16 x 300 with logits 1720 / 1697 (1686 with the line), 512 x 300
-  // 28.57 / 30.16 ms; lines from 40 to 160 MB are equal).
-  ep.through = M * (int64_t)N * (half_out ? 2 : 4) <= (128ll << 20);
+  // 28.57 / 30.16 ms; lines from 40 to 160 MB are equal.  Products with a residual, which takes as much of the
+  // cache again: 10000 x 6400 x 1600, 122 MB, 181 / 192 us, 8192 x 8192 x 1024, 128 MB, 134 / 145, 12000 x 4096 x 1024,
+  // 93 MB, 96.6 / 95.7).
+  ep.through = M * (int64_t)N * (half_out ? 2 : 4) <= (96ll << 20);
   const int cw = half_out ? 8 : 4;
   ep.tile_vec = N % cw == 0 && (!e.qkv || e.d % cw == 0) && aligned16(e.bias) && aligned16(e.residual) &&
                 aligned16(e.out) && aligned16(e.q) && aligned16(e.k) && aligned16(e.v);
