@@ -213,7 +213,7 @@ __device__ __forceinline__ void store_wave_tile_h(f4 (&acc)[2 * NB][2 * MB],
 // is free again (the kernel refills it there).  Younger than the first half's loads when band 0
 // starts: the second half's 8 loads.  Younger than the second half's loads when band 2 starts: the
 // 8 stores of bands 0 and 1 and, if `refilled`, the 8 operand loads `mid` issued.
-// DROP: as in store_wave_tile_h, but cleared in the accumulator layout, in front of the residual.  Training
+// DROP (never with GELU): as in store_wave_tile_h, but cleared in the accumulator layout, in front of the residual.  Training
 // forwards of 16800 rows x 768, projection and ffn2 on this kernel instead of one workgroup per tile: 4660 ->
 // 4330 us.
 template <int MB, int NB, bool GELU, bool DROP, typename Mid>
@@ -303,9 +303,9 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
 // loads of the next tile's k-tile 1 are issued BEFORE the epilogue's stores, so waiting for them
 // with vmcnt(EPI_STORES) -- the epilogue issues exactly 16 (fp16) or 32 (fp32) stores per lane --
 // does not wait for the stores' acknowledgements.  The bias is fetched, and waited for, before those loads are issued, so
-// that no compiler-placed wait inside the epilogue falls behind them.  Only whole row tiles (the last one
-// starts at row M - 256, see persistent_rows), no
-// residual, no dropout: the launcher sends everything else to gemm_tile.hip.
+// that no compiler-placed wait inside the epilogue falls behind them; so are the words of a dropout mask.  Only
+// whole row tiles (the last one starts at row M - 256, see persistent_rows), no residual, dropout with its mask
+// at hand and an fp16 output behind a GELU: the launcher sends everything else to gemm_tile.hip.
 // ---------------------------------------------------------------------------
 template <int MB, int NB, typename T, bool QKV, bool GELU>
 __device__ __forceinline__ void store_wave_tile32(f4 (&acc)[2 * NB][2 * MB], const f4 (&bias_r)[NB][2],
@@ -648,10 +648,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
       int lane_e = lane;
       asm volatile("" : "+v"(lane_e));
       if constexpr (HALF_SLABS) {
-        if (ep.gelu)
+        if (DROP || ep.gelu)
           store_wave_tile_h<MB, NB, QKV, true, DROP>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e, keep_w);
-        else
-          store_wave_tile_h<MB, NB, QKV, false, DROP>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e, keep_w);
+        else if constexpr (!DROP)
+          store_wave_tile_h<MB, NB, QKV, false, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e, keep_w);
       } else {
         if (ep.gelu) store_wave_tile32<MB, NB, OT, QKV, true>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
         else store_wave_tile32<MB, NB, OT, QKV, false>(acc, bias_r, ep, mw0, nw0, N, slab, lane_e);
@@ -960,11 +960,11 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
           issue(stage, m0_n, n0_n, 0);
         }
       };
-      if (ep.gelu)
-        store_wave_tile_rs<MB, NB, true, DROP>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
-                                               has_next, mid, keep_w);
-      else
+      if (DROP || !ep.gelu)
         store_wave_tile_rs<MB, NB, false, DROP>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
+                                                has_next, mid, keep_w);
+      else if constexpr (!DROP)
+        store_wave_tile_rs<MB, NB, true, false>(acc, bias_r, ep, mw0, nw0, N, res_lo, res_hi, slab, lane,
                                                 has_next, mid, keep_w);
     } else if (has_next) {
       barrier_lds();  // the barrier and the refill of `mid`
@@ -1064,13 +1064,15 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // over its own residual, which the second pass would read changed: whole row tiles and a launch behind them.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, and dropout only with its
-// mask at hand and an fp16 output.
+// mask at hand and an fp16 output, behind a GELU or in front of a residual (the two products of a block that
+// have one).
 // Sets *head to the number of rows for the persistent kernel.
 template <typename T, typename OT, bool QKV>
 int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool drop = ep.drop.p > 0.f;
-  const bool drop_ok = !QKV && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0;
+  const bool drop_ok = !QKV && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0 &&
+                       (ep.gelu != 0) != res;
   const bool persistent =
       M >= 256 && N >= 256 && N % 64 == 0 && Kp >= (res ? 192 : 128) && Kp <= (1 << 21) && ep.vec_ok &&
       (sizeof(OT) == 4 || ep.vec8_ok) && (!drop || drop_ok) &&
