@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void softmax_scalar_kernel(const T* __restrict
 template <typename T>
 __global__ __launch_bounds__(256) void pack_rows_vec_kernel(const T* __restrict__ src,
                                                             _Float16* __restrict__ dst,
-                                                            int64_t R, unsigned K8, unsigned Kp8) {
+                                                            int64_t R, unsigned K8, unsigned Kp8, int through) {
   typedef T V __attribute__((ext_vector_type(8)));
   const unsigned rows_per = 256 / Kp8 ? 256 / Kp8 : 1;  // rows a workgroup turn covers
   const unsigned lane_row = Kp8 <= 256 ? threadIdx.x / Kp8 : 0;
@@ -440,9 +440,9 @@ __global__ __launch_bounds__(256) void pack_rows_vec_kernel(const T* __restrict_
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = (_Float16)(float)v[j];
       }
-      // not written through: one store a thread and turn, with nothing behind it to hide the longer way
-      // (2048 x 1280 floats and the product with 1280 columns 20.2 us, 24.7; 4800 x 1280 alone 13.3, 16.6)
-      *reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8) = o;
+      h8* to = reinterpret_cast<h8*>(dst + (r * Kp8 + c) * 8);
+      if (through) store_through(to, o);
+      else *to = o;
     }
 }
 
@@ -773,8 +773,12 @@ static void launch_pack_rows_t(const T* src, _Float16* dst, int64_t R, int K, in
     const int64_t rows_per = 256 / (Kp / 8) ? 256 / (Kp / 8) : 1;
     int64_t blocks = (R + rows_per - 1) / rows_per;
     if (blocks > 16384) blocks = 16384;
+    // written through while the rows are few; one store a thread and turn has nothing behind it to hide the
+    // longer way when there are many (product and operand rows in fp32, plain / through: 300 x 768 x 768 6.3 / 6.0 us,
+    // 1477 x 1024 x 1024 11.0 / 10.6, 2048 x 1280 x 1280 20.2 / 24.7, 9600 x 768 x 768 28.7 / 29.8)
+    const int through = R * Kp * 2 <= (4 << 20);
     hipLaunchKernelGGL(pack_rows_vec_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, dst, R,
-                       (unsigned)(K / 8), (unsigned)(Kp / 8));
+                       (unsigned)(K / 8), (unsigned)(Kp / 8), through);
     return;
   }
   int64_t blocks = (R * (int64_t)Kp + 255) / 256;
