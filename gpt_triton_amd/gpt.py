@@ -24,8 +24,8 @@ import torch.nn as nn
 from torch.multiprocessing.reductions import StorageWeakRef
 
 from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, block_supported, blocks_forward,
-                      dropout_mask,
-                      flash_attention_v1, fused_embeddings, fused_embeddings_layer_norm, fused_ffn,
+                      blocks_workspace, dropout_mask, flash_attention_v1, fused_embeddings,
+                      fused_embeddings_layer_norm, fused_ffn,
                       fused_layer_norm, layer_norm_ffn, layer_norm_linear_supported,
                       layer_norm_matmul_and_split_qkv, lm_head, matmul_and_split_qkv, mlp_block,
                       pack_lm_head, pack_weight)
@@ -123,8 +123,9 @@ class _PackedWeights:
         hit = self.held(name, param)
         if hit is None:
             hit = pack(param.data)
-            self._entries[name] = (weakref.ref(param), StorageWeakRef(param.untyped_storage()),
-                                   param.data_ptr(), param._version, param.dtype, param.shape, hit)
+            storage = StorageWeakRef(param.untyped_storage())
+            self._entries[name] = (weakref.ref(param), storage.cdata, param.data_ptr(), param._version,
+                                   param.dtype, param.shape, hit, storage)
         return hit
 
     def held(self, name, param):
@@ -132,11 +133,11 @@ class _PackedWeights:
         entry = self._entries.get(name)
         if entry is None:
             return None
-        owner, storage, address, version, dtype, shape, hit = entry
+        owner, storage, address, version, dtype, shape, hit, _ = entry
         # an address inside a storage that is still there is that storage's: no other has it
         if (owner() is not param or param._version != version or param.data_ptr() != address or
                 param.dtype != dtype or param.shape != shape or not param.is_contiguous() or
-                _storage_expired(storage.cdata)):
+                _storage_expired(storage)):
             return None
         return hit
 
@@ -411,17 +412,17 @@ def _stack(blocks, x):
 
 def _through(stack, blocks, x, normed):
     """(x behind the blocks that went to the library together, the blocks that are left).  Every block is
-    looked over on every forward, 8 to 10 us of host work each, so they go in calls of 1, 2, 4, ... layers: the
+    looked over on every forward, 8 to 10 us of host work each, so they go in calls of 1, 3, 9, ... layers: the
     GPU works on those launched while the next are looked over.  Microseconds of a forward that is waited for /
     of one among others, modules called one by one, all blocks looked over before one call, and this: 1 x 24
-    tokens 124M 571 / 499, 438 / 315, 395 / 330; 2 x 64 570 / 500, 516 / 344, 428 / 339; 7 x 211 721 / 665, 864 /
-    687, 723 / 666; 2 x 300 tokens of the 48-layer model 4230 / 4183, 4824 / 4279, 4242 / 4188.  A weight of the
-    last layer edited in place before each forward of 2 x 64: 560, 680, 425."""
+    tokens 124M 562 / 488, 438 / 315, 407 / 306; 2 x 64 561 / 494, 516 / 344, 456 / 339; 7 x 211 712 / 654, 864 /
+    687, 716 / 655; 2 x 300 tokens of the 48-layer model 4114 / 4064, 4824 / 4279, 4130 / 4074.  A weight of the
+    last layer edited in place before each forward of 2 x 64: 560, 680, 440."""
     layers, found = stack
-    in_gemm = _ln_in_gemm(x, layers.alive[0])
-    sent, seen, size = 0, 1, 1
+    in_gemm, workspace = _ln_in_gemm(x, layers.alive[0]), blocks_workspace(x, layers.heads, layers.inner)
+    sent, seen, size, built = 0, 1, 1, 0
     while True:
-        more, built = found, layers.built
+        more = found
         while more is not None and seen < min(sent + size, len(blocks)):
             more = layers.pointers(blocks[seen])
             if more is not None:
@@ -429,15 +430,16 @@ def _through(stack, blocks, x, normed):
                 seen += 1
         if seen == len(blocks) and not layers.built:
             return blocks_forward(x, found, layers.heads, layers.inner, normed=normed,
-                                  layer_norm_in_gemm=in_gemm), []
+                                  layer_norm_in_gemm=in_gemm, workspace=workspace), []
         if found:
             # in place behind the first call, whose x is the caller's
             x = block_layers(x, found, layers.heads, layers.inner, normed=normed, layer_norm_in_gemm=in_gemm,
-                             out=x if sent else None)
+                             out=x if sent else None, workspace=workspace)
         if more is None or seen == len(blocks):
             return x, blocks[seen:]
         # packing two weights takes the host as long as a layer takes the GPU
-        normed, sent, size, found = None, seen, 1 if layers.built > built else 2 * size, []
+        normed, sent, size, found = None, seen, 1 if layers.built > built else 3 * size, []
+        built = layers.built
 
 
 @dataclass

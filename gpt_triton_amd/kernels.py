@@ -546,29 +546,36 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     return out
 
 
-def block_layers(x, pointers, num_heads, inner, normed=None, layer_norm_in_gemm=False, out=None):
+def blocks_workspace(x, num_heads, inner):
+    """(scratch that serves `block_layers` for x and these sizes, its bytes)."""
+    B, L, h = x.shape
+    nbytes = _lib.load().gptmi_blocks_workspace_bytes(B, L, num_heads, h // num_heads, inner,
+                                                      _dtype_code(x, "block_layers"))
+    return _workspace(nbytes, x), nbytes
+
+
+def block_layers(x, pointers, num_heads, inner, normed=None, layer_norm_in_gemm=False, out=None, workspace=None):
     """`attention_block` then `mlp_block` for each of some layers of a model in one call of the library, packed
     weights, no dropout; same launches, same bits.  pointers: 12 device addresses a layer, as gptmi_blocks
     lists them, of tensors that the caller has checked and keeps (`FusedGPT.forward` does).  out: where the
-    result goes, x itself included."""
+    result goes, x itself included; workspace: `blocks_workspace`, if the caller has it."""
     B, L, h = x.shape
     dev = _on_gpu(x, normed, out)
     code = _dtype_code(x, "block_layers")
     assert x.is_contiguous() and (normed is None or normed.is_contiguous() and normed.shape == x.shape)
     assert out is None or out.is_contiguous() and out.shape == x.shape and out.dtype == x.dtype
     assert len(pointers) % 12 == 0 and h % num_heads == 0
-    lib = _lib.load()
-    nbytes = lib.gptmi_blocks_workspace_bytes(B, L, num_heads, h // num_heads, inner, code)
-    ws = _workspace(nbytes, x)
+    ws, nbytes = workspace or blocks_workspace(x, num_heads, inner)
     if out is None:
         out = torch.empty_like(x)
     table = array.array("Q", pointers)
-    _call(dev, "block_layers", lib.gptmi_blocks, x.data_ptr(), _ptr(normed), table.buffer_info()[0],
+    _call(dev, "block_layers", _lib.load().gptmi_blocks, x.data_ptr(), _ptr(normed), table.buffer_info()[0],
           len(pointers) // 12, 1e-5, out.data_ptr(), B, L, num_heads, h // num_heads, inner,
           1 if layer_norm_in_gemm else 0, _ptr(ws), nbytes, code)
     return out
 
 
-def blocks_forward(x, pointers, num_heads, inner, normed=None, layer_norm_in_gemm=False):
+def blocks_forward(x, pointers, num_heads, inner, normed=None, layer_norm_in_gemm=False, workspace=None):
     """`block_layers` for a model's layers, or for those that are left of them."""
-    return block_layers(x, pointers, num_heads, inner, normed=normed, layer_norm_in_gemm=layer_norm_in_gemm)
+    return block_layers(x, pointers, num_heads, inner, normed=normed, layer_norm_in_gemm=layer_norm_in_gemm,
+                        workspace=workspace)

@@ -26,11 +26,13 @@ def through(monkeypatch):
     def run(model, x):
         calls = []
 
-        def call(x, pointers, heads, inner, normed=None, layer_norm_in_gemm=False, out=None):
-            assert (heads, inner, layer_norm_in_gemm) == (2, 512, False) and (normed is None) == bool(calls)
+        def call(x, pointers, heads, inner, normed=None, layer_norm_in_gemm=False, out=None, workspace=None):
+            assert workspace is scratch and (heads, inner, layer_norm_in_gemm) == (2, 512, False) and (normed is None) == bool(calls)
             calls.append(pointers)
             return x
 
+        scratch = (None, 0)
+        monkeypatch.setattr(gpt, "blocks_workspace", lambda x, heads, inner: scratch)
         monkeypatch.setattr(gpt, "block_layers", call)
         monkeypatch.setattr(gpt, "blocks_forward", call)
         blocks = list(model.blocks)
@@ -55,7 +57,7 @@ def addresses(blocks):
     return found
 
 
-@pytest.mark.parametrize("layers,calls", [(1, [1]), (2, [1, 1]), (3, [1, 2]), (4, [1, 2, 1]), (12, [1, 2, 4, 5])])
+@pytest.mark.parametrize("layers,calls", [(1, [1]), (2, [1, 1]), (4, [1, 3]), (12, [1, 3, 8]), (24, [1, 3, 9, 11])])
 def test_untouched_blocks_are_taken(layers, calls, through):
     assert through(*build(layers)) == (calls, 0)
 
@@ -106,7 +108,7 @@ def test_the_layers_in_front_of_another_one_are_taken(through):
                lambda block: setattr(block[0].c_attn_weight, "data", torch.zeros(384, 128).t())]
     with torch.no_grad():
         for change in changes:
-            for block, want in ((0, ([], 5)), (1, ([1], 4)), (2, ([1, 1], 3)), (4, ([1, 2, 1], 1))):
+            for block, want in ((0, ([], 5)), (1, ([1], 4)), (2, ([1, 1], 3)), (4, ([1, 3], 1))):
                 model, x = build(5)
                 change(model.blocks[block])
                 if change is changes[0]:
@@ -121,13 +123,13 @@ def test_images_that_are_not_held_are_built(edit, through, monkeypatch):
     packed = []
     monkeypatch.setattr(gpt._PackedWeights.get, "__defaults__", (lambda w: packed.append(w) or pack(w),))
     with torch.no_grad():
-        for block, calls in ((0, [1, 2, 2]), (1, [1, 2, 1, 1]), (4, [1, 2, 2])):
+        for block, calls in ((0, [1, 1, 3]), (1, [1, 3, 1]), (4, [1, 3, 1])):
             model, x = build(5)
             edit(model.blocks[block])
             packed.clear()
             assert through(model, x) == (calls, 0) and 1 <= len(packed) <= 2
             packed.clear()
-            assert through(model, x) == ([1, 2, 2], 0) and not packed
+            assert through(model, x) == ([1, 3, 1], 0) and not packed
     # none built for a module whose other weight cannot be packed
     model, x = build(2)
     model.blocks[1][0].train().eval()
