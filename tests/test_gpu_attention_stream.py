@@ -1,7 +1,7 @@
 """GPU parity of the attention kernel the headline forward runs on: fp16, head size 64, equal
-query and key lengths <= 320 and at least 64 (batch, head) pairs -- with fewer pairs, other head
-sizes or fp32 storage `flash_attention_v1` picks other kernels, which tests/test_gpu_parity.py
-covers.  Here every call has B * N >= 64:
+query and key lengths <= 320, up to 64 rows more than 512 (batch, head) pairs, beyond 288 rows more than
+85 (256 CUs) -- with fewer pairs of those lengths `flash_attention_v1` picks the ring kernel, which runs
+here beside it, and with other head sizes or fp32 storage others, which tests/test_gpu_parity.py covers:
 
   * every length either side of the 32-query chunk and 64-key tile boundaries, from 1 to the
     longest the kernel takes, both output layouts, against the oracle;
@@ -78,10 +78,13 @@ LENGTHS = [1, 2, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 191, 192, 19
            299, 300, 319, 320]
 
 
+@pytest.mark.parametrize("B,N", [(6, 12), (9, 11), (57, 9)])
 @pytest.mark.parametrize("L", LENGTHS)
-def test_stream_attention_lengths(K, gpu_device, L):
-    """72 pairs (fewer than persistent workgroups: one pair each), every boundary length."""
-    B, N = 6, 12
+def test_stream_attention_lengths(K, gpu_device, B, N, L):
+    """72 and 99 pairs (fewer than persistent workgroups: one pair each; of up to 64 rows, 72 also beyond 288,
+    on the ring kernel), every boundary length; 513 pairs of up to 64 rows."""
+    if B * N > 512 and L > 64:
+        pytest.skip("99 pairs run the streaming kernel at this length")
     q, k, v = gaussian_qkv(B, N, L, seed=1000 + L)
     print(f"stream attention: B={B} N={N} L={L}", flush=True)
     z, zm = both_layouts(K, q, k, v, gpu_device)
@@ -96,7 +99,7 @@ def test_stream_attention_lengths(K, gpu_device, L):
 @pytest.mark.parametrize("B,N", [(8, 8), (25, 12), (27, 19), (64, 12)])
 @pytest.mark.parametrize("L", [77, 300])
 def test_stream_attention_pair_counts(K, gpu_device, B, N, L):
-    """64 pairs (the fewest the kernel is picked for), 300 (some workgroups walk two pairs, most
+    """64 pairs (300 rows on the ring kernel), 300 (some workgroups walk two pairs, most
     one), 513 (two rounds and one pair of a third) and 768 (three whole rounds on 256 CUs):
     every pair against the oracle."""
     q, k, v = gaussian_qkv(B, N, L, seed=B * N + L)
@@ -112,15 +115,15 @@ def test_stream_attention_pair_counts(K, gpu_device, B, N, L):
 def test_stream_attention_reference_golden_vectors(K, gpu_device, case, heads):
     """The reference's own outputs for cases `a` ([1, 3, 150, 64]) and `c` ([1, 1, 300, 64]) of
     tests/golden/flash_attention_v1.npz: its (batch, head) pairs are placed at the first, a
-    middle and the last positions of a [7, 11] grid of otherwise random pairs (77 pairs), so the
+    middle and the last positions of a [9, 11] grid of otherwise random pairs (99 pairs), so the
     call runs on the many-pair kernel; pairs are independent, so those positions must reproduce
     the reference's vectors."""
     g = np.load(os.path.join(os.path.dirname(__file__), "golden", "flash_attention_v1.npz"))
     gq, gk, gv, gout = (g[f"{case}_{t}"] for t in ("q", "k", "v", "out"))
     L = gq.shape[2]
-    B, N = 7, 11
+    B, N = 9, 11
     q, k, v = gaussian_qkv(B, N, L, seed=77)
-    spots = [(0, 0), (3, 5), (6, 10)]
+    spots = [(0, 0), (4, 5), (8, 10)]
     for i, (b, n) in enumerate(spots):
         h = i % heads
         q[b, n], k[b, n], v[b, n] = gq[0, h], gk[0, h], gv[0, h]

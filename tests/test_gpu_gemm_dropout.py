@@ -15,13 +15,17 @@ def K(gpu_device):
 
 # 564 tiles of 256 x 256 and more, two rounds of any launch: always the persistent kernel.  Whole row tiles
 # and a last one moved up by 1 and by 255 rows; a last column tile of 64 and of 192 columns.  The first and
-# the sixth: one round, sizes that the cost model gives to it.  The last two: the second product, with a
-# residual, takes two rounds (the first, of 192 or 256 columns, does not matter).
+# the sixth: one round, sizes that the cost model gives to it.  WITH_RESIDUAL: the second product, with a
+# residual, takes two rounds (the first, of 192 or 256 columns, does not matter).  test_shapes_reach_the_kernels
+# of tests/test_gpu_gemm_ragged.py holds them to the cost model.
+WITH_RESIDUAL = [(44031, 768, 192), (43777, 832, 256)]
+SHAPES = [(4800, 768, 3072), (12032, 768, 3072), (12031, 128, 3072), (11777, 256, 3136), (12800, 192, 3008),
+          (3885, 1024, 4096)] + WITH_RESIDUAL
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("p", [0.1, 0.5])
-@pytest.mark.parametrize("M,h,inner", [(4800, 768, 3072), (12032, 768, 3072), (12031, 128, 3072), (11777, 256, 3136),
-                                       (12800, 192, 3008), (3885, 1024, 4096), (44031, 768, 192),
-                                       (43777, 832, 256)])
+@pytest.mark.parametrize("M,h,inner", SHAPES)
 def test_bits(K, gpu_device, M, h, inner, p, dtype):
     print(f"persistent GEMM with a dropout mask: M={M} h={h} inner={inner} p={p} {dtype}", flush=True)
     g = torch.Generator(device=gpu_device).manual_seed(M + h)

@@ -32,6 +32,10 @@ BETWEEN = [(1, 40, 768), (15, 768, 768), (16, 2304, 832), (17, 776, 1024), (31, 
            (2500, 3080, 256), (2561, 3080, 192), (190, 2304, 768), (600, 3080, 320)]
 
 
+# (B, L, heads, h) of qkv products that the persistent kernel takes whole
+SCATTERED = [(3, 1295, 12, 768), (16, 300, 12, 192), (37, 105, 16, 256), (1477, 1, 33, 192)]
+
+
 def cost_tables():
     source = open(os.path.join(ROOT, "gpt_triton_amd", "csrc", "gemm_tile.hip")).read()
     tables = []
@@ -39,6 +43,20 @@ def cost_tables():
         rows = re.search(r"TileCost %s\[\] = \{(.*?)\};" % name, source, re.S).group(1)
         tables += [[float(v.rstrip("f")) for v in row.split(",")] for row in re.findall(r"\{([^{}]*)\}", rows)]
     return tables
+
+
+def stream_terms():
+    """The terms of stream_cost in gemm.hip, as (coefficient, factors) with and without a residual."""
+    source = open(os.path.join(ROOT, "gpt_triton_amd", "csrc", "gemm.hip")).read()
+    with_res, without = re.search(r"return res \? (rounds.*?)\n\s*: (.*?);", source, re.S).groups()
+    # python reads the two expressions once the float suffixes are gone
+    return [re.sub(r"(?<=\d)f\b", "", e) for e in (with_res, without)]
+
+
+def two_rounds():
+    source = open(os.path.join(ROOT, "gpt_triton_amd", "csrc", "gemm.hip")).read()
+    return "float least = tiles >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);" in source and (
+        "if (rows < M) c += 1.0f + gemm_tile_cost(M - rows, N, Kp, cus);" in source)
 
 
 def pick(tiles, M, N, slices):
@@ -50,16 +68,15 @@ def pick(tiles, M, N, slices):
     return min(costs), costs.index(min(costs))
 
 
-def persistent_rows(tiles, M, N, slices, res):
-    """persistent_rows of gemm.hip for 256 CUs, no overlap."""
+def persistent_rows(tiles, M, N, slices, res, drop=False):
+    """persistent_rows of gemm.hip for 256 CUs, no overlap; with dropout all rows or none."""
+    assert two_rounds(), "the rule below is not the one of gemm.hip any more"
     cols, row_tiles = -(-N // 256), -(-M // 256)
-    whole = row_tiles * cols // 256 * 256 // cols * 256
+    whole = M if drop else row_tiles * cols // 256 * 256 // cols * 256
+    expression = stream_terms()[0 if res else 1]
 
     def stream(t):
-        rounds, fill = -(-t // 256), t / 256
-        if res:
-            return rounds * 7.42 + slices * (0.787 * rounds + 0.780 * fill)
-        return 1.67 + rounds * 4.70 + fill * 1.63 + slices * (0.917 * rounds + 0.659 * fill)
+        return eval(expression, {"rounds": -(-t // 256), "fill": t / 256, "k": slices})
 
     least, head = (math.inf if row_tiles * cols >= 512 else pick(tiles, M, N, slices)[0]), 0
     for rows in (M, min(whole, M)):
@@ -74,6 +91,7 @@ def persistent_rows(tiles, M, N, slices, res):
 
 
 def test_shapes_reach_the_kernels():
+    import test_gpu_gemm_dropout
     import test_gpu_gemm_tile
 
     tiles = cost_tables()
@@ -82,6 +100,16 @@ def test_shapes_reach_the_kernels():
         assert M % 256 != 0
         for res in (False, True):
             assert persistent_rows(tiles, M, N, Kd // 64, res) == M
+    for B, L, heads, h in SCATTERED:
+        assert B * L % 256 != 0 and persistent_rows(tiles, B * L, 3 * 64 * heads, h // 64, False) == B * L
+    for M, h, inner in test_gpu_gemm_dropout.SHAPES:
+        first = persistent_rows(tiles, M, inner, h // 64, False, drop=True)
+        second = h >= 256 and inner >= 192 and persistent_rows(tiles, M, h, inner // 64, True, drop=True)
+        assert M in (first, second)
+        if (M, h, inner) in test_gpu_gemm_dropout.WITH_RESIDUAL:
+            assert second == M
+        else:
+            assert first == M
     reached = set()
     for M, N, Kd in BETWEEN + test_gpu_gemm_tile.SHAPES:
         slices = -(-Kd // 64)
@@ -111,8 +139,7 @@ def test_ragged_rows_of_the_persistent_kernels(K, gpu_device, M, N, Kd):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-@pytest.mark.parametrize("B,L,heads,h", [(3, 1295, 12, 768), (16, 300, 12, 192), (37, 105, 16, 256),
-                                         (1477, 1, 33, 192)])
+@pytest.mark.parametrize("B,L,heads,h", SCATTERED)
 def test_ragged_rows_scattered(K, gpu_device, dtype, B, L, heads, h):
     n = heads * 64
     x, w, b, _ = operands(B * L, 3 * n, h, dtype, gpu_device, seed=B + L)
