@@ -1059,8 +1059,8 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // the cost model says is the fastest; the rows that are left follow in a launch of the tile kernel.
 // All rows also where they are no multiple of 256: the last row tile starts at row M - 256, and the rows
 // that it shares with the tile in front of it are formed twice, from the same operands in the same order,
-// so both store the same bits (4800 x 768 x 3072 with GELU: 27.0 us, 35.4 on the tile kernel; 3885 x 1024 x
-// 4096 35.2, 43.6; a second launch for the rows beyond a multiple costs 6 us and more).  Not with an output
+// so both store the same bits (4800 x 3072 x 768 with GELU: 25.2 us by itself and 29.7 within a forward, 35.1 on
+// the tile kernel; 3885 x 1024 x 4096 35.2, 43.6; a second launch for the rows beyond a multiple costs 6 us and more).  Not with an output
 // over its own residual, which the second pass would read changed: whole row tiles and a launch behind them.
 // It needs N a multiple of 64 (the wavefronts of the last column tile whose 64 columns lie past the
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, and dropout only with its

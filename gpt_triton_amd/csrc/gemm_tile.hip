@@ -583,7 +583,7 @@ int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, co
 }
 
 // ---- LayerNorm prologue ----------------------------------------------------------------------
-// 32-row tiles on 8 wavefronts: the LDS panel of the normalised rows takes 64 * K bytes (100 KB at
+// Tiles of 16 or 32 rows on 8 wavefronts: the LDS panel of 32 normalised rows takes 64 * K bytes (100 KB at
 // GPT-2 XL's 1600), three stages of weight rows 48 KB beside it -- up to K = 1024 also 96 KB, and then
 // the four-way split has a 64-wide tile.  K is split over as many groups as the plain launch splits
 // it (split = false: not at all, the rows that launch gives to the persistent kernel), so that the

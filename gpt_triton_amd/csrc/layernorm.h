@@ -11,7 +11,7 @@ namespace gptmi {
 // tile of a product (gemm_tile.hip, LNA): some 11 an element, of which 5 are left.
 //   * fp16 rows stay packed: v_fma_mix_f32 takes a half as it stands (x * 1 + s is s + x and
 //     x * 1 - mean is x - mean, rounded once, so the values are those of a conversion in front);
-//   * FULL: rows that are whole shares of all lanes (768, 1024) need no masks;
+//   * FULL: rows that are whole shares of 32 lanes (256 and 768 halves) need no masks in the operand prologue;
 //   * the divisions by H are a product with its reciprocal and one correction by the remainder, which
 //     is the correctly rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990) unless the remainder
 //     is subnormal; a mean that is not finite makes the row NaN either way, a variance beyond 2^100 is

@@ -33,18 +33,19 @@ from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, b
 # Up to this many token rows of up to this width the blocks run their LayerNorm inside the following
 # GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile, in front
 # of its first product, and one of its workgroups fills a CU.  So it pays while all column tiles run at
-# once and while normalising 32 rows costs less than a launch, up to 768: LayerNorm -> ffn1 at 24 / 128 /
-# 160 / 192 rows of 768 takes 6.5 / 8.3 / 8.5 / 13.3 us against 7.7 / 9.3 / 9.9 / 9.9 for the two
-# launches, 24 and 64 rows of 1024 8.0 and 9.3 against 7.5 and 8.6, 24 of 1600 13.1 against 12.2.
+# once and while normalising 16 or 32 rows costs less than a launch, up to 768: LayerNorm -> ffn1 at 24 / 128 /
+# 160 / 192 rows of 768 takes 5.4 / 7.5 / 7.6 / 12.2 us against 6.4 / 7.7 / 8.3 / 8.3 for the two launches, 24,
+# 64 and 128 rows of 1024 6.9, 8.3 and 8.5 against 6.7, 7.8 and 8.5, 24 of 1280 9.8 against 8.8, 24 of 1600 12.0
+# against 10.1 (8 rows of 1024 5.8 against 6.6).
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
 
 # Up to this many token rows a block is one call of the library (attention_block, mlp_block) instead
 # of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one the host
 # sets the pace of an operator-by-operator forward (some 10 us per operator against 2 us per launch
-# inside one call: 512 rows 898 against 566 us, 2048 rows 887 against 819; 1024-wide 512 rows 1759
-# against 1386).  From there to 24576 rows the two are within 2 %, but for 5 % at 6144 rows of 124M (1814
-# against 1716); the line lies beyond that, where only the memory differs: the operators give each
+# inside one call: 512 rows 926 against 567 us, 2048 rows 910 against 826; 1024-wide 512 rows 1777
+# against 1291).  From there to 24576 rows the two are within 2 %, but for 3 % at 6144 rows of 124M (1708
+# against 1662); the line lies beyond that, where only the memory differs: the operators give each
 # intermediate matrix back before they take the next.  fp32 models take the block calls at every size: their
 # intermediate matrices are fp16 there (see gptmi_attention_block).
 BLOCK_MAX_ROWS = 8192
@@ -582,7 +583,7 @@ def convert_hf_and_load_model(model_id, device):
 class GraphedForward:
     """The forward of an eval-mode FusedGPT for one input shape, captured once into a HIP graph
     and replayed per call: the 63 launches of a forward become one graph launch and their host work
-    goes (2 x 64 tokens, 124M, a pass that is waited for: 0.54 -> 0.40 ms).  Nothing in the library allocates or
+    goes (2 x 64 tokens, 124M, a pass that is waited for: 411 -> 355 us; among others both take 340).  Nothing in the library allocates or
     synchronises, so capture needs no special path; the operators' output tensors
     come from the graph's private pool.  The result of a call is overwritten by the next call --
     clone it to keep it.  No counterpart in the reference (Triton launches kernel by kernel)."""

@@ -226,7 +226,7 @@ int gptmi_linear_qkv(const void* x, const void* W, const void* bias, void* q,
 /*
  * out = gelu?(LayerNorm(x; ln_w, ln_b, eps) @ W + bias), and the same with the head-major
  * scatter of gptmi_linear_qkv: the LayerNorm runs in the GEMM's operand prologue.  Every
- * workgroup normalises the 32 rows of its tile (fp32 statistics, the arithmetic of
+ * workgroup normalises the 16 or 32 rows of its tile (fp32 statistics, the arithmetic of
  * gptmi_layernorm: the operand has the bits of that call's output) into LDS; the normalised
  * matrix never goes to memory and its kernel launch is gone.  Each column tile of a row block
  * normalises the rows again, so this pays for FEW rows, where a forward is bound by its launches
