@@ -414,14 +414,17 @@ def _stack(blocks, x):
 def _through(stack, blocks, x, normed):
     """(x behind the blocks that went to the library together, the blocks that are left).  Every block is
     looked over on every forward, 8 to 10 us of host work each, so they go in calls of 1, 3, 9, ... layers: the
-    GPU works on those launched while the next are looked over.  Microseconds of a forward that is waited for /
-    of one among others, modules called one by one, all blocks looked over before one call, and this: 1 x 24
-    tokens 124M 562 / 488, 438 / 315, 407 / 306; 2 x 64 561 / 494, 516 / 344, 456 / 339; 7 x 211 712 / 654, 864 /
-    687, 716 / 655; 2 x 300 tokens of the 48-layer model 4114 / 4064, 4824 / 4279, 4130 / 4074.  A weight of the
-    last layer edited in place before each forward of 2 x 64: 560, 680, 440."""
+    GPU works on those launched while the next are looked over.  Where the host sets the pace in any case, up
+    to some 170 rows of 768, each call counts (5 us): 2, 10, 50, ... layers.  Microseconds of a forward that is
+    waited for / of one among others, modules called one by one, all blocks looked over before one call, and
+    this: 1 x 24 tokens 124M 566 / 488, 438 / 315, 420 / 307 (in calls of 1, 3, 8 407 / 315); 2 x 128 630 / 549,
+    609 / 429, 520 / 400 (2, 10: 547 / 402); 7 x 211 712 / 654, 864 / 687, 716 / 655; 2 x 300 tokens of the 48-layer
+    model 4114 / 4064, 4824 / 4279, 4130 / 4074.  A weight of the last layer edited in place before each
+    forward of 2 x 64: 560, 680, 440."""
     layers, found = stack
     in_gemm, workspace = _ln_in_gemm(x, layers.alive[0]), blocks_workspace(x, layers.heads, layers.inner)
-    sent, seen, size, built = 0, 1, 1, 0
+    sent, seen, built = 0, 1, 0
+    size, growth = (2, 5) if x.numel() <= 1 << 17 else (1, 3)
     while True:
         more = found
         while more is not None and seen < min(sent + size, len(blocks)):
@@ -439,7 +442,7 @@ def _through(stack, blocks, x, normed):
         if more is None or seen == len(blocks):
             return x, blocks[seen:]
         # packing two weights takes the host as long as a layer takes the GPU
-        normed, sent, size, found = None, seen, 1 if layers.built > built else 3 * size, []
+        normed, sent, size, found = None, seen, 1 if layers.built > built else growth * size, []
         built = layers.built
 
 

@@ -10,14 +10,14 @@ def pack(weight):
     return PackedWeight(torch.empty(16), weight.shape, weight.dtype)
 
 
-def build(layers=3):
+def build(layers=3, rows=2048):
     model = gpt.FusedGPT(gpt.GPTConfig(n_layer=layers, n_head=2, n_embd=128, vocab_size=8, block_size=16)).eval()
     for block in model.blocks:
         for module, names in ((block[0], ("c_attn_weight", "c_proj_weight")),
                               (block[1], ("ffn1_weight", "ffn2_weight"))):
             for name in names:
                 module._packed.get(name, getattr(module, name), pack)
-    return model, torch.zeros(1, 4, 128)
+    return model, torch.zeros(1, rows, 128)
 
 
 @pytest.fixture
@@ -57,9 +57,11 @@ def addresses(blocks):
     return found
 
 
-@pytest.mark.parametrize("layers,calls", [(1, [1]), (2, [1, 1]), (4, [1, 3]), (12, [1, 3, 8]), (24, [1, 3, 9, 11])])
-def test_untouched_blocks_are_taken(layers, calls, through):
-    assert through(*build(layers)) == (calls, 0)
+@pytest.mark.parametrize("layers,few,many", [(1, [1], [1]), (2, [2], [1, 1]), (4, [2, 2], [1, 3]),
+                                             (12, [2, 10], [1, 3, 8]), (24, [2, 10, 12], [1, 3, 9, 11])])
+def test_untouched_blocks_are_taken(layers, few, many, through):
+    assert through(*build(layers, 1024)) == (few, 0)
+    assert through(*build(layers, 1025)) == (many, 0)
 
 
 @pytest.mark.parametrize("name", ["__call__", "_call_impl"])
