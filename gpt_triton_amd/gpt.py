@@ -124,6 +124,8 @@ class _PackedWeights:
         hit = self.held(name, param)
         if hit is None:
             hit = pack(param.data)
+            if param.is_cuda and torch.cuda.is_current_stream_capturing():
+                return hit  # recorded into a graph and not there yet: this forward's alone
             storage = StorageWeakRef(param.untyped_storage())
             self._entries[name] = (weakref.ref(param), storage.cdata, param.data_ptr(), param._version,
                                    param.dtype, param.shape, hit, storage)

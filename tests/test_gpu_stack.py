@@ -124,6 +124,29 @@ def test_captured_and_on_a_stream_of_its_own(G, gpu_device):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("one_call", [True, False])
+def test_first_forward_under_capture_keeps_no_images(G, gpu_device, one_call, monkeypatch):
+    """A weight image whose packing is recorded into a graph does not exist until a replay: an eager forward
+    between capture and replay builds its own."""
+    ids = torch.randint(0, 101, (2, 24), device=gpu_device)
+    if not one_call:
+        monkeypatch.setattr(G, "_stack", lambda blocks, x: None)
+    with torch.no_grad():
+        want, logits = build(G, gpu_device, torch.float16)(ids, return_logits=True)
+        model = build(G, gpu_device, torch.float16)  # the same weights
+        model.train().eval()  # drops its images
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = model(ids, return_logits=True)
+        assert not any(m._packed._entries for m in model.modules() if hasattr(m, "_packed"))
+        for _ in range(3):
+            got = model(ids, return_logits=True)
+            assert torch.equal(got[0], want) and torch.equal(got[1], logits)
+            graph.replay()
+            assert torch.equal(captured[0], want) and torch.equal(captured[1], logits)
+            torch.cuda.synchronize()
+
+
 def test_arguments_are_refused_before_any_launch(gpu_device):
     import ctypes
 
