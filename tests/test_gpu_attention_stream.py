@@ -78,13 +78,11 @@ LENGTHS = [1, 2, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 191, 192, 19
            299, 300, 319, 320]
 
 
-@pytest.mark.parametrize("B,N", [(6, 12), (9, 11), (57, 9)])
-@pytest.mark.parametrize("L", LENGTHS)
+@pytest.mark.parametrize("B,N,L", [(B, N, L) for L in LENGTHS for B, N in ((6, 12), (9, 11), (57, 9))
+                                   if B * N < 512 or L <= 64])
 def test_stream_attention_lengths(K, gpu_device, B, N, L):
     """72 and 99 pairs (fewer than persistent workgroups: one pair each; of up to 64 rows, 72 also beyond 288,
     on the ring kernel), every boundary length; 513 pairs of up to 64 rows."""
-    if B * N > 512 and L > 64:
-        pytest.skip("99 pairs run the streaming kernel at this length")
     q, k, v = gaussian_qkv(B, N, L, seed=1000 + L)
     print(f"stream attention: B={B} N={N} L={L}", flush=True)
     z, zm = both_layouts(K, q, k, v, gpu_device)
