@@ -330,7 +330,8 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
  * a few hundred tokens is bound by the host otherwise.  Replaces the loop over the blocks, gpt.py:171.
  *   params: n * 12 device pointers (a host array, read during the call): for each layer ln_w, ln_b, W_qkv,
  *           b_qkv, W_proj, b_proj of the attention block, then ln_w, ln_b, W1, b1, W2, b2 of the MLP
- *   x, out [B*L][h]   normed: LayerNorm(x) of the first layer, or NULL
+ *   x, out [B*L][h], which may be the same   normed: LayerNorm(x) of the first layer, or NULL
+ *   Everything that a layer's calls refuse is refused before the first launch.
  *   inner, fuse_layernorm, workspace: as for those two calls, for every layer
  */
 size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner, int dtype);

@@ -20,7 +20,7 @@ def build(G, device, dtype, layers=3, heads=4, width=256):
         for name, prm in model.named_parameters():
             prm.normal_(1.0 if name.endswith("layer_norm_weight") else 0.0, 0.05)
     model = model.to(device=device, dtype=dtype).eval()
-    with torch.no_grad():  # the first forward goes through the modules, which build the weight images
+    with torch.no_grad():  # the first forward builds the weight images
         model(torch.zeros((1, 8), dtype=torch.int64, device=device))
     return model
 
