@@ -993,6 +993,20 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   }
 }
 
+// Which (batch, head) pair and which query block (of q_blocks) a workgroup works on.  Workgroup ids are dealt
+// round-robin over the 8 XCDs, so id % 8 is the XCD: all blocks of a pair go to one, whose L2 then holds
+// the K and V that they share.  An XCD takes its pairs in groups of `group`, of each group the heaviest
+// (latest) query blocks first.
+struct WorkItem {
+  int bh, qb;  // bh may be `pairs` or more: none
+};
+__device__ __forceinline__ WorkItem work_item(int pairs, int q_blocks, int group) {
+  const int j = blockIdx.x >> 3, per = (pairs + 7) >> 3;  // per: pairs of an XCD, the last one of some is none
+  const int first = j / (group * q_blocks) * group, in_group = j - first * q_blocks;
+  const int size = min(group, per - first), late = in_group / size;
+  return {(first + in_group - late * size) * 8 + (int)(blockIdx.x & 7), q_blocks - 1 - late};
+}
+
 // ---------------------------------------------------------------------------
 // Ring variant for sequences too long for the streaming kernel, and for few pairs of one tile: fp16
 // storage, head size 64,
@@ -1003,7 +1017,8 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 // rows of 128 bytes, the swizzles applied on the source side -- and V stays row-major and is read
 // with the transposing LDS load.  A tile is requested three steps before its P.V products.  Two
 // workgroups per CU (198 registers; squeezed into the 168 of three wavefronts per SIMD the kernel
-// spills and is slower).  GPT-2 XL's shape (64 x 25 heads, L = 1024): 0.544 -> 0.489 ms.
+// spills and is slower).  GPT-2 XL's shape (64 x 25 heads, L = 1024): 0.511 ms with the diagonal's forms as
+// branches in the tile loop, 0.464 without, 0.40 with the pairs dealt in groups (deal_blocks).
 //
 // Loads retire in issue order, so "tiles t and t + 1 have landed" is vmcnt(4): the four loads of
 // tile t + 2 are the only younger ones (tile t + 3 is requested behind the barrier that follows
@@ -1016,7 +1031,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 template <bool BLND, bool ACC>
 __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale) {
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group) {
   constexpr int D = 64, KS = 4, DB = 2, NS = 4;
   constexpr int STAGE = 2 * BKEY * D * 2;  // 16 KB: K tile, then V tile
   constexpr int V_AT = BKEY * D * 2;       // byte offset of the V tile inside a stage
@@ -1026,9 +1041,10 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   const int ql = lane & 31, g = lane >> 5;
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
-  const int bh = blockIdx.x;
   const int q_blocks = (L + BQ - 1) / BQ;
-  const int qb = q_blocks - 1 - (int)blockIdx.y;  // heavy (late) query blocks first
+  const WorkItem item = work_item(pairs, q_blocks, group);
+  const int bh = item.bh, qb = item.qb;
+  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1093,11 +1109,10 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   // block 0 cut by the diagonal, block 1 hidden (skipped: its weights are exactly 0); 2: block 0
   // visible, block 1 cut by the diagonal.
   f16v s[2];  // S^T of the tile whose softmax comes next
-  // scores(MODE, stage): S^T = K . Q^T, one block's K fragments at a time (16 registers, not 32)
-  auto scores = [&](auto mode_tag, const char* buf) {
-    constexpr int NKB = decltype(mode_tag)::value == 1 ? 1 : 2;
+  // scores(stage): S^T = K . Q^T, one block's K fragments at a time (16 registers, not 32)
+  auto scores = [&](const char* buf) {
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
+    for (int kb = 0; kb < 2; ++kb) {
       h8 kf[KS];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -1197,50 +1212,57 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   // and the P.V products of tile t run under that softmax) instead of queueing behind the P.V
   // products.  Needs tile t + 1 published one step earlier: four stages, tile t + 3 requested at
   // step t.
+  // The loop holds nothing but entirely visible tiles and no branch: scores and accumulator stay in
+  // their registers from tile to tile (with the diagonal's forms as branches inside it, every tile ended
+  // in 48 moves that waited for its last products).  The diagonal tile's scores are always formed whole.
   const int nfull = qw0 >> 6;  // key tiles entirely below this wavefront's diagonal
-  const int diag_mode = (qw0 & 32) == 0 ? 1 : 2;
   auto stage_of = [&](int t) { return (const char*)smem + (t % NS) * STAGE; };
-  auto scores_of = [&](int t) {  // t <= nfull
-    if (t < nfull) scores(std::integral_constant<int, 0>{}, stage_of(t));
-    else if (diag_mode == 1) scores(std::integral_constant<int, 1>{}, stage_of(t));
-    else scores(std::integral_constant<int, 2>{}, stage_of(t));
+  // Tiles t and t + 1 have landed in this wavefront's part (the four loads of tile t + 2 are the only
+  // younger ones); behind the barrier that holds for every part, and nobody reads tile t - 1 any more.
+  auto arrive = [&](int t) {
+    if (t + 2 < nt) asm volatile("s_waitcnt vmcnt(4)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  auto request = [&](int t) {
+    if (t + 3 < nt) issue_tile(t + 3);
   };
   issue_tile(0);
   if (nt > 1) issue_tile(1);
   if (nt > 2) issue_tile(2);
-  for (int t = 0; t < nt; ++t) {
-    // tiles t and t + 1 have landed in this wavefront's part (the queries too: they are older;
-    // the four loads of tile t + 2 are the only younger ones); behind the barrier that holds for
-    // every part, and nobody reads tile t - 1 any more
-    if (t + 2 < nt) asm volatile("s_waitcnt vmcnt(4)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t == 0) {
-      // the compiler cannot see the wait above; touching the query registers here makes it
-      // place its own wait for them now instead of inside the first tile
+  arrive(0);
+  // the queries landed with it (they are older); the compiler cannot see that wait: touching their registers
+  // on every path in front of the loop makes it place its own here, and not at their uses inside the
+  // loop, where it would wait for all the tiles on their way
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
-    }
-    if (t + 3 < nt) issue_tile(t + 3);
-    if (wave_active && t <= nfull) {
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  request(0);
+  if (wave_active) {
+    scores(stage_of(0));
+    for (int t = 0; t < nfull; ++t) {
       const char* buf = stage_of(t);
-      if (t == 0) scores_of(0);
       read_v(buf, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (t < nfull) {
-        softmax(std::integral_constant<int, 0>{});
-        __builtin_amdgcn_sched_barrier(0);
-        scores_of(t + 1);
-        weighted(std::integral_constant<int, 0>{}, buf);
-      } else if (diag_mode == 1) {
-        softmax(std::integral_constant<int, 1>{});
-        __builtin_amdgcn_sched_barrier(0);
-        weighted(std::integral_constant<int, 1>{}, buf);
-      } else {
-        softmax(std::integral_constant<int, 2>{});
-        __builtin_amdgcn_sched_barrier(0);
-        weighted(std::integral_constant<int, 2>{}, buf);
-      }
+      softmax(std::integral_constant<int, 0>{});
+      __builtin_amdgcn_sched_barrier(0);
+      scores(stage_of(t + 1));
+      weighted(std::integral_constant<int, 0>{}, buf);
+      arrive(t + 1);
+      request(t + 1);
     }
+    const char* buf = stage_of(nfull);
+    read_v(buf, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if ((qw0 & 32) == 0) {
+      softmax(std::integral_constant<int, 1>{});
+      weighted(std::integral_constant<int, 1>{}, buf);
+    } else {
+      softmax(std::integral_constant<int, 2>{});
+      weighted(std::integral_constant<int, 2>{}, buf);
+    }
+  }
+  for (int t = wave_active ? nfull + 1 : 1; t < nt; ++t) {
+    arrive(t);
+    request(t);
   }
 
   // ---- output, as in the streaming kernel: the two lanes of a query trade halves through the
@@ -1303,7 +1325,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
 template <int D, bool BLND, bool ACC>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale) {
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group) {
   static_assert(D == 128 || D == 256, "head sizes 128 and 256");
   constexpr int KS = D / 16, DB = D / 32;
   constexpr int ROWB = D * 2;             // bytes of a row
@@ -1318,9 +1340,10 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
   const int ql = lane & 31, g = lane >> 5;
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
-  const int bh = blockIdx.y;
   const int q_blocks = (L + BQ - 1) / BQ;
-  const int qb = q_blocks - 1 - (int)blockIdx.x;  // heavy (late) query blocks first
+  const WorkItem item = work_item(pairs, q_blocks, group);
+  const int bh = item.bh, qb = item.qb;
+  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1457,24 +1480,33 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
   };
 
   const int nfull = qw0 >> 6;  // key tiles entirely below this wavefront's diagonal
-  issue_tile(0);
-  for (int t = 0; t < nt; ++t) {
-    // tile t has landed in this wavefront's part (the queries too: they are older); behind the
-    // barrier that holds for every part, and nobody reads tile t - 1 any more
+  // tile t has landed in this wavefront's part; behind the barrier that holds for every part, and nobody
+  // reads tile t - 1 any more, whose stage tile t + 1 takes
+  auto arrive = [&](int t) {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t == 0) {
-      // the compiler cannot see the wait above; touching the query registers here makes it
-      // place its own wait for them now instead of inside the first tile
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
-    }
+  };
+  auto request = [&](int t) {
     if (t + 1 < nt) issue_tile(t + 1);
-    if (wave_active && t <= nfull) {
-      const char* buf = smem + (t & 1) * STAGE;
-      if (t < nfull) step(std::integral_constant<int, 0>{}, buf);
-      else if ((qw0 & 32) == 0) step(std::integral_constant<int, 1>{}, buf);
-      else step(std::integral_constant<int, 2>{}, buf);
+  };
+  issue_tile(0);
+  arrive(0);
+  // the queries landed with it: see the ring kernel, also for the loop of visible tiles only
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  request(0);
+  if (wave_active) {
+    for (int t = 0; t < nfull; ++t) {
+      step(std::integral_constant<int, 0>{}, smem + (t & 1) * STAGE);
+      arrive(t + 1);
+      request(t + 1);
     }
+    const char* buf = smem + (nfull & 1) * STAGE;
+    if ((qw0 & 32) == 0) step(std::integral_constant<int, 1>{}, buf);
+    else step(std::integral_constant<int, 2>{}, buf);
+  }
+  for (int t = wave_active ? nfull + 1 : 1; t < nt; ++t) {
+    arrive(t);
+    request(t);
   }
 
   // ---- output, as in the streaming kernel: the two lanes of a query trade halves through the
@@ -1632,12 +1664,32 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   return 0;
 }
 
+// The workgroups for that, and the group.  Some 32 workgroups a group, half of what an XCD holds: their K and V
+// stay in its 4 MB L2 until the last block has read them (all pairs' heaviest blocks first, every block fetches
+// them anew; 64 x 25 pairs of 1024 rows: 445 us, groups of 1, 2, 4, 8, 16 pairs 417, 398, 376, 383, 394;
+// 512 x 6 of 300 rows, d = 128: 308, 229, 231, 226, 224, 233).  Below two rounds of workgroups the order decides
+// when the last one ends, and all heaviest go first (8 x 12 pairs of 1024 rows 25.6 us, groups of 4 26.8).
+// Memory holds at most some 5 million blocks' q, k, v and output.
+inline int deal_blocks(int64_t pairs, int q_blocks, unsigned* grid, int* group) {
+  const int64_t per = (pairs + 7) / 8, all = 8 * per * q_blocks;
+  if (all >= 1 << 24) {
+    set_error("flash_attn: %lld workgroups exceed the grid", (long long)all);
+    return -2;
+  }
+  const int few = (32 + q_blocks - 1) / q_blocks;
+  *group = all < 1024 || per < few ? (int)per : few;
+  *grid = (unsigned)all;
+  return 0;
+}
+
 template <bool BLND, bool ACC = false>
 int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                      int L, float scale, hipStream_t st) {
-  dim3 grid((unsigned)BN, (unsigned)((L + BQ - 1) / BQ));
-  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), grid, dim3(256), 0, st, (const _Float16*)q,
-                     (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale);
+  unsigned grid;
+  int group;
+  if (const int rc = deal_blocks(BN, (L + BQ - 1) / BQ, &grid, &group)) return rc;
+  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(grid), dim3(256), 0, st, (const _Float16*)q,
+                     (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group);
   return 0;
 }
 
@@ -1656,14 +1708,11 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
     }
     attr_done = true;
   }
-  if (BN > 65535) {  // the (batch, head) pairs go to the grid's second dimension
-    set_error("flash_attn: %lld (batch, head) pairs at head size %d: at most 65535",
-              (long long)BN, D);
-    return -2;
-  }
-  dim3 grid((unsigned)((L + BQ - 1) / BQ), (unsigned)BN);
-  hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const _Float16*)q, (const _Float16*)k,
-                     (const _Float16*)v, (_Float16*)out, heads, L, scale);
+  unsigned grid;
+  int group;
+  if (const int rc = deal_blocks(BN, (L + BQ - 1) / BQ, &grid, &group)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, st, (const _Float16*)q, (const _Float16*)k,
+                     (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group);
   return 0;
 }
 
@@ -1705,8 +1754,8 @@ int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
                   : launch_resident<D, T, false>(q, k, v, out, BN, heads, L, scale, lds, st);
     if constexpr (D >= 128 && sizeof(T) == 2) {
       // fp16, head sizes 128 and 256, longer sequences: tiles by direct loads, no staging registers
-      // (pairs in the grid's second dimension; 32-bit byte offsets inside a pair)
-      if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
+      // (32-bit byte offsets inside a pair)
+      if ((int64_t)L * D * 2 < (1ll << 31))
         return blnd ? launch_wide_attn<D, true>(q, k, v, out, BN, heads, L, scale, st)
                     : launch_wide_attn<D, false>(q, k, v, out, BN, heads, L, scale, st);
     }
@@ -1801,7 +1850,7 @@ int launch_operands_d(const void* q, const void* k, const void* v, void* out, in
   } else {
     if (const size_t lds = resident_lds_bytes(L, D))
       return launch_resident<D, T, true, true>(q, k, v, out, BN, heads, L, scale, lds, st);
-    if (BN <= 65535 && (int64_t)L * D * 2 < (1ll << 31))
+    if ((int64_t)L * D * 2 < (1ll << 31))
       return launch_wide_attn<D, true, true>(q, k, v, out, BN, heads, L, scale, st);
     return launch_tiled_as<D, T, true, 0, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
   }

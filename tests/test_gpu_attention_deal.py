@@ -1,0 +1,51 @@
+"""How the (batch, head) pairs and query blocks of the long-sequence attention kernels are dealt to workgroups:
+fewer and more than 1024 of them (one group of pairs per XCD, several), pair counts that are and are not a
+multiple of 8, a last group that is not full, and sequences that end inside a query block.  Every element
+against the textbook attention in fp32, in an output filled with NaN.
+
+Bound: the weights are rounded to fp16 (2^-11 of each, so of sum_j P_j |v_j|), and so is the output; sums
+and the exponential in fp32, 2e-5."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(gpu_device):
+    from gpt_triton_amd import kernels
+    return kernels
+
+
+def excess_over_bound(q, k, v, got):
+    """Largest |got - textbook| beyond the bound."""
+    L, scale = q.shape[2], 1 / math.sqrt(q.shape[3])
+    s = torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * scale
+    mask = torch.ones((L, L), dtype=torch.bool, device=q.device).tril()
+    p = torch.softmax(s.masked_fill(~mask, float("-inf")), dim=-1)
+    want, spread = torch.matmul(p, v.float()), torch.matmul(p, v.float().abs())
+    tol = 2.0**-11 * want.abs() + (2.0**-11 + 2e-5) * spread + 1e-6
+    return float(((got.float() - want).abs() - tol).max())
+
+
+# 64: 3 blocks of queries a pair; 128 and 256 likewise at 300 rows, 2 at 129
+@pytest.mark.parametrize("B,N,L,d", [(1, 5, 330, 64), (1, 8, 513, 64), (7, 48, 330, 64), (1, 343, 330, 64),
+                                     (8, 43, 384, 64), (4, 129, 321, 64), (1, 3, 300, 128), (1, 347, 300, 128),
+                                     (3, 171, 129, 128), (2, 172, 300, 256)])
+def test_every_pair_and_block(K, gpu_device, B, N, L, d):
+    print(f"attention dealt to workgroups: {B * N} pairs, L={L}, d={d}", flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(L + N)
+    q, k, v = (torch.randn(B, N, L, d, generator=g, device=gpu_device).half() for _ in range(3))
+    out = torch.full((B, L, N, d), float("nan"), device=gpu_device, dtype=torch.float16)
+    lib = K._lib.load()
+    rc = lib.gptmi_flash_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, N, L, L, d,
+                              1 / math.sqrt(d), 0.0, 1337, K._lib.GPTMI_O_BLND, K._lib.GPTMI_F16,
+                              torch.cuda.current_stream().cuda_stream)
+    K._lib.check(rc, "flash_attn")
+    got = out.transpose(1, 2)
+    assert not torch.isnan(got).any(), "elements never written"
+    for b in range(B):
+        worst = excess_over_bound(q[b:b + 1], k[b:b + 1], v[b:b + 1], got[b:b + 1])
+        assert worst <= 0, f"beyond the rounding bound by {worst:.3e} in batch {b}"
