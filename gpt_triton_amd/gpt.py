@@ -40,15 +40,18 @@ from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, b
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
 
-# Up to this many token rows a block is one call of the library (attention_block, mlp_block) instead
-# of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one the host
-# sets the pace of an operator-by-operator forward (some 10 us per operator against 2 us per launch
+# Up to this many elements of the residual stream a block is one call of the library (attention_block,
+# mlp_block) instead of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one
+# the host sets the pace of an operator-by-operator forward (some 10 us per operator against 2 us per launch
 # inside one call: 512 rows 926 against 567 us, 2048 rows 910 against 826; 1024-wide 512 rows 1777
-# against 1291).  From there to 24576 rows the two are within 2 %, but for 3 % at 6144 rows of 124M (1708
-# against 1662); the line lies beyond that, where only the memory differs: the operators give each
-# intermediate matrix back before they take the next.  fp32 models take the block calls at every size: their
+# against 1291).  Beyond, what a block passes through fits or nearly fits the 256 MB memory-side cache where
+# every layer writes it to the same places, as the calls do and a caching allocator does not: LayerNorm of 48 x
+# 300 rows 7.8 us instead of 18.6 behind the MLP; operators / blocks, two boxes: 48 x 300 tokens of 124M 3504 /
+# 3386 and 3557 / 3465, 64 x 300 4209 / 4033 and 4230 / 4145, 72 x 300 4429 / 4296; 1024-wide 9 x 1024 8140 / 8004.
+# From 128 x 300 on (7800 / 7788) the two are equal, and the operators, which give each intermediate
+# matrix back before they take the next, stay.  fp32 models take the block calls at every size: their
 # intermediate matrices are fp16 there (see gptmi_attention_block).
-BLOCK_MAX_ROWS = 8192
+BLOCK_MAX_ELEMENTS = 1 << 25
 
 
 def _ln_in_gemm(x, weight):
@@ -59,8 +62,8 @@ def _ln_in_gemm(x, weight):
 
 def _as_block(x, keep=None):
     width = x.shape[-1]
-    return ((keep is not None or x.dtype == torch.float32 or
-             x.numel() // width <= BLOCK_MAX_ROWS) and block_supported(x, width))
+    return ((keep is not None or x.dtype == torch.float32 or x.numel() <= BLOCK_MAX_ELEMENTS) and
+            block_supported(x, width))
 
 
 # dense fp16/bf16 tensor throughput, FLOP/s
