@@ -62,9 +62,10 @@ static LinearPlan plan_linear(int64_t M, int64_t N, int64_t K, int dtype, int wl
   return p;
 }
 
-// Packs operands as the plan says; returns the A and Bt pointers the GEMM reads.
+// Packs operands as the plan says, but for a weight that the product reads in place; returns the A and Bt
+// pointers the GEMM reads.
 static int prepare_operands(const void* x, const void* W, int64_t M, int64_t N, int64_t K,
-                            int dtype, int wlayout, void* workspace, size_t workspace_bytes,
+                            int dtype, int wlayout, bool in_place, void* workspace, size_t workspace_bytes,
                             hipStream_t st, const void** A, const void** Bt, int* Kp) {
   const LinearPlan p = plan_linear(M, N, K, dtype, wlayout);
   if (p.total > 0) {
@@ -80,7 +81,7 @@ static int prepare_operands(const void* x, const void* W, int64_t M, int64_t N, 
   }
   const bool f16 = dtype == GPTMI_F16;
   char* ws = (char*)workspace;
-  if (p.w_bytes) {
+  if (p.w_bytes && !in_place) {
     if (wlayout == GPTMI_W_KN)
       launch_pack_transpose(W, ws + p.w_off, (int)K, (int)N, p.Kp, f16, st);
     else
@@ -133,21 +134,29 @@ static void* static_scratch() {
   return ptrs[dev];
 }
 
-// gptmi_linear and gptmi_linear_static behind their argument checks: pack the operands into
-// `workspace` as the plan says, then the GEMM.
+// The operands as the plan says, packed into `workspace` or as they are, then the GEMM.
+static int product(const char* what, const void* x, const void* W, int64_t M, int64_t N, int64_t K,
+                   const GemmEpilogue& ep, int wlayout, void* workspace, size_t workspace_bytes, int dtype,
+                   hipStream_t st) {
+  const void *A, *Bt;
+  int Kp;
+  const bool in_place = wlayout == GPTMI_W_KN && gemm_reads_kn(W, M, (int)N, (int)K, ep);
+  int rc = prepare_operands(x, W, M, N, K, dtype, wlayout, in_place, workspace, workspace_bytes, st, &A, &Bt, &Kp);
+  if (rc) return rc;
+  if (((uintptr_t)A & 15) || ((uintptr_t)Bt & 15)) {
+    set_error("%s: x and W must be 16-byte aligned", what);
+    return GPTMI_ERR_INVALID;
+  }
+  rc = in_place ? launch_gemm_kn(A, Bt, M, (int)N, Kp, ep, st) : launch_gemm(A, Bt, M, (int)N, Kp, ep, st);
+  if (rc) return rc;
+  return check_launch(what);
+}
+
+// gptmi_linear and gptmi_linear_static behind their argument checks.
 static int linear_impl(const void* x, const void* W, const void* bias, const void* residual,
                        void* out, int64_t M, int64_t N, int64_t K, int gelu, float p,
                        uint64_t seed, int wlayout, void* workspace, size_t workspace_bytes,
                        int dtype, hipStream_t st) {
-  const void *A, *Bt;
-  int Kp;
-  int rc = prepare_operands(x, W, M, N, K, dtype, wlayout, workspace, workspace_bytes, st,
-                            &A, &Bt, &Kp);
-  if (rc) return rc;
-  if (((uintptr_t)A & 15) || ((uintptr_t)Bt & 15)) {
-    set_error("linear: x and W must be 16-byte aligned");
-    return GPTMI_ERR_INVALID;
-  }
   GemmEpilogue ep = {};
   ep.bias = bias;
   ep.residual = residual;
@@ -156,9 +165,7 @@ static int linear_impl(const void* x, const void* W, const void* bias, const voi
   ep.drop = Dropout{p, seed};
   ep.qkv = false;
   ep.f16 = dtype == GPTMI_F16;
-  rc = launch_gemm(A, Bt, M, (int)N, Kp, ep, st);
-  if (rc) return rc;
-  return check_launch("linear");
+  return product("linear", x, W, M, N, K, ep, wlayout, workspace, workspace_bytes, dtype, st);
 }
 
 static int check_linear_args(const void* x, const void* W, const void* out, int64_t M, int64_t N,
@@ -199,21 +206,25 @@ struct Carver {
 };
 
 // The weight images that a block's two products read: the caller's (packed), or built into its workspace.
-// K1 and K2 are multiples of 64.
+// K1 and K2 are multiples of 64.  in_place: both products read the caller's [K][N] weights as they are.
 struct BlockWeights {
   const void *W1, *W2;
   void *ws1, *ws2;
   int K1, N1, K2, N2;
   bool packed, f16;
-  const void* first() const { return packed ? W1 : ws1; }
-  const void* second() const { return packed ? W2 : ws2; }
+  bool in_place = false;
+  const void* first() const { return packed || in_place ? W1 : ws1; }
+  const void* second() const { return packed || in_place ? W2 : ws2; }
+  int multiply(const void* A, const void* B, int64_t M, int N, int K, const GemmEpilogue& ep, hipStream_t st) const {
+    return in_place ? launch_gemm_kn(A, B, M, N, K, ep, st) : launch_gemm(A, B, M, N, K, ep, st);
+  }
   void build(hipStream_t st) const {
-    if (!packed) launch_pack_transpose_pair(W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
+    if (!packed && !in_place) launch_pack_transpose_pair(W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
   }
   // together with the block's LayerNorm, to fp16
   void build_and_normalise(const void* x, const void* ln_w, const void* ln_b, void* normed, int64_t M, int h,
                            float eps, hipStream_t st) const {
-    if (packed) launch_layernorm(x, ln_w, ln_b, normed, M, h, eps, f16, true, st);
+    if (packed || in_place) launch_layernorm(x, ln_w, ln_b, normed, M, h, eps, f16, true, st);
     else
       launch_layernorm_pack_pair(x, ln_w, ln_b, normed, M, h, eps, W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
   }
@@ -481,15 +492,6 @@ int gptmi_linear_qkv(const void* x, const void* W, const void* bias, void* q, vo
     return GPTMI_ERR_UNSUPPORTED;
   }
   hipStream_t st = (hipStream_t)stream;
-  const void *A, *Bt;
-  int Kp;
-  int rc = prepare_operands(x, W, M, N, K, dtype, wlayout, workspace, workspace_bytes, st, &A,
-                            &Bt, &Kp);
-  if (rc) return rc;
-  if (((uintptr_t)A & 15) || ((uintptr_t)Bt & 15)) {
-    set_error("linear_qkv: x and W must be 16-byte aligned");
-    return GPTMI_ERR_INVALID;
-  }
   GemmEpilogue ep = {};
   ep.bias = bias;
   ep.q = q;
@@ -500,9 +502,7 @@ int gptmi_linear_qkv(const void* x, const void* W, const void* bias, void* q, vo
   ep.d = (int)d;
   ep.qkv = true;
   ep.f16 = dtype == GPTMI_F16;
-  rc = launch_gemm(A, Bt, M, (int)N, Kp, ep, st);
-  if (rc) return rc;
-  return check_launch("linear_qkv");
+  return product("linear_qkv", x, W, M, N, K, ep, wlayout, workspace, workspace_bytes, dtype, st);
 }
 
 // Shared argument checks of the two LayerNorm-prologue entry points; K = H.
@@ -648,13 +648,8 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const BlockWeights bw = {W_qkv, W_proj, pl.w_qkv, pl.w_proj, (int)h, (int)(3 * h), (int)h, (int)h,
-                           wlayout == GPTMI_W_PACKED, f16};
-  const void *Bq = bw.first(), *Bp = bw.second();
-  if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
-    set_error("attention_block: the weights must be 16-byte aligned");
-    return GPTMI_ERR_INVALID;
-  }
+  BlockWeights bw = {W_qkv, W_proj, pl.w_qkv, pl.w_proj, (int)h, (int)(3 * h), (int)h, (int)h,
+                     wlayout == GPTMI_W_PACKED, f16};
   GemmEpilogue ep = {};
   ep.bias = b_qkv;
   ep.q = pl.q;
@@ -675,6 +670,20 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     }
     prologue = prologue_aligned(x, ln_w, ln_b);
   }
+  const Dropout drop = {p, seed, keep};
+  GemmEpilogue eo = {};
+  eo.bias = b_proj;
+  eo.residual = x;
+  eo.out = out;
+  eo.drop = drop;
+  eo.f16 = f16;
+  bw.in_place = !bw.packed && !prologue && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep) &&
+                gemm_reads_kn(W_proj, M, (int)h, (int)h, eo);
+  const void *Bq = bw.first(), *Bp = bw.second();
+  if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
+    set_error("attention_block: the weights must be 16-byte aligned");
+    return GPTMI_ERR_INVALID;
+  }
   if (prologue) {
     bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
@@ -687,21 +696,14 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
       if (f16 && ((uintptr_t)normed & 15) == 0) A = normed;
       else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, f16, st);
     }
-    rc = launch_gemm(A, Bq, M, (int)(3 * h), (int)h, ep, st);
+    rc = bw.multiply(A, Bq, M, (int)(3 * h), (int)h, ep, st);
   }
   if (rc) return rc;
-  const Dropout drop = {p, seed, keep};
   const float scale = (float)(1.0 / sqrt((double)d));
   rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
            : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
   if (rc) return rc;
-  GemmEpilogue eo = {};
-  eo.bias = b_proj;
-  eo.residual = x;
-  eo.out = out;
-  eo.drop = drop;
-  eo.f16 = f16;
-  rc = launch_gemm(pl.merged, Bp, M, (int)h, (int)h, eo, st);
+  rc = bw.multiply(pl.merged, Bp, M, (int)h, (int)h, eo, st);
   if (rc) return rc;
   return check_launch("attention_block");
 }
@@ -725,13 +727,8 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   if (rc) return rc;
   const bool f16 = dtype == GPTMI_F16;
   hipStream_t st = (hipStream_t)stream;
-  const BlockWeights bw = {W1, W2, pl.w1, pl.w2, (int)H, (int)inner, (int)inner, (int)H,
-                           wlayout == GPTMI_W_PACKED, f16};
-  const void *B1 = bw.first(), *B2 = bw.second();
-  if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
-    set_error("mlp_block: the weights must be 16-byte aligned");
-    return GPTMI_ERR_INVALID;
-  }
+  BlockWeights bw = {W1, W2, pl.w1, pl.w2, (int)H, (int)inner, (int)inner, (int)H,
+                     wlayout == GPTMI_W_PACKED, f16};
   const Dropout drop = {p, seed, keep};
   GemmEpilogue e1 = {};
   e1.bias = b1;
@@ -749,21 +746,28 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
     }
     prologue = prologue_aligned(x, ln_w, ln_b);
   }
-  if (prologue) {
-    bw.build(st);
-    rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
-  } else {
-    bw.build_and_normalise(x, ln_w, ln_b, pl.normed, M, (int)H, eps, st);
-    rc = launch_gemm(pl.normed, B1, M, (int)inner, (int)H, e1, st);
-  }
-  if (rc) return rc;
   GemmEpilogue e2 = {};
   e2.bias = b2;
   e2.residual = x;
   e2.out = out;
   e2.drop = drop;
   e2.f16 = f16;
-  rc = launch_gemm(pl.inner, B2, M, (int)H, (int)inner, e2, st);
+  bw.in_place = !bw.packed && !prologue && gemm_reads_kn(W1, M, (int)inner, (int)H, e1) &&
+                gemm_reads_kn(W2, M, (int)H, (int)inner, e2);
+  const void *B1 = bw.first(), *B2 = bw.second();
+  if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
+    set_error("mlp_block: the weights must be 16-byte aligned");
+    return GPTMI_ERR_INVALID;
+  }
+  if (prologue) {
+    bw.build(st);
+    rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
+  } else {
+    bw.build_and_normalise(x, ln_w, ln_b, pl.normed, M, (int)H, eps, st);
+    rc = bw.multiply(pl.normed, B1, M, (int)inner, (int)H, e1, st);
+  }
+  if (rc) return rc;
+  rc = bw.multiply(pl.inner, B2, M, (int)H, (int)inner, e2, st);
   if (rc) return rc;
   return check_launch("mlp_block");
 }

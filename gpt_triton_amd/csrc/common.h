@@ -33,6 +33,16 @@ __device__ __forceinline__ void store_through(V* p, V v) {
     asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
 }
 
+// The transposing LDS load: within a block of 16 lanes, lane i receives element i % 4 of the 8 bytes that
+// lanes i / 4, i / 4 + 4, + 8 and + 12 point at -- with lane s pointing at the 4 columns 4 (s % 4).. of row s / 4 of
+// a row-major matrix, column i of 4 rows.
+typedef short s4v __attribute__((__vector_size__(4 * sizeof(short))));
+__device__ __forceinline__ h4 lds_read_tr16(const char* p) {
+  const s4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s4v*)(uintptr_t)p);
+  return __builtin_bit_cast(h4, r);
+}
+
 // Cross-lane steps without the LDS: an xor shuffle compiles to ds_bpermute, ~100 cycles of latency
 // per step of a reduction, and the reductions of a LayerNorm row (twelve steps) or of a softmax tile
 // sit on the critical path of their kernels.  The swaps and row rotations are VALU instructions.

@@ -674,15 +674,6 @@ struct StreamPlan {
   signed char chunk[8][2];  // query chunks (of 32) of wavefront w, -1 = none
 };
 
-typedef short s4v __attribute__((__vector_size__(4 * sizeof(short))));
-
-// four keys x one d (transposed) from a row-major V tile; see the layout note above
-__device__ __forceinline__ h4 lds_read_tr16(const char* p) {
-  const s4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) s4v*)(uintptr_t)p);
-  return __builtin_bit_cast(h4, r);
-}
-
 // 16 bytes per lane from (wavefront-uniform base) + lane_off straight into LDS at lds_off +
 // 16 * lane.  Assembly, so that the compiler's wait-count model never sees an LDS-writing memory
 // operation in flight (it would make every LDS read of the arithmetic wait for the prefetch);

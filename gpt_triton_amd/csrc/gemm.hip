@@ -1217,6 +1217,28 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp, const G
                : launch_shape<float, float, false>(A, Bt, M, N, Kp, ep, st);
 }
 
+// Wherever the tile kernel takes all rows: every size gains (microseconds, weights from HBM, transposed first /
+// in place / packed once: 16 x 768 x 2304 6.7 / 3.9 / 3.4, 16 x 3072 x 768 8.9 / 7.8 / 4.8, 128 x 768 x 3072 10.4 / 5.7
+// / 5.1, 128 x 3072 x 768 12.8 / 8.8 / 6.2, 600 x 768 x 768 8.2 / 5.4 / 5.1, 1477 x 768 x 3072 19.3 / 13.4 / 12.7, 4800 x
+// 3072 x 768 32.5 / 28.2 / 29.2).  Tiles of 16 columns lose most against the image, a line of a row of W
+// being 32 bytes of theirs.
+bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e) {
+  EpiDev ep;
+  int64_t head;
+  if (!e.f16 || K % 64 != 0 || ((uintptr_t)W & 15) != 0 || !gemm_tile_reads_kn(N, K) || make_epi(e, M, N, ep) != 0)
+    return false;
+  if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)
+             : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head)) != 0)
+    return false;
+  return head == 0;
+}
+
+int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const GemmEpilogue& e, hipStream_t st) {
+  EpiDev ep;
+  if (const int rc = make_epi(e, M, N, ep)) return rc;
+  return launch_gemm_tile_kn(A, W, M, N, K, ep, e.qkv, st);
+}
+
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,
                           const void* Bt, int64_t M, int N, int H, const GemmEpilogue& e,
                           hipStream_t st) {

@@ -202,6 +202,10 @@ inline int cu_count() {
 // one); and what the cost model says a launch takes, in microseconds.
 int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                      bool f16, bool out_f16, bool qkv, hipStream_t st);
+// The same on fp16 operands and the weight [K][N] as it stands, 16-byte aligned, where gemm_tile_reads_kn.
+bool gemm_tile_reads_kn(int N, int Kp);
+int launch_gemm_tile_kn(const void* A, const void* W, int64_t M, int N, int K, const EpiDev& ep, bool qkv,
+                        hipStream_t st);
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
                                const LnArgs& ln, bool qkv, bool split, hipStream_t st);
 float gemm_tile_cost(int64_t M, int N, int Kp, int cus);

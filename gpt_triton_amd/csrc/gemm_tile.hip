@@ -119,7 +119,13 @@ struct Tile {
 // T: storage type of bias and residual (fp16 with LNA).  OT: type of the output: T, or fp16 for
 // fp32 storage where the output is the next product's operand (no residual then).
 // WIDE: rows of 2^22 elements and more (64-bit lane addresses).
-template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE>
+//
+// KN: the weight as the caller has it, Bt = W [K][N] in fp16, instead of its packed image: no launch that
+// transposes it first (3.5 us and more, on every call with a weight that is not packed once).  A slice is then
+// 64 rows of BN columns, and a fragment is two transposing LDS loads (ds_read_b64_tr_b16: 4 rows of k x 16
+// columns each) where the image takes one load of 16 bytes; the products, their order and the sums are the
+// same, and so are the bits.
+template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE, bool KN>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     const void* __restrict__ Av, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep, LnArgs ln) {
@@ -157,21 +163,32 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     const int r = s >> 3;
     return (Off)(min(r0 + r, rows - 1) - r0) * (Off)Kp * 2u + (Off)(((s & 7) ^ ((r >> 1) & 7)) * 16);
   };
+  // KN: slot s is row s / UPB of k, position s % UPB, which holds source unit (s % UPB) ^ kn_key(row), 8
+  // columns; columns past the edge re-read the last 8.
+  constexpr int UPB = BN / 8;
+  auto kn_key = [](int r) __attribute__((always_inline)) {
+    return UPB >= 16 ? 2 * ((r & 3) | (r >> 1 & 4)) : UPB == 8 ? 2 * ((r >> 1 & 1) | (r >> 2 & 2))
+                                                   : UPB == 4 ? 2 * (r >> 3 & 1) : 0;
+  };
+  auto kn_off = [&](int s) __attribute__((always_inline)) {
+    const int r = s / UPB, u = (s % UPB) ^ kn_key(r);
+    return ((Off)r * (Off)N + (Off)(min(n0 + 8 * u, N - 8) - n0)) * 2u;
+  };
   Off a_off[A_N], b_off[B_IT];
 #pragma unroll
   for (int it = 0; it < A_IT; ++it) a_off[it] = row_off(m0, M, it * TG + tg);
 #pragma unroll
-  for (int it = 0; it < B_IT; ++it) b_off[it] = row_off(n0, N, it * TG + tg);
+  for (int it = 0; it < B_IT; ++it) b_off[it] = KN ? kn_off(it * TG + tg) : row_off(n0, N, it * TG + tg);
   const int KT = Kp / 64, ST = (KT + WK - 1) / WK;  // k-slices, k-steps
   const char* a_base = (const char*)Av + (size_t)m0 * Kp * 2;
-  const char* b_base = (const char*)(Bt + (size_t)n0 * Kp);
+  const char* b_base = (const char*)(Bt + (KN ? (size_t)n0 : (size_t)n0 * Kp));
   const unsigned wave_off = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem) +
                             (unsigned)g * SLICE + (unsigned)w * 1024u;
   // a group without a slice in the last k-step loads the last slice again and multiplies nothing
   auto issue_one = [&](int t, int stage, int n) __attribute__((always_inline)) {
-    const size_t koff = (size_t)min(t * WK + g, KT - 1) * 128;
+    const size_t slice = (size_t)min(t * WK + g, KT - 1);
     const unsigned at = wave_off + (unsigned)stage * STAGE;
-    const char* base = (n < A_IT ? a_base : b_base) + koff;
+    const char* base = n < A_IT ? a_base + slice * 128 : b_base + slice * (KN ? (size_t)N * 128 : 128);
     const Off off = n < A_IT ? a_off[n < A_IT ? n : 0] : b_off[n < A_IT ? 0 : n - A_IT];
     const unsigned lds = at + (n < A_IT ? n * (TG * 16) : B_AT + (n - A_IT) * (TG * 16));
     if constexpr (WIDE) lds_dma16(base + off, lds);
@@ -203,6 +220,15 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   const int lrow = lane & 15, lq = lane >> 4, fkey = (lrow >> 1) & 7;
   const int a_row = (wm * TM + lrow) * 128, b_row = B_AT + (wn * TN + lrow) * 128;
   const char* panel = smem + NST * STAGE;
+  // KN: of block i, lane s = lane % 16 points at the 4 columns 4 (s % 4).. of row 8 lq + s / 4 of a half slice and
+  // of the row 4 below, and gets column s of the 4 rows each
+  int kn_at[NB];
+  if constexpr (KN) {
+    const int r = 8 * lq + (lrow >> 2);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      kn_at[i] = B_AT + r * (BN * 2) + ((((wn * TN + i * 16) / 8 + ((lrow & 3) >> 1)) ^ kn_key(r)) << 4) + (lrow & 1) * 8;
+  }
   h8 fa[2][MB], fb[2][NB];  // [half slice][block]
   constexpr int NR = MB + NB, NM = MB * NB;  // fragment reads, MFMAs per half slice
   constexpr int RPM = (NR + (NM + 1) / 2 - 1) / ((NM + 1) / 2);  // reads behind an MFMA: all behind the first half of them
@@ -212,6 +238,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
     if (n < MB) {
       const char* sa = LNA ? panel + (size_t)min(t * WK + g, KT - 1) * (BM * 128) : st;
       fa[half][n < MB ? n : 0] = *reinterpret_cast<const h8*>(sa + a_row + n * 2048 + un);
+    } else if constexpr (KN) {
+      const char* at = st + kn_at[n < MB ? 0 : n - MB] + half * (32 * BN * 2);
+      const h4 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * (BN * 2));
+      fb[half][n < MB ? 0 : n - MB] = h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     } else {
       fb[half][n < MB ? 0 : n - MB] = *reinterpret_cast<const h8*>(st + b_row + (n - MB) * 2048 + un);
     }
@@ -425,10 +455,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   }
 }
 
-template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE = false>
+template <class C, typename T, typename OT, bool QKV, bool LNA, bool DROP, bool WIDE = false, bool KN = false>
 int launch_tile_cfg(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                     const LnArgs& ln, hipStream_t st) {
-  auto kern = gemm_tile_kernel<C, T, OT, QKV, LNA, DROP, WIDE>;
+  auto kern = gemm_tile_kernel<C, T, OT, QKV, LNA, DROP, WIDE, KN>;
   constexpr int stages = C::NST * ((LNA ? 0 : C::BM) + C::BN) * 128 * C::WK, sums = C::BM * C::BN * 4 * C::WK;
   static_assert(stages <= 160 * 1024 && sums <= 160 * 1024, "LDS");
   const size_t panel = LNA ? (size_t)C::BM * Kp * 2 : 0;
@@ -521,24 +551,24 @@ inline int pick_tile(int64_t M, int N, int Kp, int cus, float* cost) {
   return best;
 }
 
-template <typename T, typename OT, bool QKV, bool DROP>
+template <typename T, typename OT, bool QKV, bool DROP, bool KN>
 int launch_pick(int i, const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                 hipStream_t st) {
   const LnArgs ln = {};
   switch (i) {
-    case 0: return launch_tile_cfg<T32x16, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 1: return launch_tile_cfg<T32x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 2: return launch_tile_cfg<T64x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 3: return launch_tile_cfg<T64x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 4: return launch_tile_cfg<T64x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 5: return launch_tile_cfg<T128x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 6: return launch_tile_cfg<T192x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 7: return launch_tile_cfg<T128x256, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 8: return launch_tile_cfg<T16x16, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 9: return launch_tile_cfg<T48x32, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 10: return launch_tile_cfg<T96x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    case 11: return launch_tile_cfg<T192x64, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
-    default: return launch_tile_cfg<T256x128, T, OT, QKV, false, DROP>(A, Bt, M, N, Kp, ep, ln, st);
+    case 0: return launch_tile_cfg<T32x16, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 1: return launch_tile_cfg<T32x32, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 2: return launch_tile_cfg<T64x32, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 3: return launch_tile_cfg<T64x64, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 4: return launch_tile_cfg<T64x128, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 5: return launch_tile_cfg<T128x128, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 6: return launch_tile_cfg<T192x128, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 7: return launch_tile_cfg<T128x256, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 8: return launch_tile_cfg<T16x16, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 9: return launch_tile_cfg<T48x32, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 10: return launch_tile_cfg<T96x64, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    case 11: return launch_tile_cfg<T192x64, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
+    default: return launch_tile_cfg<T256x128, T, OT, QKV, false, DROP, false, KN>(A, Bt, M, N, Kp, ep, ln, st);
   }
 }
 
@@ -553,21 +583,31 @@ float gemm_tile_cost(int64_t M, int N, int Kp, int cus) {
   return cost;
 }
 
-template <typename T, typename OT, bool QKV>
+template <typename T, typename OT, bool QKV, bool KN = false>
 static int launch_tile_t(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                          hipStream_t st) {
   const int cus = cu_count();
   if (cus < 0) return cus;
   if constexpr (!QKV) {
     if (ep.drop.p > 0.f) {
-      if (Kp >= kWideK)
-        return launch_tile_cfg<T32x32, T, OT, false, false, true, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
-      return launch_pick<T, OT, false, true>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+      if constexpr (!KN)
+        if (Kp >= kWideK)
+          return launch_tile_cfg<T32x32, T, OT, false, false, true, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+      return launch_pick<T, OT, false, true, KN>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
     }
   }
-  if (Kp >= kWideK)
-    return launch_tile_cfg<T32x32, T, OT, QKV, false, false, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
-  return launch_pick<T, OT, QKV, false>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+  if constexpr (!KN)
+    if (Kp >= kWideK)
+      return launch_tile_cfg<T32x32, T, OT, QKV, false, false, true>(A, Bt, M, N, Kp, ep, LnArgs{}, st);
+  return launch_pick<T, OT, QKV, false, KN>(pick_tile(M, N, Kp, cus, nullptr), A, Bt, M, N, Kp, ep, st);
+}
+
+bool gemm_tile_reads_kn(int N, int Kp) { return N % 8 == 0 && N <= 1 << 22 && Kp < kWideK; }
+
+int launch_gemm_tile_kn(const void* A, const void* W, int64_t M, int N, int K, const EpiDev& ep, bool qkv,
+                        hipStream_t st) {
+  return qkv ? launch_tile_t<_Float16, _Float16, true, true>(A, W, M, N, K, ep, st)
+             : launch_tile_t<_Float16, _Float16, false, true>(A, W, M, N, K, ep, st);
 }
 
 int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,

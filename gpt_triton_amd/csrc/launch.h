@@ -64,6 +64,11 @@ struct GemmEpilogue {
 int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp,
                 const GemmEpilogue& ep, hipStream_t st);
 
+// The same product, fp16 storage, with the weight as the caller has it, W [K][N]: no packed image.  Same kernels,
+// same division of the rows, same bits.  gemm_reads_kn says where that is taken (and is the faster way).
+bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& ep);
+int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const GemmEpilogue& ep, hipStream_t st);
+
 // The same product with A = LayerNorm(x; ln_w, ln_b, eps), x [M][H] fp16 with H = K a multiple
 // of 64: every workgroup normalises the rows of its tile in its operand prologue (the bits of
 // launch_layernorm's output) and the normalised matrix never goes to memory.  fp16, no residual,

@@ -1,0 +1,73 @@
+"""Products that read a [K, N] weight as it stands: the kernels, the division of the rows and the order of the
+sums are those of the packed image, so every result is compared with the packed weight's bit for bit (which
+other tests hold against the oracle).  Rows either side of what the tile shapes take, columns that end inside a
+tile, 8 columns in all, one k-slice and several that the groups of a workgroup do not share evenly."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(gpu_device):
+    from gpt_triton_amd import kernels
+    return kernels
+
+
+def weights(device, k, n, seed):
+    g = torch.Generator(device=device).manual_seed(seed)
+    draw = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=device) * std).half()
+    return draw, draw(k, n, std=k**-0.5), draw(n)
+
+
+SHAPES = [(1, 64, 8), (1, 768, 768), (16, 3072, 768), (17, 320, 776), (33, 768, 2304), (64, 192, 72),
+          (100, 1024, 1000), (128, 768, 3072), (300, 448, 520), (511, 768, 768), (777, 1024, 1032),
+          (1477, 768, 3072), (1477, 3072, 768), (2400, 1280, 1288), (3001, 768, 768), (4800, 3072, 768),
+          (5000, 64, 264), (4800, 768, 3072), (3885, 1024, 4096), (8193, 128, 512), (9600, 768, 2304)]
+
+
+@pytest.mark.parametrize("M,k,n", SHAPES)
+def test_bits_of_the_packed_weight(K, gpu_device, M, k, n):
+    print(f"weight in place: {M} x {k} x {n}", flush=True)
+    draw, w, b = weights(gpu_device, k, n, M)
+    x, r = draw(M, k), draw(M, n)
+    image = K.pack_weight(w)
+    for bias, res, gelu in ((None, None, False), (b, None, True), (b, r, False)):
+        plain = K.fused_ffn(x, w, bias=bias, residual=res, add_gelu=gelu)
+        packed = K.fused_ffn(x, image, bias=bias, residual=res, add_gelu=gelu)
+        assert torch.isfinite(plain).all() and torch.equal(plain, packed), (bias is not None, res is not None, gelu)
+    shifted = torch.empty(k * n + 4, device=gpu_device, dtype=torch.float16)[4:].view(k, n)  # 8-byte aligned: packed
+    shifted.copy_(w)
+    assert torch.equal(K.fused_ffn(x, shifted, bias=b), K.fused_ffn(x, image, bias=b))
+
+
+@pytest.mark.parametrize("B,L,heads,d", [(1, 5, 2, 8), (2, 64, 12, 64), (3, 333, 5, 32), (7, 211, 12, 64), (16, 300, 12, 64),
+                                         (5, 777, 8, 128), (9, 1000, 6, 128)])
+def test_head_major_scatter(K, gpu_device, B, L, heads, d):
+    k = 64 * max(1, heads * d // 64)
+    print(f"weight in place, q, k, v of {heads} x {d}: {B} x {L} rows of {k}", flush=True)
+    draw, w, b = weights(gpu_device, k, 3 * heads * d, L)
+    x = draw(B, L, k)
+    for got, want in zip(K.matmul_and_split_qkv(x, w, b, heads),
+                         K.matmul_and_split_qkv(x, K.pack_weight(w), b, heads)):
+        assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,L,h,heads", [(1, 24, 128, 2), (2, 300, 768, 12), (16, 300, 768, 12), (3, 999, 1024, 16),
+                                         (56, 300, 768, 12)])
+def test_training_blocks(K, gpu_device, B, L, h, heads):
+    """Dropout with its mask at hand and drawn in place, both blocks, weights plain and packed."""
+    print(f"weight in place, training blocks: {B} x {L} rows of {h}", flush=True)
+    draw, wq, bq = weights(gpu_device, h, 3 * h, B)
+    _, wp, bp = weights(gpu_device, h, h, B + 1)
+    _, w1, b1 = weights(gpu_device, h, 4 * h, B + 2)
+    _, w2, b2 = weights(gpu_device, 4 * h, h, B + 3)
+    x, lw, lb = draw(B, L, h), draw(h), draw(h)
+    masks = (None, K.dropout_mask(B * L * 4 * h, 0.1, x)) if B * L < 2000 else (K.dropout_mask(B * L * 4 * h, 0.1, x),)
+    for keep in masks:
+        for call, ws in ((K.attention_block, (wq, bq, wp, bp)), (K.mlp_block, (w1, b1, w2, b2))):
+            images = [K.pack_weight(t) if t.dim() == 2 else t for t in ws]
+            more = (heads,) if call is K.attention_block else ()
+            plain = call(x, lw, lb, *ws, *more, dropout_prob=0.1, keep=keep)
+            packed = call(x, lw, lb, *images, *more, dropout_prob=0.1, keep=keep)
+            assert torch.isfinite(plain).all() and torch.equal(plain, packed)
