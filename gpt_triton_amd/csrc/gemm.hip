@@ -378,8 +378,36 @@ __device__ __forceinline__ void store_wave_tile32(f4 (&acc)[2 * NB][2 * MB], con
   }
 }
 
+// The weight half of a k-tile where the weight is read as the caller has it, W [K][N] in fp16 with N a multiple of
+// 256, instead of from its packed image: 64 rows of k x 256 columns.  16-byte unit u of row r lies at u ^
+// key(r), key = 2 (r & 3) + 8 (r >> 3 & 1), so that the 16 rows which a transposing load takes 32 bytes each of
+// cover all banks twice, the least for its 512 bytes.  Load n of a thread: row 16 n + tid / 32, which has the
+// key of row tid / 32.  A fragment is two transposing loads, k = 32 s + 8 (lane / 16) + 0..3 and 4..7 of columns
+// 16 i + lane % 16 of the wavefront's 64: the k of a lane, and so the products' order and bits, are the image's.
+// 4800 x 768 x 2304: transposed first 26.9 us, in place 21.7, packed once 20.9.  (In gemm_stream_res_kernel, which
+// has no register left, the two loads of a fragment spill.)
+struct KnTile {
+  unsigned lane_off;
+  int N, at;
+  __device__ __forceinline__ KnTile(int tid, int lane, int wn, int n) : N(n) {
+    auto key = [](int r) { return 2 * (r & 3) + (r & 8); };
+    const int r = tid >> 5, lrow = lane & 15, kr = 8 * (lane >> 4) + (lrow >> 2);
+    lane_off = (unsigned)r * (unsigned)n * 2u + (unsigned)(((tid & 31) ^ key(r)) << 4);
+    at = kr * 512 + (((8 * wn + ((lrow & 3) >> 1)) ^ key(kr)) << 4) + (lrow & 1) * 8;
+  }
+  __device__ __forceinline__ const char* src(const _Float16* W, int n0, int k, int n) const {
+    return (const char*)W + ((size_t)(64 * k + 16 * n) * N + n0) * 2;
+  }
+  __device__ __forceinline__ h8 fragment(const char* tile, int i, int s) const {
+    const char* p = tile + (at ^ (i * 32)) + s * (32 * 512);  // bits 5 and 6 of `at` are the unit's
+    const h4 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 4 * 512);
+    return h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  }
+};
+
 // T: type of the bias.  OT: type of the output (fp16, or T).  DROP: fp16 output, plain, the mask at hand.
-template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP>
+// KN: Bt is the weight [K][N] itself, N a multiple of 256 (see KnTile).
+template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP, bool KN>
 __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const _Float16* __restrict__ A, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep) {
@@ -435,7 +463,9 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
   // block 0 again (the shift goes into the scalar source, the lane offsets stay); its products
   // are never stored.
   const size_t blk_bytes = (size_t)64 * Kp * 2;
+  const KnTile kn(tid, lane, wn, N);
   auto b_src = [&](int n0, int k, int n) __attribute__((always_inline)) {
+    if constexpr (KN) return kn.src(Bt, n0, k, n);
     const int vb = (N - n0) >> 6;  // valid blocks of this tile (4 or more: all)
     const char* p = (const char*)Bt + ((size_t)n0 * Kp * 2 + (size_t)k * ROWB);
     return n < vb ? p : p - n * blk_bytes;
@@ -444,7 +474,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     lds_dma16_base(src, lane_off[n], wave_off + stage * STAGE + n * T_ * 16);
   };
   auto issue_b = [&](int stage, const char* src, int n) __attribute__((always_inline)) {
-    lds_dma16_base(src, lane_off[n], wave_off + stage * STAGE + BM * ROWB + n * T_ * 16);
+    lds_dma16_base(src, KN ? kn.lane_off : lane_off[n], wave_off + stage * STAGE + BM * ROWB + n * T_ * 16);
   };
   auto issue = [&](int stage, int m0, int n0, int k) __attribute__((always_inline)) {
     const char* a = a_src(m0, k);
@@ -472,6 +502,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
                                         (((s * 4 + lq) ^ fkey) << 4));
   };
   auto frag_b = [&](const char* st, int i, int s) __attribute__((always_inline)) {
+    if constexpr (KN) return kn.fragment(st + BM * ROWB, i, s);
     return *reinterpret_cast<const h8*>(st + b_row_off + i * 16 * ROWB +
                                         (((s * 4 + lq) ^ fkey) << 4));
   };
@@ -985,10 +1016,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
   }
 }
 
-template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP = false>
+template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP = false, bool KN = false>
 int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                   hipStream_t st) {
-  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV, DROP>;
+  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV, DROP, KN>;
   constexpr int smem = 2 * 512 * 128 + 8 * 4096;  // 160 KB: two stages + the epilogue slabs
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -1114,7 +1145,7 @@ EpiDev tail_epi(const EpiDev& ep, int64_t head, int N) {
   return tail;
 }
 
-template <typename T, typename OT, bool QKV>
+template <typename T, typename OT, bool QKV, bool KN = false>
 int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                  hipStream_t st) {
   const bool res = !QKV && ep.residual != nullptr;
@@ -1126,16 +1157,19 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
       if (ep.drop.p > 0.f) {  // m_head == M
         if constexpr (sizeof(T) == 2)
           if (res) return launch_stream_res<true>(A, Bt, M, N, Kp, ep, st);
-        return launch_stream<2, 4, T, OT, QKV, true>(A, Bt, M, N, Kp, ep, st);
+        return launch_stream<2, 4, T, OT, QKV, true, KN>(A, Bt, M, N, Kp, ep, st);
       }
     }
     if constexpr (sizeof(T) == 2 && !QKV)
       rc = res ? launch_stream_res<false>(A, Bt, m_head, N, Kp, ep, st)
-               : launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
+               : launch_stream<2, 4, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
     else
-      rc = launch_stream<2, 4, T, OT, QKV>(A, Bt, m_head, N, Kp, ep, st);
+      rc = launch_stream<2, 4, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
     if (rc != 0 || m_head == M) return rc;
   }
+  if constexpr (KN)
+    return launch_gemm_tile_kn((const _Float16*)A + m_head * Kp, Bt, M - m_head, N, Kp,
+                               tail_epi<T, OT, QKV>(ep, m_head, N), QKV, st);
   return launch_gemm_tile((const _Float16*)A + m_head * Kp, Bt, M - m_head, N, Kp,
                           tail_epi<T, OT, QKV>(ep, m_head, N), sizeof(T) == 2, sizeof(OT) == 2, QKV, st);
 }
@@ -1221,7 +1255,9 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp, const G
 // in place / packed once: 16 x 768 x 2304 6.7 / 3.9 / 3.4, 16 x 3072 x 768 8.9 / 7.8 / 4.8, 128 x 768 x 3072 10.4 / 5.7
 // / 5.1, 128 x 3072 x 768 12.8 / 8.8 / 6.2, 600 x 768 x 768 8.2 / 5.4 / 5.1, 1477 x 768 x 3072 19.3 / 13.4 / 12.7, 4800 x
 // 3072 x 768 32.5 / 28.2 / 29.2).  Tiles of 16 columns lose most against the image, a line of a row of W
-// being 32 bytes of theirs.
+// being 32 bytes of theirs.  In the persistent kernel without a residual, whole column tiles, up to the rows at which
+// the 1 to 2 % that it takes longer are what the transposition takes (4800 x 768 x 3072 31.4 / 26.2 / 24.8, 9600 x 768 x
+// 3072 54.7 / 49.2 / 48.5, 40000 x 768 x 3072 203 / 202 / 198).
 bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e) {
   EpiDev ep;
   int64_t head;
@@ -1230,13 +1266,14 @@ bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e
   if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)
              : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head)) != 0)
     return false;
-  return head == 0;
+  return head == 0 || (N % 256 == 0 && e.residual == nullptr && M <= 32768);
 }
 
 int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const GemmEpilogue& e, hipStream_t st) {
   EpiDev ep;
   if (const int rc = make_epi(e, M, N, ep)) return rc;
-  return launch_gemm_tile_kn(A, W, M, N, K, ep, e.qkv, st);
+  return e.qkv ? launch_shape<_Float16, _Float16, true, true>(A, W, M, N, K, ep, st)
+               : launch_shape<_Float16, _Float16, false, true>(A, W, M, N, K, ep, st);
 }
 
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,
