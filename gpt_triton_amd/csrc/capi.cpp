@@ -684,7 +684,15 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     set_error("attention_block: the weights must be 16-byte aligned");
     return GPTMI_ERR_INVALID;
   }
-  if (prologue) {
+  const float scale = (float)(1.0 / sqrt((double)d));
+  // short sequences: everything in front of the projection in one launch
+  const void* rows = normed ? normed : x;
+  const bool front = f16 && bw.packed && p == 0.f && d == 64 && attn_front_supported(B, L, heads, h) &&
+                     gemm_layernorm_supported(M, (int)h) && prologue_aligned(rows, ln_w, ln_b) &&
+                     ((uintptr_t)b_qkv & 15) == 0;
+  if (front) {
+    rc = launch_attn_front(rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st);
+  } else if (prologue) {
     bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
   } else {
@@ -699,10 +707,11 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
     rc = bw.multiply(A, Bq, M, (int)(3 * h), (int)h, ep, st);
   }
   if (rc) return rc;
-  const float scale = (float)(1.0 / sqrt((double)d));
-  rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
-           : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
-  if (rc) return rc;
+  if (!front) {
+    rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
+             : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
+    if (rc) return rc;
+  }
   rc = bw.multiply(pl.merged, Bp, M, (int)h, (int)h, eo, st);
   if (rc) return rc;
   return check_launch("attention_block");

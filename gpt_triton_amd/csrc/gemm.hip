@@ -1276,6 +1276,20 @@ int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const 
                : launch_shape<_Float16, _Float16, false, true>(A, W, M, N, K, ep, st);
 }
 
+int gemm_qkv_split(int64_t M, int N, int K, int64_t L, int heads, int d) {
+  const int cus = cu_count();
+  if (cus < 0) return cus;
+  GemmEpilogue e = {};
+  e.L = L, e.heads = heads, e.d = d;
+  e.qkv = e.f16 = true;
+  EpiDev ep;
+  int64_t head;
+  if (const int rc = make_epi(e, M, N, ep)) return rc;
+  if (const int rc = persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)) return rc;
+  if (head > 0) return head == M ? 1 : 0;
+  return gemm_tile_split(M, N, K, cus);
+}
+
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,
                           const void* Bt, int64_t M, int N, int H, const GemmEpilogue& e,
                           hipStream_t st) {

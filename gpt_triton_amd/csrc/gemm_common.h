@@ -209,5 +209,9 @@ int launch_gemm_tile_kn(const void* A, const void* W, int64_t M, int N, int K, c
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
                                const LnArgs& ln, bool qkv, bool split, hipStream_t st);
 float gemm_tile_cost(int64_t M, int N, int Kp, int cus);
+// Over how many groups launch_gemm divides K for M rows of a q, k, v product in fp16, the order of its sums; 0: not
+// the same for all rows; negative: an error.
+int gemm_qkv_split(int64_t M, int N, int K, int64_t L, int heads, int d);
+int gemm_tile_split(int64_t M, int N, int Kp, int cus);
 
 }  // namespace gptmi

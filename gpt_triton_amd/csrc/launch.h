@@ -79,6 +79,13 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
                           const void* Bt, int64_t M, int N, int H, const GemmEpilogue& ep,
                           hipStream_t st);
 
+// LayerNorm (unless x is normed), q, k, v product (packed weight image Bt [3h][h]) and causal attention of short
+// sequences in one launch: fp16, head size 64, out [B][L][heads][64], the bits of the launches it stands for.  All
+// pointers 16-byte aligned.
+bool attn_front_supported(int64_t B, int64_t L, int64_t heads, int64_t h);
+int launch_attn_front(const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
+                      const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st);
+
 // q, out: L rows per (batch, head); k, v: Lk rows.
 int launch_flash_attn(const void* q, const void* k, const void* v, void* out,
                       int64_t B, int64_t N, int64_t L, int64_t Lk, int d, float scale,
