@@ -33,7 +33,7 @@ constexpr int ROWS = 32, NST = 4, kSliceBytes = 192 * 128;
 template <int WK, bool NORMED>
 __global__ __launch_bounds__(512, 2) void attn_front_kernel(
     const _Float16* __restrict__ x, const _Float16* __restrict__ Bt, const _Float16* __restrict__ bias,
-    _Float16* __restrict__ out, int B, int heads, int L, int H, float scale, LnArgs ln) {
+    _Float16* __restrict__ out, int B, int heads, int L, int H, float scale, LnArgs ln, PrefetchArgs ahead) {
   constexpr int NB = 3, LPT = 3;  // a wavefront: 16 rows x 48 columns; its loads of a slice
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   char* panel = smem + NST * kSliceBytes;
@@ -42,6 +42,10 @@ __global__ __launch_bounds__(512, 2) void attn_front_kernel(
   const int wm = wave & 1, wn = wave >> 1;
   const int lrow = lane & 15, lq = lane >> 4;
 
+  if ((int)blockIdx.x >= B * heads) {
+    prefetch_lines<512>(ahead, (int)blockIdx.x - B * heads, (int)gridDim.x - B * heads);
+    return;
+  }
   // the sequences of a head on one XCD, whose L2 holds the head's weights
   const int item = xcd_tile(blockIdx.x, B * heads);
   const int head = item / B, b = item - head * B;
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(512, 2) void attn_front_kernel(
 
 template <int WK, bool NORMED>
 int launch_front(const void* x, const void* Bt, const void* bias, void* out, int64_t B, int heads, int L, int H,
-                 float scale, const LnArgs& ln, hipStream_t st) {
+                 float scale, const LnArgs& ln, hipStream_t st, const Prefetch* ahead) {
   auto kern = attn_front_kernel<WK, NORMED>;
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -239,8 +243,10 @@ int launch_front(const void* x, const void* Bt, const void* bias, void* out, int
     attr_done = true;
   }
   const size_t lds = (size_t)NST * kSliceBytes + (size_t)ROWS * H * 2;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(B * heads)), dim3(512), lds, st, (const _Float16*)x, (const _Float16*)Bt,
-                     (const _Float16*)bias, (_Float16*)out, (int)B, heads, L, H, scale, ln);
+  const int workers = (int)(B * heads), cus = cu_count();
+  hipLaunchKernelGGL(kern, dim3((unsigned)(workers + prefetch_workgroups(ahead, workers, cus))), dim3(512), lds, st, (const _Float16*)x, (const _Float16*)Bt,
+                     (const _Float16*)bias, (_Float16*)out, (int)B, heads, L, H, scale, ln,
+                     prefetch_args(ahead));
   return 0;
 }
 
@@ -253,11 +259,12 @@ bool attn_front_supported(int64_t B, int64_t L, int64_t heads, int64_t h) {
 }
 
 int launch_attn_front(const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
-                      const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st) {
+                      const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st,
+                      const Prefetch* ahead) {
   const int H = (int)heads * 64;
   const LnArgs ln = {ln_w, ln_b, eps, lanes_per_row(H / 8)};
   const int wk = gemm_qkv_split(B * L, 3 * H, H, L, (int)heads, 64);
-  const auto go = [&](auto kernel) { return kernel(x, Bt, bias, out, B, (int)heads, (int)L, H, scale, ln, st); };
+  const auto go = [&](auto kernel) { return kernel(x, Bt, bias, out, B, (int)heads, (int)L, H, scale, ln, st, ahead); };
   switch (wk) {
     case 4: return normed ? go(launch_front<4, true>) : go(launch_front<4, false>);
     case 2: return normed ? go(launch_front<2, true>) : go(launch_front<2, false>);

@@ -626,11 +626,11 @@ size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads
   return plan_attention(nullptr, B * L, heads * d, wlayout).total;
 }
 
-int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
+static int attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
                           const void* W_qkv, const void* b_qkv, const void* W_proj, const void* b_proj,
                           void* out, int64_t B, int64_t L, int64_t heads, int64_t d, float p,
                           uint64_t seed, const void* keep, int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace,
-                          size_t workspace_bytes, int dtype, void* stream) {
+                          size_t workspace_bytes, int dtype, void* stream, const Prefetch* ahead) {
   if (!x || !ln_w || !ln_b || !W_qkv || !W_proj || !out || B <= 0 || L <= 0 || heads <= 0 || d <= 0) {
     set_error("attention_block: invalid argument");
     return GPTMI_ERR_INVALID;
@@ -691,7 +691,7 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
                      gemm_layernorm_supported(M, (int)h) && prologue_aligned(rows, ln_w, ln_b) &&
                      ((uintptr_t)b_qkv & 15) == 0;
   if (front) {
-    rc = launch_attn_front(rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st);
+    rc = launch_attn_front(rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st, ahead);
   } else if (prologue) {
     bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
@@ -708,13 +708,22 @@ int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, c
   }
   if (rc) return rc;
   if (!front) {
-    rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st)
-             : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st);
+    rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st, ahead)
+             : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st, ahead);
     if (rc) return rc;
   }
   rc = bw.multiply(pl.merged, Bp, M, (int)h, (int)h, eo, st);
   if (rc) return rc;
   return check_launch("attention_block");
+}
+
+int gptmi_attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
+                          const void* W_qkv, const void* b_qkv, const void* W_proj, const void* b_proj,
+                          void* out, int64_t B, int64_t L, int64_t heads, int64_t d, float p, uint64_t seed,
+                          const void* keep, int64_t keep_bits, int fuse_layernorm, int wlayout,
+                          void* workspace, size_t workspace_bytes, int dtype, void* stream) {
+  return attention_block(x, normed, ln_w, ln_b, eps, W_qkv, b_qkv, W_proj, b_proj, out, B, L, heads, d, p, seed,
+                         keep, keep_bits, fuse_layernorm, wlayout, workspace, workspace_bytes, dtype, stream, nullptr);
 }
 
 size_t gptmi_mlp_block_workspace_bytes(int64_t M, int64_t H, int64_t inner, int wlayout) {
@@ -817,6 +826,32 @@ size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t
   return 2 * (size_t)round_up(M * h * (dtype == GPTMI_F16 ? 2 : 4), 256) + (a > m ? a : m);
 }
 
+// What an attention launch of few workgroups requests of the weights that come behind it.  Its other CUs bring in
+// some 15 MB while it lasts, and 40 KB more for each of its key rows; weights beyond that make it last longer than
+// they save, and half a matrix saves nothing.  The MLP's second product first, which has the longest columns, in any
+// case; then the next layer's first product, then what follows at once.  Forwards that find their weights in HBM (four
+// models in turn; wider ones always do), us, without / this: 124M 1 x 24 tokens with logits 356 -> 315, 2 x 64 366 -> 353, 8 x 24
+// 422 -> 360, 7 x 211 738 -> 686, 1 x 800 705 -> 640; 1024 wide 4 x 64 969 -> 905, 2 x 300 1367 -> 1266; 1280 wide 1 x 50 1316 ->
+// 1290 (all four weights 1390), 2 x 200 2350 -> 2241; 1600 wide 1 x 50 2058 -> 2038 (all four 2215), 1 x 300 3359 -> 3182.
+// One 124M model over and over, whose weights the memory-side cache holds: equal.
+static Prefetch weights_ahead(const void* const* layer, bool last, int64_t h, int64_t inner, int64_t L) {
+  const size_t square = (size_t)(h * h * 2), wide = (size_t)(h * inner * 2);
+  const struct {
+    const void* p;
+    size_t bytes;
+  } wanted[4] = {{layer[10], wide}, {last ? nullptr : layer[12 + 2], 3 * square}, {layer[8], wide}, {layer[4], square}};
+  const size_t most = 15000000 + 40000 * (size_t)L;
+  Prefetch ahead;
+  size_t sum = 0;
+  for (int k = 0; k < 4; ++k) {
+    if (wanted[k].p == nullptr) continue;
+    sum += wanted[k].bytes;
+    if (k > 0 && sum > most) break;
+    ahead.p[k] = wanted[k].p, ahead.bytes[k] = wanted[k].bytes;
+  }
+  return ahead;
+}
+
 int gptmi_blocks(const void* x, const void* normed, const void* const* params, int64_t n, float eps,
                  void* out, int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner,
                  int fuse_layernorm, void* workspace, size_t workspace_bytes, int dtype, void* stream) {
@@ -840,9 +875,9 @@ int gptmi_blocks(const void* x, const void* normed, const void* const* params, i
   const size_t ws_bytes = workspace_bytes - c.used;
   for (int64_t i = 0; i < n; ++i) {
     const void* const* p = params + 12 * i;
-    int rc = gptmi_attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B,
-                                   L, heads, d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws,
-                                   ws_bytes, dtype, stream);
+    const Prefetch ahead = weights_ahead(p, i + 1 == n, h, inner, L);
+    int rc = attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B, L, heads,
+                             d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream, &ahead);
     if (rc) return rc;
     // x is not read again: the layer's output may take its place
     void* y = i + 1 == n ? out : next;

@@ -4,6 +4,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include "launch.h"
+
 namespace gptmi {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -41,6 +43,32 @@ __device__ __forceinline__ h4 lds_read_tr16(const char* p) {
   const s4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) s4v*)(uintptr_t)p);
   return __builtin_bit_cast(h4, r);
+}
+
+// Lines of memory that later launches read, requested by workgroups of a launch that leaves CUs idle (see
+// launch.h): a word of each 128-byte line, spread over `blocks` workgroups of NT threads.
+struct PrefetchArgs {
+  const void* p[4];
+  unsigned lines[4];
+};
+inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
+  PrefetchArgs a = {};
+  for (int k = 0; ahead && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
+  return a;
+}
+// Workgroups for it: the CUs that a launch of `workers` leaves idle, if they are 64 or more.
+inline int prefetch_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
+  return ahead != nullptr && workers <= cus - 64 ? cus - (int)workers : 0;
+}
+template <int NT>
+__device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int block, int blocks) {
+  unsigned sink = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll 4
+    for (unsigned i = block * NT + threadIdx.x; i < pf.lines[k]; i += blocks * NT)
+      sink ^= *reinterpret_cast<const unsigned*>((const char*)pf.p[k] + (size_t)i * 128);
+  asm volatile("" : : "v"(sink));
 }
 
 // Cross-lane steps without the LDS: an xor shuffle compiles to ds_bpermute, ~100 cycles of latency

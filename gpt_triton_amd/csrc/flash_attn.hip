@@ -624,7 +624,7 @@ template <bool BLND, bool ACC, bool DROP>
 __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, int num_bh,
-    float scale, StreamPlan plan, float drop_p, const unsigned* __restrict__ keep) {
+    float scale, StreamPlan plan, float drop_p, const unsigned* __restrict__ keep, PrefetchArgs ahead) {
   constexpr int D = 64, KS = 4, DB = 2;
   constexpr int MAX_TILES = 5;  // 64-key tiles of a heavy chunk, L <= 320; a light chunk (c1) has one
   constexpr int MAX_DMA = 10;  // 16-byte loads per lane per pair: Lp / 32, Lp <= 320
@@ -883,7 +883,10 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   // the K / V loads, the light chunk's into its own registers when it is done with them.
   h8 q_heavy[KS], q_heavy_next[KS], q_light[KS];
   int bh = blockIdx.x;
-  if (bh >= num_bh) return;
+  if (bh >= num_bh) {  // a workgroup beyond the pairs
+    prefetch_lines<512>(ahead, bh - num_bh, (int)gridDim.x - num_bh);
+    return;
+  }
   // (single registers with values the compiler cannot see through, and a chain of selects: an array, or
   // loads it can join, would live in scratch memory)
   unsigned kw0 = 0, kw1 = 0, kw2 = 0, kw3 = 0, kw4 = 0, kw_light = 0;
@@ -979,7 +982,8 @@ __device__ __forceinline__ WorkItem work_item(int pairs, int q_blocks, int group
 template <bool BLND, bool ACC>
 __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group) {
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group,
+    PrefetchArgs ahead) {
   constexpr int D = 64, KS = 4, DB = 2, NS = 4;
   constexpr int STAGE = 2 * BKEY * D * 2;  // 16 KB: K tile, then V tile
   constexpr int V_AT = BKEY * D * 2;       // byte offset of the V tile inside a stage
@@ -990,6 +994,11 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
   const int q_blocks = (L + BQ - 1) / BQ;
+  const int workers = 8 * ((pairs + 7) >> 3) * q_blocks;
+  if ((int)blockIdx.x >= workers) {
+    prefetch_lines<256>(ahead, (int)blockIdx.x - workers, (int)gridDim.x - workers);
+    return;
+  }
   const WorkItem item = work_item(pairs, q_blocks, group);
   const int bh = item.bh, qb = item.qb;
   if (bh >= pairs) return;
@@ -1590,7 +1599,7 @@ inline int attn_cu_count() {
 template <bool BLND, bool ACC = false, bool DROP = false>
 int launch_stream_attn(const void* q, const void* k, const void* v, void* out, int64_t BN,
                        int heads, int L, float scale, hipStream_t st, float drop_p = 0.f,
-                       const void* keep = nullptr) {
+                       const void* keep = nullptr, const Prefetch* ahead = nullptr) {
   auto kern = flash_attn_stream_kernel<BLND, ACC, DROP>;
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
@@ -1605,10 +1614,10 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   const int cus = attn_cu_count();
   if (cus < 0) return cus;
   const int Lp = (L + BKEY - 1) / BKEY * BKEY;
-  const int grid = BN < cus ? (int)BN : cus;
+  const int grid = (BN < cus ? (int)BN : cus) + prefetch_workgroups(ahead, BN, cus);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), (size_t)Lp * 512, st,
                      (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out,
-                     heads, L, (int)BN, scale, make_stream_plan(L), drop_p, (const unsigned*)keep);
+                     heads, L, (int)BN, scale, make_stream_plan(L), drop_p, (const unsigned*)keep, prefetch_args(ahead));
   return 0;
 }
 
@@ -1632,12 +1641,14 @@ inline int deal_blocks(int64_t pairs, int q_blocks, unsigned* grid, int* group) 
 
 template <bool BLND, bool ACC = false>
 int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
-                     int L, float scale, hipStream_t st) {
+                     int L, float scale, hipStream_t st, const Prefetch* ahead) {
   unsigned grid;
   int group;
   if (const int rc = deal_blocks(BN, (L + BQ - 1) / BQ, &grid, &group)) return rc;
-  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(grid), dim3(256), 0, st, (const _Float16*)q,
-                     (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group);
+  const int cus = attn_cu_count();
+  if (cus < 0) return cus;
+  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(grid + prefetch_workgroups(ahead, grid, cus)), dim3(256), 0, st, (const _Float16*)q,
+                     (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group, prefetch_args(ahead));
   return 0;
 }
 
@@ -1674,17 +1685,18 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
 // 60 x 320 8.5 / 8.1, 96 x 320 8.6 / 8.7, 192 x 300 11.4 / 12.8 (13.1), 1536 x 300 55 / 76 (66).
 template <bool BLND, bool ACC = false>
 int launch_d64(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
-               float scale, hipStream_t st) {
+               float scale, hipStream_t st, const Prefetch* ahead) {
   const int cus = attn_cu_count();
   if (cus < 0) return cus;
   const bool ring = L > 320 || (L > 288 && 3 * BN <= cus) || (L <= BKEY && BN <= 512);
-  return ring ? launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st)
-              : launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st);
+  return ring ? launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st, ahead)
+              : launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st, 0.f, nullptr, ahead);
 }
 
 template <int D, typename T>
 int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
-             int heads, int L, int Lk, float scale, Dropout drop, bool blnd, hipStream_t st) {
+             int heads, int L, int Lk, float scale, Dropout drop, bool blnd, hipStream_t st,
+             const Prefetch* ahead) {
   const DropoutArgs da = {drop.p, (unsigned)drop.seed, (unsigned)(drop.seed >> 32)};
   if (drop.p > 0.f) {  // training-mode path: the tiled kernel carries the generator
     return blnd ? launch_tiled<D, T, true, 1>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
@@ -1694,8 +1706,8 @@ int launch_d(const void* q, const void* k, const void* v, void* out, int64_t BN,
     return blnd ? launch_tiled<D, T, true, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st)
                 : launch_tiled<D, T, false, 0>(q, k, v, out, BN, heads, L, Lk, scale, da, st);
   if constexpr (D == 64 && sizeof(T) == 2) {
-    return blnd ? launch_d64<true>(q, k, v, out, BN, heads, L, scale, st)
-                : launch_d64<false>(q, k, v, out, BN, heads, L, scale, st);
+    return blnd ? launch_d64<true>(q, k, v, out, BN, heads, L, scale, st, ahead)
+                : launch_d64<false>(q, k, v, out, BN, heads, L, scale, st, ahead);
   } else {
     if (const size_t lds = resident_lds_bytes(L, D))
       return blnd ? launch_resident<D, T, true>(q, k, v, out, BN, heads, L, scale, lds, st)
@@ -1731,13 +1743,14 @@ int launch_small_head(const void* q, const void* k, const void* v, void* out, in
 
 template <typename T>
 int launch_t(const void* q, const void* k, const void* v, void* out, int64_t BN,
-             int heads, int L, int Lk, int d, float scale, Dropout drop, bool blnd, hipStream_t st) {
+             int heads, int L, int Lk, int d, float scale, Dropout drop, bool blnd, hipStream_t st,
+             const Prefetch* ahead) {
   switch (d) {
     case 16: return launch_small_head<16, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st);
     case 32: return launch_small_head<32, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st);
-    case 64: return launch_d<64, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st);
-    case 128: return launch_d<128, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st);
-    case 256: return launch_d<256, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st);
+    case 64: return launch_d<64, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st, ahead);
+    case 128: return launch_d<128, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st, ahead);
+    case 256: return launch_d<256, T>(q, k, v, out, BN, heads, L, Lk, scale, drop, blnd, st, ahead);
     default:
       set_error("flash_attn: head size %d not built (16, 32, 64, 128 and 256 are)", d);
       return -2;
@@ -1789,12 +1802,12 @@ int launch_masked(const void* q, const void* k, const void* v, void* out, int64_
 // model's kernels round their operands to anyway, see launch_flash_attn_operands.
 template <int D>
 int launch_operands_d(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
-                      int L, float scale, DropoutArgs da, hipStream_t st) {
+                      int L, float scale, DropoutArgs da, hipStream_t st, const Prefetch* ahead) {
   typedef _Float16 T;
   if (da.p > 0.f)
     return launch_tiled_as<D, T, true, 1, false, D, true>(q, k, v, out, BN, heads, L, L, scale, da, st);
   if constexpr (D == 64) {
-    return launch_d64<true, true>(q, k, v, out, BN, heads, L, scale, st);
+    return launch_d64<true, true>(q, k, v, out, BN, heads, L, scale, st, ahead);
   } else {
     if (const size_t lds = resident_lds_bytes(L, D))
       return launch_resident<D, T, true, true>(q, k, v, out, BN, heads, L, scale, lds, st);
@@ -1816,7 +1829,8 @@ int launch_operands_small(const void* q, const void* k, const void* v, void* out
 }  // namespace
 
 int launch_flash_attn_operands(const void* q, const void* k, const void* v, void* out, int64_t B,
-                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st) {
+                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st,
+                               const Prefetch* ahead) {
   const int64_t BN = B * N;
   if (BN > 0x7fffffffll || L > (1 << 24)) {
     set_error("flash_attn: B*N=%lld or L=%lld beyond the grid limits", (long long)BN, (long long)L);
@@ -1828,9 +1842,9 @@ int launch_flash_attn_operands(const void* q, const void* k, const void* v, void
   switch (d) {
     case 16: return launch_operands_small<16>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
     case 32: return launch_operands_small<32>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
-    case 64: return launch_operands_d<64>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
-    case 128: return launch_operands_d<128>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
-    case 256: return launch_operands_d<256>(q, k, v, out, BN, (int)N, (int)L, scale, da, st);
+    case 64: return launch_operands_d<64>(q, k, v, out, BN, (int)N, (int)L, scale, da, st, ahead);
+    case 128: return launch_operands_d<128>(q, k, v, out, BN, (int)N, (int)L, scale, da, st, ahead);
+    case 256: return launch_operands_d<256>(q, k, v, out, BN, (int)N, (int)L, scale, da, st, ahead);
     default:
       set_error("flash_attn: head size %d not built (16, 32, 64, 128 and 256 are)", d);
       return -2;
@@ -1839,7 +1853,7 @@ int launch_flash_attn_operands(const void* q, const void* k, const void* v, void
 
 int launch_flash_attn(const void* q, const void* k, const void* v, void* out, int64_t B,
                       int64_t N, int64_t L, int64_t Lk, int d, float scale, Dropout drop,
-                      bool out_blnd, bool f16, hipStream_t st) {
+                      bool out_blnd, bool f16, hipStream_t st, const Prefetch* ahead) {
   const int64_t BN = B * N;
   if (BN > 0x7fffffffll || L > (1 << 24) || Lk > (1 << 24)) {
     set_error("flash_attn: B*N=%lld, Lq=%lld or Lk=%lld beyond the grid limits", (long long)BN,
@@ -1851,9 +1865,9 @@ int launch_flash_attn(const void* q, const void* k, const void* v, void* out, in
     return launch_masked<false>(q, k, v, out, BN, (int)N, (int)L, d, scale, da, drop.keep, st);
   }
   return f16 ? launch_t<_Float16>(q, k, v, out, BN, (int)N, (int)L, (int)Lk, d, scale, drop,
-                                  out_blnd, st)
+                                  out_blnd, st, ahead)
              : launch_t<float>(q, k, v, out, BN, (int)N, (int)L, (int)Lk, d, scale, drop, out_blnd,
-                               st);
+                               st, ahead);
 }
 
 }  // namespace gptmi

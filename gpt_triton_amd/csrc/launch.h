@@ -6,6 +6,13 @@
 
 namespace gptmi {
 
+// What the launches behind this one will read (weights): a launch of few workgroups has others request it from HBM
+// into the memory-side cache meanwhile.
+struct Prefetch {
+  const void* p[4] = {};
+  size_t bytes[4] = {};
+};
+
 // Dropout of one launch: probability p (0 = none) and the 64-bit seed of the generator.
 struct Dropout {
   float p;
@@ -84,12 +91,13 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
 // pointers 16-byte aligned.
 bool attn_front_supported(int64_t B, int64_t L, int64_t heads, int64_t h);
 int launch_attn_front(const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
-                      const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st);
+                      const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st,
+                      const Prefetch* ahead = nullptr);
 
 // q, out: L rows per (batch, head); k, v: Lk rows.
 int launch_flash_attn(const void* q, const void* k, const void* v, void* out,
                       int64_t B, int64_t N, int64_t L, int64_t Lk, int d, float scale,
-                      Dropout drop, bool out_blnd, bool f16, hipStream_t st);
+                      Dropout drop, bool out_blnd, bool f16, hipStream_t st, const Prefetch* ahead = nullptr);
 
 
 // The attention of an fp32 model on fp16 copies of q, k, v: the fp32 kernels round q, k and v to fp16
@@ -97,6 +105,7 @@ int launch_flash_attn(const void* q, const void* k, const void* v, void* out,
 // in front and the output rounded here the values are the same and half the bytes move.  fp32 softmax
 // arithmetic as for fp32 storage; equal lengths; out [B][L][N][d] fp16.
 int launch_flash_attn_operands(const void* q, const void* k, const void* v, void* out, int64_t B,
-                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st);
+                               int64_t N, int64_t L, int d, float scale, Dropout drop, hipStream_t st,
+                               const Prefetch* ahead = nullptr);
 
 }  // namespace gptmi
