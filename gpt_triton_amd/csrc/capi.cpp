@@ -826,8 +826,8 @@ size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t
   return 2 * (size_t)round_up(M * h * (dtype == GPTMI_F16 ? 2 : 4), 256) + (a > m ? a : m);
 }
 
-// What an attention launch of few workgroups requests of the weights that come behind it.  Its other CUs bring in
-// some 15 MB while it lasts, and 40 KB more for each of its key rows; weights beyond that make it last longer than
+// What an attention launch requests of the weights that come behind it (prefetch_workgroups).  Where it has few
+// workgroups, the other CUs bring in some 15 MB while it lasts, and 40 KB more for each of its key rows; weights beyond that make it last longer than
 // they save, and half a matrix saves nothing.  The MLP's second product first, which has the longest columns, in any
 // case; then the next layer's first product, then what follows at once.  Forwards that find their weights in HBM (four
 // models in turn; wider ones always do), us, without / this: 124M 1 x 24 tokens with logits 356 -> 315, 2 x 64 366 -> 353, 8 x 24

@@ -45,8 +45,8 @@ __device__ __forceinline__ h4 lds_read_tr16(const char* p) {
   return __builtin_bit_cast(h4, r);
 }
 
-// Lines of memory that later launches read, requested by workgroups of a launch that leaves CUs idle (see
-// launch.h): a word of each 128-byte line, spread over `blocks` workgroups of NT threads.
+// Lines of memory that later launches read, requested by workgroups of a launch that leaves CUs idle, or does at
+// its end (see launch.h): a word of each 128-byte line, spread over `blocks` workgroups of NT threads.
 struct PrefetchArgs {
   const void* p[4];
   unsigned lines[4];
@@ -56,9 +56,12 @@ inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
   for (int k = 0; ahead && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
   return a;
 }
-// Workgroups for it: the CUs that a launch of `workers` leaves idle, if they are 64 or more.
+// Workgroups for it, behind the `workers` of the launch: the CUs that these leave idle, or 128 that find room as the
+// last of them end (64 gain less: 28 x 300 tokens of 124M none / 64 / 128 2072 / 1923 / 1901 us, 32 x 300 in fp32 2440 / 2266 /
+// 2268, 16 x 512 2054 / 1922 / 1899, 64 x 300 3977 / 3940 / 3928; 1024 wide 8 x 1024 6024 / 5661 / 5623, 1280 wide 4 x 700 5855 / 5514 /
+// 5361).
 inline int prefetch_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
-  return ahead != nullptr && workers <= cus - 64 ? cus - (int)workers : 0;
+  return ahead == nullptr ? 0 : workers <= cus - 64 ? cus - (int)workers : 128;
 }
 template <int NT>
 __device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int block, int blocks) {

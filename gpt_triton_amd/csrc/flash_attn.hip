@@ -624,7 +624,8 @@ template <bool BLND, bool ACC, bool DROP>
 __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, int num_bh,
-    float scale, StreamPlan plan, float drop_p, const unsigned* __restrict__ keep, PrefetchArgs ahead) {
+    float scale, StreamPlan plan, float drop_p, const unsigned* __restrict__ keep, int workers,
+    PrefetchArgs ahead) {
   constexpr int D = 64, KS = 4, DB = 2;
   constexpr int MAX_TILES = 5;  // 64-key tiles of a heavy chunk, L <= 320; a light chunk (c1) has one
   constexpr int MAX_DMA = 10;  // 16-byte loads per lane per pair: Lp / 32, Lp <= 320
@@ -883,8 +884,8 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   // the K / V loads, the light chunk's into its own registers when it is done with them.
   h8 q_heavy[KS], q_heavy_next[KS], q_light[KS];
   int bh = blockIdx.x;
-  if (bh >= num_bh) {  // a workgroup beyond the pairs
-    prefetch_lines<512>(ahead, bh - num_bh, (int)gridDim.x - num_bh);
+  if (bh >= workers) {
+    prefetch_lines<512>(ahead, bh - workers, (int)gridDim.x - workers);
     return;
   }
   // (single registers with values the compiler cannot see through, and a chain of selects: an array, or
@@ -908,7 +909,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   int buf = 0;
   bool stored = false;  // this wavefront's heavy chunk stored its 4 x 16 bytes right before
   while (true) {
-    const int bh_next = bh + (int)gridDim.x;
+    const int bh_next = bh + workers;
     const bool has_next = bh_next < num_bh;
     // Everything this wavefront LOADED has landed (the pair's K / V units and queries); behind the
     // barrier that holds for every wavefront, and nobody reads the other buffer any more.  Loads
@@ -1614,10 +1615,18 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   const int cus = attn_cu_count();
   if (cus < 0) return cus;
   const int Lp = (L + BKEY - 1) / BKEY * BKEY;
-  const int grid = (BN < cus ? (int)BN : cus) + prefetch_workgroups(ahead, BN, cus);
+  const int workers = BN < cus ? (int)BN : cus;
+  // One full round of pairs ends all at once, and what comes behind it then is not hidden: 64 prefetching workgroups
+  // instead of 128 (20 x 300 tokens of 124M none / 64 / 128 1523 / 1487 / 1516 us), and none behind short pairs for
+  // weights that a model may find in the memory-side cache (21 x 128 tokens of 124M, its weights there / in HBM, 763 /
+  // 913 without, 808 / 845 with).
+  int further = prefetch_workgroups(ahead, BN, cus);
+  if (ahead != nullptr && BN > cus - 64 && BN <= cus) further = L <= 128 && ahead->bytes[0] <= 5000000 ? 0 : 64;
+  const int grid = workers + further;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), (size_t)Lp * 512, st,
                      (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out,
-                     heads, L, (int)BN, scale, make_stream_plan(L), drop_p, (const unsigned*)keep, prefetch_args(ahead));
+                     heads, L, (int)BN, scale, make_stream_plan(L), drop_p, (const unsigned*)keep, workers,
+                     prefetch_args(ahead));
   return 0;
 }
 

@@ -6,8 +6,8 @@
 
 namespace gptmi {
 
-// What the launches behind this one will read (weights): a launch of few workgroups has others request it from HBM
-// into the memory-side cache meanwhile.
+// What the launches behind this one will read (weights): an attention launch has further workgroups request it from
+// HBM into the memory-side cache, on the CUs that it leaves idle.
 struct Prefetch {
   const void* p[4] = {};
   size_t bytes[4] = {};
