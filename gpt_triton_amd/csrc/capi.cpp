@@ -229,6 +229,15 @@ struct BlockWeights {
       launch_layernorm_pack_pair(x, ln_w, ln_b, normed, M, h, eps, W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
   }
 };
+// A block packs its plain weights in its LayerNorm's own launch, which leaves the images in the memory-side
+// cache; a product that reads [K][N] in place takes 2-5 us more where few rows meet a long K, as its narrow
+// tiles then read short pieces of the weights' rows.  Whole forwards with plain weights, us, packed / in place:
+// width 768: 24 rows 569 / 535, 128 rows 567 / 533, 488 rows 638 / 583; width 1600: 40 rows 2778 / 2657, 300
+// rows 3838 / 3683; width 1024: 186 rows 1174 / 1224, 512 rows 1328 / 1506, 1024 rows 1813 / 1906, 1500 rows
+// 2266 / 2269; width 1280: 50 rows 1748 / 1897, 300 rows 2361 / 2433, 1024 rows 3713 / 3595.
+static bool reads_in_place(int64_t M, int64_t h) {
+  return h <= 768 || h > 1280 || M >= (h > 1024 ? 1024 : 1536);
+}
 static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
   return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
 }
@@ -677,7 +686,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   eo.out = out;
   eo.drop = drop;
   eo.f16 = f16;
-  bw.in_place = !bw.packed && !prologue && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep) &&
+  bw.in_place = !bw.packed && !prologue && reads_in_place(M, h) && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep) &&
                 gemm_reads_kn(W_proj, M, (int)h, (int)h, eo);
   const void *Bq = bw.first(), *Bp = bw.second();
   if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
@@ -770,7 +779,7 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e2.out = out;
   e2.drop = drop;
   e2.f16 = f16;
-  bw.in_place = !bw.packed && !prologue && gemm_reads_kn(W1, M, (int)inner, (int)H, e1) &&
+  bw.in_place = !bw.packed && !prologue && reads_in_place(M, H) && gemm_reads_kn(W1, M, (int)inner, (int)H, e1) &&
                 gemm_reads_kn(W2, M, (int)H, (int)inner, e2);
   const void *B1 = bw.first(), *B2 = bw.second();
   if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
