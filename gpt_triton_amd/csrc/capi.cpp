@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "gemm_common.h"
 #include "launch.h"
 
 namespace gptmi {
@@ -237,6 +238,16 @@ struct BlockWeights {
 // 2266 / 2269; width 1280: 50 rows 1748 / 1897, 300 rows 2361 / 2433, 1024 rows 3713 / 3595.
 static bool reads_in_place(int64_t M, int64_t h) {
   return h <= 768 || h > 1280 || M >= (h > 1024 ? 1024 : 1536);
+}
+// The one launch in front of a short sequences' projection: of few pairs it takes longer than the two it stands
+// for, but an eager forward that small waits for the host, which then has a launch less a block.  A graph's replay
+// does not.  124M, weights from HBM, us, in two launches / in one: eager 1 x 24 tokens 313 / 297, 2 x 24 319 / 309, 4 x 32
+// 346 / 331; replayed 1 x 24 290 / 302, 2 x 24 306 / 317, 3 x 30 340 / 336, 4 x 32 352 / 342, 8 x 24 409 / 368.
+static bool front_pays(int64_t pairs, hipStream_t st) {
+  if (pairs > 32) return true;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+  return status == hipStreamCaptureStatusNone;
 }
 static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
   return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
@@ -698,7 +709,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   const void* rows = normed ? normed : x;
   const bool front = f16 && bw.packed && p == 0.f && d == 64 && attn_front_supported(B, L, heads, h) &&
                      gemm_layernorm_supported(M, (int)h) && prologue_aligned(rows, ln_w, ln_b) &&
-                     ((uintptr_t)b_qkv & 15) == 0;
+                     ((uintptr_t)b_qkv & 15) == 0 && front_pays(B * heads, st);
   if (front) {
     rc = launch_attn_front(rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st, ahead);
   } else if (prologue) {
@@ -835,21 +846,29 @@ size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t
   return 2 * (size_t)round_up(M * h * (dtype == GPTMI_F16 ? 2 : 4), 256) + (a > m ? a : m);
 }
 
-// What an attention launch requests of the weights that come behind it (prefetch_workgroups).  Where it has few
-// workgroups, the other CUs bring in some 15 MB while it lasts, and 40 KB more for each of its key rows; weights beyond that make it last longer than
-// they save, and half a matrix saves nothing.  The MLP's second product first, which has the longest columns, in any
-// case; then the next layer's first product, then what follows at once.  Forwards that find their weights in HBM (four
-// models in turn; wider ones always do), us, without / this: 124M 1 x 24 tokens with logits 356 -> 315, 2 x 64 366 -> 353, 8 x 24
-// 422 -> 360, 7 x 211 738 -> 686, 1 x 800 705 -> 640; 1024 wide 4 x 64 969 -> 905, 2 x 300 1367 -> 1266; 1280 wide 1 x 50 1316 ->
-// 1290 (all four weights 1390), 2 x 200 2350 -> 2241; 1600 wide 1 x 50 2058 -> 2038 (all four 2215), 1 x 300 3359 -> 3182.
-// One 124M model over and over, whose weights the memory-side cache holds: equal.
-static Prefetch weights_ahead(const void* const* layer, bool last, int64_t h, int64_t inner, int64_t L) {
+// What an attention launch requests of the weights that come behind it (prefetch_workgroups): the MLP's second
+// product first, which has the longest columns, then the next layer's first product, then what follows at once; half a
+// matrix saves nothing, and what the launch has to wait for costs what it saves.  Launches of as many workgroups as
+// CUs and those of the front kernel last long enough for some 15 MB and 40 KB more for each key row, launches of
+// few pairs for 120 KB a key row, and the second product alone is worth a wait of its 14 MB or less.  Forwards that
+// find their weights in HBM (four models in turn; wider ones always do), us, nothing / the second product alone /
+// this: 124M 1 x 24 tokens 342 / 335 / 303, 2 x 64 370 / 357 / 356 (15 MB: 368), 7 x 211 751 / 724 / 674, 1 x 800
+// 713 / 695 / 651; 100 x 40 1274 / - / 1164 (120 KB a row: 1217); 1024 wide 1 x 41 707 / 698 / 697 (15 MB: 715), 4 x 160
+// 1390 / - / 1237, 2 x 200 1168 / 1148 / 1115; 1280 wide 2 x 60 1641 / 1545, 2 x 200 2376 / 2320 / 2239; 1600 wide
+// 1 x 41 1925 / 1959 / 1925, 1 x 150 2616 / 2478 / 2478, 1 x 300 3349 / 3174 / 3100, 1 x 500 4287 / 3851 / 3851 (60 MB:
+// 3972).  One 124M model over and over, whose weights the memory-side cache holds: equal.
+static Prefetch weights_ahead(const void* const* layer, bool last, int64_t B, int64_t L, int64_t heads, int64_t h,
+                              int64_t inner, hipStream_t st) {
   const size_t square = (size_t)(h * h * 2), wide = (size_t)(h * inner * 2);
   const struct {
     const void* p;
     size_t bytes;
   } wanted[4] = {{layer[10], wide}, {last ? nullptr : layer[12 + 2], 3 * square}, {layer[8], wide}, {layer[4], square}};
-  const size_t most = 15000000 + 40000 * (size_t)L;
+  const size_t rows = (size_t)L, alone = 15000000 + 40000 * rows;
+  if (wide > alone) return Prefetch();
+  const bool lasting = B * heads > cu_count() - 64 || (attn_front_supported(B, L, heads, h) && front_pays(B * heads, st));
+  const size_t by_row = 120000 * rows < 40000000 ? 120000 * rows : 40000000;
+  const size_t most = lasting && alone > by_row ? alone : by_row;
   Prefetch ahead;
   size_t sum = 0;
   for (int k = 0; k < 4; ++k) {
@@ -884,7 +903,7 @@ int gptmi_blocks(const void* x, const void* normed, const void* const* params, i
   const size_t ws_bytes = workspace_bytes - c.used;
   for (int64_t i = 0; i < n; ++i) {
     const void* const* p = params + 12 * i;
-    const Prefetch ahead = weights_ahead(p, i + 1 == n, h, inner, L);
+    const Prefetch ahead = weights_ahead(p, i + 1 == n, B, L, heads, h, inner, (hipStream_t)stream);
     int rc = attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B, L, heads,
                              d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream, &ahead);
     if (rc) return rc;

@@ -57,9 +57,9 @@ inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
   return a;
 }
 // Workgroups for it, behind the `workers` of the launch: the CUs that these leave idle, or 128 that find room as the
-// last of them end (64 gain less: 28 x 300 tokens of 124M none / 64 / 128 2072 / 1923 / 1901 us, 32 x 300 in fp32 2440 / 2266 /
-// 2268, 16 x 512 2054 / 1922 / 1899, 64 x 300 3977 / 3940 / 3928; 1024 wide 8 x 1024 6024 / 5661 / 5623, 1280 wide 4 x 700 5855 / 5514 /
-// 5361).
+// last of them end (64 gain less: 28 x 300 tokens of 124M none / 64 / 128 2072 / 1923 / 1901 us, 32 x 300 in fp32
+// 2440 / 2266 / 2268, 16 x 512 2054 / 1922 / 1899, 64 x 300 3977 / 3940 / 3928; 1024 wide 8 x 1024 6024 / 5661 /
+// 5623, 1280 wide 4 x 700 5855 / 5514 / 5361).
 inline int prefetch_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
   return ahead == nullptr ? 0 : workers <= cus - 64 ? cus - (int)workers : 128;
 }

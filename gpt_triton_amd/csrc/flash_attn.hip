@@ -961,9 +961,8 @@ __device__ __forceinline__ WorkItem work_item(int pairs, int q_blocks, int group
 
 // ---------------------------------------------------------------------------
 // Ring variant for sequences too long for the streaming kernel, and for few pairs of one tile: fp16
-// storage, head size 64,
-// equal query and key lengths, no dropout.  One workgroup = 4 wavefronts = one (batch, head) x
-// 128 queries, as in the tiled kernel, but the 64-key tiles of K and V travel the way the
+// storage, head size 64, equal query and key lengths, no dropout.  One workgroup = 4 wavefronts = one
+// (batch, head) x 128 queries, as in the tiled kernel, but the 64-key tiles of K and V travel the way the
 // streaming kernel moves them: by direct global->LDS loads (no staging registers, no LDS store
 // instructions) into a ring of four 16 KB stages -- K tile [64][64] then V tile [64][64] halves,
 // rows of 128 bytes, the swizzles applied on the source side -- and V stays row-major and is read
