@@ -135,7 +135,9 @@ int gptmi_softmax(const void* x, void* out, int64_t M, int64_t H, int dtype,
 /*
  * Bytes of workspace gptmi_linear / gptmi_linear_qkv need for these sizes
  * (0 if none).  The workspace holds the fp16, K-contiguous, zero-padded copy of
- * the weight (and of x when x is fp32 or K is not a multiple of 64).
+ * the weight (and of x when x is fp32 or K is not a multiple of 64).  An aligned fp16
+ * W[K][N] is read in place where a kernel can (K a multiple of 64, N of 8); the size does
+ * not depend on that.
  */
 size_t gptmi_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype,
                                     int wlayout);
@@ -149,8 +151,8 @@ size_t gptmi_packed_weight_bytes(int64_t N, int64_t K);
  * Writes the packed image of W (layout GPTMI_W_KN or GPTMI_W_NK, storage `dtype`)
  * into `packed` (gptmi_packed_weight_bytes(N, K) bytes, 256-byte aligned): the
  * weight rounded to fp16, K-contiguous, zero padded to a multiple of 64.  It is
- * what gptmi_linear builds in its workspace on every call; packing once and
- * passing GPTMI_W_PACKED skips that step for weights that do not change.
+ * what gptmi_linear builds in its workspace on every call unless it can read W in place;
+ * packing once and passing GPTMI_W_PACKED skips that step for weights that do not change.
  * No counterpart in the reference (its Triton kernel reads W[K][N] in place,
  * kernels.py:231-234).
  */
@@ -195,7 +197,7 @@ int gptmi_linear(const void* x, const void* W, const void* bias,
  *     gptmi_linear_static_capacity() are refused with GPTMI_ERR_WORKSPACE (fp16, K % 64 == 0,
  *     W[K][N]: N*K*2 <= 8 MiB, e.g. every GEMM of GPT-2 124M; GPTMI_W_PACKED needs no scratch).
  *   - Every call on a GPU shares that GPU's array and keeps nothing in it between calls (the
- *     images are rewritten in full by each call).  Calls that overlap on one GPU -- two streams,
+ *     images are rewritten in full by each call that needs them).  Calls that overlap on one GPU -- two streams,
  *     two host threads -- race on it; calls on one stream are ordered and safe.
  *   - The first call on a device resolves the array's address there (hipGetSymbolAddress); make
  *     that call outside a graph capture.
