@@ -5,19 +5,6 @@
 
 namespace gptmi {
 
-// exp(x) for x <= 0, -inf and NaN: 2^n 2^a with n the integer nearest to x log2(e), |a| <= 1/2; n comes out of
-// the low bits of a sum with 1.5 * 2^23 and stops at -200, where the result is 0 in fp32.  What expf does in
-// 13 operations beside the hardware's exp2, mostly for what lies above 0, in 7.  From 0 to -87 0.95 ulp at most
-// and 0.305 rms (expf 0.85 and 0.300); the attention's distance from 64 bits is that of expf to five digits
-// (300 rows, d = 64 1.39249e-4 and 1.39248e-4, 7.47355e-5 and 7.47356e-5 with sharper weights).  With
-// NormaliseHalf, attention of 32 x 12 pairs of 300 rows 30.5 -> 25.3 us, fp32 forward of 32 x 300 2489 -> 2431.
-__device__ __forceinline__ float exp_nonpositive(float x) {
-  constexpr float kLog2e = 1.44269502162933349609375f, kRest = 1.925963033500012e-8f, kShift = 12582912.f;
-  const float t = fmaxf(fmaf(x, kLog2e, kShift), kShift - 200.f);
-  const float a = fmaf(x, kRest, fmaf(x, kLog2e, kShift - t));
-  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(a), __float_as_int(t) - __float_as_int(kShift));
-}
-
 // The softmax arithmetic, in three forms.
 // ACC = false, SCALED = false (fp16 storage): running max on the raw scores, scale * log2(e) folded
 // into one fused multiply-add in front of the hardware's exp2, a reciprocal for the denominator -- the
@@ -30,8 +17,8 @@ __device__ __forceinline__ float exp_nonpositive(float x) {
 // product rounded per max, tiles of different max disagree by that rounding (fp16, scaled scores of
 // 500000: 3.6e-3).
 //   ACC = true (fp32 storage, and the fp16 copies of q, k, v that the block functions of fp32 models
-//   hand on): an exp as exact as the library's and a true division, so fewer fp16 rounding flips of P against the
-//   reference's np.exp.
+//   hand on): library exp and a true division, so fewer fp16 rounding flips of P against the
+//   reference's np.exp.  (Argument reductions of fewer operations were less exact: 0.95 ulp against expf's 0.85.)
 //   ACC = false (fp16 storage with dropout): the hardware's exp2.
 template <bool ACC, bool SCALED = ACC>
 struct Softmax {
@@ -44,12 +31,12 @@ struct Softmax {
   __device__ __forceinline__ float base(float m) const { return SCALED ? m : m * c; }
   // the weight of score s = score(.) for base b = base(m)
   __device__ __forceinline__ float weight(float s, float b) const {
-    if constexpr (SCALED) return ACC ? exp_nonpositive(s - b) : __expf(s - b);
+    if constexpr (SCALED) return ACC ? expf(s - b) : __expf(s - b);
     else return __builtin_amdgcn_exp2f(fmaf(s, c, -b));
   }
   // the rescaling when the running max goes from `old` to m
   __device__ __forceinline__ float rescale(float old, float m) const {
-    if constexpr (SCALED) return ACC ? exp_nonpositive(old - m) : __expf(old - m);
+    if constexpr (SCALED) return ACC ? expf(old - m) : __expf(old - m);
     else return __builtin_amdgcn_exp2f((old - m) * c);
   }
 };

@@ -59,3 +59,24 @@ def test_infinite_and_nan_keys(K, gpu_device, L):
     k[:, :, 50] = float("nan")
     bad = torch.isnan(K.flash_attention_v1(q, k, v))
     assert bool(bad[:, :, 50:].all()) and not bool(bad[:, :, :50].any())
+
+
+@pytest.mark.parametrize("d,L", [(16, 2), (64, 2), (64, 330), (256, 40), (256, 330)])  # resident and tiled kernels
+def test_the_exponential_is_the_library_s(K, gpu_device, d, L):
+    """Row 1 sees scores 0 and s, exact in fp32, and values 1 and 0: its output is 1 / (1 + exp(s)) with the library's
+    exponential to the last bit (operations of lower error bounds differ from it, of higher ones too).  s from
+    -0.7 up, where the sum shows every other last bit of exp(s), and a tail to -16."""
+    N = 2048
+    print(f"fp32 attention, last bits of the exponential: d={d}, L={L}", flush=True)
+    g = torch.Generator().manual_seed(d + L)
+    a = (1 + torch.rand(N, generator=g)).half().double()
+    s = -0.7 * torch.rand(N, generator=g, dtype=torch.float64)
+    s[::8] *= 23
+    b = (s / a * d**0.5).half().double()
+    s = a * b / d**0.5  # 22 bits, and a power of two
+    assert torch.equal(s.float().double(), s)
+    q, k, v = (torch.zeros(1, N, L, d) for _ in range(3))
+    q[0, :, 1, 0], k[0, :, 1, 0], v[0, :, 0] = a.float(), b.float(), 1
+    got = K.flash_attention_v1(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device))[0, :, 1, 0].cpu()
+    want = (1 / (1 + torch.exp(s.float().to(gpu_device)))).cpu()
+    assert torch.equal(got, want), f"{int((got != want).sum())} of {N} rows"
