@@ -24,6 +24,7 @@
 // global loads are in flight while the current one is consumed.
 #include <type_traits>
 
+#include "attn_deal.h"
 #include "common.h"
 #include "launch.h"
 #include "softmax.h"
@@ -945,20 +946,6 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   }
 }
 
-// Which (batch, head) pair and which query block (of q_blocks) a workgroup works on.  Workgroup ids are dealt
-// round-robin over the 8 XCDs, so id % 8 is the XCD: all blocks of a pair go to one, whose L2 then holds
-// the K and V that they share.  An XCD takes its pairs in groups of `group`, of each group the heaviest
-// (latest) query blocks first.
-struct WorkItem {
-  int bh, qb;  // bh may be `pairs` or more: none
-};
-__device__ __forceinline__ WorkItem work_item(int pairs, int q_blocks, int group) {
-  const int j = blockIdx.x >> 3, per = (pairs + 7) >> 3;  // per: pairs of an XCD, the last one of some is none
-  const int first = j / (group * q_blocks) * group, in_group = j - first * q_blocks;
-  const int size = min(group, per - first), late = in_group / size;
-  return {(first + in_group - late * size) * 8 + (int)(blockIdx.x & 7), q_blocks - 1 - late};
-}
-
 // ---------------------------------------------------------------------------
 // Ring variant for sequences too long for the streaming kernel, and for few pairs of one tile: fp16
 // storage, head size 64, equal query and key lengths, no dropout.  One workgroup = 4 wavefronts = one
@@ -994,14 +981,13 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
   const int q_blocks = (L + BQ - 1) / BQ;
-  const int workers = 8 * ((pairs + 7) >> 3) * q_blocks;
+  const int workers = pairs * q_blocks;
   if ((int)blockIdx.x >= workers) {
     prefetch_lines<256>(ahead, (int)blockIdx.x - workers, (int)gridDim.x - workers);
     return;
   }
-  const WorkItem item = work_item(pairs, q_blocks, group);
+  const WorkItem item = work_item((int)blockIdx.x, pairs, q_blocks, group);
   const int bh = item.bh, qb = item.qb;
-  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1298,9 +1284,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
   const int q_blocks = (L + BQ - 1) / BQ;
-  const WorkItem item = work_item(pairs, q_blocks, group);
+  const WorkItem item = work_item((int)blockIdx.x, pairs, q_blocks, group);
   const int bh = item.bh, qb = item.qb;
-  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1629,34 +1614,21 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   return 0;
 }
 
-// The workgroups for that, and the group.  Some 32 workgroups a group, half of what an XCD holds: their K and V
-// stay in its 4 MB L2 until the last block has read them (all pairs' heaviest blocks first, every block fetches
-// them anew; 64 x 25 pairs of 1024 rows: 445 us, groups of 1, 2, 4, 8, 16 pairs 417, 398, 376, 383, 394;
-// 512 x 6 of 300 rows, d = 128: 308, 229, 231, 226, 224, 233).  Below two rounds of workgroups the order decides
-// when the last one ends, and all heaviest go first (8 x 12 pairs of 1024 rows 25.6 us, groups of 4 26.8).
-// Memory holds at most some 5 million blocks' q, k, v and output.
-inline int deal_blocks(int64_t pairs, int q_blocks, unsigned* grid, int* group) {
-  const int64_t per = (pairs + 7) / 8, all = 8 * per * q_blocks;
-  if (all >= 1 << 24) {
-    set_error("flash_attn: %lld workgroups exceed the grid", (long long)all);
-    return -2;
-  }
-  const int few = (32 + q_blocks - 1) / q_blocks;
-  *group = all < 1024 || per < few ? (int)per : few;
-  *grid = (unsigned)all;
-  return 0;
+inline int grid_exceeded(int64_t pairs, int L) {
+  set_error("flash_attn: %lld pairs of %d rows exceed the grid", (long long)pairs, L);
+  return -2;
 }
 
 template <bool BLND, bool ACC = false>
 int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                      int L, float scale, hipStream_t st, const Prefetch* ahead) {
-  unsigned grid;
-  int group;
-  if (const int rc = deal_blocks(BN, (L + BQ - 1) / BQ, &grid, &group)) return rc;
+  Deal deal;
+  if (!deal_blocks(BN, (L + BQ - 1) / BQ, &deal)) return grid_exceeded(BN, L);
   const int cus = attn_cu_count();
   if (cus < 0) return cus;
-  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(grid + prefetch_workgroups(ahead, grid, cus)), dim3(256), 0, st, (const _Float16*)q,
-                     (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group, prefetch_args(ahead));
+  hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(deal.grid + prefetch_workgroups(ahead, deal.grid, cus)),
+                     dim3(256), 0, st, (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L,
+                     scale, (int)BN, deal.group, prefetch_args(ahead));
   return 0;
 }
 
@@ -1675,11 +1647,10 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
     }
     attr_done = true;
   }
-  unsigned grid;
-  int group;
-  if (const int rc = deal_blocks(BN, (L + BQ - 1) / BQ, &grid, &group)) return rc;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, st, (const _Float16*)q, (const _Float16*)k,
-                     (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, group);
+  Deal deal;
+  if (!deal_blocks(BN, (L + BQ - 1) / BQ, &deal)) return grid_exceeded(BN, L);
+  hipLaunchKernelGGL(kern, dim3(deal.grid), dim3(256), lds, st, (const _Float16*)q, (const _Float16*)k,
+                     (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, deal.group);
   return 0;
 }
 

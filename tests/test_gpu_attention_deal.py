@@ -49,3 +49,10 @@ def test_every_pair_and_block(K, gpu_device, B, N, L, d):
     for b in range(B):
         worst = excess_over_bound(q[b:b + 1], k[b:b + 1], v[b:b + 1], got[b:b + 1])
         assert worst <= 0, f"beyond the rounding bound by {worst:.3e} in batch {b}"
+
+
+# pairs tied to no XCD behind and without tied ones: fewer than 8 pairs, one pair more than 8, no whole eights
+@pytest.mark.parametrize("B,N,L,d", [(1, 1, 4096, 64), (1, 9, 14600, 64), (1, 1, 2000, 128), (2, 21, 700, 256),
+                                     (1, 131, 1000, 128)])
+def test_pairs_of_no_xcd(K, gpu_device, B, N, L, d):
+    test_every_pair_and_block(K, gpu_device, B, N, L, d)
