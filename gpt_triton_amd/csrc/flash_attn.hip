@@ -969,7 +969,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
 template <bool BLND, bool ACC>
 __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group,
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int dealt, int group,
     PrefetchArgs ahead) {
   constexpr int D = 64, KS = 4, DB = 2, NS = 4;
   constexpr int STAGE = 2 * BKEY * D * 2;  // 16 KB: K tile, then V tile
@@ -981,13 +981,14 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
   const int q_blocks = (L + BQ - 1) / BQ;
-  const int workers = pairs * q_blocks;
+  const int workers = dealt * q_blocks;
   if ((int)blockIdx.x >= workers) {
     prefetch_lines<256>(ahead, (int)blockIdx.x - workers, (int)gridDim.x - workers);
     return;
   }
-  const WorkItem item = work_item((int)blockIdx.x, pairs, q_blocks, group);
+  const WorkItem item = work_item((int)blockIdx.x, dealt, q_blocks, group);
   const int bh = item.bh, qb = item.qb;
+  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1268,7 +1269,8 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
 template <int D, bool BLND, bool ACC>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
     const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int group) {
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int dealt,
+    int group) {
   static_assert(D == 128 || D == 256, "head sizes 128 and 256");
   constexpr int KS = D / 16, DB = D / 32;
   constexpr int ROWB = D * 2;             // bytes of a row
@@ -1284,8 +1286,9 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
   const unsigned smem_base = (unsigned)(uintptr_t)smem;
 
   const int q_blocks = (L + BQ - 1) / BQ;
-  const WorkItem item = work_item((int)blockIdx.x, pairs, q_blocks, group);
+  const WorkItem item = work_item((int)blockIdx.x, dealt, q_blocks, group);
   const int bh = item.bh, qb = item.qb;
+  if (bh >= pairs) return;
   const int q0 = qb * BQ;
   const int qw0 = q0 + wave * 32, q = qw0 + ql;
   const bool wave_active = qw0 < L;
@@ -1628,7 +1631,7 @@ int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int
   if (cus < 0) return cus;
   hipLaunchKernelGGL((flash_attn_ring_kernel<BLND, ACC>), dim3(deal.grid + prefetch_workgroups(ahead, deal.grid, cus)),
                      dim3(256), 0, st, (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L,
-                     scale, (int)BN, deal.group, prefetch_args(ahead));
+                     scale, (int)BN, deal.pairs, deal.group, prefetch_args(ahead));
   return 0;
 }
 
@@ -1650,7 +1653,7 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
   Deal deal;
   if (!deal_blocks(BN, (L + BQ - 1) / BQ, &deal)) return grid_exceeded(BN, L);
   hipLaunchKernelGGL(kern, dim3(deal.grid), dim3(256), lds, st, (const _Float16*)q, (const _Float16*)k,
-                     (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, deal.group);
+                     (const _Float16*)v, (_Float16*)out, heads, L, scale, (int)BN, deal.pairs, deal.group);
   return 0;
 }
 
