@@ -207,38 +207,47 @@ struct Carver {
 };
 
 // The weight images that a block's two products read: the caller's (packed), or built into its workspace.
-// K1 and K2 are multiples of 64.  in_place: both products read the caller's [K][N] weights as they are.
+// K1 and K2 are multiples of 64.  in_place: the first product reads the caller's [K][N] weight as it is.
+//
+// The first is read as the caller has it, [K][N], wherever it can be: its rows of 3 h or 4 h hold whole lines for a tile, and
+// the 0.1 to 2 us more that the product lasts are less than its share of the packing.  The second one's rows are
+// short where its K is long (K = 4 h): read in place it lasts 1 to 8 us more, at widths that are a power of 2 up to 15,
+// while its image is built in the LayerNorm's own launch, which has room, and stays in the memory-side cache.  Where
+// there is no such launch (normalised rows handed in, layernorm_packs) it is read in place too.  Blocks with plain
+// weights from HBM, us a layer, both packed / first in place / both in place: width 512, 50 rows 27.8 / 25.6 / 25.3;
+// 768: 24 34.3 / 31.4 / 33.2, 512 48.8 / 42.5 / 49.9, 2048 66.8 / 67.2 / 73.6; 896: 186 45.6 / 39.0 / 41.6;
+// 1024: 24 40.2 / 37.2 / 40.8, 512 51.5 / 51.0 / 58.9, 4800 164.9 / 163.5 / 168.5; 1280: 300 63.0 / 59.1 / 65.0, 777
+// 88.4 / 83.0 / 79.5; 1600: 100 60.9 / 54.6 / 54.6, 777 113.1 / 109.5 / 103.6, 1500 158.4 / 153.2 / 157.5; 2048: 300
+// 105.3 / 96.6 / 103.2, 8192 808.8 / 817.2 / 808.6.  No launch to pack in: attention blocks of 768 with 300 rows handed
+// in 21.4 / 18.4 / 15.5, of 1600 31.8 / 30.0 / 23.8; both blocks of 3200, 300 rows 262 / 211 / 180.
 struct BlockWeights {
   const void *W1, *W2;
   void *ws1, *ws2;
   int K1, N1, K2, N2;
   bool packed, f16;
-  bool in_place = false;
-  const void* first() const { return packed || in_place ? W1 : ws1; }
-  const void* second() const { return packed || in_place ? W2 : ws2; }
-  int multiply(const void* A, const void* B, int64_t M, int N, int K, const GemmEpilogue& ep, hipStream_t st) const {
-    return in_place ? launch_gemm_kn(A, B, M, N, K, ep, st) : launch_gemm(A, B, M, N, K, ep, st);
+  bool first_in_place = false, second_in_place = false;
+  const void* first() const { return packed || first_in_place ? W1 : ws1; }
+  const void* second() const { return packed || second_in_place ? W2 : ws2; }
+  int multiply_first(const void* A, int64_t M, const GemmEpilogue& ep, hipStream_t st) const {
+    return first_in_place ? launch_gemm_kn(A, W1, M, N1, K1, ep, st) : launch_gemm(A, first(), M, N1, K1, ep, st);
   }
+  int multiply_second(const void* A, int64_t M, const GemmEpilogue& ep, hipStream_t st) const {
+    return second_in_place ? launch_gemm_kn(A, W2, M, N2, K2, ep, st) : launch_gemm(A, second(), M, N2, K2, ep, st);
+  }
+  // columns to be packed
+  int n1() const { return packed || first_in_place ? 0 : N1; }
+  int n2() const { return packed || second_in_place ? 0 : N2; }
   void build(hipStream_t st) const {
-    if (!packed && !in_place) launch_pack_transpose_pair(W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
+    if (n1() + n2() > 0) launch_pack_transpose_pair(W1, ws1, K1, n1(), W2, ws2, K2, n2(), f16, st);
   }
   // together with the block's LayerNorm, to fp16
   void build_and_normalise(const void* x, const void* ln_w, const void* ln_b, void* normed, int64_t M, int h,
                            float eps, hipStream_t st) const {
-    if (packed || in_place) launch_layernorm(x, ln_w, ln_b, normed, M, h, eps, f16, true, st);
+    if (n1() + n2() == 0) launch_layernorm(x, ln_w, ln_b, normed, M, h, eps, f16, true, st);
     else
-      launch_layernorm_pack_pair(x, ln_w, ln_b, normed, M, h, eps, W1, ws1, K1, N1, W2, ws2, K2, N2, f16, st);
+      launch_layernorm_pack_pair(x, ln_w, ln_b, normed, M, h, eps, W1, ws1, K1, n1(), W2, ws2, K2, n2(), f16, st);
   }
 };
-// A block packs its plain weights in its LayerNorm's own launch, which leaves the images in the memory-side
-// cache; a product that reads [K][N] in place takes 2-5 us more where few rows meet a long K, as its narrow
-// tiles then read short pieces of the weights' rows.  Whole forwards with plain weights, us, packed / in place:
-// width 768: 24 rows 569 / 535, 128 rows 567 / 533, 488 rows 638 / 583; width 1600: 40 rows 2778 / 2657, 300
-// rows 3838 / 3683; width 1024: 186 rows 1174 / 1224, 512 rows 1328 / 1506, 1024 rows 1813 / 1906, 1500 rows
-// 2266 / 2269; width 1280: 50 rows 1748 / 1897, 300 rows 2361 / 2433, 1024 rows 3713 / 3595.
-static bool reads_in_place(int64_t M, int64_t h) {
-  return h <= 768 || h > 1280 || M >= (h > 1024 ? 1024 : 1536);
-}
 // The one launch in front of a short sequences' projection: of few pairs it takes longer than the two it stands
 // for, but an eager forward that small waits for the host, which then has a launch less a block.  A graph's replay
 // does not.  124M, weights from HBM, us, in two launches / in one: eager 1 x 24 tokens 313 / 297, 2 x 24 319 / 309, 4 x 32
@@ -697,8 +706,8 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   eo.out = out;
   eo.drop = drop;
   eo.f16 = f16;
-  bw.in_place = !bw.packed && !prologue && reads_in_place(M, h) && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep) &&
-                gemm_reads_kn(W_proj, M, (int)h, (int)h, eo);
+  bw.first_in_place = !bw.packed && !prologue && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep);
+  bw.second_in_place = bw.first_in_place && (normed || !layernorm_packs((int)h)) && gemm_reads_kn(W_proj, M, (int)h, (int)h, eo);
   const void *Bq = bw.first(), *Bp = bw.second();
   if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
     set_error("attention_block: the weights must be 16-byte aligned");
@@ -724,7 +733,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
       if (f16 && ((uintptr_t)normed & 15) == 0) A = normed;
       else launch_pack_rows(normed, pl.normed, M, (int)h, (int)h, f16, st);
     }
-    rc = bw.multiply(A, Bq, M, (int)(3 * h), (int)h, ep, st);
+    rc = bw.multiply_first(A, M, ep, st);
   }
   if (rc) return rc;
   if (!front) {
@@ -732,7 +741,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
              : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st, ahead);
     if (rc) return rc;
   }
-  rc = bw.multiply(pl.merged, Bp, M, (int)h, (int)h, eo, st);
+  rc = bw.multiply_second(pl.merged, M, eo, st);
   if (rc) return rc;
   return check_launch("attention_block");
 }
@@ -790,8 +799,8 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e2.out = out;
   e2.drop = drop;
   e2.f16 = f16;
-  bw.in_place = !bw.packed && !prologue && reads_in_place(M, H) && gemm_reads_kn(W1, M, (int)inner, (int)H, e1) &&
-                gemm_reads_kn(W2, M, (int)H, (int)inner, e2);
+  bw.first_in_place = !bw.packed && !prologue && gemm_reads_kn(W1, M, (int)inner, (int)H, e1);
+  bw.second_in_place = bw.first_in_place && !layernorm_packs((int)H) && gemm_reads_kn(W2, M, (int)H, (int)inner, e2);
   const void *B1 = bw.first(), *B2 = bw.second();
   if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
     set_error("mlp_block: the weights must be 16-byte aligned");
@@ -802,10 +811,10 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, B1, M, (int)inner, (int)H, e1, st);
   } else {
     bw.build_and_normalise(x, ln_w, ln_b, pl.normed, M, (int)H, eps, st);
-    rc = bw.multiply(pl.normed, B1, M, (int)inner, (int)H, e1, st);
+    rc = bw.multiply_first(pl.normed, M, e1, st);
   }
   if (rc) return rc;
-  rc = bw.multiply(pl.inner, B2, M, (int)H, (int)inner, e2, st);
+  rc = bw.multiply_second(pl.inner, M, e2, st);
   if (rc) return rc;
   return check_launch("mlp_block");
 }

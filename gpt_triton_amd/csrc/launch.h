@@ -37,7 +37,7 @@ void launch_pack_rows(const void* src, void* dst, int64_t R, int K, int Kp, bool
                       hipStream_t st);
 void launch_pack_transpose(const void* src, void* dst, int K, int N, int Kp, bool f16,
                            hipStream_t st);
-// two weights, K1 and K2 multiples of 64
+// two weights, K1 and K2 multiples of 64; N1 or N2 may be 0
 void launch_pack_transpose_pair(const void* s1, void* d1, int K1, int N1, const void* s2, void* d2, int K2,
                                 int N2, bool f16, hipStream_t st);
 
@@ -46,6 +46,8 @@ void launch_pack_transpose_pair(const void* s1, void* d1, int K1, int N1, const 
 void launch_layernorm_pack_pair(const void* x, const void* w, const void* b, void* out, int64_t M, int H,
                                 float eps, const void* s1, void* d1, int K1, int N1, const void* s2, void* d2,
                                 int K2, int N2, bool f16, hipStream_t st);
+// whether fp16 rows of this width leave room for that
+bool layernorm_packs(int H);
 
 // Epilogue description of one GEMM launch: out = gelu?(acc + bias) + residual,
 // stored either as a plain [M][N] matrix or scattered into q/k/v [B][heads][L][d].

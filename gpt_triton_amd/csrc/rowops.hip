@@ -824,8 +824,8 @@ static void launch_pack_pair_t(const void* s1, void* d1, int K1, int N1, const v
 void launch_pack_transpose_pair(const void* s1, void* d1, int K1, int N1, const void* s2, void* d2, int K2,
                                 int N2, bool f16, hipStream_t st) {
   if (!pack_vec_ok(s1, d1, N1, K1) || !pack_vec_ok(s2, d2, N2, K2)) {
-    launch_pack_transpose(s1, d1, K1, N1, K1, f16, st);
-    launch_pack_transpose(s2, d2, K2, N2, K2, f16, st);
+    if (N1 > 0) launch_pack_transpose(s1, d1, K1, N1, K1, f16, st);
+    if (N2 > 0) launch_pack_transpose(s2, d2, K2, N2, K2, f16, st);
   } else if (f16) {
     launch_pack_pair_t<_Float16>(s1, d1, K1, N1, s2, d2, K2, N2, st);
   } else {
@@ -847,8 +847,10 @@ static void lnp_go(const void* x, const void* w, const void* b, void* out, int64
                        (const T*)b, (_Float16*)out, M, H, eps, tiles, p1, p2);
 }
 
-// False where the two do not go into one launch: unaligned rows, parameters or weights, rows of more than
-// 4 chunks a lane (the registers of longer ones would leave the packing few wavefronts), too many blocks.
+constexpr int kPackChunks = 4;  // of a lane: the registers of longer rows would leave the packing few wavefronts
+bool layernorm_packs(int H) { return H <= kPackChunks * 64 * Vec<_Float16>::N; }
+
+// False where the two do not go into one launch: unaligned rows, parameters or weights, long rows, too many blocks.
 template <typename T>
 static bool launch_layernorm_pack_t(const void* x, const void* w, const void* b, void* out, int64_t M, int H,
                                     float eps, const void* s1, void* d1, int K1, int N1, const void* s2,
@@ -859,7 +861,7 @@ static bool launch_layernorm_pack_t(const void* x, const void* w, const void* b,
     return false;
   const int lpr = lanes_per_row(H / VN), need = (H / VN + lpr - 1) / lpr;
   const int64_t blocks = lpr == 32 ? (M + 7) / 8 : (M + 3) / 4;
-  if (need > 4 || blocks >= (1ll << 30)) return false;
+  if (need > kPackChunks || blocks >= (1ll << 30)) return false;
   const PackArgs<T> p1 = pack_args<T>(s1, d1, K1, N1, K1), p2 = pack_args<T>(s2, d2, K2, N2, K2);
   if (need <= 1) lnp_go<T, 1>(x, w, b, out, M, H, eps, lpr, blocks, p1, p2, st);
   else if (need <= 2) lnp_go<T, 2>(x, w, b, out, M, H, eps, lpr, blocks, p1, p2, st);

@@ -73,3 +73,24 @@ def test_training_blocks(K, gpu_device, B, L, h, heads):
             plain = call(x, lw, lb, *ws, *more, dropout_prob=0.1, keep=keep)
             packed = call(x, lw, lb, *images, *more, dropout_prob=0.1, keep=keep)
             assert torch.isfinite(plain).all() and torch.equal(plain, packed)
+
+
+@pytest.mark.parametrize("B,L,h,heads", [(1, 24, 768, 12), (3, 341, 896, 14), (1, 100, 1280, 20), (2, 777, 1600, 25),
+                                         (2, 150, 2048, 32), (3, 50, 2112, 33), (1, 300, 2560, 20)])
+def test_blocks_of_any_width(K, gpu_device, B, L, h, heads):
+    """The second weight of a block packed in the LayerNorm's launch and, behind rows that are handed in normalised and
+    rows too wide for that, read in place; a second weight that has to be packed by itself."""
+    print(f"weight in place, blocks: {B} x {L} rows of {h}", flush=True)
+    draw, wq, bq = weights(gpu_device, h, 3 * h, B)
+    _, wp, bp = weights(gpu_device, h, h, B + 1)
+    _, w1, b1 = weights(gpu_device, h, 4 * h, B + 2)
+    _, w2, b2 = weights(gpu_device, 4 * h, h, B + 3)
+    x, lw, lb, y = draw(B, L, h), draw(h), draw(h), draw(B, L, h)
+    for call, ws, rest in ((K.attention_block, (wq, bq, wp, bp, heads), {}), (K.mlp_block, (w1, b1, w2, b2), {}),
+                           (K.attention_block, (wq, bq, wp, bp, heads), {"normed": y})):
+        images = [K.pack_weight(t) if torch.is_tensor(t) and t.dim() == 2 else t for t in ws]
+        shifted = torch.empty(ws[2].numel() + 4, device=gpu_device, dtype=torch.float16)[4:].view(ws[2].shape)
+        shifted.copy_(ws[2])  # 8-byte aligned
+        want = call(x, lw, lb, *images, **rest)
+        assert torch.isfinite(want).all() and torch.equal(call(x, lw, lb, *ws, **rest), want)
+        assert torch.equal(call(x, lw, lb, *ws[:2], shifted, *ws[3:], **rest), want)
