@@ -1251,6 +1251,10 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp, const G
                : launch_shape<float, float, false>(A, Bt, M, N, Kp, ep, st);
 }
 
+static bool disjoint(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  return (uintptr_t)a + a_bytes <= (uintptr_t)b || (uintptr_t)b + b_bytes <= (uintptr_t)a;
+}
+
 // Wherever the tile kernel takes all rows: every size gains (microseconds, weights from HBM, transposed first /
 // in place / packed once: 16 x 768 x 2304 6.7 / 3.9 / 3.4, 16 x 3072 x 768 8.9 / 7.8 / 4.8, 128 x 768 x 3072 10.4 / 5.7
 // / 5.1, 128 x 3072 x 768 12.8 / 8.8 / 6.2, 600 x 768 x 768 8.2 / 5.4 / 5.1, 1477 x 768 x 3072 19.3 / 13.4 / 12.7, 4800 x
@@ -1258,9 +1262,14 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp, const G
 // being 32 bytes of theirs.  In the persistent kernel without a residual, whole column tiles, up to the rows at which
 // the 1 to 2 % that it takes longer are what the transposition takes (4800 x 768 x 3072 31.4 / 26.2 / 24.8, 9600 x 768 x
 // 3072 54.7 / 49.2 / 48.5, 40000 x 768 x 3072 203 / 202 / 198).
+// Not where an output lies over the weight, whose image is complete before the first output is stored.
 bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e) {
   EpiDev ep;
   int64_t head;
+  const size_t w_bytes = (size_t)K * N * 2, out_bytes = (size_t)M * N * 2, part = out_bytes / 3;
+  if (e.qkv ? !disjoint(W, w_bytes, e.q, part) || !disjoint(W, w_bytes, e.k, part) || !disjoint(W, w_bytes, e.v, part)
+            : !disjoint(W, w_bytes, e.out, out_bytes))
+    return false;
   if (!e.f16 || K % 64 != 0 || ((uintptr_t)W & 15) != 0 || !gemm_tile_reads_kn(N, K) || make_epi(e, M, N, ep) != 0)
     return false;
   if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)

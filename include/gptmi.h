@@ -170,7 +170,8 @@ int gptmi_pack_weight(const void* W, void* packed, int64_t N, int64_t K, int wla
  *   x [M][K]   W [K][N] (GPTMI_W_KN), [N][K] (GPTMI_W_NK) or packed (GPTMI_W_PACKED)
  *   bias [N] or NULL
  *   residual [M][N] or NULL     out [M][N] (may be the residual's own memory: every
- *                               element is read before it is written)
+ *                               element is read before it is written, or that of a W in layout
+ *                               GPTMI_W_KN, which is copied first then; no other operand's)
  * workspace: at least gptmi_linear_workspace_bytes(...) bytes, 256-byte aligned
  * (may be NULL when that is 0).
  * Any M >= 1 (below 2^31 - 512), 1 <= N <= 2^26, 1 <= K <= 2^30 (GPTMI_ERR_UNSUPPORTED beyond)

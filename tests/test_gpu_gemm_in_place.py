@@ -94,3 +94,50 @@ def test_blocks_of_any_width(K, gpu_device, B, L, h, heads):
         want = call(x, lw, lb, *images, **rest)
         assert torch.isfinite(want).all() and torch.equal(call(x, lw, lb, *ws, **rest), want)
         assert torch.equal(call(x, lw, lb, *ws[:2], shifted, *ws[3:], **rest), want)
+
+
+@pytest.mark.parametrize("M,k,n", [(100, 768, 768), (128, 768, 3072), (600, 3072, 768), (4800, 6400, 768), (4700, 6400, 768)])
+def test_output_over_the_weight(K, gpu_device, M, k, n):
+    """A weight that the output lies over is copied before it is multiplied, the output at its start and across its
+    end, in products and as the second of a block, where it is read in place otherwise."""
+    print(f"output over the weight: {M} x {k} x {n}", flush=True)
+    draw, w, b = weights(gpu_device, k, n, M)
+    x = draw(M, k)
+    want = K.fused_ffn(x, w, bias=b)
+    room = torch.empty(k * n + M * n, device=gpu_device, dtype=torch.float16)
+    for at in (0, k * n - min(M, k) * n // 2 // 8 * 8):
+        room[:k * n] = w.view(-1)
+        out = room[at:at + M * n].view(M, n)
+        K._linear(x, room[:k * n].view(k, n), b, None, out, False, 0.0, K._lib.GPTMI_W_KN, "over the weight")
+        assert torch.equal(out, want)
+    if n % 192 == 0:
+        parts = K.matmul_and_split_qkv(x.view(1, M, k), w, b, n // 192)
+        lib, ws = K._lib.load(), torch.empty(k * n * 2 + 256, device=gpu_device, dtype=torch.uint8)
+        ws = ws[-ws.data_ptr() % 256:]
+        room[:k * n] = w.view(-1)
+        q, kk, v = room[:M * n].view(3, M * n // 3)
+        rc = lib.gptmi_linear_qkv(x.data_ptr(), room.data_ptr(), b.data_ptr(), q.data_ptr(), kk.data_ptr(), v.data_ptr(),
+                                  1, M, n // 192, 64, k, K._lib.GPTMI_W_KN, ws.data_ptr(), k * n * 2, K._lib.GPTMI_F16,
+                                  torch.cuda.current_stream().cuda_stream)
+        K._lib.check(rc, "linear_qkv")
+        for got, part in zip((q, kk, v), parts):
+            assert torch.equal(got, part.view(-1))
+
+
+def test_block_over_its_weight(K, gpu_device):
+    B, L, h, heads = 2, 150, 768, 12
+    print("block's output over its second weight", flush=True)
+    draw, wq, bq = weights(gpu_device, h, 3 * h, 1)
+    _, wp, bp = weights(gpu_device, h, h, 2)
+    x, y, lw, lb = draw(B, L, h), draw(B, L, h), draw(h), draw(h)
+    want = K.attention_block(x, lw, lb, wq, bq, wp, bp, heads, normed=y)
+    lib = K._lib.load()
+    nbytes = lib.gptmi_attention_block_workspace_bytes(B, L, heads, h // heads, K._lib.GPTMI_W_KN)
+    ws = torch.empty(nbytes + 256, device=gpu_device, dtype=torch.uint8)
+    ws = ws[-ws.data_ptr() % 256:]
+    rc = lib.gptmi_attention_block(x.data_ptr(), y.data_ptr(), lw.data_ptr(), lb.data_ptr(), 1e-5, wq.data_ptr(),
+                                   bq.data_ptr(), wp.data_ptr(), bp.data_ptr(), wp.data_ptr(), B, L, heads, h // heads, 0.0,
+                                   1337, None, 0, 0, K._lib.GPTMI_W_KN, ws.data_ptr(), nbytes, K._lib.GPTMI_F16,
+                                   torch.cuda.current_stream().cuda_stream)
+    K._lib.check(rc, "attention_block")
+    assert torch.equal(wp.view(-1)[:B * L * h], want.view(-1))
