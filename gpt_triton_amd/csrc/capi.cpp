@@ -855,40 +855,6 @@ size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t
   return 2 * (size_t)round_up(M * h * (dtype == GPTMI_F16 ? 2 : 4), 256) + (a > m ? a : m);
 }
 
-// What an attention launch requests of the weights that come behind it (prefetch_workgroups): the MLP's second
-// product first, which has the longest columns, then the next layer's first product, then what follows at once; half a
-// matrix saves nothing, and what the launch has to wait for costs what it saves.  Launches of as many workgroups as
-// CUs and those of the front kernel last long enough for some 15 MB and 40 KB more for each key row, launches of
-// few pairs for 120 KB a key row, and the second product alone is worth a wait of its 14 MB or less.  Forwards that
-// find their weights in HBM (four models in turn; wider ones always do), us, nothing / the second product alone /
-// this: 124M 1 x 24 tokens 342 / 335 / 303, 2 x 64 370 / 357 / 356 (15 MB: 368), 7 x 211 751 / 724 / 674, 1 x 800
-// 713 / 695 / 651; 100 x 40 1274 / - / 1164 (120 KB a row: 1217); 1024 wide 1 x 41 707 / 698 / 697 (15 MB: 715), 4 x 160
-// 1390 / - / 1237, 2 x 200 1168 / 1148 / 1115; 1280 wide 2 x 60 1641 / 1545, 2 x 200 2376 / 2320 / 2239; 1600 wide
-// 1 x 41 1925 / 1959 / 1925, 1 x 150 2616 / 2478 / 2478, 1 x 300 3349 / 3174 / 3100, 1 x 500 4287 / 3851 / 3851 (60 MB:
-// 3972).  One 124M model over and over, whose weights the memory-side cache holds: equal.
-static Prefetch weights_ahead(const void* const* layer, bool last, int64_t B, int64_t L, int64_t heads, int64_t h,
-                              int64_t inner, hipStream_t st) {
-  const size_t square = (size_t)(h * h * 2), wide = (size_t)(h * inner * 2);
-  const struct {
-    const void* p;
-    size_t bytes;
-  } wanted[4] = {{layer[10], wide}, {last ? nullptr : layer[12 + 2], 3 * square}, {layer[8], wide}, {layer[4], square}};
-  const size_t rows = (size_t)L, alone = 15000000 + 40000 * rows;
-  if (wide > alone) return Prefetch();
-  const bool lasting = B * heads > cu_count() - 64 || (attn_front_supported(B, L, heads, h) && front_pays(B * heads, st));
-  const size_t by_row = 120000 * rows < 40000000 ? 120000 * rows : 40000000;
-  const size_t most = lasting && alone > by_row ? alone : by_row;
-  Prefetch ahead;
-  size_t sum = 0;
-  for (int k = 0; k < 4; ++k) {
-    if (wanted[k].p == nullptr) continue;
-    sum += wanted[k].bytes;
-    if (k > 0 && sum > most) break;
-    ahead.p[k] = wanted[k].p, ahead.bytes[k] = wanted[k].bytes;
-  }
-  return ahead;
-}
-
 int gptmi_blocks(const void* x, const void* normed, const void* const* params, int64_t n, float eps,
                  void* out, int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner,
                  int fuse_layernorm, void* workspace, size_t workspace_bytes, int dtype, void* stream) {
@@ -910,9 +876,12 @@ int gptmi_blocks(const void* x, const void* normed, const void* const* params, i
   void *mid = c.take(mat), *next = c.take(mat);
   char* ws = (char*)workspace + c.used;
   const size_t ws_bytes = workspace_bytes - c.used;
+  const bool lasting = B * heads > cu_count() - 64 ||
+                       (attn_front_supported(B, L, heads, h) && front_pays(B * heads, (hipStream_t)stream));
+  const AheadPlan plan = plan_ahead(L, lasting, h, inner);
   for (int64_t i = 0; i < n; ++i) {
     const void* const* p = params + 12 * i;
-    const Prefetch ahead = weights_ahead(p, i + 1 == n, B, L, heads, h, inner, (hipStream_t)stream);
+    const Prefetch ahead = weights_ahead(p, i + 1 == n, plan);
     int rc = attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B, L, heads,
                              d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream, &ahead);
     if (rc) return rc;

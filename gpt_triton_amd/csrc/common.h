@@ -53,7 +53,7 @@ struct PrefetchArgs {
 };
 inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
   PrefetchArgs a = {};
-  for (int k = 0; ahead && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
+  for (int k = 0; ahead != nullptr && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
   return a;
 }
 // Workgroups for it, behind the `workers` of the launch: the CUs that these leave idle, or 128 that find room as the
@@ -61,7 +61,7 @@ inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
 // 2440 / 2266 / 2268, 16 x 512 2054 / 1922 / 1899, 64 x 300 3977 / 3940 / 3928; 1024 wide 8 x 1024 6024 / 5661 /
 // 5623, 1280 wide 4 x 700 5855 / 5514 / 5361).
 inline int prefetch_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
-  return ahead == nullptr ? 0 : workers <= cus - 64 ? cus - (int)workers : 128;
+  return ahead == nullptr || ahead->empty() ? 0 : workers <= cus - 64 ? cus - (int)workers : 128;
 }
 template <int NT>
 __device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int block, int blocks) {

@@ -1603,12 +1603,12 @@ int launch_stream_attn(const void* q, const void* k, const void* v, void* out, i
   if (cus < 0) return cus;
   const int Lp = (L + BKEY - 1) / BKEY * BKEY;
   const int workers = BN < cus ? (int)BN : cus;
-  // One full round of pairs ends all at once, and what comes behind it then is not hidden: 64 prefetching workgroups
-  // instead of 128 (20 x 300 tokens of 124M none / 64 / 128 1523 / 1487 / 1516 us), and none behind short pairs for
-  // weights that a model may find in the memory-side cache (21 x 128 tokens of 124M, its weights there / in HBM, 763 /
-  // 913 without, 808 / 845 with).
-  int further = prefetch_workgroups(ahead, BN, cus);
-  if (ahead != nullptr && BN > cus - 64 && BN <= cus) further = L <= 128 && ahead->bytes[0] <= 5000000 ? 0 : 64;
+  // One full round of pairs ends all at once, and what comes behind it then is not hidden: none for weights that
+  // may be in the memory-side cache (us, none / 64 / 128 workgroups: 124M, its weights there, 21 x 128 tokens 823 / 859 /
+  // 849, 20 x 300 1565 / 1585 / 1581; in HBM 935 / 919 / 892, 1611 / 1605 / 1604; 1024 wide 15 x 128 2081 / 2057 / 2028,
+  // 15 x 300 3805 / 3845 / 3738; 1280 wide 12 x 200 5568 / 5398 / 5327)
+  const bool one_round = BN > cus - 64 && BN <= cus;
+  const int further = one_round && ahead != nullptr && ahead->may_be_cached ? 0 : prefetch_workgroups(ahead, BN, cus);
   const int grid = workers + further;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), (size_t)Lp * 512, st,
                      (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out,

@@ -4,14 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace gptmi {
+#include "weights_ahead.h"
 
-// What the launches behind this one will read (weights): an attention launch has further workgroups request it from
-// HBM into the memory-side cache, on the CUs that it leaves idle.
-struct Prefetch {
-  const void* p[4] = {};
-  size_t bytes[4] = {};
-};
+namespace gptmi {
 
 // Dropout of one launch: probability p (0 = none) and the 64-bit seed of the generator.
 struct Dropout {

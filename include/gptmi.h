@@ -335,6 +335,8 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
  *           b_qkv, W_proj, b_proj of the attention block, then ln_w, ln_b, W1, b1, W2, b2 of the MLP
  *   x, out [B*L][h], which may be the same   normed: LayerNorm(x) of the first layer, or NULL
  *   Everything that a layer's calls refuse is refused before the first launch.
+ *   Attention launches of head size 64 also read ahead of the weights that come behind them, all of them
+ *   within the n layers' images, where that is found to pay.
  *   inner, fuse_layernorm, workspace: as for those two calls, for every layer
  */
 size_t gptmi_blocks_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d, int64_t inner, int dtype);
