@@ -252,20 +252,20 @@ int launch_front(const void* x, const void* Bt, const void* bias, void* out, int
 
 }  // namespace
 
-bool attn_front_supported(int64_t B, int64_t L, int64_t heads, int64_t h) {
-  if (L > ROWS || h > 768 || heads * 64 != h) return false;
+int attn_front_split(int64_t B, int64_t L, int64_t heads, int64_t h) {
+  if (L > ROWS || h > 768 || heads * 64 != h) return 0;
   const int cus = cu_count();
-  return cus > 0 && B * heads <= cus && gemm_qkv_split(B * L, (int)(3 * h), (int)h, L, (int)heads, 64) > 0;
+  const int wk = cus > 0 && B * heads <= cus ? gemm_qkv_split(B * L, (int)(3 * h), (int)h, L, (int)heads, 64) : 0;
+  return wk > 0 ? wk : 0;
 }
 
-int launch_attn_front(const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
+int launch_attn_front(int split, const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
                       const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st,
                       const Prefetch* ahead) {
   const int H = (int)heads * 64;
   const LnArgs ln = {ln_w, ln_b, eps, lanes_per_row(H / 8)};
-  const int wk = gemm_qkv_split(B * L, 3 * H, H, L, (int)heads, 64);
   const auto go = [&](auto kernel) { return kernel(x, Bt, bias, out, B, (int)heads, (int)L, H, scale, ln, st, ahead); };
-  switch (wk) {
+  switch (split) {
     case 4: return normed ? go(launch_front<4, true>) : go(launch_front<4, false>);
     case 2: return normed ? go(launch_front<2, true>) : go(launch_front<2, false>);
     default: return normed ? go(launch_front<1, true>) : go(launch_front<1, false>);

@@ -258,6 +258,11 @@ static bool front_pays(int64_t pairs, hipStream_t st) {
   if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
   return status == hipStreamCaptureStatusNone;
 }
+// The split of that launch (attn_front_split), 0 where it is not taken.
+static int front_split(int64_t B, int64_t L, int64_t heads, int64_t d, bool f16, hipStream_t st) {
+  const int split = f16 && d == 64 ? attn_front_split(B, L, heads, heads * d) : 0;
+  return split > 0 && gemm_layernorm_supported(B * L, (int)(heads * d)) && front_pays(B * heads, st) ? split : 0;
+}
 static size_t image_bytes(int64_t N, int64_t K, int wlayout) {
   return wlayout == GPTMI_W_PACKED ? 0 : (size_t)(N * round_up(K, 64) * 2);
 }
@@ -655,11 +660,18 @@ size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads
   return plan_attention(nullptr, B * L, heads * d, wlayout).total;
 }
 
+// What gptmi_blocks knows of a layer: front_split, the same for all of them, and what to request ahead.
+struct Stack {
+  int front;
+  Prefetch ahead;
+};
+
 static int attention_block(const void* x, const void* normed, const void* ln_w, const void* ln_b, float eps,
                           const void* W_qkv, const void* b_qkv, const void* W_proj, const void* b_proj,
                           void* out, int64_t B, int64_t L, int64_t heads, int64_t d, float p,
                           uint64_t seed, const void* keep, int64_t keep_bits, int fuse_layernorm, int wlayout, void* workspace,
-                          size_t workspace_bytes, int dtype, void* stream, const Prefetch* ahead) {
+                          size_t workspace_bytes, int dtype, void* stream, const Stack* stack) {
+  const Prefetch* ahead = stack ? &stack->ahead : nullptr;
   if (!x || !ln_w || !ln_b || !W_qkv || !W_proj || !out || B <= 0 || L <= 0 || heads <= 0 || d <= 0) {
     set_error("attention_block: invalid argument");
     return GPTMI_ERR_INVALID;
@@ -716,11 +728,10 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   const float scale = (float)(1.0 / sqrt((double)d));
   // short sequences: everything in front of the projection in one launch
   const void* rows = normed ? normed : x;
-  const bool front = f16 && bw.packed && p == 0.f && d == 64 && attn_front_supported(B, L, heads, h) &&
-                     gemm_layernorm_supported(M, (int)h) && prologue_aligned(rows, ln_w, ln_b) &&
-                     ((uintptr_t)b_qkv & 15) == 0 && front_pays(B * heads, st);
-  if (front) {
-    rc = launch_attn_front(rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st, ahead);
+  const int front = !bw.packed || p > 0.f || !prologue_aligned(rows, ln_w, ln_b) || ((uintptr_t)b_qkv & 15) != 0 ? 0
+                    : stack ? stack->front : front_split(B, L, heads, d, f16, st);
+  if (front > 0) {
+    rc = launch_attn_front(front, rows, normed != nullptr, ln_w, ln_b, eps, Bq, b_qkv, pl.merged, B, L, heads, scale, st, ahead);
   } else if (prologue) {
     bw.build(st);
     rc = launch_gemm_layernorm(x, ln_w, ln_b, eps, Bq, M, (int)(3 * h), (int)h, ep, st);
@@ -736,7 +747,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
     rc = bw.multiply_first(A, M, ep, st);
   }
   if (rc) return rc;
-  if (!front) {
+  if (front == 0) {
     rc = f16 ? launch_flash_attn(pl.q, pl.k, pl.v, pl.merged, B, heads, L, L, (int)d, scale, drop, true, true, st, ahead)
              : launch_flash_attn_operands(pl.q, pl.k, pl.v, pl.merged, B, heads, L, (int)d, scale, drop, st, ahead);
     if (rc) return rc;
@@ -876,14 +887,13 @@ int gptmi_blocks(const void* x, const void* normed, const void* const* params, i
   void *mid = c.take(mat), *next = c.take(mat);
   char* ws = (char*)workspace + c.used;
   const size_t ws_bytes = workspace_bytes - c.used;
-  const bool lasting = B * heads > cu_count() - 64 ||
-                       (attn_front_supported(B, L, heads, h) && front_pays(B * heads, (hipStream_t)stream));
-  const AheadPlan plan = plan_ahead(L, lasting, h, inner);
+  Stack stack = {front_split(B, L, heads, d, dtype == GPTMI_F16, (hipStream_t)stream), Prefetch()};
+  const AheadPlan plan = plan_ahead(L, B * heads > cu_count() - 64 || stack.front > 0, h, inner);
   for (int64_t i = 0; i < n; ++i) {
     const void* const* p = params + 12 * i;
-    const Prefetch ahead = weights_ahead(p, i + 1 == n, plan);
+    stack.ahead = weights_ahead(p, i + 1 == n, plan);
     int rc = attention_block(x, i == 0 ? normed : nullptr, p[0], p[1], eps, p[2], p[3], p[4], p[5], mid, B, L, heads,
-                             d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream, &ahead);
+                             d, 0.0f, 1337, nullptr, 0, fuse_layernorm, GPTMI_W_PACKED, ws, ws_bytes, dtype, stream, &stack);
     if (rc) return rc;
     // x is not read again: the layer's output may take its place
     void* y = i + 1 == n ? out : next;

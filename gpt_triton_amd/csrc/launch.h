@@ -85,9 +85,9 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
 
 // LayerNorm (unless x is normed), q, k, v product (packed weight image Bt [3h][h]) and causal attention of short
 // sequences in one launch: fp16, head size 64, out [B][L][heads][64], the bits of the launches it stands for.  All
-// pointers 16-byte aligned.
-bool attn_front_supported(int64_t B, int64_t L, int64_t heads, int64_t h);
-int launch_attn_front(const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
+// pointers 16-byte aligned.  split: attn_front_split's, the product's groups of k-slices, or 0 for what it does not take.
+int attn_front_split(int64_t B, int64_t L, int64_t heads, int64_t h);
+int launch_attn_front(int split, const void* x, bool normed, const void* ln_w, const void* ln_b, float eps, const void* Bt,
                       const void* bias, void* out, int64_t B, int64_t L, int64_t heads, float scale, hipStream_t st,
                       const Prefetch* ahead = nullptr);
 
