@@ -56,3 +56,30 @@ def test_every_pair_and_block(K, gpu_device, B, N, L, d):
                                      (1, 131, 1000, 128)])
 def test_pairs_of_no_xcd(K, gpu_device, B, N, L, d):
     test_every_pair_and_block(K, gpu_device, B, N, L, d)
+
+
+def test_more_pairs_than_a_grid_dimension(K, gpu_device):
+    """65600 pairs of 129 rows, the fewest that the wide kernel takes at d = 128."""
+    test_every_pair_and_block(K, gpu_device, 41, 1600, 129, 128)
+
+
+# the ring kernel, fewer and more than 1024 blocks, whole eights of pairs and not; the wide kernel likewise
+@pytest.mark.parametrize("B,heads,L,d", [(3, 3, 330, 64), (43, 8, 330, 64), (49, 7, 330, 64), (5, 3, 300, 128), (87, 4, 300, 128),
+                                         (2, 3, 129, 256), (174, 2, 300, 256)])
+def test_blocks_of_fp32_models(K, gpu_device, B, heads, L, d):
+    """The forms with the fp32 softmax, which an attention block of fp32 storage runs on its fp16 q, k, v: weights of
+    one identity each make these the normalised rows and the projection the attention's output."""
+    print(f"fp32 attention block dealt to workgroups: {B * heads} pairs, L={L}, d={d}", flush=True)
+    h = heads * d
+    g = torch.Generator(device=gpu_device).manual_seed(L + B)
+    x = torch.randn(B, L, h, generator=g, device=gpu_device)
+    one, zero = torch.ones(h, device=gpu_device), torch.zeros(3 * h, device=gpu_device)
+    eye = torch.eye(h, device=gpu_device)
+    y = K.fused_layer_norm(x, one, zero[:h])
+    got = K.attention_block(x, one, zero[:h], eye.repeat(1, 3).contiguous(), zero, eye, zero[:h], heads) - x
+    assert torch.isfinite(got).all()
+    q = y.half().view(B, L, heads, d).transpose(1, 2).contiguous()
+    got = got.view(B, L, heads, d).transpose(1, 2)
+    for b in range(B):
+        worst = excess_over_bound(q[b:b + 1], q[b:b + 1], q[b:b + 1], got[b:b + 1])
+        assert worst <= 0, f"beyond the rounding bound by {worst:.3e} in batch {b}"

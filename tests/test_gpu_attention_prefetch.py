@@ -1,6 +1,7 @@
 """Layers in one call, whose attention launches have further workgroups that touch the weights behind them: the bits of
 the layers called one by one, where such workgroups fill idle CUs and where they follow a full round, for each of the
-attention kernels that take them, with the weight images at the very end of their allocations."""
+attention kernels that take them.  What they touch does not show in the output: test_weights_ahead.py holds it to
+the images."""
 import pytest
 import torch
 
@@ -11,7 +12,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,L,heads,dtype", [(2, 20, 4, "fp16"), (64, 24, 4, "fp16"), (3, 60, 4, "fp16"), (100, 50, 4, "fp16"),
                                              (2, 400, 4, "fp16"), (20, 500, 4, "fp16"), (150, 330, 4, "fp16"),
                                              (5, 200, 4, "fp16"), (60, 150, 4, "fp16"), (62, 128, 4, "fp16"),
-                                             (90, 300, 4, "fp16"), (2, 100, 4, "fp32"), (80, 200, 4, "fp32")])
+                                             (90, 300, 4, "fp16"), (2, 100, 4, "fp32"), (80, 200, 4, "fp32"),
+                                             # nothing to request; one round of pairs of layers too large for the cache
+                                             (2, 40, 25, "fp16"), (15, 128, 16, "fp16")])
 def test_layers_in_one_call(gpu_device, B, L, heads, dtype):
     from gpt_triton_amd import kernels as K
     print(f"prefetching layers: {B} x {L} rows, {heads} heads, {dtype}", flush=True)
