@@ -209,17 +209,21 @@ struct Carver {
 // The weight images that a block's two products read: the caller's (packed), or built into its workspace.
 // K1 and K2 are multiples of 64.  in_place: the first product reads the caller's [K][N] weight as it is.
 //
-// The first is read as the caller has it, [K][N], wherever it can be: its rows of 3 h or 4 h hold whole lines for a tile, and
-// the 0.1 to 2 us more that the product lasts are less than its share of the packing.  The second one's rows are
+// The first is read as the caller has it, [K][N], wherever it can be: its rows of 3 h or 4 h hold whole lines for a
+// tile, and the 0.1 to 2 us more that the product lasts are less than its share of the packing.  The second one's rows are
 // short where its K is long (K = 4 h): read in place it lasts 1 to 8 us more, at widths that are a power of 2 up to 15,
 // while its image is built in the LayerNorm's own launch, which has room, and stays in the memory-side cache.  Where
-// there is no such launch (normalised rows handed in, layernorm_packs) it is read in place too.  Blocks with plain
+// there is no such launch (normalised rows handed in, layernorm_packs) it is read in place too.  With more than some 6
+// rows for a column the products gain from the images what packing both costs (few_rows).  Blocks with plain
 // weights from HBM, us a layer, both packed / first in place / both in place: width 512, 50 rows 27.8 / 25.6 / 25.3;
 // 768: 24 34.3 / 31.4 / 33.2, 512 48.8 / 42.5 / 49.9, 2048 66.8 / 67.2 / 73.6; 896: 186 45.6 / 39.0 / 41.6;
 // 1024: 24 40.2 / 37.2 / 40.8, 512 51.5 / 51.0 / 58.9, 4800 164.9 / 163.5 / 168.5; 1280: 300 63.0 / 59.1 / 65.0, 777
 // 88.4 / 83.0 / 79.5; 1600: 100 60.9 / 54.6 / 54.6, 777 113.1 / 109.5 / 103.6, 1500 158.4 / 153.2 / 157.5; 2048: 300
 // 105.3 / 96.6 / 103.2, 8192 808.8 / 817.2 / 808.6.  No launch to pack in: attention blocks of 768 with 300 rows handed
-// in 21.4 / 18.4 / 15.5, of 1600 31.8 / 30.0 / 23.8; both blocks of 3200, 300 rows 262 / 211 / 180.
+// in 21.4 / 18.4 / 15.5, of 1600 31.8 / 30.0 / 23.8; both blocks of 3200, 300 rows 262 / 211 / 180.  Both packed / first in
+// place with dropout, many rows: 768: 3000 102.2 / 100.6, 4800 119.9 / 121.7, 8192 204.9 / 209.1; 1024: 4800 196.7 /
+// 194.3, 12000 380 / 381; 1280: 6000 292.0 / 290.4, 16384 791 / 792; 1600: 8192 591.5 / 590.6, 16384 1120 / 1129.
+static bool few_rows(int64_t M, int64_t h) { return M <= 6 * h; }
 struct BlockWeights {
   const void *W1, *W2;
   void *ws1, *ws2;
@@ -718,7 +722,7 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   eo.out = out;
   eo.drop = drop;
   eo.f16 = f16;
-  bw.first_in_place = !bw.packed && !prologue && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep);
+  bw.first_in_place = !bw.packed && !prologue && (normed || few_rows(M, h)) && gemm_reads_kn(W_qkv, M, (int)(3 * h), (int)h, ep);
   bw.second_in_place = bw.first_in_place && (normed || !layernorm_packs((int)h)) && gemm_reads_kn(W_proj, M, (int)h, (int)h, eo);
   const void *Bq = bw.first(), *Bp = bw.second();
   if (((uintptr_t)Bq & 15) || ((uintptr_t)Bp & 15)) {
@@ -810,7 +814,7 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e2.out = out;
   e2.drop = drop;
   e2.f16 = f16;
-  bw.first_in_place = !bw.packed && !prologue && gemm_reads_kn(W1, M, (int)inner, (int)H, e1);
+  bw.first_in_place = !bw.packed && !prologue && few_rows(M, H) && gemm_reads_kn(W1, M, (int)inner, (int)H, e1);
   bw.second_in_place = bw.first_in_place && !layernorm_packs((int)H) && gemm_reads_kn(W2, M, (int)H, (int)inner, e2);
   const void *B1 = bw.first(), *B2 = bw.second();
   if (((uintptr_t)B1 & 15) || ((uintptr_t)B2 & 15)) {
