@@ -8,8 +8,9 @@
 // accumulators to LDS, and one wavefront attends.  A head's panel of weights (295 KB at 768) passes through
 // one CU, and takes what the launch lasts beside the LayerNorm, so: one round of workgroups, and rows of up to 768
 // (forwards of 1 x 32, 4 x 32 and 16 x 32 tokens 1024 wide 795, 860 and 1143 us, 672, 823 and 1200 in the launches
-// it would replace).  At 768, before -> after: 1 x 24 tokens 328 -> 292 us, 2 x 24 329 -> 298, 4 x 32 343 -> 322, 8 x 24 413 ->
-// 346, 16 x 24 421 -> 385, 21 x 32 501 -> 451.
+// it would replace).  At 768, replayed, in the launches / so: 1 x 24 tokens 285 / 298 us, 2 x 24 301 / 311, 3 x 30 335 /
+// 331, 4 x 32 348 / 336, 8 x 24 403 / 363, 21 x 32 553 / 525: with few pairs, 12 workgroups pulling 295 KB of weights each,
+// it is the longer way for the GPU, and pays where the host sets the pace (front_pays).
 //
 // Bits: those of the launches it stands for.  The LayerNorm is theirs (normalise_panel); the product's
 // k-slices of 64 are summed in WK groups (slice t in group t % WK) that are added in order, as the tile that the

