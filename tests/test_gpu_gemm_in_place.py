@@ -55,8 +55,9 @@ def test_head_major_scatter(K, gpu_device, B, L, heads, d):
 
 @pytest.mark.parametrize("B,L,h,heads", [(1, 24, 128, 2), (2, 300, 768, 12), (16, 300, 768, 12), (3, 999, 1024, 16),
                                          (56, 300, 768, 12),
-                                         # either side of the rows from which these widths read in place
-                                         (5, 307, 1024, 16), (3, 512, 1024, 16), (3, 341, 1280, 20), (4, 256, 1280, 20)])
+                                         (5, 307, 1024, 16), (3, 512, 1024, 16), (3, 341, 1280, 20), (4, 256, 1280, 20),
+                                         # either side of the rows from which a block packs both weights
+                                         (6, 768, 768, 12), (6, 769, 768, 12)])
 def test_training_blocks(K, gpu_device, B, L, h, heads):
     """Dropout with its mask at hand and drawn in place, both blocks, weights plain and packed."""
     print(f"weight in place, training blocks: {B} x {L} rows of {h}", flush=True)
