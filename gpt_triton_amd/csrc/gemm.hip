@@ -1035,7 +1035,7 @@ int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const
   if (num_cus < 0) return num_cus;
   const int tiles_m = (int)((M + 255) / 256), tiles_n = (N + 255) / 256;
   const int num_tiles = tiles_m * tiles_n;
-  const int group_w = column_group(tiles_n, 256, Kp);
+  const int group_w = column_group(M, N, Kp, QKV, 256, 256, num_cus);
   const int grid = num_tiles < num_cus ? num_tiles : num_cus;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), smem, st, (const _Float16*)A,
                      (const _Float16*)Bt, (int)M, N, Kp, tiles_m, tiles_n, group_w, ep);
@@ -1061,7 +1061,7 @@ int launch_stream_res(const void* A, const void* Bt, int64_t M, int N, int Kp, c
   if (num_cus < 0) return num_cus;
   const int tiles_m = (int)((M + 255) / 256), tiles_n = (N + 255) / 256;
   const int num_tiles = tiles_m * tiles_n;
-  const int group_w = column_group(tiles_n, 256, Kp);
+  const int group_w = column_group(M, N, Kp, false, 256, 256, num_cus);
   const int grid = num_tiles < num_cus ? num_tiles : num_cus;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), smem, st, (const _Float16*)A,
                      (const _Float16*)Bt, (int)M, N, Kp, tiles_m, tiles_n, group_w, ep);

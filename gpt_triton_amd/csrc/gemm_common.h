@@ -1,6 +1,7 @@
 // What the GEMM translation units share: the epilogue description, the direct global->LDS loads
 // with their hand-counted waits, the tile order, and the CU count of the persistent launches.
 #pragma once
+#include <math.h>
 #include <stdlib.h>
 
 #include "common.h"
@@ -160,12 +161,35 @@ __device__ __forceinline__ int xcd_tile(int pid, int num_tiles) {
   return xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
 }
 
-// Width, in column tiles, of the groups the tile order walks through.  The weight panels of
-// one group (group_w * BN rows of Kp halves) should stay in a 4 MB L2 beside the activation
-// panels in flight, so they get about 2.4 MB; every group re-reads the activations once, so
+// Width, in column tiles, of the groups the tile order walks through.
+//
+// A launch whose tiles all run at once (no more than CUs): an XCD has one contiguous range of R tiles, and reads the
+// weight panels of its columns and the activation panels of its rows into its L2 once each, so the fewest bytes are
+// those of a patch of as nearly the same bytes either way: w = sqrt(R BM / BN) columns.  Groups of one column, all
+// its rows one after the other, where the rows of w columns are no more than the range, or hardly (then a column is
+// read by one XCD alone).  Weights from HBM, the activations in the L2s, us, column fastest throughout / so: 128 x 2304 x
+// 768 4.66 / 4.22, 300 x 768 x 768 4.12 / 3.68, 128 x 768 x 3072 7.2 / 7.0, 3885 x 1024 x 4096 38.3 / 35.8.
+// In a forward the row order has something for it too: an XCD then finds rows in its L2 that it has just written.  So
+// the patches are for few rows, for products whose weight does not fit beside that in an L2 of 4 MB, and for
+// those that are no deeper than wide, without the scatter.  Forwards replayed, column fastest / patches in the q, k, v
+// product / projection / ffn1 / ffn2: 2 x 64 tokens of 124M 357 / 352 / 356 / 349 / 358, 8 x 40 420 / 424 / 420 / 422 / 427,
+// 2 x 300 525 / 529 / 523 / 525 / 529, 1 x 800 670 / 674 / 669 / 667 / 670; 1024 wide 3 x 300 1502 / 1493 / 1494 / 1505 /
+// 1479, 5 x 777 3490 / 3493 / 3488 / 3488 / 3459; 1600 wide 1 x 300 3140 / 3130 / 3125 / 3120 / 3120, 3 x 300 4983 / 4986 /
+// 4984 / 4955 / 4931.
+//
+// More tiles than that: the weight panels of one group (group_w * BN rows of Kp halves) should stay in a 4 MB L2
+// beside the activation panels in flight, so they get about 2.4 MB; every group re-reads the activations once, so
 // the groups are as few and as even as that allows.  Panels too long for two of them to fit
 // (large K) keep the plain column-fastest order.
-inline int column_group(int tiles_n, int bn, int Kp) {
+inline int column_group(int64_t M, int N, int Kp, bool scatter, int bm, int bn, int cus) {
+  const int64_t tiles_m = (M + bm - 1) / bm;
+  const int tiles_n = (N + bn - 1) / bn;
+  if (tiles_m * tiles_n <= cus && (M <= 128 || (int64_t)N * Kp > 5 << 19 || (!scatter && Kp <= N))) {
+    const float range = (float)((tiles_m * tiles_n + 7) / 8), w = sqrtf(range * (float)bm / (float)bn);
+    if (w * (float)tiles_m <= 1.25f * range) return 1;
+    const int groups = (int)((float)tiles_n / w + 0.5f);
+    return groups <= 1 ? tiles_n : (tiles_n + groups - 1) / groups;
+  }
   const int64_t panel = (int64_t)bn * Kp * 2;
   const int fit = (int)((2400 << 10) / panel);
   if (fit < 2 || tiles_n <= fit) return tiles_n;

@@ -402,7 +402,9 @@ int launch_tile_cfg(const void* A, const void* Bt, int64_t M, int N, int Kp, con
     set_error("gemm: %lld x %lld output tiles exceed the grid", (long long)tiles_m, (long long)tiles_n);
     return -2;
   }
-  const int group_w = column_group((int)tiles_n, C::BN, Kp);
+  const int cus = cu_count();
+  if (cus < 0) return cus;
+  const int group_w = column_group(M, N, Kp, QKV, C::BM, C::BN, cus);
   hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(C::THREADS), smem, st, A,
                      (const _Float16*)Bt, (int)M, N, Kp, (int)tiles_m, (int)tiles_n, group_w, ep, ln);
   return 0;
