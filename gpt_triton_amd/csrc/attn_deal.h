@@ -3,10 +3,12 @@
 #pragma once
 #include <stdint.h>
 
+#ifndef GPTMI_HOST_DEVICE
 #ifdef __HIPCC__
 #define GPTMI_HOST_DEVICE __attribute__((host, device, always_inline))
 #else
 #define GPTMI_HOST_DEVICE
+#endif
 #endif
 
 namespace gptmi {

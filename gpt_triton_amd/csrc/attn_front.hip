@@ -44,7 +44,7 @@ __global__ __launch_bounds__(512, 2) void attn_front_kernel(
   const int lrow = lane & 15, lq = lane >> 4;
 
   if ((int)blockIdx.x >= B * heads) {
-    prefetch_lines<512>(ahead, (int)blockIdx.x - B * heads, (int)gridDim.x - B * heads);
+    prefetch_lines<512>(ahead, B * heads);
     return;
   }
   // the sequences of a head on one XCD, whose L2 holds the head's weights

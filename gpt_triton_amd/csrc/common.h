@@ -45,32 +45,36 @@ __device__ __forceinline__ h4 lds_read_tr16(const char* p) {
   return __builtin_bit_cast(h4, r);
 }
 
-// Lines of memory that later launches read, requested by workgroups of a launch that leaves CUs idle, or does at
-// its end (see launch.h): a word of each 128-byte line, spread over `blocks` workgroups of NT threads.
-struct PrefetchArgs {
-  const void* p[4];
-  unsigned lines[4];
-};
-inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
-  PrefetchArgs a = {};
-  for (int k = 0; ahead != nullptr && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
-  return a;
-}
-// Workgroups for it, behind the `workers` of the launch: the CUs that these leave idle, or 128 that find room as the
+// Workgroups for what a launch requests ahead, behind its `workers`: the CUs that these leave idle, or 128 that find room as the
 // last of them end (64 gain less: 28 x 300 tokens of 124M none / 64 / 128 2072 / 1923 / 1901 us, 32 x 300 in fp32
 // 2440 / 2266 / 2268, 16 x 512 2054 / 1922 / 1899, 64 x 300 3977 / 3940 / 3928; 1024 wide 8 x 1024 6024 / 5661 /
 // 5623, 1280 wide 4 x 700 5855 / 5514 / 5361).
 inline int prefetch_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
   return ahead == nullptr || ahead->empty() ? 0 : workers <= cus - 64 ? cus - (int)workers : 128;
 }
+// The workgroups from `first` on of a launch: a word of each 128-byte line, and a thread has 8 loads on their way at a
+// time.  As loops over the four matrices, each load was waited for before the next was made, a microsecond or two
+// apiece: forwards, weights from HBM, 60 x 24 tokens of 124M 729 -> 717 us, 21 x 64 644 -> 628, 28 x 300 2020 -> 2006, 1024 wide
+// 15 x 300 3778 -> 3738, 1600 wide 1 x 200 2759 -> 2733, 4 x 512 8812 -> 8706; others equal.
 template <int NT>
-__device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int block, int blocks) {
+__device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int first) {
+  typedef const __attribute__((address_space(1))) unsigned* Word;
+  const unsigned xcd = blockIdx.x & 7, skipped = (xcd - (unsigned)first) & 7;  // ids in front of the XCD's first one
+  const unsigned block = (blockIdx.x - (unsigned)first) >> 3, blocks = (gridDim.x - (unsigned)first - skipped + 7) >> 3;
+  const AheadLines lines(pf, xcd);
   unsigned sink = 0;
+  constexpr unsigned B = 8;
+  const unsigned step = blocks * NT;
+  for (unsigned i = block * NT + threadIdx.x; i < lines.all(); i += B * step) {
+    unsigned w[B];
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll 4
-    for (unsigned i = block * NT + threadIdx.x; i < pf.lines[k]; i += blocks * NT)
-      sink ^= *reinterpret_cast<const unsigned*>((const char*)pf.p[k] + (size_t)i * 128);
+    for (unsigned j = 0; j < B; ++j) {
+      const unsigned n = i + j * step;
+      w[j] = *(Word)(uintptr_t)lines.at(n < lines.all() ? n : lines.all() - 1);
+    }
+#pragma unroll
+    for (unsigned j = 0; j < B; ++j) sink ^= w[j];
+  }
   asm volatile("" : : "v"(sink));
 }
 

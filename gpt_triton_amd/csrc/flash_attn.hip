@@ -886,7 +886,7 @@ __global__ __launch_bounds__(512, 2) void flash_attn_stream_kernel(
   h8 q_heavy[KS], q_heavy_next[KS], q_light[KS];
   int bh = blockIdx.x;
   if (bh >= workers) {
-    prefetch_lines<512>(ahead, bh - workers, (int)gridDim.x - workers);
+    prefetch_lines<512>(ahead, workers);
     return;
   }
   // (single registers with values the compiler cannot see through, and a chain of selects: an array, or
@@ -983,7 +983,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring_kernel(
   const int q_blocks = (L + BQ - 1) / BQ;
   const int workers = dealt * q_blocks;
   if ((int)blockIdx.x >= workers) {
-    prefetch_lines<256>(ahead, (int)blockIdx.x - workers, (int)gridDim.x - workers);
+    prefetch_lines<256>(ahead, workers);
     return;
   }
   const WorkItem item = work_item((int)blockIdx.x, dealt, q_blocks, group);

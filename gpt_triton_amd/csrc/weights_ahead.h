@@ -4,6 +4,14 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#ifndef GPTMI_HOST_DEVICE
+#ifdef __HIPCC__
+#define GPTMI_HOST_DEVICE __attribute__((host, device, always_inline))
+#else
+#define GPTMI_HOST_DEVICE
+#endif
+#endif
+
 namespace gptmi {
 
 // What the launches behind this one will read (weights): an attention launch has further workgroups request it from
@@ -13,6 +21,40 @@ struct Prefetch {
   size_t bytes[4] = {};
   bool may_be_cached = false;  // the memory-side cache may hold it from the model's last forward
   bool empty() const { return bytes[0] == 0; }
+};
+
+// The same as a kernel takes it, in lines of 128 bytes.
+struct PrefetchArgs {
+  const void* p[4];
+  unsigned lines[4];  // multiples of 8, for both sides of a matrix are multiples of 64
+};
+inline PrefetchArgs prefetch_args(const Prefetch* ahead) {
+  PrefetchArgs a = {};
+  for (int k = 0; ahead != nullptr && k < 4; ++k) a.p[k] = ahead->p[k], a.lines[k] = (unsigned)(ahead->bytes[k] / 128);
+  return a;
+}
+// What goes through one of the 8 XCDs: an eighth of each matrix, in order (the part that the products of few rows read
+// there, which then lies in its L2 as well), one matrix behind the other.
+class AheadLines {
+ public:
+  GPTMI_HOST_DEVICE AheadLines(const PrefetchArgs& pf, unsigned xcd) {
+    unsigned all = 0;
+#pragma GCC unroll 4
+    for (int k = 0; k < 4; ++k) {
+      const unsigned eighth = pf.lines[k] >> 3;
+      base_[k] = (uintptr_t)pf.p[k] + ((uintptr_t)xcd * eighth - all) * 128;
+      all += eighth;
+      end_[k] = all;
+    }
+  }
+  GPTMI_HOST_DEVICE unsigned all() const { return end_[3]; }
+  GPTMI_HOST_DEVICE uintptr_t at(unsigned n) const {  // address of the n-th of them
+    return (n < end_[0] ? base_[0] : n < end_[1] ? base_[1] : n < end_[2] ? base_[2] : base_[3]) + (uintptr_t)n * 128;
+  }
+
+ private:
+  uintptr_t base_[4];
+  unsigned end_[4];
 };
 
 // Sizes that are the same for all layers of a call; rows: of a key, lasting: see weights_ahead.
