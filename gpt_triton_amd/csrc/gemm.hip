@@ -287,7 +287,7 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
 }
 
 // ---------------------------------------------------------------------------
-// Streaming variant of the 256x256x64 kernel: one workgroup per CU walks tiles
+// Streaming variant of the 256x256x64 kernel (BM = 192: 192x256x64): one workgroup per CU walks tiles
 // blockIdx.x, blockIdx.x + gridDim.x, ...  The two operand stages keep alternating across tile
 // boundaries, so the first two k-tiles of the NEXT output tile are requested while the current
 // one finishes, and the epilogue runs with those loads in flight.  What this removes, per tile
@@ -301,10 +301,10 @@ __device__ __forceinline__ void store_wave_tile_rs(f4 (&acc)[2 * NB][2 * MB], co
 //
 // Load/store counter.  Loads and stores of a wavefront retire in issue order on this ISA.  The
 // loads of the next tile's k-tile 1 are issued BEFORE the epilogue's stores, so waiting for them
-// with vmcnt(EPI_STORES) -- the epilogue issues exactly 16 (fp16) or 32 (fp32) stores per lane --
+// with vmcnt(EPI_STORES) -- the epilogue issues exactly 16 (fp16) or 32 (fp32) stores per lane, 12 or 24 of 192 rows --
 // does not wait for the stores' acknowledgements.  The bias is fetched, and waited for, before those loads are issued, so
 // that no compiler-placed wait inside the epilogue falls behind them; so are the words of a dropout mask.  Only
-// whole row tiles (the last one starts at row M - 256, see persistent_rows), no residual, dropout with its mask
+// whole row tiles (the last one starts at row M - BM, see persistent_rows), no residual, dropout with its mask
 // at hand and an fp16 output behind a GELU: the launcher sends everything else to gemm_tile.hip.
 // ---------------------------------------------------------------------------
 template <int MB, int NB, typename T, bool QKV, bool GELU>
@@ -407,17 +407,17 @@ struct KnTile {
 
 // T: type of the bias.  OT: type of the output (fp16, or T).  DROP: fp16 output, plain, the mask at hand.
 // KN: Bt is the weight [K][N] itself, N a multiple of 256 (see KnTile).
-template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP, bool KN>
+template <int BM, int WM, int WN, typename T, typename OT, bool QKV, bool DROP, bool KN>
 __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const _Float16* __restrict__ A, const _Float16* __restrict__ Bt, int M, int N, int Kp,
     int tiles_m, int tiles_n, int group_w, EpiDev ep) {
-  constexpr int BM = 256, BN = 256, ROWB = 128, T_ = 512, KS = 4;
+  constexpr int BN = 256, ROWB = 128, T_ = 512;
   static_assert(WM * WN == 8, "8 wavefronts");
   static_assert(!DROP || (!QKV && sizeof(OT) == 2), "dropout with a plain fp16 output");
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int MB = TM / 32, NB = TN / 32;
-  constexpr int A_IT = 4, B_IT = 4, LPT = A_IT + B_IT;  // 16-byte loads per thread per k-tile
-  constexpr int STAGE = (BM + BN) * ROWB;               // 64 KB
+  constexpr int A_IT = BM / 64, B_IT = 4, LPT = A_IT + B_IT;  // 16-byte loads per thread per k-tile
+  constexpr int STAGE = (BM + BN) * ROWB;                     // 64 KB, 56 of 192 rows
   constexpr int SLABS = 2 * STAGE;                      // epilogue slabs start behind the stages
   constexpr bool HALF_SLABS = sizeof(OT) == 2;          // fp16 output: store_wave_tile_h
   constexpr int EPI_STORES = HALF_SLABS ? MB * NB * 2 : MB * NB * 4;  // stores per lane per epilogue
@@ -433,13 +433,13 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 
   // Operand-tile slot s = it * 512 + tid: row it * 64 + tid / 8, 16-byte position tid % 8,
   // which holds source chunk (tid % 8) ^ ((row >> 1) & 7) -- the key does not depend on `it`.
-  // M is 256 or more, the last row tile starts at M - 256 and N is a multiple of 64, so no
+  // M is 256 or more, the last row tile starts at M - BM and N is a multiple of 64, so no
   // row is clamped: a load address is a per-tile scalar base (first row of the tile, k-tile
   // offset) plus one of four per-thread 32-bit offsets shared by A and B.
   const int r0 = tid >> 3;
-  unsigned lane_off[A_IT];
+  unsigned lane_off[B_IT];
 #pragma unroll
-  for (int it = 0; it < A_IT; ++it)
+  for (int it = 0; it < B_IT; ++it)
     lane_off[it] = (unsigned)(r0 + it * 64) * (unsigned)Kp * 2u +
                    (unsigned)(((tid & 7) ^ ((r0 >> 1) & 7)) * 16);
   const unsigned wave_off =
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     m0 = min((in_grp / grp_w) * BM, M - BM);
     n0 = (grp * group_w + in_grp % grp_w) * BN;
   };
-  // A k-tile is eight 16-byte loads per lane: four for the A rows, four for the B rows.  The
+  // A k-tile is eight 16-byte loads per lane: four for the A rows (three of 192), four for the B rows.  The
   // source of a half is a scalar (first row of the tile, first byte of the k-tile), computed once
   // and not per load: the scalar work of a load that goes between two MFMAs must fit under one.
   auto a_src = [&](int m0, int k) __attribute__((always_inline)) {
@@ -492,13 +492,13 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
   const int lrow = lane & 15, lq = lane >> 4, fkey = (lrow >> 1) & 7;
   const int a_row_off = (wm * TM + lrow) * ROWB;
   const int b_row_off = BM * ROWB + (wn * TN + lrow) * ROWB;
-  // A slice = one 32-wide k-step s times one half h of the sub-tile's rows: 4 A blocks (af; a
+  // A slice = one 32-wide k-step s times one half h of the sub-tile's rows: MB A blocks (af; a
   // block's register takes the next slice's block as soon as its four MFMAs are issued) times 4 B
   // blocks (bf[s], good for both halves of step s).
-  static_assert(TM == 128 && TN == 64, "128 x 64 sub-tiles");
-  h8 af[4], bf[2][4];
+  static_assert((TM == 128 || TM == 96) && TN == 64, "128 x 64 or 96 x 64 sub-tiles");
+  h8 af[MB], bf[2][4];
   auto frag_a = [&](const char* st, int h, int jl, int s) __attribute__((always_inline)) {
-    return *reinterpret_cast<const h8*>(st + a_row_off + (h * 64 + jl * 16) * ROWB +
+    return *reinterpret_cast<const h8*>(st + a_row_off + (h * (TM / 2) + jl * 16) * ROWB +
                                         (((s * 4 + lq) ^ fkey) << 4));
   };
   auto frag_b = [&](const char* st, int i, int s) __attribute__((always_inline)) {
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
   auto read_first = [&](int stage) __attribute__((always_inline)) {
     const char* st = smem + stage * STAGE;
 #pragma unroll
-    for (int jl = 0; jl < 4; ++jl) af[jl] = frag_a(st, 0, jl, 0);
+    for (int jl = 0; jl < MB; ++jl) af[jl] = frag_a(st, 0, jl, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) bf[0][i] = frag_b(st, i, 0);
   };
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-    // One slice, a quarter of a k-tile: 16 MFMAs of 16 x 16 x 32 in eight pairs (a pair takes the
+    // One slice, a quarter of a k-tile: 16 (12) MFMAs of 16 x 16 x 32 in eight (six) pairs (a pair takes the
     // matrix pipe as long as one 32 x 32 x 16, and this shape draws less power for the same
     // products: on random operands the chip holds a higher clock).  Behind the pairs, one each, go
     // the fragment reads for slice `rks` of `rstage`: a read issued in the shadow of an MFMA costs
@@ -556,14 +556,14 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
       const int t = (rks + 3) & 3, s = t >> 1, h = t & 1;
       const char* st = smem + rstage * STAGE;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+      for (int q = 0; q < 2 * MB; ++q) {
         const int jl = q >> 1;
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const int ii = (q & 1) * 2 + p;
           const int i = (jl & 1) ? 3 - ii : ii;  // one operand changes per MFMA
-          acc[i][4 * h + jl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[s][i], af[jl],
-                                                                      acc[i][4 * h + jl], 0, 0, 0);
+          acc[i][MB * h + jl] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[s][i], af[jl],
+                                                                      acc[i][MB * h + jl], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (fetch) {
@@ -573,6 +573,10 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
           if (q & 1) af[jl] = frag_a(st, rks & 1, jl, rks >> 1);
           else if (t == 1) bf[1][jl] = frag_b(st, jl, 1);
           else if (t == 3) bf[0][jl] = frag_b(st, jl, 0);
+          if (MB == 3 && q == 1) {  // three pairs' first halves, four B blocks
+            if (t == 1) bf[1][3] = frag_b(st, 3, 1);
+            else if (t == 3) bf[0][3] = frag_b(st, 3, 0);
+          }
         }
         extra(q);
         __builtin_amdgcn_sched_barrier(0);
@@ -586,6 +590,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
     const char* b_half[B_IT] = {};  // B half still to be issued into the other stage
     auto with_b_half = [&](int q) __attribute__((always_inline)) {
       if (q & 1) issue_b(stage ^ 1, b_half[q / 2], q / 2);
+      else if (MB == 3 && q == 4) issue_b(stage ^ 1, b_half[3], 3);
     };
     // k-slices 0..2 of the k-tile in `stage`; `extra0` goes with the first
     auto first_slices = [&](auto&& extra0) __attribute__((always_inline)) {
@@ -1016,11 +1021,11 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_res_kernel(
   }
 }
 
-template <int WM, int WN, typename T, typename OT, bool QKV, bool DROP = false, bool KN = false>
+template <int BM, typename T, typename OT, bool QKV, bool DROP = false, bool KN = false>
 int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const EpiDev& ep,
                   hipStream_t st) {
-  auto kern = gemm_stream_kernel<WM, WN, T, OT, QKV, DROP, KN>;
-  constexpr int smem = 2 * 512 * 128 + 8 * 4096;  // 160 KB: two stages + the epilogue slabs
+  auto kern = gemm_stream_kernel<BM, 2, 4, T, OT, QKV, DROP, KN>;
+  constexpr int smem = 2 * (BM + 256) * 128 + 8 * 4096;  // two stages + the epilogue slabs: 160 KB, or 144
   static bool attr_done = false;  // idempotent; a race only repeats the call
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1033,9 +1038,9 @@ int launch_stream(const void* A, const void* Bt, int64_t M, int N, int Kp, const
   }
   const int num_cus = cu_count();
   if (num_cus < 0) return num_cus;
-  const int tiles_m = (int)((M + 255) / 256), tiles_n = (N + 255) / 256;
+  const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (N + 255) / 256;
   const int num_tiles = tiles_m * tiles_n;
-  const int group_w = column_group(M, N, Kp, QKV, 256, 256, num_cus);
+  const int group_w = column_group(M, N, Kp, QKV, BM, 256, num_cus);
   const int grid = num_tiles < num_cus ? num_tiles : num_cus;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), smem, st, (const _Float16*)A,
                      (const _Float16*)Bt, (int)M, N, Kp, tiles_m, tiles_n, group_w, ep);
@@ -1068,11 +1073,14 @@ int launch_stream_res(const void* A, const void* Bt, int64_t M, int N, int Kp, c
   return 0;
 }
 
-// Cost in microseconds of a persistent launch over `tiles` 256 x 256 tiles, in the terms of the
+// Cost in microseconds of a persistent launch over `tiles` tiles of 256 or 192 rows x 256, in the terms of the
 // cost model of gemm_tile.hip: every workgroup walks ceil(tiles / CUs) of them, and tile and k-slice take
-// longer the more of the chip works (L2 and clock).  Fitted to the same products from 256 rows on.
-inline float stream_cost(int64_t tiles, int Kp, bool res, int cus) {
+// longer the more of the chip works (L2 and clock).  Fitted to the same products from 256 rows on; the tiles of 192
+// rows relative to those of 256, at 181 sizes from 256 to 26000 rows (2 % off; of the two the one that the
+// model takes is the faster one, 6 % faster on average than 256 rows always).
+inline float stream_cost(int64_t tiles, int Kp, bool res, int cus, int bm) {
   const float rounds = (float)((tiles + cus - 1) / cus), fill = (float)tiles / (float)cus, k = (float)(Kp / 64);
+  if (bm == 192) return 1.67f + rounds * 2.82f + fill * 0.98f + k * (0.853f * rounds + 0.488f * fill);
   return res ? rounds * 7.42f + k * (0.787f * rounds + 0.780f * fill)
              : 1.67f + rounds * 4.70f + fill * 1.63f + k * (0.917f * rounds + 0.659f * fill);
 }
@@ -1097,9 +1105,14 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // edge store nothing), two k-tiles (three with a residual), vector epilogues, and dropout only with its
 // mask at hand and an fp16 output, behind a GELU or in front of a residual (the two products of a block that
 // have one).
-// Sets *head to the number of rows for the persistent kernel.
+// Tiles of 192 rows move 17 % more bytes a product and lose 5 % of the rate, but leave fewer CUs without a tile where
+// those of 256 fill the rounds badly (fp16, 256 / 192 rows, us: 4800 x 2304 x 768, 171 / 225 tiles, 23.3 / 21.7; 3885 x
+// 3072 x 1024, 192 / 252, 32.3 / 29.8; 4000 x 3072 x 768 25.7 / 22.7; 9600 x 2304 x 768, 342 / 450, 44.0 / 38.7, and 43.5
+// with the rows beyond one round on the tile kernel; 12000 x 3072 x 768, 564 / 756, 73.3 / 64.9; 4800 x 3072 x 768, 228 /
+// 300, 27.8 / 37.8).  Without a residual and without dropout, up to 6 rounds, beyond which there is nothing to gain.
+// Sets *head to the number of rows for the persistent kernel and *bm to its tiles' rows.
 template <typename T, typename OT, bool QKV>
-int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
+int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, int* bm) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool drop = ep.drop.p > 0.f;
   const bool drop_ok = !QKV && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0 &&
@@ -1109,6 +1122,7 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
       (sizeof(OT) == 4 || ep.vec8_ok) && (!drop || drop_ok) &&
       (!res || (sizeof(T) == 2 && (((uintptr_t)ep.residual) & 15) == 0));
   *head = 0;
+  *bm = 256;
   if (!persistent) return 0;
   const int cus = cu_count();
   if (cus < 0) return cus;
@@ -1116,18 +1130,21 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head) {
   const int64_t all = res && overlap(ep.out, ep.residual, M, N, sizeof(OT)) ? M / 256 * 256 : M;
   if (drop && all != M) return 0;  // all or none: the mask counts from row 0
   const int64_t tiles = (all + 255) / 256 * tiles_n;
-  // rows of the row tiles that fill whole rounds
-  const int64_t whole = drop ? all : tiles / cus * cus / tiles_n * 256;
   // Two whole rounds and more: always persistent.  Under a load that long the chip's clock falls, and
   // with it the tile kernel, which moves more bytes per product (65536 x 1600 x 1600 with a residual:
   // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
   // 20480 x 1024 x 4096, is the other way round, 196 against 183).
   float least = tiles >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
-  for (const int64_t rows : {all, whole < all ? whole : all}) {
-    if (rows == 0) continue;
-    float c = stream_cost((rows + 255) / 256 * tiles_n, Kp, res, cus);
-    if (rows < M) c += 1.0f + gemm_tile_cost(M - rows, N, Kp, cus);
-    if (c < least) least = c, *head = rows;
+  for (const int tm : {256, 192}) {
+    if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus)) break;
+    // rows of the row tiles that fill whole rounds
+    const int64_t whole = drop ? all : (all + tm - 1) / tm * tiles_n / cus * cus / tiles_n * tm;
+    for (const int64_t rows : {all, whole < all ? whole : all}) {
+      if (rows == 0) continue;
+      float c = stream_cost((rows + tm - 1) / tm * tiles_n, Kp, res, cus, tm);
+      if (rows < M) c += 1.0f + gemm_tile_cost(M - rows, N, Kp, cus);
+      if (c < least) least = c, *head = rows, *bm = tm;
+    }
   }
   return 0;
 }
@@ -1150,21 +1167,26 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
                  hipStream_t st) {
   const bool res = !QKV && ep.residual != nullptr;
   int64_t m_head;
-  if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head)) return rc;
+  int bm;
+  if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head, &bm)) return rc;
   if (m_head > 0) {
     int rc;
     if constexpr (sizeof(OT) == 2 && !QKV) {
       if (ep.drop.p > 0.f) {  // m_head == M
         if constexpr (sizeof(T) == 2)
           if (res) return launch_stream_res<true>(A, Bt, M, N, Kp, ep, st);
-        return launch_stream<2, 4, T, OT, QKV, true, KN>(A, Bt, M, N, Kp, ep, st);
+        return launch_stream<256, T, OT, QKV, true, KN>(A, Bt, M, N, Kp, ep, st);
       }
     }
-    if constexpr (sizeof(T) == 2 && !QKV)
-      rc = res ? launch_stream_res<false>(A, Bt, m_head, N, Kp, ep, st)
-               : launch_stream<2, 4, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
-    else
-      rc = launch_stream<2, 4, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
+    if (bm == 192) {
+      rc = launch_stream<192, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
+    } else {
+      if constexpr (sizeof(T) == 2 && !QKV)
+        rc = res ? launch_stream_res<false>(A, Bt, m_head, N, Kp, ep, st)
+                 : launch_stream<256, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
+      else
+        rc = launch_stream<256, T, OT, QKV, false, KN>(A, Bt, m_head, N, Kp, ep, st);
+    }
     if (rc != 0 || m_head == M) return rc;
   }
   if constexpr (KN)
@@ -1180,7 +1202,8 @@ template <bool QKV>
 int launch_shape_layernorm(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
                            const LnArgs& ln, hipStream_t st) {
   int64_t m_head;
-  if (const int rc = persistent_rows<_Float16, _Float16, QKV>(M, N, H, ep, &m_head)) return rc;
+  int bm;
+  if (const int rc = persistent_rows<_Float16, _Float16, QKV>(M, N, H, ep, &m_head, &bm)) return rc;
   if (m_head > 0) {
     const int rc = launch_gemm_layernorm_tile(x, Bt, m_head, N, H, ep, ln, QKV, false, st);
     if (rc != 0 || m_head == M) return rc;
@@ -1266,14 +1289,15 @@ static bool disjoint(const void* a, size_t a_bytes, const void* b, size_t b_byte
 bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e) {
   EpiDev ep;
   int64_t head;
+  int bm;
   const size_t w_bytes = (size_t)K * N * 2, out_bytes = (size_t)M * N * 2, part = out_bytes / 3;
   if (e.qkv ? !disjoint(W, w_bytes, e.q, part) || !disjoint(W, w_bytes, e.k, part) || !disjoint(W, w_bytes, e.v, part)
             : !disjoint(W, w_bytes, e.out, out_bytes))
     return false;
   if (!e.f16 || K % 64 != 0 || ((uintptr_t)W & 15) != 0 || !gemm_tile_reads_kn(N, K) || make_epi(e, M, N, ep) != 0)
     return false;
-  if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)
-             : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head)) != 0)
+  if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head, &bm)
+             : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head, &bm)) != 0)
     return false;
   return head == 0 || (N % 256 == 0 && e.residual == nullptr && M <= 32768);
 }
@@ -1293,8 +1317,9 @@ int gemm_qkv_split(int64_t M, int N, int K, int64_t L, int heads, int d) {
   e.qkv = e.f16 = true;
   EpiDev ep;
   int64_t head;
+  int bm;
   if (const int rc = make_epi(e, M, N, ep)) return rc;
-  if (const int rc = persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head)) return rc;
+  if (const int rc = persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head, &bm)) return rc;
   if (head > 0) return head == M ? 1 : 0;
   return gemm_tile_split(M, N, K, cus);
 }
