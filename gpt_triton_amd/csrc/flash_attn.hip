@@ -1485,6 +1485,273 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void flash_attn_wide_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Ring variant with 16 queries a wavefront.  A wavefront's path through its key tiles is a chain (score products,
+// max, weights, P.V products, one behind the other), and where the query blocks leave the chip half empty that
+// chain is the launch.  With v_mfma_f32_16x16x32 instead of 32x32x16 a lane has 16 of a tile's scores instead of 32 and
+// the chain is about half as long; the price is that K and V are read from LDS for 16 queries at a time.
+// Four wavefronts, 64 queries a workgroup; tiles, ring, barriers and the order inside a wavefront as in
+// flash_attn_ring_kernel, but for K's fragments, which are requested in front of the softmax too.  A 64-key tile
+// takes 0.67 us of a wavefront that has its SIMD to itself, 0.92 there (in fp32 arithmetic 1.0 and 1.6); 8 stages instead
+// of 4 changed nothing.  12 pairs of 1024 rows 16.9 -> 13.4 us, 84 of 211 6.4 -> 5.8, in fp32 arithmetic 29.3 -> 19.7 and 12 of
+// 300 11.0 -> 7.9.
+//
+// The results are flash_attn_ring_kernel's bit for bit, though a query's keys are spread over four lanes instead of two:
+//   * one 16x16x32 product adds its 32 terms as two 32x32x16 products one behind the other add theirs (compared on
+//     200000 random sums);
+//   * lane (ql, lq) = (lane % 16, lane / 16) has query ql and the scores of 32-key block lq / 2 which there lane group g =
+//     lq % 2 has: row m of the b-th 16-row block of K's fragments is key 32 (m / 8) + 8 b + m % 8;
+//   * the weights of a lane group's two blocks are added in order: lanes 0..31 add theirs, lanes 32..63 go on from there;
+//   * of the weights as fp16, the lanes of block 0 trade their second half for the first half of those of block 1
+//     (permlane32_swap), which makes them the second operands of the blocks' products, keys in the ring kernel's order.
+// K's unit u of row r lies at u ^ (r >> 1 & 7) ^ 4 (r >> 5), for 16 lanes read 8 rows and those 32 further on; V's at u ^
+// 2 (r >> 1 & 3), so that the 8 rows which 32 lanes read 32 bytes of each cover all banks once.
+// ---------------------------------------------------------------------------
+constexpr int kRing16Rows = 64;  // queries a workgroup
+template <bool BLND, bool ACC>
+__global__ __launch_bounds__(256, 2) void flash_attn_ring16_kernel(
+    const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
+    const _Float16* __restrict__ V, _Float16* __restrict__ O, int heads, int L, float scale, int pairs, int dealt, int group,
+    PrefetchArgs ahead) {
+  constexpr int D = 64, KS = 2, DB = 4, KB = 4, NS = 4;
+  constexpr int STAGE = 2 * BKEY * D * 2;  // 16 KB: K tile, then V tile
+  constexpr int V_AT = BKEY * D * 2;       // byte offset of the V tile inside a stage
+  __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ql = lane & 15, lq = lane >> 4;
+  const unsigned smem_base = (unsigned)(uintptr_t)smem;
+
+  const int q_blocks = (L + kRing16Rows - 1) / kRing16Rows;
+  const int workers = dealt * q_blocks;
+  if ((int)blockIdx.x >= workers) {
+    prefetch_lines<256>(ahead, workers);
+    return;
+  }
+  const WorkItem item = work_item((int)blockIdx.x, dealt, q_blocks, group);
+  const int bh = item.bh, q0 = item.qb * kRing16Rows;
+  if (bh >= pairs) return;
+  const int qw0 = q0 + wave * 16, q = qw0 + ql;
+  const bool wave_active = qw0 < L;
+  const int last_q = q0 + kRing16Rows - 1 < L - 1 ? q0 + kRing16Rows - 1 : L - 1;
+  const int nt = last_q / BKEY + 1;  // key tiles 0..nt-1 touch this query block
+
+  // queries first (the oldest loads in flight): lane (ql, lq) holds d = 32 ks + 8 lq + 0..7
+  h8 qf[KS];
+  {
+    const _Float16* qp = Q + ((int64_t)bh * L + (q < L ? q : L - 1)) * D + lq * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const h8*>(qp + ks * 32);
+  }
+
+  // a tile is 16 loads of 1 KB (8 rows each), K rows then V rows; wavefront w issues loads 4 w .. 4 w + 3
+  const bool brings_v = wave >= 2;
+  const char* src = (const char*)((brings_v ? V : K) + (int64_t)bh * L * D);
+  const int lrow = lane >> 3;
+  const unsigned unit16 = brings_v ? (unsigned)(((lane & 7) ^ (2 * ((lrow >> 1) & 3))) << 4)
+                                   : (unsigned)(((lane & 7) ^ (lane >> 4)) << 4);
+  auto issue_tile = [&](int t) {
+    const unsigned dst = smem_base + (unsigned)((t % NS) * STAGE) + (unsigned)(wave * 4) * 1024u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int rel = (wave & 1) * 4 + j;  // 8-row group inside the K (or V) tile
+      int row = t * BKEY + rel * 8 + lrow;
+      row = row < L ? row : L - 1;  // keys past the end are masked, the values finite
+      const unsigned u = brings_v ? unit16 : (unit16 ^ ((unsigned)((rel ^ (rel >> 2)) & 1) << 6));
+      attn_dma16(src, (unsigned)row * 128u + u, dst + j * 1024);
+    }
+  };
+
+  // block b, half ks of the columns: k_off[ks ^ (b & 1)] + 1024 b
+  int k_off[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    k_off[ks] = (32 * (ql >> 3) + (ql & 7)) * 128 + (((ks * 4 + lq) ^ ((ql >> 1) & 3) ^ (4 * (ql >> 3))) << 4);
+  const int vrow = 16 * (lq >> 1) + 4 * (lq & 1) + (ql >> 2);
+  int v_off[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i)
+    v_off[i] = V_AT + vrow * 128 + (((2 * i + ((ql & 3) >> 1)) ^ (2 * ((vrow >> 1) & 3))) << 4) + (ql & 1) * 8;
+  const Softmax<ACC> sm(scale);
+
+  f4 oacc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) oacc[i] = f4{0.f, 0.f, 0.f, 0.f};
+  float mrun = -INFINITY, den = 0.f;
+
+  f4 s[KB];  // S^T of the tile whose softmax comes next
+  h8 kf[KB][KS];
+  auto read_k = [&](const char* buf) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[kb][ks] = *reinterpret_cast<const h8*>(buf + kb * 1024 + k_off[ks ^ (kb & 1)]);
+  };
+  auto scores = [&]() {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) s[kb] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[kb][ks], qf[ks], s[kb], 0, 0, 0);
+  };
+  h4 vlo[2][DB], vhi[2][DB];
+  auto read_v = [&](const char* buf) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        vlo[kk][i] = lds_read_tr16(buf + kk * 4096 + v_off[i]);
+        vhi[kk][i] = lds_read_tr16(buf + kk * 4096 + 1024 + v_off[i]);
+      }
+  };
+  // mask (the tile that the diagonal cuts), running max, P = exp(S - max) summed into the denominator and rounded
+  // to fp16, accumulator rescaled
+  h8 pf[2];
+  f4 weights[KB];
+  float mult, lower;  // the accumulator's factor; lanes 0..31: the sum of their weights
+  auto softmax = [&](auto diagonal) {
+    if constexpr (decltype(diagonal)::value) {
+      // of this lane's keys, 8 b + r behind the first: those up to `visible`
+      const int visible = (qw0 & 63) + ql - 32 * (lq >> 1) - 4 * (lq & 1);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[kb][r] = 8 * kb + r <= visible ? s[kb][r] : -INFINITY;
+    }
+    float bmax = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[kb][r] = sm.score(s[kb][r]);
+        bmax = fmaxf(bmax, s[kb][r]);
+      }
+    const LanePair mx = row_swap(bmax);
+    bmax = half_max(fmaxf(mx.a, mx.b));
+    const float mnew = bmax > mrun ? bmax : mrun;
+    const float mb = sm.base(mnew);
+    mult = sm.rescale(mrun, mnew);
+    lower = 0.f;
+    h8 half[2];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = sm.weight(s[kb][r], mb);
+        weights[kb][r] = p;
+        lower += p;
+        half[kb >> 1][(kb & 1) * 4 + r] = (_Float16)p;
+      }
+    const u4 first = __builtin_bit_cast(u4, half[0]), second = __builtin_bit_cast(u4, half[1]);
+    u4 block0, block1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const auto t = __builtin_amdgcn_permlane32_swap(first[e], second[e], false, false);
+      block0[e] = t[0];
+      block1[e] = t[1];
+    }
+    pf[0] = __builtin_bit_cast(h8, block0);
+    pf[1] = __builtin_bit_cast(h8, block1);
+    mrun = mnew;
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) oacc[i][r] *= mult;
+  };
+  // the rest of the denominator, which nothing waits for: behind the next tile's score products
+  auto denominator = [&]() {
+    float psum = half_swap(lower).a;  // that of lanes 0..31, from which the others go on
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) psum += weights[kb][r];
+    const LanePair ps = row_swap(psum);
+    psum = half_swap(ps.a + ps.b).b;  // that of lanes 32..63
+    den = den * mult + psum;
+  };
+  auto weighted = [&]() {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < DB; ++i) {
+        const h4 lo = vlo[kk][i], hi = vhi[kk][i];
+        const h8 vf = h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        oacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[kk], oacc[i], 0, 0, 0);
+      }
+  };
+
+  const int nfull = qw0 >> 6;  // key tiles entirely below this wavefront's diagonal
+  auto stage_of = [&](int t) { return (const char*)smem + (t % NS) * STAGE; };
+  auto arrive = [&](int t) {
+    if (t + 2 < nt) asm volatile("s_waitcnt vmcnt(4)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  auto request = [&](int t) {
+    if (t + 3 < nt) issue_tile(t + 3);
+  };
+  issue_tile(0);
+  if (nt > 1) issue_tile(1);
+  if (nt > 2) issue_tile(2);
+  arrive(0);
+  // see flash_attn_ring_kernel
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+  request(0);
+  if (wave_active) {
+    read_k(stage_of(0));
+    scores();
+    for (int t = 0; t < nfull; ++t) {
+      read_k(stage_of(t + 1));
+      read_v(stage_of(t));
+      __builtin_amdgcn_sched_barrier(0);
+      softmax(std::false_type{});
+      __builtin_amdgcn_sched_barrier(0);
+      scores();
+      denominator();
+      weighted();
+      arrive(t + 1);
+      request(t + 1);
+    }
+    read_v(stage_of(nfull));
+    __builtin_amdgcn_sched_barrier(0);
+    softmax(std::true_type{});
+    denominator();
+    weighted();
+  }
+  for (int t = wave_active ? nfull + 1 : 1; t < nt; ++t) {
+    arrive(t);
+    request(t);
+  }
+
+  // a lane has, of each 16 d, 4 of its query's row: neighbouring lane groups trade halves through the 16-lane swap
+  // and store 16 bytes each
+  const NormaliseHalf<ACC> norm(den);
+  if (q < L) {
+    int64_t row_off;
+    if (BLND) {
+      const int b = bh / heads, n = bh - b * heads;
+      row_off = (((int64_t)b * L + q) * heads + n) * D;
+    } else {
+      row_off = ((int64_t)bh * L + q) * D;
+    }
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {
+      h4 x, y;  // d = 32 pr + 4 lq + 0..3 and the same + 16
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[j] = (_Float16)norm(oacc[2 * pr][j]);
+        y[j] = (_Float16)norm(oacc[2 * pr + 1][j]);
+      }
+      const u2 xd = __builtin_bit_cast(u2, x), yd = __builtin_bit_cast(u2, y);
+      const auto r0 = __builtin_amdgcn_permlane16_swap(xd[0], yd[0], false, false);
+      const auto r1 = __builtin_amdgcn_permlane16_swap(xd[1], yd[1], false, false);
+      // even lq: own x, then the next group's x (d + 4..7); odd lq: the group's y in front, then own y
+      *reinterpret_cast<u4*>(O + row_off + 32 * pr + 16 * (lq & 1) + 4 * (lq & 2)) = u4{r0[0], r1[0], r0[1], r1[1]};
+    }
+  }
+}
+
 // Deals the query chunks of a sequence of L <= 320 rows to the 8 wavefronts: chunk c costs
 // c + 1 blocks; heaviest first, each to the SIMD (wavefronts w and w + 4) with the smallest
 // load so far that still has a free slot, inside the SIMD to the lighter wavefront.
@@ -1635,6 +1902,19 @@ int launch_ring_attn(const void* q, const void* k, const void* v, void* out, int
   return 0;
 }
 
+template <bool BLND, bool ACC = false>
+int launch_ring16_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
+                       int L, float scale, hipStream_t st, const Prefetch* ahead) {
+  Deal deal;
+  if (!deal_blocks(BN, (L + kRing16Rows - 1) / kRing16Rows, &deal)) return grid_exceeded(BN, L);
+  const int cus = attn_cu_count();
+  if (cus < 0) return cus;
+  hipLaunchKernelGGL((flash_attn_ring16_kernel<BLND, ACC>), dim3(deal.grid + prefetch_workgroups(ahead, deal.grid, cus)),
+                     dim3(256), 0, st, (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, (_Float16*)out, heads, L,
+                     scale, (int)BN, deal.pairs, deal.group, prefetch_args(ahead));
+  return 0;
+}
+
 template <int D, bool BLND, bool ACC = false>
 int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads,
                      int L, float scale, hipStream_t st) {
@@ -1658,19 +1938,28 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
 }
 
 // fp16 q, k, v of equal lengths at head size 64, no dropout.  Up to 320 rows two (batch, head) pairs fit
-// the LDS: the streaming kernel.  Longer ones take their key tiles through the ring, and so does a single
-// tile of up to 512 pairs, where nothing is left to overlap and the ring's workgroup, with half the
-// wavefronts, is through sooner, and more than 288 rows (the last of ten chunks sets the streaming kernel's
-// pace) while the ring's three workgroups a pair find CUs of their own.  Microseconds, streaming / ring (the
-// resident kernel): 12 x 24 rows 3.6 / 3.1 (3.7), 24 x 64 3.9 / 3.5 (4.0), 192 x 64 4.2 / 3.7 (4.3), 768 x 64
-// 7.9 / 8.0 (9.3), 12 x 128 4.7 / 4.6 (5.0), 12 x 211 5.9 / 6.2 (6.9), 24 x 288 7.4 / 7.4, 12 x 300 8.1 / 7.7 (9.6),
-// 60 x 320 8.5 / 8.1, 96 x 320 8.6 / 8.7, 192 x 300 11.4 / 12.8 (13.1), 1536 x 300 55 / 76 (66).
+// the LDS: the streaming kernel.  Longer ones take their key tiles through the ring, and so do up to 512 pairs of
+// two tiles, whose workgroups all run at once.  While 64-row blocks fill the CUs about twice, 16 queries a wavefront are
+// through sooner; beyond, K and V read from LDS twice as often cost more than the shorter chain gives, later for long
+// sequences, for the fp32 arithmetic, whose chain is longer, and for a single tile.  The same bits from all three.
+// Microseconds, streaming / ring / 16 queries:
+//   24 x 64 rows 4.1 / 3.7 / 3.5, 512 x 64 6.1 / 4.7 / 4.5, 1500 x 64 12.8 / 12.2 / 11.9, 12 x 128 4.8 / 4.6 / 4.2, 256 x 128 5.5 /
+//   5.3 / 5.1, 300 x 128 7.8 / 7.1 / 7.7, 512 x 128 9.8 / 9.3 / 10.4, 84 x 211 6.4 / 6.3 / 5.8, 128 x 256 7.1 / 7.0 / 6.5, 150 x
+//   256 7.8 / 8.0 / 8.6, 12 x 300 8.0 / 6.9 / 5.9, 102 x 320 9.2 / 8.4 / 7.7, 154 x 320 10.4 / 10.1 / 11.1, 192 x 300 11.2 / 12.7 /
+//   12.1; ring / 16 queries: 73 x 400 9.5 / 8.3, 110 x 400 10.7 / 12.5, 75 x 512 11.6 / 10.3, 96 x 512 12.1 / 13.2, 128 x
+//   512 13.2 / 16.6, 12 x 1024 16.9 / 13.4, 48 x 1024 19.9 / 18.6, 64 x 1024 20.8 / 26.4;
+//   in fp32 arithmetic 24 x 64 5.0 / 4.5 / 4.0, 12 x 300 12.5 / 11.0 / 7.9, 171 x 192 9.0 / 10.1 / 8.5, 154 x 320 15.1 / 16.2 / 14.8,
+//   205 x 320 16.7 / 20.8 / 19.2; 12 x 1024 29.3 / 19.7, 96 x 512 19.0 / 17.7, 48 x 1024 32.1 / 28.1, 64 x 1024 33.0 / 39.9.
 template <bool BLND, bool ACC = false>
 int launch_d64(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
                float scale, hipStream_t st, const Prefetch* ahead) {
   const int cus = attn_cu_count();
   if (cus < 0) return cus;
-  const bool ring = L > 320 || (L > 288 && 3 * BN <= cus) || (L <= BKEY && BN <= 512);
+  const int64_t blocks = BN * ((L + kRing16Rows - 1) / kRing16Rows);
+  // (a scale that is not positive turns the mask's -inf into something else, differently in each kernel)
+  if (scale > 0.f && 2 * blocks <= (L <= BKEY ? 12 : ACC ? 6 : L > 448 ? 5 : 4) * (int64_t)cus)
+    return launch_ring16_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st, ahead);
+  const bool ring = L > 320 || (L <= 2 * BKEY && BN <= 512);
   return ring ? launch_ring_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st, ahead)
               : launch_stream_attn<BLND, ACC>(q, k, v, out, BN, heads, L, scale, st, 0.f, nullptr, ahead);
 }
