@@ -1598,12 +1598,15 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring16_kernel(
   h4 vlo[2][DB], vhi[2][DB];
   auto read_v = [&](const char* buf) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int i = 0; i < DB; ++i) {
+      unsigned at = (unsigned)(uintptr_t)buf + (unsigned)v_off[i];
+      asm("" : "+v"(at));  // one address for four loads (their offsets are the instructions'): without it one each
 #pragma unroll
-      for (int i = 0; i < DB; ++i) {
-        vlo[kk][i] = lds_read_tr16(buf + kk * 4096 + v_off[i]);
-        vhi[kk][i] = lds_read_tr16(buf + kk * 4096 + 1024 + v_off[i]);
+      for (int kk = 0; kk < 2; ++kk) {
+        vlo[kk][i] = lds_read_tr16((const char*)(uintptr_t)at + kk * 4096);
+        vhi[kk][i] = lds_read_tr16((const char*)(uintptr_t)at + kk * 4096 + 1024);
       }
+    }
   };
   // mask (the tile that the diagonal cuts), running max, P = exp(S - max) summed into the denominator and rounded
   // to fp16, accumulator rescaled
