@@ -355,6 +355,15 @@ static bool prologue_aligned(const void* x, const void* ln_w, const void* ln_b) 
   return (((uintptr_t)x | (uintptr_t)ln_w | (uintptr_t)ln_b) & 15) == 0;
 }
 
+// fp32 models' blocks with packed weights run their LayerNorm inside the product behind it without being asked, where
+// FusedGPT asks for it in fp16 (gpt._ln_in_gemm): a launch less, the same bits.  Forwards, two launches / one, weights
+// from HBM, us: 124M 1 x 24 tokens eager 351 / 339, replayed 305 / 290, 2 x 64 eager 400 / 351 (where the host sets the
+// pace; otherwise 353 / 363), replayed 359 / 359, 1 x 160 386 / 383, 1 x 192 418 / 480; 1024 wide 1 x 24 eager 772 /
+// 645, replayed 649 / 631, 1 x 32 656 / 630, 1 x 48 674 / 708, 2 x 64 797 / 806.
+static bool prologue_f32(int64_t M, int64_t h, bool packed, float p) {
+  return packed && p == 0.f && h <= 1024 && M <= (h <= 768 ? 160 : 32) && gemm_layernorm_supported(M, (int)h, false);
+}
+
 }  // namespace gptmi
 
 using namespace gptmi;
@@ -714,8 +723,10 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
-    prologue = prologue_aligned(x, ln_w, ln_b);
+  } else if (!f16 && !normed) {
+    prologue = prologue_f32(M, h, bw.packed, p);
   }
+  prologue = prologue && prologue_aligned(x, ln_w, ln_b);
   const Dropout drop = {p, seed, keep};
   GemmEpilogue eo = {};
   eo.bias = b_proj;
@@ -807,8 +818,10 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
-    prologue = prologue_aligned(x, ln_w, ln_b);
+  } else if (!f16) {
+    prologue = prologue_f32(M, H, bw.packed, p);
   }
+  prologue = prologue && prologue_aligned(x, ln_w, ln_b);
   GemmEpilogue e2 = {};
   e2.bias = b2;
   e2.residual = x;

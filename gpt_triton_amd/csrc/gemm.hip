@@ -1198,18 +1198,18 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
 
 // The rows divided as the plain launch divides them, so that every row's sum is formed in the same
 // order: those of the persistent kernel by the form that does not split K.
-template <bool QKV>
+template <typename T, bool QKV>
 int launch_shape_layernorm(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
                            const LnArgs& ln, hipStream_t st) {
   int64_t m_head;
   int bm;
-  if (const int rc = persistent_rows<_Float16, _Float16, QKV>(M, N, H, ep, &m_head, &bm)) return rc;
+  if (const int rc = persistent_rows<T, _Float16, QKV>(M, N, H, ep, &m_head, &bm)) return rc;
   if (m_head > 0) {
-    const int rc = launch_gemm_layernorm_tile(x, Bt, m_head, N, H, ep, ln, QKV, false, st);
+    const int rc = launch_gemm_layernorm_tile(x, Bt, m_head, N, H, ep, ln, sizeof(T) == 2, QKV, false, st);
     if (rc != 0 || m_head == M) return rc;
   }
-  return launch_gemm_layernorm_tile((const _Float16*)x + m_head * H, Bt, M - m_head, N, H,
-                                    tail_epi<_Float16, _Float16, QKV>(ep, m_head, N), ln, QKV, true, st);
+  return launch_gemm_layernorm_tile((const T*)x + m_head * H, Bt, M - m_head, N, H,
+                                    tail_epi<T, _Float16, QKV>(ep, m_head, N), ln, sizeof(T) == 2, QKV, true, st);
 }
 
 }  // namespace
@@ -1327,8 +1327,8 @@ int gemm_qkv_split(int64_t M, int N, int K, int64_t L, int heads, int d) {
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,
                           const void* Bt, int64_t M, int N, int H, const GemmEpilogue& e,
                           hipStream_t st) {
-  if (!e.f16 || e.residual != nullptr || e.drop.p > 0.f || !gemm_layernorm_supported(M, H)) {
-    set_error("gemm with LayerNorm prologue: fp16, no residual, no dropout, H=%d a multiple of "
+  if (!(e.f16 || e.out_f16) || e.residual != nullptr || e.drop.p > 0.f || !gemm_layernorm_supported(M, H, e.f16)) {
+    set_error("gemm with LayerNorm prologue: fp16 output, no residual, no dropout, H=%d a multiple of "
               "64 whose 32-row panel fits the LDS", H);
     return -2;
   }
@@ -1338,9 +1338,12 @@ int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, flo
   }
   EpiDev ep;
   if (const int rc = make_epi(e, M, N, ep)) return rc;
-  const LnArgs ln = {ln_w, ln_b, eps, lanes_per_row(H / 8)};
-  return e.qkv ? launch_shape_layernorm<true>(x, Bt, M, N, H, ep, ln, st)
-               : launch_shape_layernorm<false>(x, Bt, M, N, H, ep, ln, st);
+  const LnArgs ln = {ln_w, ln_b, eps, lanes_per_row(H / (e.f16 ? 8 : 4))};
+  if (e.f16)
+    return e.qkv ? launch_shape_layernorm<_Float16, true>(x, Bt, M, N, H, ep, ln, st)
+                 : launch_shape_layernorm<_Float16, false>(x, Bt, M, N, H, ep, ln, st);
+  return e.qkv ? launch_shape_layernorm<float, true>(x, Bt, M, N, H, ep, ln, st)
+               : launch_shape_layernorm<float, false>(x, Bt, M, N, H, ep, ln, st);
 }
 
 }  // namespace gptmi

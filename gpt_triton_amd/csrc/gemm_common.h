@@ -231,7 +231,7 @@ bool gemm_tile_reads_kn(int N, int Kp);
 int launch_gemm_tile_kn(const void* A, const void* W, int64_t M, int N, int K, const EpiDev& ep, bool qkv,
                         hipStream_t st);
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
-                               const LnArgs& ln, bool qkv, bool split, hipStream_t st);
+                               const LnArgs& ln, bool f16, bool qkv, bool split, hipStream_t st);
 float gemm_tile_cost(int64_t M, int N, int Kp, int cus);
 // Over how many groups launch_gemm divides K for M rows of a q, k, v product in fp16, the order of its sums; 0: not
 // the same for all rows; negative: an error.

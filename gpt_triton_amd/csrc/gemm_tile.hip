@@ -40,7 +40,7 @@ struct Tile {
   static constexpr int THREADS = 64 * WM_ * WN_ * WK_;
 };
 
-// T: storage type of bias and residual (fp16 with LNA).  OT: type of the output: T, or fp16 for
+// T: storage type of bias and residual, and with LNA of the rows and the LayerNorm's parameters.  OT: type of the output: T, or fp16 for
 // fp32 storage where the output is the next product's operand (no residual then).
 // WIDE: rows of 2^22 elements and more (64-bit lane addresses).
 //
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(
   };
 
   if constexpr (LNA) {
-    normalise_panel<BM, NT>((const _Float16*)Av, M, Kp, m0, ln, smem + NST * STAGE, tid);
+    normalise_panel<BM, NT>((const T*)Av, M, Kp, m0, ln, smem + NST * STAGE, tid);
     wait_vmcnt<0>();
     __syncthreads();
   } else {
@@ -580,31 +580,34 @@ inline int pick_ln(int64_t M, int N, int K, bool split, int cus) {
   return K <= 1024 && (M + 31) / 32 * cols > cus ? 1 : 0;
 }
 
-template <bool QKV>
+template <typename T, bool QKV>
 int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiDev& ep, const LnArgs& ln,
               bool split, hipStream_t st) {
   const int cus = cu_count();
   if (cus < 0) return cus;
   switch (pick_ln(M, N, K, split, cus)) {
-    case 0: return launch_tile_cfg<Ln32x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    case 1: return launch_tile_cfg<Ln32x64w, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    case 2: return launch_tile_cfg<Ln32x64, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    case 4: return launch_tile_cfg<Ln16x32, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
-    default: return launch_tile_cfg<Ln32x128, _Float16, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 0: return launch_tile_cfg<Ln32x32, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 1: return launch_tile_cfg<Ln32x64w, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 2: return launch_tile_cfg<Ln32x64, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 4: return launch_tile_cfg<Ln16x32, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    default: return launch_tile_cfg<Ln32x128, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
   }
 }
 }  // namespace
 
-bool gemm_layernorm_supported(int64_t M, int H) {
+bool gemm_layernorm_supported(int64_t M, int H, bool f16) {
   if (H <= 0 || H % 64 != 0 || M <= 0) return false;
-  const int nchunks = H / 8, lpr = lanes_per_row(nchunks);
+  const int nchunks = H / (f16 ? 8 : 4), lpr = lanes_per_row(nchunks);
   return (nchunks + lpr - 1) / lpr <= 4 && (size_t)kLnStages + 64 * (size_t)H <= 160 * 1024;
 }
 
 int launch_gemm_layernorm_tile(const void* x, const void* Bt, int64_t M, int N, int H, const EpiDev& ep,
-                               const LnArgs& ln, bool qkv, bool split, hipStream_t st) {
-  return qkv ? launch_ln<true>(x, Bt, M, N, H, ep, ln, split, st)
-             : launch_ln<false>(x, Bt, M, N, H, ep, ln, split, st);
+                               const LnArgs& ln, bool f16, bool qkv, bool split, hipStream_t st) {
+  if (f16)
+    return qkv ? launch_ln<_Float16, true>(x, Bt, M, N, H, ep, ln, split, st)
+               : launch_ln<_Float16, false>(x, Bt, M, N, H, ep, ln, split, st);
+  return qkv ? launch_ln<float, true>(x, Bt, M, N, H, ep, ln, split, st)
+             : launch_ln<float, false>(x, Bt, M, N, H, ep, ln, split, st);
 }
 
 }  // namespace gptmi

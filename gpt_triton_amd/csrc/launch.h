@@ -73,12 +73,12 @@ int launch_gemm(const void* A, const void* Bt, int64_t M, int N, int Kp,
 bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& ep);
 int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const GemmEpilogue& ep, hipStream_t st);
 
-// The same product with A = LayerNorm(x; ln_w, ln_b, eps), x [M][H] fp16 with H = K a multiple
+// The same product with A = LayerNorm(x; ln_w, ln_b, eps), x [M][H] in the storage type with H = K a multiple
 // of 64: every workgroup normalises the rows of its tile in its operand prologue (the bits of
-// launch_layernorm's output) and the normalised matrix never goes to memory.  fp16, no residual,
+// launch_layernorm's fp16 output) and the normalised matrix never goes to memory.  fp16 output, no residual,
 // no dropout; meant for few rows, where a LayerNorm launch costs more than normalising the rows
 // once per column tile.  gemm_layernorm_supported says whether (M, H) is taken.
-bool gemm_layernorm_supported(int64_t M, int H);
+bool gemm_layernorm_supported(int64_t M, int H, bool f16 = true);
 int launch_gemm_layernorm(const void* x, const void* ln_w, const void* ln_b, float eps,
                           const void* Bt, int64_t M, int N, int H, const GemmEpilogue& ep,
                           hipStream_t st);

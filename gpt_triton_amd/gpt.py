@@ -33,12 +33,15 @@ from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, b
 # Up to this many token rows of up to this width the blocks run their LayerNorm inside the following
 # GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile, in front
 # of its first product, and one of its workgroups fills a CU.  So it pays while all column tiles run at
-# once and while normalising 16 or 32 rows costs less than a launch, up to 768: LayerNorm -> ffn1 at 24 / 128 /
-# 160 / 192 rows of 768 takes 5.4 / 7.5 / 7.6 / 12.2 us against 6.4 / 7.7 / 8.3 / 8.3 for the two launches, 24,
-# 64 and 128 rows of 1024 6.9, 8.3 and 8.5 against 6.7, 7.8 and 8.5, 24 of 1280 9.8 against 8.8, 24 of 1600 12.0
-# against 10.1 (8 rows of 1024 5.8 against 6.6).
+# once and while normalising 16 or 32 rows costs less than a launch: 160 rows up to 768, up to 1024 the rows of
+# one row block.  LayerNorm -> ffn1 at 24 / 128 / 160 / 192 rows of 768 takes 5.4 / 7.5 / 7.6 / 12.2 us against 6.4 /
+# 7.7 / 8.3 / 8.3 for the two launches, 24 of 1280 9.8 against 8.8, 24 of 1600 12.0 against 10.1.  Forwards of the
+# 1024-wide model, two launches / one, us: 1 x 8 tokens replayed 636 / 622, eager 778 / 632, 1 x 24 651 / 630 and 781 /
+# 651, 1 x 41 673 / 702 and 778 / 698, 2 x 64 803 / 805 and 803 / 807 (eager ones of few rows wait for the host).
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
+LN_PROLOGUE_FEW_ROWS = 32
+LN_PROLOGUE_FEW_WIDTH = 1024
 
 # Up to this many elements of the residual stream a block is one call of the library (attention_block,
 # mlp_block) instead of one per operator.  Up to about 2000 rows of the 124M model and 1000 of the 1024-wide one
@@ -58,7 +61,9 @@ BLOCK_MAX_ELEMENTS = 1 << 25
 
 def _ln_in_gemm(x, weight):
     width = x.shape[-1]
-    return (width <= LN_PROLOGUE_MAX_WIDTH and x.numel() // width <= LN_PROLOGUE_MAX_ROWS and
+    few = width > LN_PROLOGUE_MAX_WIDTH
+    rows = min(LN_PROLOGUE_MAX_ROWS, LN_PROLOGUE_FEW_ROWS) if few else LN_PROLOGUE_MAX_ROWS
+    return (width <= LN_PROLOGUE_FEW_WIDTH and x.numel() // width <= rows and
             layer_norm_linear_supported(x, weight))
 
 
