@@ -562,9 +562,11 @@ int launch_gemm_tile(const void* A, const void* Bt, int64_t M, int N, int Kp, co
 // tiles of 32 x 32 took 13.4 us against 9.3 for the LayerNorm launch and the plain one, as 192 of
 // 32 x 64 8.3 (7.3 with the arithmetic of layernorm.h as it stands).  Normalising is a third of the
 // launch, so while tiles of 16 rows still run at once, they do (24 rows x 768 x 2304: 5.6 us as 72 tiles
-// of 32 x 32, 5.0 as 144 of 16 x 32).
+// of 32 x 32, 5.0 as 144 of 16 x 32), and beyond that those of 16 x 64 (us, 32 rows / so: 64 x 768 x 3072 6.4 / 6.1, 80 x
+// 768 x 3072 6.9 / 6.1, 64 x 768 x 2304 5.5 / 5.0, 112 x 768 x 2304 5.9 / 5.0).
 namespace {
 typedef Tile<16,  32, 1, 2, 4, 3> Ln16x32;
+typedef Tile<16,  64, 1, 2, 4, 3> Ln16x64;
 typedef Tile<32,  32, 1, 2, 4, 3> Ln32x32;
 typedef Tile<32,  64, 1, 2, 4, 3> Ln32x64w;
 typedef Tile<32,  64, 1, 4, 2, 3> Ln32x64;
@@ -577,6 +579,7 @@ inline int pick_ln(int64_t M, int N, int K, bool split, int cus) {
   if (wk < 4) return wk == 1 ? 3 : 2;
   const int64_t cols = (N + 31) / 32;
   if ((M + 15) / 16 * cols <= cus) return 4;
+  if ((M + 15) / 16 * ((N + 63) / 64) <= cus) return 5;
   return K <= 1024 && (M + 31) / 32 * cols > cus ? 1 : 0;
 }
 
@@ -590,6 +593,7 @@ int launch_ln(const void* x, const void* Bt, int64_t M, int N, int K, const EpiD
     case 1: return launch_tile_cfg<Ln32x64w, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 2: return launch_tile_cfg<Ln32x64, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     case 4: return launch_tile_cfg<Ln16x32, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
+    case 5: return launch_tile_cfg<Ln16x64, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
     default: return launch_tile_cfg<Ln32x128, T, _Float16, QKV, true, false>(x, Bt, M, N, K, ep, ln, st);
   }
 }
