@@ -359,9 +359,9 @@ static bool prologue_aligned(const void* x, const void* ln_w, const void* ln_b) 
 // FusedGPT asks for it in fp16 (gpt._ln_in_gemm): a launch less, the same bits.  Forwards, two launches / one, weights
 // from HBM, us: 124M 1 x 24 tokens eager 351 / 339, replayed 305 / 290, 2 x 64 eager 400 / 351 (where the host sets the
 // pace; otherwise 353 / 363), replayed 359 / 359, 1 x 160 386 / 383, 1 x 192 418 / 480; 1024 wide 1 x 24 eager 772 /
-// 645, replayed 649 / 631, 1 x 32 656 / 630, 1 x 48 674 / 708, 2 x 64 797 / 806.
+// 645, replayed 649 / 631, 1 x 32 656 / 630, 1 x 64 692 / 677, eager 795 / 672, 2 x 64 797 / 806.
 static bool prologue_f32(int64_t M, int64_t h, bool packed, float p) {
-  return packed && p == 0.f && h <= 1024 && M <= (h <= 768 ? 160 : 32) && gemm_layernorm_supported(M, (int)h, false);
+  return packed && p == 0.f && h <= 1024 && M <= (h <= 768 ? 160 : 64) && gemm_layernorm_supported(M, (int)h, false);
 }
 
 }  // namespace gptmi

@@ -33,14 +33,15 @@ from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, b
 # Up to this many token rows of up to this width the blocks run their LayerNorm inside the following
 # GEMM (same bits, a launch less).  The fused form normalises a row block once per column tile, in front
 # of its first product, and one of its workgroups fills a CU.  So it pays while all column tiles run at
-# once and while normalising 16 or 32 rows costs less than a launch: 160 rows up to 768, up to 1024 the rows of
-# one row block.  LayerNorm -> ffn1 at 24 / 128 / 160 / 192 rows of 768 takes 5.4 / 7.5 / 7.6 / 12.2 us against 6.4 /
+# once and while normalising 16 or 32 rows costs less than a launch: 160 rows up to 768, up to 1024 as many as take
+# tiles of 16 rows.  LayerNorm -> ffn1 at 24 / 128 / 160 / 192 rows of 768 takes 5.4 / 7.5 / 7.6 / 12.2 us against 6.4 /
 # 7.7 / 8.3 / 8.3 for the two launches, 24 of 1280 9.8 against 8.8, 24 of 1600 12.0 against 10.1.  Forwards of the
 # 1024-wide model, two launches / one, us: 1 x 8 tokens replayed 636 / 622, eager 778 / 632, 1 x 24 651 / 630 and 781 /
-# 651, 1 x 41 673 / 702 and 778 / 698, 2 x 64 803 / 805 and 803 / 807 (eager ones of few rows wait for the host).
+# 651, 1 x 41 671 / 671 and 785 / 667, 1 x 64 689 / 675 and 793 / 670, 1 x 80 745 / 754 and 791 / 749, 2 x 64 803 / 805 and 803 /
+# 807 (eager ones of few rows wait for the host).
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
-LN_PROLOGUE_FEW_ROWS = 32
+LN_PROLOGUE_FEW_ROWS = 64
 LN_PROLOGUE_FEW_WIDTH = 1024
 
 # Up to this many elements of the residual stream a block is one call of the library (attention_block,

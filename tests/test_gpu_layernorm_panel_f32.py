@@ -31,7 +31,7 @@ def operands(rows, h, device, special):
 
 
 SIZES = [(rows, h) for h in (64, 320, 768) for rows in (1, 16, 17, 32, 33, 48, 49, 80, 81, 112, 113, 128, 160, 161)] + [
-    (rows, h) for h in (832, 1024) for rows in (1, 24, 32, 33)]
+    (rows, h) for h in (832, 1024) for rows in (1, 24, 32, 33, 64, 65)]
 
 
 @pytest.mark.parametrize("rows,h", SIZES)
