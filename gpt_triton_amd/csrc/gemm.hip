@@ -8,7 +8,7 @@
 // the q/k/v relayout of matmul_and_split_qkv, kernels.py:347-367, which is done
 // here by the store instead of by three copies.
 //
-// This file holds the persistent kernels for problems that fill the chip with 256 x 256 tiles
+// This file holds the persistent kernels for problems that fill the chip with 256 x 256 (or 192 x 256) tiles
 // (gemm_stream_kernel without and gemm_stream_res_kernel with a residual): one workgroup per CU walks
 // tiles and the pipeline runs across tile boundaries.  gemm_tile.hip holds the kernel with one
 // workgroup per tile for everything else.  launch_shape (at the end) divides the rows between them.
@@ -1091,6 +1091,9 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
   return (p < q ? q - p : p - q) < (uintptr_t)M * (uintptr_t)N * elem;
 }
 
+// Whether the persistent kernel, without a residual, takes the weight [K][N] as it stands (see gemm_reads_kn).
+inline bool stream_reads_kn(int64_t M, int N) { return N % 256 == 0 && M <= 32768; }
+
 // Divides the rows between the persistent kernel and the tile kernel.  The persistent kernel takes
 // 256-row tiles: all rows, as many tiles as fill whole rounds of the CUs (every workgroup walks
 // ceil(tiles / CUs) tiles, so a few tiles beyond a whole number of rounds cost a full round: the
@@ -1110,9 +1113,11 @@ inline bool overlap(const void* a, const void* b, int64_t M, int N, size_t elem)
 // 3072 x 1024, 192 / 252, 32.3 / 29.8; 4000 x 3072 x 768 25.7 / 22.7; 9600 x 2304 x 768, 342 / 450, 44.0 / 38.7, and 43.5
 // with the rows beyond one round on the tile kernel; 12000 x 3072 x 768, 564 / 756, 73.3 / 64.9; 4800 x 3072 x 768, 228 /
 // 300, 27.8 / 37.8).  Without a residual and without dropout, up to 6 rounds, beyond which there is nothing to gain.
+// kn: whether the weight can be read in place is asked (gemm_reads_kn), or it is: where the persistent kernel cannot, what
+// tiles of 192 rows save is less than the image costs.
 // Sets *head to the number of rows for the persistent kernel and *bm to its tiles' rows.
 template <typename T, typename OT, bool QKV>
-int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, int* bm) {
+int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, int* bm, bool kn = false) {
   const bool res = !QKV && ep.residual != nullptr;
   const bool drop = ep.drop.p > 0.f;
   const bool drop_ok = !QKV && sizeof(OT) == 2 && ep.keep != nullptr && ((uintptr_t)ep.keep & 3) == 0 &&
@@ -1136,7 +1141,7 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, i
   // 20480 x 1024 x 4096, is the other way round, 196 against 183).
   float least = tiles >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
   for (const int tm : {256, 192}) {
-    if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus)) break;
+    if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus || (kn && !stream_reads_kn(M, N)))) break;
     // rows of the row tiles that fill whole rounds
     const int64_t whole = drop ? all : (all + tm - 1) / tm * tiles_n / cus * cus / tiles_n * tm;
     for (const int64_t rows : {all, whole < all ? whole : all}) {
@@ -1168,7 +1173,7 @@ int launch_shape(const void* A, const void* Bt, int64_t M, int N, int Kp, const 
   const bool res = !QKV && ep.residual != nullptr;
   int64_t m_head;
   int bm;
-  if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head, &bm)) return rc;
+  if (const int rc = persistent_rows<T, OT, QKV>(M, N, Kp, ep, &m_head, &bm, KN)) return rc;
   if (m_head > 0) {
     int rc;
     if constexpr (sizeof(OT) == 2 && !QKV) {
@@ -1296,10 +1301,10 @@ bool gemm_reads_kn(const void* W, int64_t M, int N, int K, const GemmEpilogue& e
     return false;
   if (!e.f16 || K % 64 != 0 || ((uintptr_t)W & 15) != 0 || !gemm_tile_reads_kn(N, K) || make_epi(e, M, N, ep) != 0)
     return false;
-  if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head, &bm)
-             : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head, &bm)) != 0)
+  if ((e.qkv ? persistent_rows<_Float16, _Float16, true>(M, N, K, ep, &head, &bm, true)
+             : persistent_rows<_Float16, _Float16, false>(M, N, K, ep, &head, &bm, true)) != 0)
     return false;
-  return head == 0 || (N % 256 == 0 && e.residual == nullptr && M <= 32768);
+  return head == 0 || (e.residual == nullptr && stream_reads_kn(M, N));
 }
 
 int launch_gemm_kn(const void* A, const void* W, int64_t M, int N, int K, const GemmEpilogue& e, hipStream_t st) {

@@ -31,6 +31,9 @@ CASES = [(1, 1600, 1), (3, 1600, 15), (7, 1540, 16), (5, 1540, 17), (1530, 1540,
          (13, 300, 100), (256, 520, 128), (12, 513, 129), (84, 200, 211), (102, 110, 289), (12, 192, 300),
          (102, 103, 320), (12, 90, 321), (73, 74, 448), (80, 81, 449), (12, 90, 511), (12, 90, 513), (39, 64, 1024),
          (2, 20, 2100)]
+# the streaming kernel's lengths: either side of every 32-row chunk and 64-key tile
+CASES += [(4, 1540, L) for L in (31, 32, 48, 63)]
+CASES += [(4, 700, L) for L in (66, 95, 96, 97, 127, 159, 160, 161, 191, 192, 193, 223, 224, 225, 255, 256, 257, 287, 288)]
 
 
 @pytest.mark.parametrize("few,many,L", CASES)

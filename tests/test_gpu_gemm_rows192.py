@@ -17,20 +17,21 @@ PLANS = [((4800, 2304, 768), (4800, 192)), ((4032, 3072, 192), (4032, 192)), ((4
          ((9600, 2304, 768), (9600, 192)), ((383, 25600, 192), (383, 192)), ((24592, 256, 128), (24592, 192)),
          ((16337, 320, 128), (16337, 192)), ((6700, 3072, 768), None), ((8200, 3072, 1024), None),
          ((7200, 2304, 768), None), ((4800, 3072, 768), (4800, 256)), ((153600, 2304, 768), None),
-         ((2900, 4096, 1024), (2900, 192))]
+         ((2900, 4096, 1024), (2900, 192)), ((1700, 4800, 1600), (1700, 192)),
+         ((2064, 3200, 256), (2064, 192))]
 
 
-def plan(tiles, M, N, slices):
-    """persistent_rows of gemm.hip for 256 CUs, no residual, no dropout."""
+def plan(tiles, M, N, slices, kn=False):
+    """persistent_rows of gemm.hip for 256 CUs, no residual, no dropout; kn: the weight in place, if it can be."""
     with open(os.path.join(ragged.ROOT, "gpt_triton_amd", "csrc", "gemm.hip")) as f:
         source = f.read()
-    assert "if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus)) break;" in source
+    assert "if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus || (kn && !stream_reads_kn(M, N)))) break;" in source
     e192 = re.sub(r"(?<=\d)f\b", "", re.search(r"if \(bm == 192\) return (.*?);", source).group(1))
     cols = -(-N // 256)
     tiles256 = -(-M // 256) * cols
     least, head, bm = (math.inf if tiles256 >= 512 else ragged.pick(tiles, M, N, slices)[0]), 0, 256
     for tm, expression in ((256, ragged.stream_terms()[1]), (192, e192)):
-        if tm == 192 and tiles256 > 6 * 256:
+        if tm == 192 and (tiles256 > 6 * 256 or kn and (N % 256 != 0 or M > 32768)):
             break
         whole = -(-M // tm) * cols // 256 * 256 // cols * tm
         for rows in (M, min(whole, M)):
@@ -53,6 +54,8 @@ def test_where_the_rule_takes_them():
         assert want is None or (head, bm) == want
     # rows left to the tile kernel behind tiles of 192
     assert plan(tiles, 6700, 3072, 12)[1] == 192 and 0 < plan(tiles, 6700, 3072, 12)[0] < 6700
+    # a weight that the persistent kernel cannot read in place: the tile kernel does, as it did
+    assert plan(tiles, 2064, 3200, 4) == (2064, 192) and plan(tiles, 2064, 3200, 4, kn=True) == (0, 256)
     # many rounds: tiles of 256 only
     assert plan(tiles, 153600, 2304, 12)[1] == 256
     # and every shape of the tile kernel is still reached by the sizes that the other tests take
