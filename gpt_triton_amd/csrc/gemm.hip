@@ -1113,6 +1113,9 @@ inline bool stream_reads_kn(int64_t M, int N) { return N % 256 == 0 && M <= 3276
 // 3072 x 1024, 192 / 252, 32.3 / 29.8; 4000 x 3072 x 768 25.7 / 22.7; 9600 x 2304 x 768, 342 / 450, 44.0 / 38.7, and 43.5
 // with the rows beyond one round on the tile kernel; 12000 x 3072 x 768, 564 / 756, 73.3 / 64.9; 4800 x 3072 x 768, 228 /
 // 300, 27.8 / 37.8).  Without a residual and without dropout, up to 6 rounds, beyond which there is nothing to gain.
+// Nor where the rows that those of 256 leave to the tile kernel get a tile that divides K: the sums of its two or four groups
+// are the more exact ones (K 3072 and more, relative to 64 bits 2.5e-7 against 3.5e-7), and no row is to lose them
+// (7200 x 1088 x 4352, the last rows of 11384 x 3072 x 768; one in 55 of the sizes of 192 rows, which then take 2 % longer).
 // kn: whether the weight can be read in place is asked (gemm_reads_kn), or it is: where the persistent kernel cannot, what
 // tiles of 192 rows save is less than the image costs.
 // Sets *head to the number of rows for the persistent kernel and *bm to its tiles' rows.
@@ -1140,8 +1143,10 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, i
   // 336 against 419 us, and 2.4 rounds of 20480 x 1600 x 6400 430 against 445; one round and a bit,
   // 20480 x 1024 x 4096, is the other way round, 196 against 183).
   float least = tiles >= 2 * (int64_t)cus ? INFINITY : gemm_tile_cost(M, N, Kp, cus);
+  auto one_sum = [&](int64_t rows) { return rows == M || gemm_tile_split(M - rows, N, Kp, cus) == 1; };
   for (const int tm : {256, 192}) {
     if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus || (kn && !stream_reads_kn(M, N)))) break;
+    if (tm == 192 && !one_sum(*head)) break;
     // rows of the row tiles that fill whole rounds
     const int64_t whole = drop ? all : (all + tm - 1) / tm * tiles_n / cus * cus / tiles_n * tm;
     for (const int64_t rows : {all, whole < all ? whole : all}) {

@@ -1,0 +1,59 @@
+"""The order of a row's sum where the persistent kernel takes tiles of 192 rows (csrc/gemm.hip): rows whose K the tile
+kernel divides over two or four groups, which gives the more exact sums, keep them.  On the CPU the rule, over many sizes;
+on the GPU the bits, on random operands."""
+import pytest
+import torch
+
+import test_gpu_gemm_ragged as ragged
+from test_gpu_gemm_in_place import weights
+from test_gpu_gemm_rows192 import plan, split
+
+
+def first_plan(tiles, M, N, slices):
+    """Rows of the persistent kernel with tiles of 256 rows only."""
+    return ragged.persistent_rows(tiles, M, N, slices, False)
+
+
+SIZES = [(M, N, Kd) for N, Kd in ((2304, 768), (3072, 768), (768, 3072), (3072, 1024), (1024, 4096), (1280, 5120), (4800, 1600),
+                                  (1088, 4352), (1344, 3072), (2880, 768)) for M in range(256, 26000, 177)]
+
+
+def test_no_row_loses_its_split():
+    tiles, taken, left = ragged.cost_tables(), 0, 0
+    for M, N, Kd in SIZES:
+        head, bm = plan(tiles, M, N, Kd // 64)
+        if bm != 192:
+            continue
+        taken += 1
+        assert split(tiles, M - first_plan(tiles, M, N, Kd // 64), N, Kd // 64) == 1, (M, N, Kd)
+    print(f"{taken} of {len(SIZES)} sizes take tiles of 192 rows")
+    assert taken > len(SIZES) // 20
+
+
+@pytest.fixture(scope="module")
+def K(gpu_device):
+    from gpt_triton_amd import kernels
+    return kernels
+
+
+# M, N, K; the first of the rows that the tile kernel takes, with K divided
+DIVIDED = [(7200, 1088, 4352, 0), (5924, 1344, 3072, 0), (11384, 3072, 768, 10752)]
+
+
+def test_the_shapes_below():
+    tiles = ragged.cost_tables()
+    for M, N, Kd, start in DIVIDED:
+        assert plan(tiles, M, N, Kd // 64) == (start, 256) and split(tiles, M - start, N, Kd // 64) > 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,Kd,start", DIVIDED)
+def test_divided_sums_stay_divided(K, gpu_device, M, N, Kd, start):
+    print(f"divided sums {M} x {N} x {Kd}", flush=True)
+    draw, w, b = weights(gpu_device, Kd, N, M)
+    x = draw(M, Kd)
+    image = K.pack_weight(w)
+    whole = K.fused_ffn(x, image)
+    assert torch.isfinite(whole).all() and torch.equal(whole[start:], K.fused_ffn(x[start:].contiguous(), image))
+    if start == 0:  # the weight in place is the tile kernel's for these columns
+        assert torch.equal(whole, K.fused_ffn(x, w))
