@@ -1117,7 +1117,8 @@ inline bool stream_reads_kn(int64_t M, int N) { return N % 256 == 0 && M <= 3276
 // are the more exact ones (K 3072 and more, relative to 64 bits 2.5e-7 against 3.5e-7), and no row is to lose them
 // (7200 x 1088 x 4352, the last rows of 11384 x 3072 x 768; one in 55 of the sizes of 192 rows, which then take 2 % longer).
 // kn: whether the weight can be read in place is asked (gemm_reads_kn), or it is: where the persistent kernel cannot, what
-// tiles of 192 rows save is less than the image costs.
+// tiles of 192 rows save is less than the image costs.  The image of such a weight takes them only with whole sums everywhere,
+// which are those of the plan without them: a weight and its image give the same bits.
 // Sets *head to the number of rows for the persistent kernel and *bm to its tiles' rows.
 template <typename T, typename OT, bool QKV>
 int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, int* bm, bool kn = false) {
@@ -1153,7 +1154,7 @@ int persistent_rows(int64_t M, int N, int Kp, const EpiDev& ep, int64_t* head, i
       if (rows == 0) continue;
       float c = stream_cost((rows + tm - 1) / tm * tiles_n, Kp, res, cus, tm);
       if (rows < M) c += 1.0f + gemm_tile_cost(M - rows, N, Kp, cus);
-      if (c < least) least = c, *head = rows, *bm = tm;
+      if (c < least && (tm == 256 || stream_reads_kn(M, N) || one_sum(rows))) least = c, *head = rows, *bm = tm;
     }
   }
   return 0;

@@ -32,6 +32,7 @@ def plan(tiles, M, N, slices, kn=False):
         source = f.read()
     assert "if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus || (kn && !stream_reads_kn(M, N)))) break;" in source
     assert "if (tm == 192 && !one_sum(*head)) break;" in source
+    assert "if (c < least && (tm == 256 || stream_reads_kn(M, N) || one_sum(rows))) least = c, *head = rows, *bm = tm;" in source
     e192 = re.sub(r"(?<=\d)f\b", "", re.search(r"if \(bm == 192\) return (.*?);", source).group(1))
     cols = -(-N // 256)
     tiles256 = -(-M // 256) * cols
@@ -49,7 +50,8 @@ def plan(tiles, M, N, slices, kn=False):
             c = eval(expression, {"rounds": -(-t // 256), "fill": t / 256, "k": slices})
             if rows < M:
                 c += 1.0 + ragged.pick(tiles, M - rows, N, slices)[0]
-            if c < least:
+            in_place = N % 256 == 0 and M <= 32768
+            if c < least and (tm == 256 or in_place or split(tiles, M - rows, N, slices) == 1):
                 least, head, bm = c, rows, tm
     return head, bm
 

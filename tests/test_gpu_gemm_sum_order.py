@@ -1,6 +1,6 @@
 """The order of a row's sum where the persistent kernel takes tiles of 192 rows (csrc/gemm.hip): rows whose K the tile
-kernel divides over two or four groups, which gives the more exact sums, keep them.  On the CPU the rule, over many sizes;
-on the GPU the bits, on random operands."""
+kernel divides over two or four groups, which gives the more exact sums, keep them, and a weight and its packed image give
+the same bits.  On the CPU the rule, over many sizes; on the GPU the bits, on random operands."""
 import pytest
 import torch
 
@@ -30,6 +30,26 @@ def test_no_row_loses_its_split():
     assert taken > len(SIZES) // 20
 
 
+def sums(tiles, M, N, slices, kn):
+    """(first row, number of sums) of the rows that are formed alike; None where a weight is packed instead."""
+    head, _ = plan(tiles, M, N, slices, kn)
+    if kn and head and (N % 256 != 0 or M > 32768):
+        return None
+    groups = split(tiles, M - head, N, slices)
+    return [(0, 1)] if groups == 1 else [(0, 1), (head, groups)] if head else [(0, groups)]
+
+
+def test_a_weight_and_its_image_sum_alike():
+    tiles, both = ragged.cost_tables(), 0
+    for N, Kd in ((1088, 4352), (1152, 4608), (1344, 5376), (1728, 6912), (2624, 768), (2880, 768), (3008, 768), (2304, 768), (4800, 1600)):
+        for M in list(range(256, 36000, 97)) + list(range(7000, 9000, 8)):
+            plain = sums(tiles, M, N, Kd // 64, True)
+            if plain is not None:
+                both += 1
+                assert plain == sums(tiles, M, N, Kd // 64, False), (M, N, Kd)
+    assert both > 1000
+
+
 @pytest.fixture(scope="module")
 def K(gpu_device):
     from gpt_triton_amd import kernels
@@ -57,3 +77,20 @@ def test_divided_sums_stay_divided(K, gpu_device, M, N, Kd, start):
     assert torch.isfinite(whole).all() and torch.equal(whole[start:], K.fused_ffn(x[start:].contiguous(), image))
     if start == 0:  # the weight in place is the tile kernel's for these columns
         assert torch.equal(whole, K.fused_ffn(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,Kd", [(7176, 1088, 4352), (7232, 1088, 4352), (8992, 2624, 768), (8200, 2880, 768), (8212, 2880, 768),
+                                    (8200, 3072, 1024), (2064, 3200, 256)])
+def test_a_weight_and_its_image(K, gpu_device, M, N, Kd):
+    print(f"a weight and its image {M} x {N} x {Kd}", flush=True)
+    draw, w, b = weights(gpu_device, Kd, N, M)
+    x = draw(M, Kd)
+    image = K.pack_weight(w)
+    for gelu in (False, True):
+        plain = K.fused_ffn(x, w, bias=b, add_gelu=gelu)
+        assert torch.isfinite(plain).all() and torch.equal(plain, K.fused_ffn(x, image, bias=b, add_gelu=gelu))
+    if N % 192 == 0:
+        for got, want in zip(K.matmul_and_split_qkv(x.view(1, M, Kd), w, b, N // 192),
+                             K.matmul_and_split_qkv(x.view(1, M, Kd), image, b, N // 192)):
+            assert torch.equal(got, want)
