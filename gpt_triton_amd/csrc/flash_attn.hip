@@ -1673,15 +1673,19 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring16_kernel(
     psum = half_swap(ps.a + ps.b).b;  // that of lanes 32..63
     den = den * mult + psum;
   };
-  auto weighted = [&]() {
+  // of the tile that the diagonal cuts, queries 0..31 leave out the second block of keys, as flash_attn_ring_kernel does:
+  // its weights are 0, but a row of V that is not finite would be felt
+  auto weighted = [&](auto diagonal) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int kk = 0; kk < 2; ++kk) {
+      if (decltype(diagonal)::value && kk == 1 && (qw0 & 32) == 0) break;
 #pragma unroll
       for (int i = 0; i < DB; ++i) {
         const h4 lo = vlo[kk][i], hi = vhi[kk][i];
         const h8 vf = h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         oacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[kk], oacc[i], 0, 0, 0);
       }
+    }
   };
 
   const int nfull = qw0 >> 6;  // key tiles entirely below this wavefront's diagonal
@@ -1712,7 +1716,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring16_kernel(
       __builtin_amdgcn_sched_barrier(0);
       scores();
       denominator();
-      weighted();
+      weighted(std::false_type{});
       arrive(t + 1);
       request(t + 1);
     }
@@ -1720,7 +1724,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_ring16_kernel(
     __builtin_amdgcn_sched_barrier(0);
     softmax(std::true_type{});
     denominator();
-    weighted();
+    weighted(std::true_type{});
   }
   for (int t = wave_active ? nfull + 1 : 1; t < nt; ++t) {
     arrive(t);
