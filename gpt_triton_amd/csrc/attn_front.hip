@@ -245,9 +245,9 @@ int launch_front(const void* x, const void* Bt, const void* bias, void* out, int
   }
   const size_t lds = (size_t)NST * kSliceBytes + (size_t)ROWS * H * 2;
   const int workers = (int)(B * heads), cus = cu_count();
-  hipLaunchKernelGGL(kern, dim3((unsigned)(workers + prefetch_workgroups(ahead, workers, cus))), dim3(512), lds, st, (const _Float16*)x, (const _Float16*)Bt,
-                     (const _Float16*)bias, (_Float16*)out, (int)B, heads, L, H, scale, ln,
-                     prefetch_args(ahead));
+  hipLaunchKernelGGL(kern, dim3((unsigned)(workers + front_ahead_workgroups(ahead, workers, cus))), dim3(512), lds, st,
+                     (const _Float16*)x, (const _Float16*)Bt, (const _Float16*)bias, (_Float16*)out, (int)B, heads, L, H, scale,
+                     ln, prefetch_args(ahead));
   return 0;
 }
 

@@ -57,6 +57,17 @@ class AheadLines {
   unsigned end_[4];
 };
 
+// Workgroups for it behind the `workers` of the front kernel (LayerNorm, product and attention of short sequences), which
+// pull their weights through CUs of their own, one workgroup each: requests from all idle CUs at once stand in their way,
+// from 64 they do not, and from few what they ask for is late.  With fewer than 32 CUs idle they wait for the workers to
+// end, and more of them are through sooner.  Forwards of 124M that the GPU sets the pace of, all idle CUs (beyond 192
+// workers 128) / 128 / 64 / 32, us: 1 x 8 tokens 276 / 271 / 264 / 263, 1 x 24 with logits 301 / 296 / 289 / 288, weights from HBM 1 x
+// 24 294 / 288 / 285 / 286, 8 x 24 360 / 358 / 354 / 357, 16 x 32 412 / 413 / 412 / 414, 18 x 32 434 / 434 / 427 / 421, 19 x 32
+// 456 / 455 / 464 / 498, 21 x 32 505 / 506 / 524 / 557.
+inline int front_ahead_workgroups(const Prefetch* ahead, int64_t workers, int cus) {
+  return ahead == nullptr || ahead->empty() ? 0 : workers <= cus - 32 ? 64 : 128;
+}
+
 // Sizes that are the same for all layers of a call; rows: of a key, lasting: see weights_ahead.
 struct AheadPlan {
   size_t square, wide, most;  // bytes of W_proj, W1 or W2; of all that is requested behind W2
