@@ -21,26 +21,17 @@ PLANS = [((4800, 2304, 768), (4800, 192)), ((4032, 3072, 192), (4032, 192)), ((4
          ((2064, 3200, 256), (2064, 192))]
 
 
-def split(tiles, M, N, slices):
-    """Over how many sums the tile kernel divides K for M rows; none are one."""
-    return tiles[ragged.pick(tiles, M, N, slices)[1]][2] if M > 0 else 1
-
-
 def plan(tiles, M, N, slices, kn=False):
     """persistent_rows of gemm.hip for 256 CUs, no residual, no dropout; kn: the weight in place, if it can be."""
     with open(os.path.join(ragged.ROOT, "gpt_triton_amd", "csrc", "gemm.hip")) as f:
         source = f.read()
     assert "if (tm == 192 && (res || drop || tiles > 6 * (int64_t)cus || (kn && !stream_reads_kn(M, N)))) break;" in source
-    assert "if (tm == 192 && !one_sum(*head)) break;" in source
-    assert "if (c < least && (tm == 256 || stream_reads_kn(M, N) || one_sum(rows))) least = c, *head = rows, *bm = tm;" in source
     e192 = re.sub(r"(?<=\d)f\b", "", re.search(r"if \(bm == 192\) return (.*?);", source).group(1))
     cols = -(-N // 256)
     tiles256 = -(-M // 256) * cols
     least, head, bm = (math.inf if tiles256 >= 512 else ragged.pick(tiles, M, N, slices)[0]), 0, 256
     for tm, expression in ((256, ragged.stream_terms()[1]), (192, e192)):
         if tm == 192 and (tiles256 > 6 * 256 or kn and (N % 256 != 0 or M > 32768)):
-            break
-        if tm == 192 and split(tiles, M - head, N, slices) > 1:
             break
         whole = -(-M // tm) * cols // 256 * 256 // cols * tm
         for rows in (M, min(whole, M)):
@@ -50,8 +41,7 @@ def plan(tiles, M, N, slices, kn=False):
             c = eval(expression, {"rounds": -(-t // 256), "fill": t / 256, "k": slices})
             if rows < M:
                 c += 1.0 + ragged.pick(tiles, M - rows, N, slices)[0]
-            in_place = N % 256 == 0 and M <= 32768
-            if c < least and (tm == 256 or in_place or split(tiles, M - rows, N, slices) == 1):
+            if c < least:
                 least, head, bm = c, rows, tm
     return head, bm
 
