@@ -355,11 +355,13 @@ static bool prologue_aligned(const void* x, const void* ln_w, const void* ln_b) 
   return (((uintptr_t)x | (uintptr_t)ln_w | (uintptr_t)ln_b) & 15) == 0;
 }
 
-// fp32 models' blocks with packed weights run their LayerNorm inside the product behind it without being asked, where
-// FusedGPT asks for it in fp16 (gpt._ln_in_gemm): a launch less, the same bits.  Forwards, two launches / one, weights
-// from HBM, us: 124M 1 x 24 tokens eager 351 / 339, replayed 305 / 290, 2 x 64 eager 400 / 351 (where the host sets the
-// pace; otherwise 353 / 363), replayed 359 / 359, 1 x 160 386 / 383, 1 x 192 418 / 480; 1024 wide 1 x 24 eager 772 /
-// 645, replayed 649 / 631, 1 x 32 656 / 630, 1 x 64 692 / 677, eager 795 / 672, 2 x 64 797 / 806.
+// fp32 models' blocks with packed weights run their LayerNorm inside the product behind it without being asked, up to
+// the rows that FusedGPT asks for it at in fp16 (gpt.LN_PROLOGUE_MAX_ROWS and those beside it; a caller declines with -1):
+// a launch less, the same bits.  Forwards, two launches / one, weights from HBM, us, queued behind other work | replayed |
+// waited for: 124M 1 x 24 tokens 297 / 284 | 306 / 292 | 473 / 444, 1 x 80 326 / 304 | 333 / 312 | 478 / 445, 1 x 112 348 /
+// 335 | 358 / 343 | 506 / 470, 2 x 64 357 / 357 | 364 / 366 | 508 / 493, 1 x 144 371 / 364 | 379 / 373 | 522 / 500, 1 x 160 380 /
+// 374 | 390 / 383 | 531 / 503, replayed 1 x 192 418 / 480; 1024 wide 1 x 8 626 / 627 | 635 / 637 | 842 / 777, 1 x 24 643 / 631 |
+// 651 / 639 | 845 / 772, 1 x 64 686 / 675 | 690 / 682 | 868 / 805, 2 x 64 797 / 806 on the GPU.
 static bool prologue_f32(int64_t M, int64_t h, bool packed, float p) {
   return packed && p == 0.f && h <= 1024 && M <= (h <= 768 ? 160 : 64) && gemm_layernorm_supported(M, (int)h, false);
 }
@@ -716,14 +718,14 @@ static int attention_block(const void* x, const void* normed, const void* ln_w, 
   ep.qkv = true;
   ep.f16 = f16;
   ep.out_f16 = true;
-  bool prologue = fuse_layernorm && !normed;
+  bool prologue = fuse_layernorm > 0 && !normed;
   if (prologue) {
     if (!f16 || !gemm_layernorm_supported(M, (int)h)) {
       set_error("attention_block: the LayerNorm prologue takes fp16 storage and the row widths of "
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
-  } else if (!f16 && !normed) {
+  } else if (!f16 && !normed && fuse_layernorm == 0) {
     prologue = prologue_f32(M, h, bw.packed, p);
   }
   prologue = prologue && prologue_aligned(x, ln_w, ln_b);
@@ -811,14 +813,14 @@ int gptmi_mlp_block(const void* x, const void* ln_w, const void* ln_b, float eps
   e1.drop = drop;
   e1.f16 = f16;
   e1.out_f16 = true;
-  bool prologue = fuse_layernorm != 0;
+  bool prologue = fuse_layernorm > 0;
   if (prologue) {
     if (!f16 || p > 0.f || !gemm_layernorm_supported(M, (int)H)) {
       set_error("mlp_block: the LayerNorm prologue takes fp16 storage, no dropout and the row widths of "
                 "gptmi_layernorm_linear_supported");
       return GPTMI_ERR_UNSUPPORTED;
     }
-  } else if (!f16) {
+  } else if (!f16 && fuse_layernorm == 0) {
     prologue = prologue_f32(M, H, bw.packed, p);
   }
   prologue = prologue && prologue_aligned(x, ln_w, ln_b);
@@ -867,7 +869,7 @@ static int check_blocks(const void* const* params, int64_t n, int64_t B, int64_t
       return GPTMI_ERR_INVALID;
     }
   }
-  if (fuse_layernorm && (dtype != GPTMI_F16 || !gemm_layernorm_supported(B * L, (int)h))) {
+  if (fuse_layernorm > 0 && (dtype != GPTMI_F16 || !gemm_layernorm_supported(B * L, (int)h))) {
     set_error("blocks: the LayerNorm prologue takes fp16 storage and the row widths of "
               "gptmi_layernorm_linear_supported");
     return GPTMI_ERR_UNSUPPORTED;

@@ -38,7 +38,8 @@ from .kernels import (HEAD_SIZES, PackedWeight, attention_block, block_layers, b
 # 7.7 / 8.3 / 8.3 for the two launches, 24 of 1280 9.8 against 8.8, 24 of 1600 12.0 against 10.1.  Forwards of the
 # 1024-wide model, two launches / one, us: 1 x 8 tokens replayed 636 / 622, eager 778 / 632, 1 x 24 651 / 630 and 781 /
 # 651, 1 x 41 671 / 671 and 785 / 667, 1 x 64 689 / 675 and 793 / 670, 1 x 80 745 / 754 and 791 / 749, 2 x 64 803 / 805 and 803 /
-# 807 (eager ones of few rows wait for the host).
+# 807 (eager ones of few rows wait for the host).  fp32 models' blocks do it without being asked, up to the same limits in the
+# library (prologue_f32 in csrc/capi.cpp); LN_PROLOGUE_MAX_ROWS = 0 turns it off in both types.
 LN_PROLOGUE_MAX_ROWS = 160
 LN_PROLOGUE_MAX_WIDTH = 768
 LN_PROLOGUE_FEW_ROWS = 64
@@ -64,6 +65,8 @@ def _ln_in_gemm(x, weight):
     width = x.shape[-1]
     few = width > LN_PROLOGUE_MAX_WIDTH
     rows = min(LN_PROLOGUE_MAX_ROWS, LN_PROLOGUE_FEW_ROWS) if few else LN_PROLOGUE_MAX_ROWS
+    if LN_PROLOGUE_MAX_ROWS == 0:
+        return None
     return (width <= LN_PROLOGUE_FEW_WIDTH and x.numel() // width <= rows and
             layer_norm_linear_supported(x, weight))
 
@@ -298,12 +301,14 @@ class FusedMLP(nn.Module):
                 p > 0.0 and keep.serves(x, x.numel() // width * max(inner, width), p)):
             keep = None
         as_block = inner % 64 == 0
-        if as_block and p == 0.0 and _ln_in_gemm(x, w1):
+        in_gemm = as_block and p == 0.0 and _ln_in_gemm(x, w1)
+        if in_gemm:
             return layer_norm_ffn(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
                                   bias=prm["ffn1_bias"], add_gelu=True, then=(w2, prm["ffn2_bias"]))
         if as_block and _as_block(x, keep):
             return mlp_block(x, prm["layer_norm_weight"], prm["layer_norm_bias"], w1,
-                             prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p, keep=keep)
+                             prm["ffn1_bias"], w2, prm["ffn2_bias"], dropout_prob=p, layer_norm_in_gemm=in_gemm,
+                             keep=keep)
         y = fused_layer_norm(x, prm["layer_norm_weight"].data, prm["layer_norm_bias"].data)
         y = fused_ffn(y, w1, bias=prm["ffn1_bias"].data, residual=None, add_gelu=True,
                       dropout_prob=p)

@@ -478,11 +478,16 @@ def _block_layout(first, second, what):
     return _lib.GPTMI_W_PACKED if packed else _lib.GPTMI_W_KN
 
 
+def _in_gemm_code(layer_norm_in_gemm):
+    return -1 if layer_norm_in_gemm is None else 1 if layer_norm_in_gemm else 0
+
+
 def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, proj_bias, num_heads,
                     dropout_prob=0.0, normed=None, layer_norm_in_gemm=False, keep=None):
     """x + dropout(proj(attention(qkv(LayerNorm(x))))) for x [B, L, h]: the operators of an attention
     block (gpt.py:39-60) behind one call of the library, with their bits in fp16 (fp32: up to the fp16
-    rounding of the projection's operands).  `normed`: LayerNorm(x), if the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`; keep: a
+    rounding of the projection's operands).  `normed`: LayerNorm(x), if the caller has it; layer_norm_in_gemm: as in `layer_norm_matmul_and_split_qkv`
+    (False: fp32 blocks of few rows with packed weights all the same; None: in no case); keep: a
     `dropout_mask` for dropout_prob of at least max(x.numel(), L * L) offsets, read instead of
     generating the masks here."""
     B, L, h = x.shape
@@ -510,7 +515,7 @@ def attention_block(x, ln_weight, ln_bias, qkv_weight, qkv_bias, proj_weight, pr
           ln_weight.data_ptr(), ln_bias.data_ptr(), 1e-5, qkv_weight.data_ptr(), qkv_bias.data_ptr(),
           proj_weight.data_ptr(), proj_bias.data_ptr(), out.data_ptr(), B, L, num_heads, d,
           float(dropout_prob), 1337, *_keep_args(keep, x, dropout_prob, "attention_block"),
-          1 if layer_norm_in_gemm else 0, layout, _ptr(ws), nbytes, code)
+          _in_gemm_code(layer_norm_in_gemm), layout, _ptr(ws), nbytes, code)
     return out
 
 
@@ -518,7 +523,7 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
               layer_norm_in_gemm=False, keep=None):
     """x + dropout(W2 . dropout(gelu(W1 . LayerNorm(x)))): the operators of an MLP block
     (gpt.py:91-111) behind one call of the library, with their bits; layer_norm_in_gemm: as in
-    `layer_norm_ffn`; keep: as in `attention_block`, of at least (rows of x) * max(inner, h) offsets."""
+    `layer_norm_ffn` and `attention_block`; keep: as in `attention_block`, of at least (rows of x) * max(inner, h) offsets."""
     h = x.shape[-1]
     dtype = x.dtype
     inner = weight1.shape[1]
@@ -541,7 +546,7 @@ def mlp_block(x, ln_weight, ln_bias, weight1, bias1, weight2, bias2, dropout_pro
     _call(dev, "mlp_block", lib.gptmi_mlp_block, x.data_ptr(), ln_weight.data_ptr(),
           ln_bias.data_ptr(), 1e-5, weight1.data_ptr(), bias1.data_ptr(), weight2.data_ptr(),
           bias2.data_ptr(), out.data_ptr(), M, h, inner, float(dropout_prob), 1337,
-          *_keep_args(keep, x, dropout_prob, "mlp_block"), 1 if layer_norm_in_gemm else 0, layout,
+          *_keep_args(keep, x, dropout_prob, "mlp_block"), _in_gemm_code(layer_norm_in_gemm), layout,
           _ptr(ws), nbytes, code)
     return out
 
@@ -571,7 +576,7 @@ def block_layers(x, pointers, num_heads, inner, normed=None, layer_norm_in_gemm=
     table = array.array("Q", pointers)
     _call(dev, "block_layers", _lib.load().gptmi_blocks, x.data_ptr(), _ptr(normed), table.buffer_info()[0],
           len(pointers) // 12, 1e-5, out.data_ptr(), B, L, num_heads, h // num_heads, inner,
-          1 if layer_norm_in_gemm else 0, _ptr(ws), nbytes, code)
+          _in_gemm_code(layer_norm_in_gemm), _ptr(ws), nbytes, code)
     return out
 
 

@@ -310,7 +310,8 @@ int gptmi_dropout_mask(void* mask, int64_t n, float p, uint64_t seed, void* stre
  *                   kernels generate the mask themselves
  *   fuse_layernorm: 1 = the LayerNorm prologue (see gptmi_layernorm_linear_supported) where x, ln_w
  *                   and ln_b are 16-byte aligned, the LayerNorm kernel otherwise; fp32 blocks with
- *                   packed weights, few rows and no dropout use it with 0 too, with the same bits
+ *                   packed weights, few rows and no dropout use it with 0 too, with the same bits;
+ *                   -1 = the LayerNorm kernel in every case
  * workspace: the given number of bytes, 256-byte aligned.
  */
 size_t gptmi_attention_block_workspace_bytes(int64_t B, int64_t L, int64_t heads, int64_t d,
