@@ -1,14 +1,13 @@
-"""GPU parity of the attention kernel the headline forward runs on: fp16, head size 64, equal
-query and key lengths <= 320, up to 64 rows more than 512 (batch, head) pairs, beyond 288 rows more than
-85 (256 CUs) -- with fewer pairs of those lengths `flash_attention_v1` picks the ring kernel, which runs
-here beside it, and with other head sizes or fp32 storage others, which tests/test_gpu_parity.py covers:
+"""GPU parity of attention at head size 64 in fp16, equal query and key lengths <= 320.  The headline forward
+runs on the streaming kernel; with as few pairs as the lengths and the reference's vectors have below
+`flash_attention_v1` picks the one with 16 queries a wavefront (tests/test_gpu_kernels_by_size.py has both among more
+pairs, on the streaming kernel), and with other head sizes or fp32 storage others, which tests/test_gpu_parity.py covers:
 
   * every length either side of the 32-query chunk and 64-key tile boundaries, from 1 to the
     longest the kernel takes, both output layouts, against the oracle;
   * pair counts below, between multiples of and above the number of persistent workgroups;
   * the reference's own outputs (tests/golden/flash_attention_v1.npz, written by the reference's
-    kernel under Triton's CPU interpreter) placed among random pairs, so that the reference's
-    vectors are compared on this kernel and not only on the few-pair ones;
+    kernel under Triton's CPU interpreter) placed among random pairs;
   * the benchmark shape [512, 12, 300, 64]: every element of every pair against the textbook
     attention evaluated by torch in fp32 on the GPU, the output pre-filled with NaN; the same
     check at the same bytes for head sizes 128 and 256 ([512, 6, 300, 128], [512, 3, 300, 256]),
