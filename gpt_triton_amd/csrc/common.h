@@ -81,7 +81,8 @@ __device__ __forceinline__ void prefetch_lines(const PrefetchArgs& pf, int first
 // Cross-lane steps without the LDS: an xor shuffle compiles to ds_bpermute, ~100 cycles of latency
 // per step of a reduction, and the reductions of a LayerNorm row (twelve steps) or of a softmax tile
 // sit on the critical path of their kernels.  The swaps and row rotations are VALU instructions.
-//   half_swap(v): v of lane ^ 32 and the lane's own, in some order (what a commutative step needs)
+//   half_swap(v): v of lane % 32 (a) and of lane % 32 + 32 (b), for both lanes in this order (the attention kernel with 16
+//                 queries a wavefront adds in it)
 struct LanePair {
   float a, b;
 };
@@ -91,7 +92,7 @@ __device__ __forceinline__ LanePair half_swap(float v) {
   const unsigned x = r[0], y = r[1];
   return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
 }
-__device__ __forceinline__ LanePair row_swap(float v) {  // lane ^ 16
+__device__ __forceinline__ LanePair row_swap(float v) {  // a: of the lane without its bit 4, b: with it
   const unsigned u = __builtin_bit_cast(unsigned, v);
   const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
   const unsigned x = r[0], y = r[1];

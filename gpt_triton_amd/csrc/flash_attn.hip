@@ -1946,17 +1946,24 @@ int launch_wide_attn(const void* q, const void* k, const void* v, void* out, int
 
 // fp16 q, k, v of equal lengths at head size 64, no dropout.  Up to 320 rows two (batch, head) pairs fit
 // the LDS: the streaming kernel.  Longer ones take their key tiles through the ring, and so do up to 512 pairs of
-// two tiles, whose workgroups all run at once.  While 64-row blocks fill the CUs about twice, 16 queries a wavefront are
+// two tiles, whose workgroups all run at once, in both arithmetics.  While 64-row blocks fill the CUs about twice, 16 queries a wavefront are
 // through sooner; beyond, K and V read from LDS twice as often cost more than the shorter chain gives, later for long
-// sequences, for the fp32 arithmetic, whose chain is longer, and for a single tile.  The same bits from all three.
+// sequences, for the fp32 arithmetic, whose chain is longer, and for a single tile.  The lines lie where nothing gets slower:
+// they are one number each, the crossing moves with the length (fp16: near 680 blocks of 512 rows, 760 of 640, 860 of 1024, fp32
+// arithmetic beyond 830 of 512, 960 of 1024, for lines at 640 and 768), and between the two up to a fifth is left (44 x 1024).
+// Two tiles in fp32 arithmetic beyond the line cross with the length too (300 pairs of 65 rows ring 7.5, 16 queries
+// 7.8, of 128 rows 9.3 and 8.4); the streaming kernel is behind both.  The same bits from all three.
 // Microseconds, streaming / ring / 16 queries:
 //   24 x 64 rows 4.1 / 3.7 / 3.5, 512 x 64 6.1 / 4.7 / 4.5, 1500 x 64 12.8 / 12.2 / 11.9, 12 x 128 4.8 / 4.6 / 4.2, 256 x 128 5.5 /
 //   5.3 / 5.1, 300 x 128 7.8 / 7.1 / 7.7, 512 x 128 9.8 / 9.3 / 10.4, 84 x 211 6.4 / 6.3 / 5.8, 128 x 256 7.1 / 7.0 / 6.5, 150 x
 //   256 7.8 / 8.0 / 8.6, 12 x 300 8.0 / 6.9 / 5.9, 102 x 320 9.2 / 8.4 / 7.7, 154 x 320 10.4 / 10.1 / 11.1, 192 x 300 11.2 / 12.7 /
 //   12.1; ring / 16 queries: 73 x 400 9.5 / 8.3, 110 x 400 10.7 / 12.5, 75 x 512 11.6 / 10.3, 96 x 512 12.1 / 13.2, 128 x
-//   512 13.2 / 16.6, 12 x 1024 16.9 / 13.4, 48 x 1024 19.9 / 18.6, 64 x 1024 20.8 / 26.4;
-//   in fp32 arithmetic 24 x 64 5.0 / 4.5 / 4.0, 12 x 300 12.5 / 11.0 / 7.9, 171 x 192 9.0 / 10.1 / 8.5, 154 x 320 15.1 / 16.2 / 14.8,
-//   205 x 320 16.7 / 20.8 / 19.2; 12 x 1024 29.3 / 19.7, 96 x 512 19.0 / 17.7, 48 x 1024 32.1 / 28.1, 64 x 1024 33.0 / 39.9.
+//   512 13.2 / 16.6, 64 x 640 12.3 / 10.1, 76 x 640 12.6 / 12.8, 12 x 1024 16.9 / 13.4, 44 x 1024 17.7 / 14.4, 48 x 1024 17.7 / 16.3,
+//   56 x 1024 19.0 / 19.5, 64 x 1024 20.8 / 26.4;
+//   in fp32 arithmetic 24 x 64 5.0 / 4.5 / 4.0, 256 x 128 6.9 / 6.7 / 5.9, 385 x 72 9.0 / 7.8 / 7.9, 385 x 128 10.8 / 9.6 / 8.8, 512
+//   x 72 9.2 / 7.9 / 8.2, 512 x 128 11.3 / 10.0 / 10.6, 12 x 300 12.5 / 11.0 / 7.9, 171 x 192 9.0 / 10.1 / 8.5, 154 x 320 15.1 / 16.2 / 14.8,
+//   205 x 320 16.7 / 20.8 / 19.2; 12 x 1024 29.3 / 19.7, 96 x 512 19.0 / 17.7, 104 x 512 17.5 / 17.0,
+//   48 x 1024 32.1 / 28.1, 60 x 1024 30.9 / 29.9, 64 x 1024 33.0 / 39.9.
 template <bool BLND, bool ACC = false>
 int launch_d64(const void* q, const void* k, const void* v, void* out, int64_t BN, int heads, int L,
                float scale, hipStream_t st, const Prefetch* ahead) {

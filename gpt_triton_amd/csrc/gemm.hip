@@ -433,7 +433,7 @@ __global__ __launch_bounds__(512, 2) void gemm_stream_kernel(
 
   // Operand-tile slot s = it * 512 + tid: row it * 64 + tid / 8, 16-byte position tid % 8,
   // which holds source chunk (tid % 8) ^ ((row >> 1) & 7) -- the key does not depend on `it`.
-  // M is 256 or more, the last row tile starts at M - BM and N is a multiple of 64, so no
+  // M is BM or more, the last row tile starts at M - BM and N is a multiple of 64, so no
   // row is clamped: a load address is a per-tile scalar base (first row of the tile, k-tile
   // offset) plus one of four per-thread 32-bit offsets shared by A and B.
   const int r0 = tid >> 3;

@@ -67,7 +67,7 @@ __device__ __forceinline__ void normalise_rows(const T* __restrict__ x, int M, i
   }
 }
 
-// At most 4 chunks per lane: rows of up to 224 chunks (gemm_layernorm_supported), 64 lanes beyond 128.
+// At most 4 chunks per lane: rows of up to 256 chunks (gemm_layernorm_supported), 64 lanes beyond 128.
 template <int BM, int NT, typename T>
 __device__ __forceinline__ void normalise_panel(const T* x, int M, int H, int m0, const LnArgs& ln,
                                                 char* panel, int tid) {
