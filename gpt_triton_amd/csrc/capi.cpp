@@ -256,7 +256,9 @@ struct BlockWeights {
 // for, but an eager forward that small waits for the host, which then has a launch less a block.  A graph's replay
 // does not.  124M, weights from HBM, us, in two launches / in one: eager 1 x 24 tokens 333 / 293, 2 x 24 333 / 305 (a pass
 // that is waited for 433 / 430, 450 / 443; on a host that takes 1.5 us a launch instead of 2.5 all equal), 4 x 32 344 /
-// 331; replayed 1 x 24 285 / 298, 2 x 24 301 / 311, 3 x 30 335 / 331, 4 x 32 348 / 336, 8 x 24 403 / 363.
+// 331; replayed 1 x 24 285 / 298, 2 x 24 301 / 311, 3 x 30 335 / 331, 4 x 32 348 / 336, 8 x 24 403 / 363, all with requests
+// ahead from every idle CU.  With 64 workgroups for them (front_ahead_workgroups) the two are close: replayed in two
+// launches / eager in one behind other work 1 x 8 286 / 283, 1 x 24 289 / 290, 1 x 32 290 / 290, 2 x 24 298 / 292.
 static bool front_pays(int64_t pairs, hipStream_t st) {
   if (pairs > 32) return true;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
